@@ -1035,6 +1035,7 @@ int restore_ckpt(pic_ctx *ctx, const Ckpt &c) {
   for (int s = 0; s < 2; ++s) {
     ctx->n[s] = c.n[s];
     ctx->sorted_end[s] = c.sorted_end[s];
+    ctx->row_end[s] = 0;  // the cell starts are those of a later sort
     ctx->cur[s] = c.cur[s];
     ctx->drift_halves[s] = c.drift_halves[s];
     const int64_t n = c.n[s];

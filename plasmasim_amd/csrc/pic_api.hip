@@ -326,7 +326,8 @@ static void free_all(pic_ctx *ctx) {
   if (ctx->prim_tmp) (void)hipFree(ctx->prim_tmp);
   if (ctx->dev_counter) (void)hipFree(ctx->dev_counter);
   for (int sp = 0; sp < 2; ++sp)
-    if (ctx->tile_start[sp]) (void)hipFree(ctx->tile_start[sp]);
+    for (uint32_t *t : {ctx->tile_start[sp], ctx->row_start[sp]})
+      if (t) (void)hipFree(t);
   if (ctx->host_counter) (void)hipHostFree(ctx->host_counter);
   if (ctx->diag_partial) (void)hipFree(ctx->diag_partial);
   if (ctx->thrust_acc) (void)hipFree(ctx->thrust_acc);
@@ -477,6 +478,8 @@ extern "C" int pic_create(const pic_config *cfg, pic_ctx **out) {
     for (int sp = 0; sp < 2; ++sp) {
       CREATE_HIP(hipMalloc(&ctx->tile_start[sp], (size_t)(nt + 1) * sizeof(uint32_t)));
       CREATE_HIP(hipMemset(ctx->tile_start[sp], 0, (size_t)(nt + 1) * sizeof(uint32_t)));
+      if (nt == 1 && ncell_in < ((int64_t)1 << 30))
+        CREATE_HIP(hipMalloc(&ctx->row_start[sp], (size_t)(ncell_in + 1) * sizeof(uint32_t)));
     }
   }
   CREATE_HIP(hipMalloc(&ctx->dev_counter, 8 * sizeof(int64_t)));
@@ -925,7 +928,8 @@ extern "C" int pic_thrust_ave_enable(pic_ctx *ctx, int on) {
   const TileGeom tg = tile_geom(ctx);
   // workgroups of one pass: the tiles and the tail chunks of up to the
   // capacity's slots
-  const int64_t slots = (int64_t)tg.ntiles() + div_up(ctx->cap, kTailChunk) + 1;
+  const int64_t boxes = tg.ntiles() == 1 ? row_geom(tg).ntiles() : tg.ntiles();
+  const int64_t slots = boxes + div_up(ctx->cap, tail_chunk(ctx->cfg.ppc, false)) + 1;
   if (!ctx->thrust_acc) PIC_HIP(ctx, hipMalloc(&ctx->thrust_acc, 16 * sizeof(double)));
   if (ctx->thrust_part_slots < slots) {
     if (ctx->thrust_part) (void)hipFree(ctx->thrust_part);

@@ -341,6 +341,7 @@ extern "C" int pic_checkpoint_load(pic_ctx *ctx, const char *path) {
   ctx->inflow_event = h.inflow_event;
   for (int s = 0; s < 2; ++s) {
     ctx->sorted_end[s] = same_tiles && h.ntiles > 0 ? h.sorted_end[s] : 0;
+    ctx->row_end[s] = 0;  // the file holds no cell starts
     // the windows of restored tiles follow the drift from where the writer's
     // stood, so a resumed run deposits exactly as an uninterrupted one
     ctx->drift_halves[s] = ctx->sorted_end[s] > 0 ? h.drift_halves[s] : 0;

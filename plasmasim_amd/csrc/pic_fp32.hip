@@ -622,7 +622,12 @@ __device__ inline void thrust_store(const float (&th)[6], double *out, int bid) 
 // PERM: the pass also applies a sort's permutation: slot i takes its
 // particle from slot perm[i] of the arrays Q and stores the result in P (the
 // other buffer of the species), so the sort needs no separate copy
-template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool DET, bool THRUST, bool PERM>
+// ROWS: the store is sorted as one tile; a workgroup takes a box of cell
+// columns (row_geom), its threads divided evenly over the box's columns, so
+// that all of them load at once.  31 x 27 x 45 x 8 ppc on one workgroup
+// (the one tile's) took 7.26 ms per launch; in boxes 73 us.
+template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool DET, bool THRUST, bool PERM,
+          bool ROWS>
 __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
     Grid32 G, TileGeom tg, Particles32 P, TileRun tr, Push32 kp,
     typename GlobT<DET>::T *jx, typename GlobT<DET>::T *jy,
@@ -640,7 +645,7 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
   if (tid == 0) {
     int64_t s, e;
     Win w;
-    tile_setup(bid, tr, tg, kWin,
+    tile_setup<ROWS>(bid, tr, tg, kWin,
                [&](int64_t i, int &k, int &l, int &m) {
                  const int32_t cl = PERM ? Q.cell[perm[i]] : P.cell[i];
                  if (cl < 0) return false;
@@ -717,14 +722,19 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
   constexpr int N = PIC_PPT32;
   constexpr int SH = N == 8 ? 3 : N == 4 ? 2 : N == 2 ? 1 : 0;
   // slot indices fit in int32 (the host bounds the stored count)
-  const int s32 = (int)s, e32 = (int)e;
+  int s32 = (int)s, e32 = (int)e, lane = tid, lanes = blockDim.x;
+  if (ROWS && bid < tr.ntiles) {
+    lanes = kPassBlock / (tg.TX * tg.TY);
+    row_range(tr, tg, g.NX, g.NY, g.NZ, bid, tid / lanes, s32, e32);
+    lane = tid % lanes;
+  }
   const int q0 = s32 >> SH, q1 = (e32 + N - 1) >> SH;
   // 32-bit byte offsets from the uniform array bases (SGPR-base loads and
   // stores, no 64-bit address arithmetic per array)
   const auto vat = [](auto *base, uint32_t byte) {
     return (decltype(base))((char *)base + byte);
   };
-  for (int q = q0 + tid; q < q1; q += blockDim.x) {
+  for (int q = q0 + lane; q < q1; q += lanes) {
     const int i0 = q << SH;
     const uint32_t bo = (uint32_t)i0 * 4u;
     vi cs;
@@ -1790,9 +1800,21 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   tr.tile_start = ctx->tile_start[sp];
   tr.sorted_end = ctx->sorted_end[sp];
   tr.ntiles = tr.sorted_end > 0 ? tg.ntiles() : 0;
+  // one tile: boxes of rows while the sort's cell starts are current,
+  // otherwise chunks as an unsorted tail
+  const bool rows = tr.ntiles == 1 && ctx->row_start[sp] &&
+                    ctx->row_end[sp] == tr.sorted_end;
+  if (rows) {
+    tg = row_geom(tg);
+    tr.tile_start = ctx->row_start[sp];
+    tr.ntiles = tg.ntiles();
+  } else if (tr.ntiles == 1) {
+    tr.ntiles = 0;
+  }
   if (tr.ntiles == 0) tr.sorted_end = 0;
   tr.n = n;
-  tr.ntail = (int)div_up(n - tr.sorted_end, kTailChunk);
+  tr.chunk = tail_chunk(ctx->cfg.ppc, ctx->geom.NX % 4 == 0 && ctx->geom.NY % 4 == 0);
+  tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
   const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
   if (nb == 0) return settle(ctx, sp);
   // with a pending permutation the pass reads the current buffer through it
@@ -1830,61 +1852,55 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     // tiles be classified
     if (kp.box_margin + 2 >= 0.2 * std::min(c.nx, c.ny)) kp.box_margin = 1 << 20;
   }
+  // DET, then the pass: push and J, drift and n, the boundary, or all three
+  // (only a fused pass applies a permutation, and a store sorted as one
+  // tile has none to apply)
+#define L(DET, ROWS, ...)                                                              \
+  switch (sel) {                                                                       \
+    case 7:                                                                            \
+      if (pm)                                                                          \
+        k_particles32<true, true, true, DET, true, true, false>                        \
+            <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
+      else                                                                             \
+        k_particles32<true, true, true, DET, true, false, ROWS>                        \
+            <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
+      break;                                                                           \
+    case 4:                                                                            \
+      k_particles32<true, false, false, DET, false, false, ROWS>                       \
+          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
+      break;                                                                           \
+    case 2:                                                                            \
+      k_particles32<false, true, false, DET, false, false, ROWS>                       \
+          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
+      break;                                                                           \
+    case 1:                                                                            \
+      k_particles32<false, false, true, DET, false, false, ROWS>                       \
+          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
+      break;                                                                           \
+    default:                                                                           \
+      return set_error(ctx, PIC_E_ARG, "particle pass %d", sel);                       \
+  }
   if (det) {
-    unsigned long long *base = S->fx;
     const int64_t pl = ctx->geom.plane;
-    const int off = sp == PIC_ION ? 0 : 3;
-    unsigned long long *jx = base + (off + 0) * pl, *jy = base + (off + 1) * pl,
-                       *jz = base + (off + 2) * pl,
-                       *nd = base + (6 + (sp == PIC_ION ? 0 : 1)) * pl;
-#define L(A, B, C) \
-  k_particles32<A, B, C, true, false, false><<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm)
-    switch (sel == 7 ? 8 : sel) {
-      case 8:
-        if (pm)
-          k_particles32<true, true, true, true, true, true>
-              <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm);
-        else
-          k_particles32<true, true, true, true, true, false>
-              <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm);
-        break;
-      case 6: L(true, true, false); break;
-      case 4: L(true, false, false); break;
-      case 2: L(false, true, false); break;
-      case 1: L(false, false, true); break;
-      case 3: L(false, true, true); break;
-      case 5: L(true, false, true); break;
-      default: return 0;
+    unsigned long long *j = S->fx + (sp == PIC_ION ? 0 : 3) * pl,
+                       *nd = S->fx + (sp == PIC_ION ? 6 : 7) * pl;
+    if (rows) {
+      L(true, true, j, j + pl, j + 2 * pl, nd)
+    } else {
+      L(true, false, j, j + pl, j + 2 * pl, nd)
     }
-#undef L
     if (do_push_j || do_drift_n) S->fx_dirty = true;
   } else {
     Fields<float> F = fields<float>(ctx);
-    float *jx = F.f[sp == PIC_ION ? PIC_JIX : PIC_JEX];
-    float *jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
-    float *jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
+    const int j = sp == PIC_ION ? PIC_JIX : PIC_JEX;
     float *nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
-#define L(A, B, C) \
-  k_particles32<A, B, C, false, false, false><<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm)
-    switch (sel == 7 ? 8 : sel) {
-      case 8:
-        if (pm)
-          k_particles32<true, true, true, false, true, true>
-              <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm);
-        else
-          k_particles32<true, true, true, false, true, false>
-              <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, jx, jy, jz, nd, tp, Q, pm);
-        break;
-      case 6: L(true, true, false); break;
-      case 4: L(true, false, false); break;
-      case 2: L(false, true, false); break;
-      case 1: L(false, false, true); break;
-      case 3: L(false, true, true); break;
-      case 5: L(true, false, true); break;
-      default: return 0;
+    if (rows) {
+      L(false, true, F.f[j], F.f[j + 1], F.f[j + 2], nd)
+    } else {
+      L(false, false, F.f[j], F.f[j + 1], F.f[j + 2], nd)
     }
-#undef L
   }
+#undef L
   PIC_LAUNCH_CHECK(ctx);
   if (pm) {
     ctx->cur[sp] = 1 - ctx->cur[sp];
@@ -2089,6 +2105,9 @@ static int sort_impl(pic_ctx *ctx, int sp, bool defer) {
   rc = tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
                    ctx->tile_start[sp]);
   if (rc) return rc;
+  if (ctx->row_start[sp] &&
+      (rc = tile_bounds(ctx, ctx->keys_alt, n, 1u, (int)ncell, ctx->row_start[sp])))
+    return rc;
   // the kept count is the start of the drop tile
   PIC_HIP(ctx, hipMemcpyAsync(ctx->host_counter, ctx->tile_start[sp] + nt,
                               sizeof(uint32_t), hipMemcpyDeviceToHost,
@@ -2103,6 +2122,7 @@ static int sort_impl(pic_ctx *ctx, int sp, bool defer) {
   ctx->cur[sp] = 1 - ctx->cur[sp];
   ctx->n[sp] = valid;
   ctx->sorted_end[sp] = valid;
+  ctx->row_end[sp] = valid;
   return 0;
 }
 

@@ -310,103 +310,6 @@ __device__ inline void boris(const StepConst &k, const double f[6], double &x,
   z += vz * dt * 0.5;
 }
 
-__device__ inline void add(double *p, double v) { unsafeAtomicAdd(p, v); }
-
-// shape_func_{ion,electron}0_j_2 (:3397-3553)
-__device__ inline void deposit_j(const Geom &g, double *jx, double *jy,
-                                 double *jz, double x, double y, double z,
-                                 double vx, double vy, double vz, double wgt,
-                                 double q, double dx) {
-  const double dx3 = dx * dx * dx;
-  const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
-  int k = (int)(x / dx);
-  int l = (int)(y / dx - 0.5);
-  int m = (int)(z / dx - 0.5);
-  const double qn = q * wgt / dx3;
-  double temp = qn * vx;
-  double kkkp = ((k + 1) * dx - x);
-  double lllp = (((l + 1) + 0.5) * dx - y);
-  double mmmp = (((m + 1) + 0.5) * dx - z);
-  double pk = (x - k * dx);
-  double pl = (y - (l + 0.5) * dx);
-  double pm = (z - (m + 0.5) * dx);
-  double tk = temp * kkkp, tp = temp * pk;
-  int64_t i = g.idx(k, l, m);
-  add(jx + i, (tk) * (lllp * mmmp));
-  add(jx + i + 1, (tk) * (lllp * pm));
-  add(jx + i + dl, (tk) * (pl * mmmp));
-  add(jx + i + dl + 1, (tk) * (pl * pm));
-  add(jx + i + dk, (tp) * (lllp * mmmp));
-  add(jx + i + dk + 1, (tp) * (lllp * pm));
-  add(jx + i + dk + dl, (tp) * (pl * mmmp));
-  add(jx + i + dk + dl + 1, (tp) * (pl * pm));
-
-  k = (int)(x / dx - 0.5);
-  l = (int)(y / dx);
-  temp = qn * vy;
-  kkkp = (((k + 1) + 0.5) * dx - x);
-  lllp = ((l + 1) * dx - y);
-  pk = (x - (k + 0.5) * dx);
-  pl = (y - l * dx);
-  tk = temp * kkkp;
-  tp = temp * pk;
-  i = g.idx(k, l, m);
-  add(jy + i, (tk) * (lllp * mmmp));
-  add(jy + i + 1, (tk) * (lllp * pm));
-  add(jy + i + dl, (tk) * (pl * mmmp));
-  add(jy + i + dl + 1, (tk) * (pl * pm));
-  add(jy + i + dk, (tp) * (lllp * mmmp));
-  add(jy + i + dk + 1, (tp) * (lllp * pm));
-  add(jy + i + dk + dl, (tp) * (pl * mmmp));
-  add(jy + i + dk + dl + 1, (tp) * (pl * pm));
-
-  l = (int)(y / dx - 0.5);
-  m = (int)(z / dx);
-  temp = qn * vz;
-  lllp = (((l + 1) + 0.5) * dx - y);
-  mmmp = ((m + 1) * dx - z);
-  pl = (y - (l + 0.5) * dx);
-  pm = (z - m * dx);
-  tk = temp * kkkp;
-  tp = temp * pk;
-  i = g.idx(k, l, m);
-  add(jz + i, (tk) * (lllp * mmmp));
-  add(jz + i + 1, (tk) * (lllp * pm));
-  add(jz + i + dl, (tk) * (pl * mmmp));
-  add(jz + i + dl + 1, (tk) * (pl * pm));
-  add(jz + i + dk, (tp) * (lllp * mmmp));
-  add(jz + i + dk + 1, (tp) * (lllp * pm));
-  add(jz + i + dk + dl, (tp) * (pl * mmmp));
-  add(jz + i + dk + dl + 1, (tp) * (pl * pm));
-}
-
-// shape_func_{ion,electron}0_n_2 (:3333-3395)
-__device__ inline void deposit_n(const Geom &g, double *n, double x, double y,
-                                 double z, double wgt, double dx) {
-  const double dx3 = dx * dx * dx;
-  const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
-  const int k = (int)(x / dx - 0.5);
-  const int l = (int)(y / dx - 0.5);
-  const int m = (int)(z / dx - 0.5);
-  const double temp = wgt / dx3;
-  const double kkkp = (((k + 1) + 0.5) * dx - x);
-  const double lllp = (((l + 1) + 0.5) * dx - y);
-  const double mmmp = (((m + 1) + 0.5) * dx - z);
-  const double pk = (x - (k + 0.5) * dx);
-  const double pl = (y - (l + 0.5) * dx);
-  const double pm = (z - (m + 0.5) * dx);
-  const double tk = temp * kkkp, tp = temp * pk;
-  const int64_t i = g.idx(k, l, m);
-  add(n + i, (tk) * (lllp * mmmp));
-  add(n + i + 1, (tk) * (lllp * pm));
-  add(n + i + dl, (tk) * (pl * mmmp));
-  add(n + i + dl + 1, (tk) * (pl * pm));
-  add(n + i + dk, (tp) * (lllp * mmmp));
-  add(n + i + dk + 1, (tp) * (lllp * pm));
-  add(n + i + dk + dl, (tp) * (pl * mmmp));
-  add(n + i + dk + dl + 1, (tp) * (pl * pm));
-}
-
 // Array-safety rule (the oracle states the same): nodes base..base+1 stay
 // inside the array when -0.5 < x/dx < S-1 on every axis.
 __device__ inline bool in_array(const Geom &g, double x, double y, double z,
@@ -421,73 +324,6 @@ __device__ inline bool in_gate(const Geom &g, double x, double y, double z,
                                double dx) {
   return x < (g.NX + 4) * dx && x >= 0. && y < (g.NY + 4) * dx && y >= 0. &&
          z < (g.NZ + 4) * dx && z >= 0.;
-}
-
-// One particle pass.  PUSH_J: hot loop A (:731-812); DRIFT_N: hot loop B
-// (:818-867); BOUNDARY: sr_particle (:2041-2531) on one rank.  The fused
-// form (all three) is exact because none of the field updates between those
-// loops in fdtd() reads or writes particle state.
-template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY>
-__global__ __launch_bounds__(256) void k_particles(
-    Geom g, Fields<double> F, Particles64 P, int64_t n, StepConst kc,
-    double *jx, double *jy, double *jz, double *nd) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double z = P.z[i];
-  if (isnan(z)) return;  // dead until the next compaction
-  double x = P.x[i], y = P.y[i];
-  double vx = P.vx[i], vy = P.vy[i], vz = P.vz[i];
-  const double dx = kc.dx;
-  const double dth = kc.dt * 0.5;
-  if (PUSH_J) {
-    if (x < kc.blo[0] || x > kc.bhi[0] || y < kc.blo[1] || y > kc.bhi[1] ||
-        z < kc.blo[2] || z > kc.bhi[2] || !in_array(g, x, y, z, dx)) {
-      x += vx * dth;
-      y += vy * dth;
-      z += vz * dth;
-    } else {
-      double f[6];
-      gather(F, g, x, y, z, dx, f);
-      boris(kc, f, x, y, z, vx, vy, vz);
-    }
-    if (in_gate(g, x, y, z, dx) && in_array(g, x, y, z, dx))
-      deposit_j(g, jx, jy, jz, x, y, z, vx, vy, vz, kc.weight, kc.q, dx);
-  }
-  if (DRIFT_N) {
-    x += vx * dth;
-    y += vy * dth;
-    z += vz * dth;
-    if (in_gate(g, x, y, z, dx) && in_array(g, x, y, z, dx))
-      deposit_n(g, nd, x, y, z, kc.weight, dx);
-  }
-  if (BOUNDARY) {
-    const double dx2 = 2. * dx;
-    const double gx2 = (g.NX + 2) * dx, gy2 = (g.NY + 2) * dx,
-                 gz2 = (g.NZ + 2) * dx;
-    bool dead = !(z < gz2 && z >= dx2);
-    if (!dead) {
-      if (x >= gx2) {
-        if (kc.periodic[0]) x = x - g.NX * dx; else dead = true;
-      } else if (x < dx2) {
-        if (kc.periodic[0]) x = x + g.NX * dx; else dead = true;
-      }
-      if (y >= gy2) {
-        if (kc.periodic[1]) y = y - g.NY * dx; else dead = true;
-      } else if (y < dx2) {
-        if (kc.periodic[1]) y = y + g.NY * dx; else dead = true;
-      }
-    }
-    if (dead) {
-      P.z[i] = __longlong_as_double(0x7ff8000000000000LL);
-      return;
-    }
-  }
-  P.x[i] = x;
-  P.y[i] = y;
-  P.z[i] = z;
-  P.vx[i] = vx;
-  P.vy[i] = vy;
-  P.vz[i] = vz;
 }
 
 // ---------------------------------------------------------------------------
@@ -567,7 +403,11 @@ __device__ inline void thrust_store64(const double (&th)[6], double *out, int bi
 // particles of the central box: their positions and velocities at the start
 // of the pass are that step's end state, E is unchanged since, and Fp holds
 // the total B of its end (E planes shared with F).
-template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST>
+// ROWS: as in the FP32 form, boxes of cell columns of a store sorted as one
+// tile, the threads divided evenly over a box's columns.  32^3 x 16 ppc in
+// chunks of 2048 slots, whose boxes fit no window, took 475 us per launch
+// and in boxes 90 us; 8 x 8 x 16 x 4 ppc 70 us and 18 us.
+template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST, bool ROWS>
 __global__ __launch_bounds__(256) void k_particles_tiled(
     Geom g, TileGeom tg, Fields<double> F, Particles64 P, TileRun tr,
     StepConst kc, double *jx, double *jy, double *jz, double *nd,
@@ -581,7 +421,7 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
   if (tid == 0) {
     int64_t s, e;
     Win w;
-    tile_setup(bid, tr, tg, kWin64,
+    tile_setup<ROWS>(bid, tr, tg, kWin64,
                [&](int64_t i, int &k, int &l, int &m) {
                  const double x = P.x[i], y = P.y[i], z = P.z[i];
                  if (!in_array(g, x, y, z, dx)) return false;
@@ -608,7 +448,16 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
   for (int i = tid; i < 4 * WN; i += blockDim.x) acc[(i / WN) * kWin64 + i % WN] = 0.0;
   __syncthreads();
   const double dth = kc.dt * 0.5;
-  for (int64_t i = s + tid; i < e; i += blockDim.x) {
+  int64_t i0 = s + tid, i1 = e;
+  int lanes = blockDim.x;
+  if (ROWS && bid < tr.ntiles) {
+    lanes = kBlock / (tg.TX * tg.TY);
+    int rs, re;
+    row_range(tr, tg, g.NX, g.NY, g.NZ, bid, tid / lanes, rs, re);
+    i0 = rs + tid % lanes;
+    i1 = re;
+  }
+  for (int64_t i = i0; i < i1; i += lanes) {
     double z = P.z[i];
     if (isnan(z)) continue;
     double x = P.x[i], y = P.y[i];
@@ -1043,15 +892,27 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   double *jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
   double *jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
   double *nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
-  const TileGeom tg = tile_geom(ctx);
+  TileGeom tg = tile_geom(ctx);
   TileRun tr;
   tr.tile_start = ctx->tile_start[sp];
   tr.sorted_end = ctx->sorted_end[sp];
-  // a single tile (the reference's order) is processed as tail chunks
-  tr.ntiles = (tr.sorted_end > 0 && tg.ntiles() > 1) ? tg.ntiles() : 0;
+  tr.ntiles = tr.sorted_end > 0 ? tg.ntiles() : 0;
+  // a single tile (the reference's order): boxes of rows while the sort's
+  // cell starts are current, otherwise chunks as an unsorted tail (slots of
+  // the rows are 32-bit)
+  const bool rows = tr.ntiles == 1 && ctx->row_start[sp] &&
+                    ctx->row_end[sp] == tr.sorted_end && n <= ((int64_t)1 << 30);
+  if (rows) {
+    tg = row_geom(tg);
+    tr.tile_start = ctx->row_start[sp];
+    tr.ntiles = tg.ntiles();
+  } else if (tr.ntiles == 1) {
+    tr.ntiles = 0;
+  }
   if (tr.ntiles == 0) tr.sorted_end = 0;
   tr.n = n;
-  tr.ntail = (int)div_up(n - tr.sorted_end, kTailChunk);
+  tr.chunk = tail_chunk(ctx->cfg.ppc, false);
+  tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
   const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
   const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
   // the fused pass of pic_step adds the previous step's thrust_fave
@@ -1066,22 +927,22 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     for (int q = 0; q < 3; ++q) Fp.f[PIC_BX + q] = (double *)bp + q * ctx->geom.plane;
     tp = ctx->thrust_part;
   }
-#define LAUNCH(A, B, C)                                                    \
-  k_particles_tiled<A, B, C, false><<<nb, kBlock, 0, ctx->stream>>>(        \
-      ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp)
+#define LAUNCH(A, B, C, T)                                                  \
+  do {                                                                      \
+    if (rows)                                                               \
+      k_particles_tiled<A, B, C, T, true><<<nb, kBlock, 0, ctx->stream>>>(  \
+          ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp);             \
+    else                                                                    \
+      k_particles_tiled<A, B, C, T, false><<<nb, kBlock, 0, ctx->stream>>>( \
+          ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp);             \
+  } while (0)
   switch (thrust ? 8 : sel) {
-    case 8:
-      k_particles_tiled<true, true, true, true><<<nb, kBlock, 0, ctx->stream>>>(
-          ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp);
-      break;
-    case 7: LAUNCH(true, true, true); break;
-    case 6: LAUNCH(true, true, false); break;
-    case 4: LAUNCH(true, false, false); break;
-    case 2: LAUNCH(false, true, false); break;
-    case 1: LAUNCH(false, false, true); break;
-    case 3: LAUNCH(false, true, true); break;
-    case 5: LAUNCH(true, false, true); break;
-    default: return 0;
+    case 8: LAUNCH(true, true, true, true); break;
+    case 7: LAUNCH(true, true, true, false); break;
+    case 4: LAUNCH(true, false, false, false); break;
+    case 2: LAUNCH(false, true, false, false); break;
+    case 1: LAUNCH(false, false, true, false); break;
+    default: return set_error(ctx, PIC_E_ARG, "particle pass %d", sel);
   }
 #undef LAUNCH
   PIC_LAUNCH_CHECK(ctx);
@@ -1236,6 +1097,9 @@ int sort(pic_ctx *ctx, int sp) {
   rc = tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
                    ctx->tile_start[sp]);
   if (rc) return rc;
+  if (ctx->row_start[sp] &&
+      (rc = tile_bounds(ctx, ctx->keys_alt, n, 1u, (int)ncell, ctx->row_start[sp])))
+    return rc;
   // the kept count is the start of the drop tile
   PIC_HIP(ctx, hipMemcpyAsync(ctx->host_counter, ctx->tile_start[sp] + nt,
                               sizeof(uint32_t), hipMemcpyDeviceToHost,
@@ -1250,6 +1114,7 @@ int sort(pic_ctx *ctx, int sp) {
   ctx->cur[sp] = 1 - ctx->cur[sp];
   ctx->n[sp] = valid;
   ctx->sorted_end[sp] = valid;
+  ctx->row_end[sp] = valid;
   return 0;
 }
 

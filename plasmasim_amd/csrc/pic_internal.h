@@ -148,6 +148,11 @@ struct pic_ctx {
   // sort; [0, sorted_end) is tile-sorted, later slots are the inflow tail
   uint32_t *tile_start[2] = {nullptr, nullptr};   // ntiles + 1 per species
   int64_t sorted_end[2] = {0, 0};
+  // one tile over the interior: each cell's first slot after the last sort
+  // (cells + 1 entries), valid while row_end == sorted_end > 0; whatever
+  // sets sorted_end other than a sort sets row_end to 0
+  uint32_t *row_start[2] = {nullptr, nullptr};
+  int64_t row_end[2] = {0, 0};
   int32_t drift_halves[2] = {0, 0};  // half-step drifts since the tile sort
   int64_t sort_tile_count = 0;   // sorts done by the tile sort
   pic::tsort::Bufs *ts64 = nullptr;  // the FP64 form's tile-sort lists (pic_tsort.h)

@@ -16,16 +16,65 @@
 namespace pic {
 
 constexpr int kMargin = 3;
-constexpr int kTailChunk = 2048;
+constexpr int kTailChunk = 2048;  // most slots per workgroup of the tail
 constexpr int kStray = 8;
 
+// Slots per workgroup of the unsorted inflow tail.  An inflow batch walks
+// its two-layer slab in blocks of 4 x 4 x 2 cells (blocked) or along y in
+// columns of 2 cells, ppc slots per cell; the window holds 3 blocks or 16
+// columns (kStray cells to either side of the middle sample), so a chunk of
+// more slots than that has no window and adds every contribution to the
+// global planes.
+inline int tail_chunk(int ppc, bool blocked) {
+  const int64_t most = (int64_t)(blocked ? 64 : 32) * ppc;
+  int c = kTailChunk;
+  while (c > 256 && c > most) c >>= 1;
+  return c;
+}
+
 struct TileRun {
-  const uint32_t *tile_start;  // ntiles + 1 entries
+  const uint32_t *tile_start;  // ntiles + 1 entries (rows: one per cell, + 1)
   int ntiles;
   int64_t sorted_end;          // [0, sorted_end) is tile-sorted
   int64_t n;                   // stored slots
-  int ntail;                   // tail chunks of kTailChunk
+  int ntail;                   // tail chunks
+  int chunk;                   // slots per tail chunk
 };
+
+// A store sorted as one tile (the reference's order: cells along z, then y,
+// then x) has no tile ranges of its own.  The pass takes it in boxes of
+// TX x TY columns of TZ cells; a box's particles are TX * TY ranges of the
+// store, found in the table of each cell's first slot that the sort leaves.
+// Boxes may reach over the grid's upper faces (the sizes need not divide).
+// 4 x 4 x 8 is the largest box whose window fits both forms; where that
+// gives fewer boxes than the chip holds workgroups (3 per CU), 2 x 2 x 8.
+inline TileGeom row_geom(const TileGeom &one) {
+  const auto up = [](int a, int b) { return (a + b - 1) / b; };
+  TileGeom t = one;
+  const int NX = one.TX, NY = one.TY, NZ = one.TZ;
+  for (int w = 4; w >= 2; w -= 2) {
+    t.TX = t.TY = w;
+    t.TZ = 8;
+    t.NTX = up(NX, w);
+    t.NTY = up(NY, w);
+    t.NTZ = up(NZ, 8);
+    if (t.ntiles() >= 768) break;
+  }
+  t.LX = t.LY = t.LZ = -1;
+  return t;
+}
+
+// slot range of column r (< TX * TY) of box bid
+__device__ inline void row_range(const TileRun &tr, const TileGeom &tg, int NX, int NY,
+                                 int NZ, int bid, int r, int &s, int &e) {
+  const int tz = bid % tg.NTZ, ty = (bid / tg.NTZ) % tg.NTY, tx = bid / (tg.NTZ * tg.NTY);
+  const int k = tx * tg.TX + r / tg.TY, l = ty * tg.TY + r % tg.TY;
+  s = e = 0;
+  if (k >= NX || l >= NY) return;
+  const int64_t c = ((int64_t)k * NY + l) * NZ;
+  s = (int)tr.tile_start[c + tz * tg.TZ];
+  e = (int)tr.tile_start[c + min((tz + 1) * tg.TZ, NZ)];
+}
 
 // LDS window: origin (cells) and extents (nodes), and the cell range whose
 // stencils fit inside it
@@ -61,15 +110,16 @@ __device__ inline int xcd_remap(int b, int nt, int nb) {
 }
 
 // Range and window of workgroup bid.  cell_of(i, k, l, m) returns false for
-// a dead slot.  Runs on one thread.
-template <typename CellOf>
+// a dead slot.  Runs on one thread.  ROWS: the workgroups below ntiles are
+// boxes of rows (row_geom), whose ranges row_range gives; s < e here.
+template <bool ROWS, typename CellOf>
 __device__ inline void tile_setup(int bid, const TileRun &tr, const TileGeom &tg,
                                   int win_max, CellOf cell_of, int64_t &s,
                                   int64_t &e, Win &w) {
   int ak0, ak1, al0, al1, am0, am1;  // anchor box (cells)
   if (bid < tr.ntiles) {
-    s = tr.tile_start[bid];
-    e = tr.tile_start[bid + 1];
+    s = ROWS ? 0 : tr.tile_start[bid];
+    e = ROWS ? 1 : tr.tile_start[bid + 1];
     const int tz = bid % tg.NTZ, ty = (bid / tg.NTZ) % tg.NTY,
               tx = bid / (tg.NTZ * tg.NTY);
     ak0 = 2 + tx * tg.TX + tg.shift[0];
@@ -80,8 +130,8 @@ __device__ inline void tile_setup(int bid, const TileRun &tr, const TileGeom &tg
     am1 = am0 + tg.TZ - 1;
   } else {
     const int c = bid - tr.ntiles;
-    s = tr.sorted_end + (int64_t)c * kTailChunk;
-    e = s + kTailChunk < tr.n ? s + kTailChunk : tr.n;
+    s = tr.sorted_end + (int64_t)c * tr.chunk;
+    e = s + tr.chunk < tr.n ? s + tr.chunk : tr.n;
     ak0 = al0 = am0 = 1 << 20;
     ak1 = al1 = am1 = -1;
     // 8 samples; those more than kStray cells from a middle sample on some

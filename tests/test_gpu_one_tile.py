@@ -1,0 +1,80 @@
+"""Stores sorted as one tile over the interior (the reference's order): the
+particle pass takes them in boxes of cell columns, whose sizes need not
+divide the grid, and the inflow tail in chunks."""
+import numpy as np
+import pytest
+
+import plasmasim_amd as ps
+from helpers import rel_l2
+
+pytestmark = pytest.mark.gpu
+FIELDS = ["ex", "ey", "ez", "bx", "by", "bz", "jix", "jiy", "jiz", "jex", "jey", "jez", "ni",
+          "ne"]
+
+
+def state(n, tile, precision, fused=True):
+    c = ps.preset(1)
+    c.nx, c.ny, c.nz = n
+    c.ppc = 5
+    c.absorb[2] = 2
+    c.ballistic_lo[2], c.ballistic_hi[2] = 6.0, c.nz - 2.0
+    c.inflow_every, c.sort_every = 3, 5
+    c.precision = precision
+    c.deposit = ps.PIC_DEPOSIT_DETERMINISTIC
+    for a in range(3):
+        c.tile[a] = tile[a]
+    s = ps.Simulation(c)
+    s.load_particles()
+    s.begin()
+    s.thrust_ave(True)
+    if fused:
+        s.step(12)
+    else:
+        for _ in range(3):
+            s.renew_grid()
+            for sp in (0, 1):
+                s.push_deposit_j(sp)
+            for sp in (0, 1):
+                s.drift_deposit_n(sp)
+            s.fold_current()
+            s.particle_boundary()
+    return s
+
+
+# (grid, a tiling of it that runs on tile ranges): the smallest grid, one cell
+# over and under the boxes' sizes, sizes that nothing divides, many boxes
+@pytest.mark.parametrize("n, tile", [((4, 4, 8), (4, 4, 4)), ((5, 7, 9), (5, 7, 3)),
+                                     ((9, 3 * 5, 17 * 2), (3, 5, 2)),
+                                     ((31, 27, 45), (1, 3, 15)), ((48, 36, 64), (4, 4, 8))])
+@pytest.mark.parametrize("fused", [True, False])
+def test_one_tile_equals_tiles(n, tile, fused):
+    """FP32 with the fixed summation order: bit for bit the fields of the
+    tiled run (sorts, inflows and both kinds of tail between).  FP64: sums in
+    another order, 32 contributions of 2^-53 each per node and step."""
+    a = state(n, (0, 0, 0), ps.PIC_FP32, fused)
+    b = state(n, tile, ps.PIC_FP32, fused)
+    for k in FIELDS:
+        assert np.array_equal(a.download_field(k), b.download_field(k)), k
+    if fused:
+        fa, fb = a.thrust_ave_get()[0], b.thrust_ave_get()[0]
+        # per-lane fp32 sums of another grouping: 2^-24 of the largest part
+        assert np.abs(fa - fb).max() <= 1e-5 * max(np.abs(fb).max(), 1e-30)
+    a = state(n, (0, 0, 0), ps.PIC_FP64, fused)
+    b = state(n, tile, ps.PIC_FP64, fused)
+    for k in FIELDS:
+        assert rel_l2(a.download_field(k), b.download_field(k)) <= 1e-12, k
+
+
+def test_one_tile_resumes_without_cell_starts(tmp_path):
+    """A loaded checkpoint carries no cell starts: the pass takes the store
+    in chunks until the next sort, with the same result."""
+    a = state((20, 12, 24), (0, 0, 0), ps.PIC_FP32)
+    f = str(tmp_path / "c.bin")
+    a.checkpoint_save(f)
+    b = ps.Simulation(a.cfg)
+    b.checkpoint_load(f)
+    a.thrust_ave(False)
+    a.step(3)
+    b.step(3)
+    for k in FIELDS:
+        assert np.array_equal(a.download_field(k), b.download_field(k)), k
