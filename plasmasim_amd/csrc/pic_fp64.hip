@@ -273,22 +273,34 @@ __device__ inline void gather(const Fields<double> &F, const Geom &g, double x,
                    Z.hu, Z.hl) * inv_dx3;
 }
 
-// cal_track4 (:2804-2870)
-__device__ inline void boris(const StepConst &k, const double f[6], double &x,
-                             double &y, double &z, double &vx, double &vy,
-                             double &vz) {
-  const double C = k.c, dt = k.dt;
-  const double T = 0.5 * k.q * dt / k.mass;
+// Constants of one species' pass, formed on the host by the reference's
+// operations (a uniform FP64 product on the device would hold two vector
+// registers through the whole loop).
+struct PassConst {
+  double dx, dt, dth, c;
+  double cc;              // C^2
+  double T, TT, T2;       // q dt / (2 m), its square, 2 T
+  double eimf_x, eimf_y;  // V * IMF terms of E (:2817-2818)
+  double qn, wn;          // q w / dx^3, w / dx^3
+  double blo[3], bhi[3];  // ballistic zone
+  double box_lo[3], box_hi[3];  // thrust_fave's box (open)
+  int periodic[2];
+};
+
+// cal_track4 (:2804-2870), velocity
+__device__ inline void boris(const PassConst &k, const double f[6], double &vx,
+                             double &vy, double &vz) {
+  const double C = k.c, T = k.T;
   double ex = f[0], ey = f[1], ez = f[2];
   const double bx = f[3], by = f[4], bz = f[5];
-  ex += k.vdrift_z * k.imf_y;
-  ey += -k.vdrift_z * k.imf_x;
-  double gamma1 = C / sqrt(C * C - vx * vx - vy * vy - vz * vz);
+  ex += k.eimf_x;
+  ey += k.eimf_y;
+  double gamma1 = C / sqrt(k.cc - vx * vx - vy * vy - vz * vz);
   if (isnan(gamma1)) gamma1 = 0.;
   double ux = gamma1 * vx, uy = gamma1 * vy, uz = gamma1 * vz;
-  double gamma2 = C / sqrt(C * C + ux * ux + uy * uy + uz * uz);
+  double gamma2 = C / sqrt(k.cc + ux * ux + uy * uy + uz * uz);
   const double bux = gamma2 * (bx), buy = gamma2 * (by), buz = gamma2 * (bz);
-  const double S = 2. * T / (1. + T * T * (bux * bux + buy * buy + buz * buz));
+  const double S = k.T2 / (1. + k.TT * (bux * bux + buy * buy + buz * buz));
   ux += (ex) * T;
   uy += (ey) * T;
   uz += (ez) * T;
@@ -301,13 +313,10 @@ __device__ inline void boris(const StepConst &k, const double f[6], double &x,
   upx += (ex) * T;
   upy += (ey) * T;
   upz += (ez) * T;
-  gamma2 = C / sqrt(C * C + upx * upx + upy * upy + upz * upz);
+  gamma2 = C / sqrt(k.cc + upx * upx + upy * upy + upz * upz);
   vx = gamma2 * upx;
   vy = gamma2 * upy;
   vz = gamma2 * upz;
-  x += vx * dt * 0.5;
-  y += vy * dt * 0.5;
-  z += vz * dt * 0.5;
 }
 
 // Array-safety rule (the oracle states the same): nodes base..base+1 stay
@@ -319,65 +328,219 @@ __device__ inline bool in_array(const Geom &g, double x, double y, double z,
          zd > -0.5 && zd < g.SZ - 1;
 }
 
-// deposit gate (:747-749)
-__device__ inline bool in_gate(const Geom &g, double x, double y, double z,
-                               double dx) {
-  return x < (g.NX + 4) * dx && x >= 0. && y < (g.NY + 4) * dx && y >= 0. &&
-         z < (g.NZ + 4) * dx && z >= 0.;
-}
-
 // ---------------------------------------------------------------------------
-// tiled particle pass: one workgroup per sort tile, J and n accumulated in an
-// LDS window with FP64 atomics, then added to the planes (see pic_tiles.h)
+// particle pass: one workgroup per sort tile, J and n accumulated in an LDS
+// window with FP64 atomics, then added to the planes (see pic_tiles.h)
+//
+// No unit is saturated (128^3 x 64 ppc: VALU 41 %, LDS 42 %, L1 46 % busy at
+// three waves per SIMD), the waves wait on each in turn; the pass is written
+// for few instructions (830 per particle) with the reference's operations and
+// rounding: one stencil per position shared by the gathers and the previous
+// step's force; constants formed on the host; each lane's walk of the
+// stencils set up once per workgroup, one swap of the weights per axis; and
+// in normalised units (UNIT: dx = 1, where x / dx and w * dx are x and w
+// exactly; planes and arrays below 4 GiB) no divisions by dx and 32-bit byte
+// offsets from uniform bases.  165 VGPRs, from 239 at two waves per SIMD.
+// 20 steps at 128^3 x 64 ppc 377 -> 345 ms, at 32^3 x 16 ppc 7.1 -> 5.8 ms.
 
 constexpr int kWin64 = 1400;  // window capacity in nodes (4 x double each)
 
 #define PIC_LDS __attribute__((address_space(3)))
 #define PIC_GLB __attribute__((address_space(1)))
 
-__device__ inline void lds_add64(double *p, double v) {
-  __hip_atomic_fetch_add((PIC_LDS double *)p, v, __ATOMIC_RELAXED,
+typedef unsigned long long u64;
+
+__device__ __forceinline__ void lds_add64(char *acc, int byte, double v) {
+  __hip_atomic_fetch_add((PIC_LDS double *)(acc + byte), v, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ inline void glob_add64(double *p, double v) {
+__device__ __forceinline__ void glob_add64(double *p, double v) {
   __hip_atomic_fetch_add((PIC_GLB double *)p, v, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <bool UNIT>
+struct Off {
+  using T = int64_t;
+};
+template <>
+struct Off<true> {
+  using T = uint32_t;
+};
+template <typename T, typename O>
+__device__ __forceinline__ T *at(T *base, O byte) {
+  return (T *)((char *)base + byte);
+}
+
+// Gather of one staggered component around the byte offset i of its stencil
+// base (shape_func_v2 :3223-3273): the products and sums of gather1.
+template <typename O>
+__device__ __forceinline__ double gather1o(const double *F, O i, O dl, O dk, double wa0,
+                                           double wa1, double wb0, double wb1,
+                                           double wc0, double wc1) {
+  const double *f0 = at(F, i), *f1 = at(F, i + dl), *f2 = at(F, i + dk),
+               *f3 = at(F, i + dk + dl);
+  const double p1 = f0[0] * (wa0 * wb0 * wc0) + f0[1] * (wa0 * wb0 * wc1);
+  const double p2 = f1[0] * (wa0 * wb1 * wc0) + f1[1] * (wa0 * wb1 * wc1);
+  const double p3 = f2[0] * (wa1 * wb0 * wc0) + f2[1] * (wa1 * wb0 * wc1);
+  const double p4 = f3[0] * (wa1 * wb1 * wc0) + f3[1] * (wa1 * wb1 * wc1);
+  return p1 + p2 + p3 + p4;
+}
+
+// The lane's walk over the 8 nodes of a stencil in the LDS window: lane j
+// takes them mirrored along the axes set in j & 7, so that lanes holding
+// particles of one cell add to different nodes.
+struct Walk64 {
+  int first;   // byte offset of the first visited node from the stencil base
+  int off[8];  // byte offsets of the visits from the first node
+  bool mx, my, mz;
+};
+
+__device__ inline Walk64 make_walk64(int WY, int WZ) {
+  Walk64 k;
+  const int sw = threadIdx.x & 7;
+  k.mx = sw & 4;
+  k.my = sw & 2;
+  k.mz = sw & 1;
+  const int sz = 8, sy = 8 * WZ, sx = 8 * WY * WZ;
+  const int dx = k.mx ? -sx : sx, dy = k.my ? -sy : sy, dz = k.mz ? -sz : sz;
+  k.first = (k.mx ? sx : 0) + (k.my ? sy : 0) + (k.mz ? sz : 0);
+  k.off[0] = 0;
+  k.off[1] = dz;
+  k.off[2] = dy;
+  k.off[3] = dy + dz;
+  k.off[4] = dx;
+  k.off[5] = dx + dz;
+  k.off[6] = dx + dy;
+  k.off[7] = dx + dy + dz;
+  return k;
+}
+
 // The 8 contributions (temp*wa)*(wb*wc) of one component, as the reference
-// forms them (:3412-3425); lane j visits the nodes in the order n ^ (j & 7)
-// so that lanes holding particles of one cell hit different LDS nodes.
-__device__ inline void dep8_64(double *lds, double *glob, bool in_lds,
-                               const Win &w, const Geom &g, int a, int b,
-                               int c, double wa0, double wa1, double wb0,
-                               double wb1, double wc0, double wc1,
-                               double temp) {
+// forms them (:3412-3425), in the lane's walk order.
+__device__ __forceinline__ void lds_dep8_64(char *acc, int base, const Walk64 &k,
+                                            double temp, double wa0, double wa1,
+                                            double wb0, double wb1, double wc0,
+                                            double wc1) {
+  const double A0 = k.mx ? wa1 : wa0, A1 = k.mx ? wa0 : wa1;
+  const double B0 = k.my ? wb1 : wb0, B1 = k.my ? wb0 : wb1;
+  const double C0 = k.mz ? wc1 : wc0, C1 = k.mz ? wc0 : wc1;
+  const double ta0 = temp * A0, ta1 = temp * A1;
+  const double bc00 = B0 * C0, bc01 = B0 * C1, bc10 = B1 * C0, bc11 = B1 * C1;
+  const int p = base + k.first;
+  lds_add64(acc, p + k.off[0], ta0 * bc00);
+  lds_add64(acc, p + k.off[1], ta0 * bc01);
+  lds_add64(acc, p + k.off[2], ta0 * bc10);
+  lds_add64(acc, p + k.off[3], ta0 * bc11);
+  lds_add64(acc, p + k.off[4], ta1 * bc00);
+  lds_add64(acc, p + k.off[5], ta1 * bc01);
+  lds_add64(acc, p + k.off[6], ta1 * bc10);
+  lds_add64(acc, p + k.off[7], ta1 * bc11);
+}
+
+// the same stencil straight into a global plane
+__device__ __noinline__ void glob_dep8_64(double *glob, int64_t i, int64_t dl, int64_t dk,
+                                          double temp, double wa0, double wa1, double wb0,
+                                          double wb1, double wc0, double wc1) {
   const double ta0 = temp * wa0, ta1 = temp * wa1;
-  if (in_lds) {
-    const int WZ = w.WZ, WYZ = w.WY * w.WZ;
-    const int i = ((a - w.k0) * w.WY + (b - w.l0)) * WZ + (c - w.m0);
-    const int sw = threadIdx.x & 7;
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      const int id = n ^ sw;
-      const double ta = (id & 4) ? ta1 : ta0;
-      const double wb = (id & 2) ? wb1 : wb0;
-      const double wc = (id & 1) ? wc1 : wc0;
-      const int off = ((id & 4) ? WYZ : 0) + ((id & 2) ? WZ : 0) + (id & 1);
-      lds_add64(lds + i + off, (ta) * (wb * wc));
+  glob_add64(glob + i, (ta0) * (wb0 * wc0));
+  glob_add64(glob + i + 1, (ta0) * (wb0 * wc1));
+  glob_add64(glob + i + dl, (ta0) * (wb1 * wc0));
+  glob_add64(glob + i + dl + 1, (ta0) * (wb1 * wc1));
+  glob_add64(glob + i + dk, (ta1) * (wb0 * wc0));
+  glob_add64(glob + i + dk + 1, (ta1) * (wb0 * wc1));
+  glob_add64(glob + i + dk + dl, (ta1) * (wb1 * wc0));
+  glob_add64(glob + i + dk + dl + 1, (ta1) * (wb1 * wc1));
+}
+
+// The particles outside the window (pend), straight into the global planes.
+// A few, scattered over the waves: the wave takes them one at a time, each
+// active lane adding one node of one component, instead of idling behind a
+// lane's 8 or 24 atomics; more than kCoopMax in one wave go lane by lane (as
+// in the FP32 pass).  Reached by every active lane of the wave.
+constexpr int kCoopMax = 8;
+
+__device__ __forceinline__ double lane_get(double v, int src) {
+  const u64 b = (u64)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, src);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), src);
+  return __longlong_as_double((long long)(((u64)hi << 32) | lo));
+}
+
+__device__ __forceinline__ void glob_coop64(const Geom &g, bool pend, bool current,
+                                            double dx, double x, double y, double z,
+                                            double q0, double q1, double q2, double *jx,
+                                            double *jy, double *jz, double *nd) {
+  u64 todo = __builtin_amdgcn_ballot_w64(pend);
+  if (todo == 0) return;
+  const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
+  if (__builtin_popcountll(todo) > kCoopMax) {
+    if (pend) {
+      const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx), Z = axis_weights(z, dx);
+      if (current) {
+        glob_dep8_64(jx, g.idx(X.bi, Y.bh, Z.bh), dl, dk, q0, X.iu, X.il, Y.hu, Y.hl, Z.hu,
+                     Z.hl);
+        glob_dep8_64(jy, g.idx(X.bh, Y.bi, Z.bh), dl, dk, q1, X.hu, X.hl, Y.iu, Y.il, Z.hu,
+                     Z.hl);
+        glob_dep8_64(jz, g.idx(X.bh, Y.bh, Z.bi), dl, dk, q2, X.hu, X.hl, Y.hu, Y.hl, Z.iu,
+                     Z.il);
+      } else {
+        glob_dep8_64(nd, g.idx(X.bh, Y.bh, Z.bh), dl, dk, q0, X.hu, X.hl, Y.hu, Y.hl, Z.hu,
+                     Z.hl);
+      }
     }
-  } else {
-    const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
-    const int64_t i = g.idx(a, b, c);
-    glob_add64(glob + i, (ta0) * (wb0 * wc0));
-    glob_add64(glob + i + 1, (ta0) * (wb0 * wc1));
-    glob_add64(glob + i + dl, (ta0) * (wb1 * wc0));
-    glob_add64(glob + i + dl + 1, (ta0) * (wb1 * wc1));
-    glob_add64(glob + i + dk, (ta1) * (wb0 * wc0));
-    glob_add64(glob + i + dk + 1, (ta1) * (wb0 * wc1));
-    glob_add64(glob + i + dk + dl, (ta1) * (wb1 * wc0));
-    glob_add64(glob + i + dk + dl + 1, (ta1) * (wb1 * wc1));
+    return;
   }
+  const u64 ex = __builtin_amdgcn_read_exec();
+  const int rank = (int)__builtin_amdgcn_mbcnt_hi(
+      (uint32_t)(ex >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ex, 0u));
+  const int nact = __builtin_popcountll(ex);
+  const int nn = current ? 24 : 8;
+  do {
+    const int src = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    const AxisW X = axis_weights(lane_get(x, src), dx), Y = axis_weights(lane_get(y, src), dx),
+                Z = axis_weights(lane_get(z, src), dx);
+    const double s0 = lane_get(q0, src);
+    double s1 = 0.0, s2 = 0.0;
+    if (current) {
+      s1 = lane_get(q1, src);
+      s2 = lane_get(q2, src);
+    }
+    for (int t = rank; t < nn; t += nact) {
+      // node t: component t >> 3 (3: density), corner bits (x, y, z) of
+      // t & 7; the component's own axis takes the integer-node weights
+      const int c = current ? t >> 3 : 3;
+      const bool ux = t & 4, uy = t & 2, uz = t & 1;
+      const double wx = c == 0 ? (ux ? X.il : X.iu) : (ux ? X.hl : X.hu);
+      const double wy = c == 1 ? (uy ? Y.il : Y.iu) : (uy ? Y.hl : Y.hu);
+      const double wz = c == 2 ? (uz ? Z.il : Z.iu) : (uz ? Z.hl : Z.hu);
+      const double q = c == 1 ? s1 : c == 2 ? s2 : s0;
+      double *dst = c == 0 ? jx : c == 1 ? jy : c == 2 ? jz : nd;
+      const int64_t i = g.idx(c == 0 ? X.bi : X.bh, c == 1 ? Y.bi : Y.bh, c == 2 ? Z.bi : Z.bh) +
+                        (ux ? dk : 0) + (uy ? dl : 0) + (uz ? 1 : 0);
+      glob_add64(dst + i, (q * wx) * (wy * wz));
+    }
+  } while (todo);
+}
+
+// A deposit's place: inside the array and the gate (:747-749), which reduce
+// to 0 <= x and x/dx < S-1 per axis.
+__device__ __forceinline__ bool dep_ok(const Geom &g, double x, double y, double z, int k,
+                                       int l, int m) {
+  return x >= 0. && k < g.SX - 1 && y >= 0. && l < g.SY - 1 && z >= 0. && m < g.SZ - 1;
+}
+
+// a deposit at cell c touches the nodes c - 1 to c + 1: cells within the
+// anchor +- (kMargin - 1) keep them inside the window
+__device__ __forceinline__ bool win_holds(const Win &w, int k, int l, int m) {
+  return w.on && (unsigned)(k - w.vk0 + 1) <= (unsigned)(w.vk1 - w.vk0 + 2) &&
+         (unsigned)(l - w.vl0 + 1) <= (unsigned)(w.vl1 - w.vl0 + 2) &&
+         (unsigned)(m - w.vm0 + 1) <= (unsigned)(w.vm1 - w.vm0 + 2);
+}
+
+__device__ __forceinline__ int win_byte(const Win &w, int k, int l, int m) {
+  return (((k - w.k0) * w.WY + (l - w.l0)) * w.WZ + (m - w.m0)) * 8;
 }
 
 // thrust_fave partials of one workgroup (six per-thread sums added over the
@@ -399,25 +562,36 @@ __device__ inline void thrust_store64(const double (&th)[6], double *out, int bi
   }
 }
 
+// the planes a pass reads and adds to: E, total B, the total B at the end of
+// the previous step (THRUST)
+struct PassFields {
+  const double *e[3], *b[3], *bp[3];
+  double *jx, *jy, *jz, *nd;
+};
+
+// One particle pass.  PUSH_J: hot loop A (:731-812); DRIFT_N: hot loop B
+// (:818-867); BOUNDARY: sr_particle (:2041-2531) on one rank.  The fused
+// form (all three) is exact because none of the field updates between those
+// loops in fdtd() reads or writes particle state.
 // THRUST: also add thrust_fave (:5124-5285) of the previous step for the
 // particles of the central box: their positions and velocities at the start
-// of the pass are that step's end state, E is unchanged since, and Fp holds
-// the total B of its end (E planes shared with F).
+// of the pass are that step's end state, E is unchanged since, and bp holds
+// the total B of its end.
 // ROWS: as in the FP32 form, boxes of cell columns of a store sorted as one
 // tile, the threads divided evenly over a box's columns.  32^3 x 16 ppc in
 // chunks of 2048 slots, whose boxes fit no window, took 475 us per launch
 // and in boxes 90 us; 8 x 8 x 16 x 4 ppc 70 us and 18 us.
-template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST, bool ROWS>
+template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST, bool ROWS, bool UNIT>
 __global__ __launch_bounds__(256) void k_particles_tiled(
-    Geom g, TileGeom tg, Fields<double> F, Particles64 P, TileRun tr,
-    StepConst kc, double *jx, double *jy, double *jz, double *nd,
-    Fields<double> Fp, double *thrust_part) {
-  __shared__ double acc[4 * kWin64];
+    Geom g, TileGeom tg, PassFields F, Particles64 P, TileRun tr, PassConst kc,
+    double *thrust_part) {
+  using O = typename Off<UNIT>::T;
+  __shared__ double acc_mem[4 * kWin64];
   __shared__ Win sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
   const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
-  const double dx = kc.dx;
+  const double dx = UNIT ? 1.0 : kc.dx;
   if (tid == 0) {
     int64_t s, e;
     Win w;
@@ -443,11 +617,29 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
     if (THRUST && tid < 6) thrust_part[(int64_t)bid * 6 + tid] = 0.0;
     return;
   }
-  const Win w = sw;
+  // the window into scalar registers
+  Win w;
+  w.on = __builtin_amdgcn_readfirstlane(sw.on ? 1 : 0) != 0;
+  w.k0 = __builtin_amdgcn_readfirstlane(sw.k0);
+  w.l0 = __builtin_amdgcn_readfirstlane(sw.l0);
+  w.m0 = __builtin_amdgcn_readfirstlane(sw.m0);
+  w.WX = __builtin_amdgcn_readfirstlane(sw.WX);
+  w.WY = __builtin_amdgcn_readfirstlane(sw.WY);
+  w.WZ = __builtin_amdgcn_readfirstlane(sw.WZ);
+  w.vk0 = __builtin_amdgcn_readfirstlane(sw.vk0);
+  w.vk1 = __builtin_amdgcn_readfirstlane(sw.vk1);
+  w.vl0 = __builtin_amdgcn_readfirstlane(sw.vl0);
+  w.vl1 = __builtin_amdgcn_readfirstlane(sw.vl1);
+  w.vm0 = __builtin_amdgcn_readfirstlane(sw.vm0);
+  w.vm1 = __builtin_amdgcn_readfirstlane(sw.vm1);
   const int WN = w.on ? w.WX * w.WY * w.WZ : 0;
-  for (int i = tid; i < 4 * WN; i += blockDim.x) acc[(i / WN) * kWin64 + i % WN] = 0.0;
+  for (int i = tid; i < 4 * WN; i += blockDim.x) acc_mem[(i / WN) * kWin64 + i % WN] = 0.0;
   __syncthreads();
-  const double dth = kc.dt * 0.5;
+  char *acc = (char *)acc_mem;
+  const Walk64 wk = make_walk64(w.WY, w.WZ);
+  const int wsl = 8 * w.WZ, wsk = 8 * w.WY * w.WZ;  // window strides
+  const O fl = (O)g.SZ * 8, fk = (O)g.SY * g.SZ * 8;  // plane strides
+  const double dth = kc.dth;
   int64_t i0 = s + tid, i1 = e;
   int lanes = blockDim.x;
   if (ROWS && bid < tr.ntiles) {
@@ -458,89 +650,129 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
     i1 = re;
   }
   for (int64_t i = i0; i < i1; i += lanes) {
-    double z = P.z[i];
-    if (isnan(z)) continue;
-    double x = P.x[i], y = P.y[i];
-    double vx = P.vx[i], vy = P.vy[i], vz = P.vz[i];
-    const bool safe0 = in_array(g, x, y, z, dx);
-    const bool lds_ok =
-        safe0 && in_win(w, (int)(x / dx), (int)(y / dx), (int)(z / dx));
-    if (THRUST && safe0 && x < g.NX * dx * 0.8 && x > g.NX * dx * 0.2 &&
-        y < g.NY * dx * 0.8 && y > g.NY * dx * 0.2 && z < g.NZ * dx * 0.8 &&
-        z > g.NZ * dx * 0.2) {
-      double f[6];
-      gather(Fp, g, x, y, z, dx, f);
-      th[0] += f[0];
-      th[1] += f[1];
-      th[2] += f[2];
-      th[3] += vy * f[5] - vz * f[4];
-      th[4] += vz * f[3] - vx * f[5];
-      th[5] += vx * f[4] - vy * f[3];
+    const O pb = (O)i * 8;
+    double z = *at(P.z, pb);
+    if (isnan(z)) continue;  // dead until the next compaction
+    double x = *at(P.x, pb), y = *at(P.y, pb);
+    double vx = *at(P.vx, pb), vy = *at(P.vy, pb), vz = *at(P.vz, pb);
+    if (PUSH_J) {
+      const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx), Z = axis_weights(z, dx);
+      // in_array by the cells: x/dx < S-1 for the cell below S-1
+      const bool safe0 = x / dx > -0.5 && X.bi < g.SX - 1 && y / dx > -0.5 &&
+                         Y.bi < g.SY - 1 && z / dx > -0.5 && Z.bi < g.SZ - 1;
+      const bool push = safe0 && !(x < kc.blo[0] || x > kc.bhi[0] || y < kc.blo[1] ||
+                                   y > kc.bhi[1] || z < kc.blo[2] || z > kc.bhi[2]);
+      const bool box = THRUST && safe0 && x < kc.box_hi[0] && x > kc.box_lo[0] &&
+                       y < kc.box_hi[1] && y > kc.box_lo[1] && z < kc.box_hi[2] &&
+                       z > kc.box_lo[2];
+      if (push || box) {
+        const double inv_dx3 = 1. / (dx * dx * dx);
+        // byte offset of the cell's node and of one node down per axis
+        const O o = (((O)X.bi * g.SY + Y.bi) * g.SZ + Z.bi) * 8;
+        const O hx = X.bh != X.bi ? fk : 0, hy = Y.bh != Y.bi ? fl : 0,
+                hz = Z.bh != Z.bi ? 8 : 0;
+        const O ox = o - hx, oy = o - hy, oz = o - hz;
+        double f[6];
+        f[0] = gather1o<O>(F.e[0], oy - hz, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.hu, Z.hl) * inv_dx3;
+        f[1] = gather1o<O>(F.e[1], ox - hz, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+        f[2] = gather1o<O>(F.e[2], ox - hy, fl, fk, X.hu, X.hl, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+        if (THRUST && box) {
+          // the weights of x renamed: the compiler would otherwise form the
+          // node weights once for this gather and the push's and hold them
+          // across both
+          double xiu = X.iu, xil = X.il, xhu = X.hu, xhl = X.hl;
+          asm("" : "+v"(xiu), "+v"(xil), "+v"(xhu), "+v"(xhl));
+          const double bx = gather1o<O>(F.bp[0], ox, fl, fk, xhu, xhl, Y.iu, Y.il, Z.iu, Z.il) * inv_dx3;
+          const double by = gather1o<O>(F.bp[1], oy, fl, fk, xiu, xil, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+          const double bz = gather1o<O>(F.bp[2], oz, fl, fk, xiu, xil, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+          th[0] += f[0];
+          th[1] += f[1];
+          th[2] += f[2];
+          th[3] += vy * bz - vz * by;
+          th[4] += vz * bx - vx * bz;
+          th[5] += vx * by - vy * bx;
+        }
+        if (push) {
+          f[3] = gather1o<O>(F.b[0], ox, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.iu, Z.il) * inv_dx3;
+          f[4] = gather1o<O>(F.b[1], oy, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+          f[5] = gather1o<O>(F.b[2], oz, fl, fk, X.iu, X.il, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+          boris(kc, f, vx, vy, vz);
+        }
+      }
+      x += vx * kc.dt * 0.5;
+      y += vy * kc.dt * 0.5;
+      z += vz * kc.dt * 0.5;
     }
     if (PUSH_J) {
-      if (x < kc.blo[0] || x > kc.bhi[0] || y < kc.blo[1] || y > kc.bhi[1] ||
-          z < kc.blo[2] || z > kc.bhi[2] || !safe0) {
-        x += vx * dth;
-        y += vy * dth;
-        z += vz * dth;
-      } else {
-        double f[6];
-        gather(F, g, x, y, z, dx, f);
-        boris(kc, f, x, y, z, vx, vy, vz);
+      // shape_func_*0_j_2 (:3397-3553) with the reference's weights
+      const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx), Z = axis_weights(z, dx);
+      const bool dep = dep_ok(g, x, y, z, X.bi, Y.bi, Z.bi);
+      const bool in_lds = win_holds(w, X.bi, Y.bi, Z.bi);
+      const double qn = kc.qn;
+      if (dep && in_lds) {
+        const int c = win_byte(w, X.bi, Y.bi, Z.bi);
+        const int hx = X.bh != X.bi ? wsk : 0, hy = Y.bh != Y.bi ? wsl : 0,
+                  hz = Z.bh != Z.bi ? 8 : 0;
+        lds_dep8_64(acc + 0 * 8 * kWin64, c - hy - hz, wk, qn * vx, X.iu, X.il, Y.hu, Y.hl,
+                    Z.hu, Z.hl);
+        lds_dep8_64(acc + 1 * 8 * kWin64, c - hx - hz, wk, qn * vy, X.hu, X.hl, Y.iu, Y.il,
+                    Z.hu, Z.hl);
+        lds_dep8_64(acc + 2 * 8 * kWin64, c - hx - hy, wk, qn * vz, X.hu, X.hl, Y.hu, Y.hl,
+                    Z.iu, Z.il);
       }
-      if (in_gate(g, x, y, z, dx) && in_array(g, x, y, z, dx)) {
-        // shape_func_*0_j_2 (:3397-3553) with the reference's weights
-        const double qn = kc.q * kc.weight / (dx * dx * dx);
-        const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx),
-                    Z = axis_weights(z, dx);
-        dep8_64(acc + 0 * kWin64, jx, lds_ok, w, g, X.bi, Y.bh, Z.bh, X.iu,
-                X.il, Y.hu, Y.hl, Z.hu, Z.hl, qn * vx);
-        dep8_64(acc + 1 * kWin64, jy, lds_ok, w, g, X.bh, Y.bi, Z.bh, X.hu,
-                X.hl, Y.iu, Y.il, Z.hu, Z.hl, qn * vy);
-        dep8_64(acc + 2 * kWin64, jz, lds_ok, w, g, X.bh, Y.bh, Z.bi, X.hu,
-                X.hl, Y.hu, Y.hl, Z.iu, Z.il, qn * vz);
-      }
+      glob_coop64(g, dep && !in_lds, true, dx, x, y, z, qn * vx, qn * vy, qn * vz, F.jx, F.jy,
+                  F.jz, F.nd);
     }
     if (DRIFT_N) {
       x += vx * dth;
       y += vy * dth;
       z += vz * dth;
-      if (in_gate(g, x, y, z, dx) && in_array(g, x, y, z, dx)) {
-        // shape_func_*0_n_2 (:3333-3395)
-        const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx),
-                    Z = axis_weights(z, dx);
-        dep8_64(acc + 3 * kWin64, nd, lds_ok, w, g, X.bh, Y.bh, Z.bh, X.hu,
-                X.hl, Y.hu, Y.hl, Z.hu, Z.hl, kc.weight / (dx * dx * dx));
+      // shape_func_*0_n_2 (:3333-3395)
+      const AxisW X = axis_weights(x, dx), Y = axis_weights(y, dx), Z = axis_weights(z, dx);
+      const bool dep = dep_ok(g, x, y, z, X.bi, Y.bi, Z.bi);
+      const bool in_lds = win_holds(w, X.bi, Y.bi, Z.bi);
+      const double wn = kc.wn;
+      if (dep && in_lds) {
+        const int c = win_byte(w, X.bi, Y.bi, Z.bi) - (X.bh != X.bi ? wsk : 0) -
+                      (Y.bh != Y.bi ? wsl : 0) - (Z.bh != Z.bi ? 8 : 0);
+        lds_dep8_64(acc + 3 * 8 * kWin64, c, wk, wn, X.hu, X.hl, Y.hu, Y.hl, Z.hu, Z.hl);
       }
+      glob_coop64(g, dep && !in_lds, false, dx, x, y, z, wn, 0.0, 0.0, F.jx, F.jy, F.jz, F.nd);
     }
     if (BOUNDARY) {
-      const double dx2 = 2. * dx;
-      const double gx2 = (g.NX + 2) * dx, gy2 = (g.NY + 2) * dx,
-                   gz2 = (g.NZ + 2) * dx;
-      bool dead = !(z < gz2 && z >= dx2);
-      if (!dead) {
-        if (x >= gx2) {
-          if (kc.periodic[0]) x = x - g.NX * dx; else dead = true;
-        } else if (x < dx2) {
-          if (kc.periodic[0]) x = x + g.NX * dx; else dead = true;
-        }
-        if (y >= gy2) {
-          if (kc.periodic[1]) y = y - g.NY * dx; else dead = true;
-        } else if (y < dx2) {
-          if (kc.periodic[1]) y = y + g.NY * dx; else dead = true;
-        }
+      bool dead, xhi, xlo, yhi, ylo;
+      if (UNIT) {  // the upper faces by the cells: the same comparisons
+        dead = !(z >= 2.) || (int)z >= g.NZ + 2;
+        xhi = (int)x >= g.NX + 2;
+        xlo = x < 2.;
+        yhi = (int)y >= g.NY + 2;
+        ylo = y < 2.;
+      } else {
+        const double dx2 = 2. * dx;
+        dead = !(z < (g.NZ + 2) * dx && z >= dx2);
+        xhi = x >= (g.NX + 2) * dx;
+        xlo = x < dx2;
+        yhi = y >= (g.NY + 2) * dx;
+        ylo = y < dx2;
       }
+      dead = dead || ((xhi || xlo) && !kc.periodic[0]) || ((yhi || ylo) && !kc.periodic[1]);
+      if (xhi) x = x - g.NX * dx;
+      else if (xlo) x = x + g.NX * dx;
+      if (yhi) y = y - g.NY * dx;
+      else if (ylo) y = y + g.NY * dx;
       if (dead) {
-        P.z[i] = __longlong_as_double(0x7ff8000000000000LL);
+        *at(P.z, pb) = __longlong_as_double(0x7ff8000000000000LL);
         continue;
       }
     }
-    P.x[i] = x;
-    P.y[i] = y;
-    P.z[i] = z;
-    P.vx[i] = vx;
-    P.vy[i] = vy;
-    P.vz[i] = vz;
+    *at(P.x, pb) = x;
+    *at(P.y, pb) = y;
+    *at(P.z, pb) = z;
+    if (PUSH_J) {
+      *at(P.vx, pb) = vx;
+      *at(P.vy, pb) = vy;
+      *at(P.vz, pb) = vz;
+    }
   }
   if (THRUST) thrust_store64(th, thrust_part, bid);
   if (!w.on) return;
@@ -548,9 +780,11 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
   const int WYZ = w.WY * w.WZ;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    double *dst = c == 0 ? jx : c == 1 ? jy : c == 2 ? jz : nd;
+    if (!PUSH_J && c < 3) continue;
+    if (!DRIFT_N && c == 3) continue;
+    double *dst = c == 0 ? F.jx : c == 1 ? F.jy : c == 2 ? F.jz : F.nd;
     for (int j = tid; j < WN; j += blockDim.x) {
-      const double v = acc[c * kWin64 + j];
+      const double v = acc_mem[c * kWin64 + j];
       if (v == 0.0) continue;
       const int kk = w.k0 + j / WYZ, ll = w.l0 + (j / w.WZ) % w.WY,
                 mm = w.m0 + j % w.WZ;
@@ -887,12 +1121,46 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   if (n == 0) return 0;
   Fields<double> F = fields<double>(ctx);
   Particles64 P = p64(ctx, sp, ctx->cur[sp]);
-  StepConst kc = step_const(ctx, sp);
-  double *jx = F.f[sp == PIC_ION ? PIC_JIX : PIC_JEX];
-  double *jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
-  double *jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
-  double *nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
+  const StepConst sc = step_const(ctx, sp);
+  PassConst kc;
+  {
+    const double dx = sc.dx;
+    kc.dx = dx;
+    kc.dt = sc.dt;
+    kc.dth = sc.dt * 0.5;
+    kc.c = sc.c;
+    kc.cc = sc.c * sc.c;
+    kc.T = 0.5 * sc.q * sc.dt / sc.mass;
+    kc.TT = kc.T * kc.T;
+    kc.T2 = 2. * kc.T;
+    kc.eimf_x = sc.vdrift_z * sc.imf_y;
+    kc.eimf_y = -sc.vdrift_z * sc.imf_x;
+    kc.qn = sc.q * sc.weight / (dx * dx * dx);
+    kc.wn = sc.weight / (dx * dx * dx);
+    const int N[3] = {ctx->geom.NX, ctx->geom.NY, ctx->geom.NZ};
+    for (int a = 0; a < 3; ++a) {
+      kc.blo[a] = sc.blo[a];
+      kc.bhi[a] = sc.bhi[a];
+      kc.box_lo[a] = N[a] * dx * 0.2;
+      kc.box_hi[a] = N[a] * dx * 0.8;
+    }
+    kc.periodic[0] = sc.periodic[0];
+    kc.periodic[1] = sc.periodic[1];
+  }
+  PassFields pf;
+  const double *kept = (const double *)ctx->thrust_bprev;
+  for (int q = 0; q < 3; ++q) {
+    pf.e[q] = F.f[PIC_EX + q];
+    pf.b[q] = F.f[PIC_BX + q];
+    pf.bp[q] = kept + q * ctx->geom.plane;
+  }
+  pf.jx = F.f[sp == PIC_ION ? PIC_JIX : PIC_JEX];
+  pf.jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
+  pf.jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
+  pf.nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
   TileGeom tg = tile_geom(ctx);
+  add_drift_shift(tg, ctx->cfg, ctx->drift_halves[sp]);
+  ctx->drift_halves[sp] += (do_push_j ? 1 : 0) + (do_drift_n ? 1 : 0);
   TileRun tr;
   tr.tile_start = ctx->tile_start[sp];
   tr.sorted_end = ctx->sorted_end[sp];
@@ -917,24 +1185,31 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
   // the fused pass of pic_step adds the previous step's thrust_fave
   const bool thrust = ctx->thrust_now && sel == 7;
-  Fields<double> Fp = F;
   double *tp = nullptr;
   if (thrust) {
     if ((int64_t)nb > ctx->thrust_part_slots)
       return set_error(ctx, PIC_E_CAPACITY, "thrust: %u workgroups, %lld partial slots",
                        nb, (long long)ctx->thrust_part_slots);
-    const double *bp = (const double *)ctx->thrust_bprev;
-    for (int q = 0; q < 3; ++q) Fp.f[PIC_BX + q] = (double *)bp + q * ctx->geom.plane;
     tp = ctx->thrust_part;
   }
-#define LAUNCH(A, B, C, T)                                                  \
-  do {                                                                      \
-    if (rows)                                                               \
-      k_particles_tiled<A, B, C, T, true><<<nb, kBlock, 0, ctx->stream>>>(  \
-          ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp);             \
-    else                                                                    \
-      k_particles_tiled<A, B, C, T, false><<<nb, kBlock, 0, ctx->stream>>>( \
-          ctx->geom, tg, F, P, tr, kc, jx, jy, jz, nd, Fp, tp);             \
+  // normalised units with 32-bit byte offsets, or any dx with 64-bit ones
+  const bool unit = ctx->cfg.dx == 1.0 && n < ((int64_t)1 << 29) &&
+                    ctx->geom.plane < ((int64_t)1 << 29);
+#define LAUNCH2(A, B, C, T, R)                                                   \
+  do {                                                                           \
+    if (unit)                                                                    \
+      k_particles_tiled<A, B, C, T, R, true><<<nb, kBlock, 0, ctx->stream>>>(    \
+          ctx->geom, tg, pf, P, tr, kc, tp);                                     \
+    else                                                                         \
+      k_particles_tiled<A, B, C, T, R, false><<<nb, kBlock, 0, ctx->stream>>>(   \
+          ctx->geom, tg, pf, P, tr, kc, tp);                                     \
+  } while (0)
+#define LAUNCH(A, B, C, T)                                                       \
+  do {                                                                           \
+    if (rows)                                                                    \
+      LAUNCH2(A, B, C, T, true);                                                 \
+    else                                                                         \
+      LAUNCH2(A, B, C, T, false);                                                \
   } while (0)
   switch (thrust ? 8 : sel) {
     case 8: LAUNCH(true, true, true, true); break;
@@ -944,6 +1219,7 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     case 1: LAUNCH(false, false, true, false); break;
     default: return set_error(ctx, PIC_E_ARG, "particle pass %d", sel);
   }
+#undef LAUNCH2
 #undef LAUNCH
   PIC_LAUNCH_CHECK(ctx);
   if (thrust) {
@@ -1060,6 +1336,7 @@ void tsort_free(pic_ctx *ctx) {
 int sort(pic_ctx *ctx, int sp) {
   const Geom &g = ctx->geom;
   const int64_t n = ctx->n[sp];
+  ctx->drift_halves[sp] = 0;
   if (n == 0) return 0;
   Particles64 src = p64(ctx, sp, ctx->cur[sp]);
   const TileGeom tg = tile_geom(ctx);

@@ -175,9 +175,4 @@ __device__ inline void tile_setup(int bid, const TileRun &tr, const TileGeom &tg
   }
 }
 
-__device__ inline bool in_win(const Win &w, int k, int l, int m) {
-  return w.on && k >= w.vk0 && k <= w.vk1 && l >= w.vl0 && l <= w.vl1 &&
-         m >= w.vm0 && m <= w.vm1;
-}
-
 }  // namespace pic

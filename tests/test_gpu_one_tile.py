@@ -6,6 +6,7 @@ import pytest
 
 import plasmasim_amd as ps
 from helpers import rel_l2
+from oracle_lib import Oracle
 
 pytestmark = pytest.mark.gpu
 FIELDS = ["ex", "ey", "ez", "bx", "by", "bz", "jix", "jiy", "jiz", "jex", "jey", "jez", "ni",
@@ -78,3 +79,30 @@ def test_one_tile_resumes_without_cell_starts(tmp_path):
     b.step(3)
     for k in FIELDS:
         assert np.array_equal(a.download_field(k), b.download_field(k)), k
+
+
+@pytest.mark.parametrize("dx", [1.0, 0.75])
+@pytest.mark.parametrize("tile", [(0, 0, 0), (4, 4, 8)])
+def test_fp64_pass_in_other_units(dx, tile):
+    """FP64 pass in normalised units and with dx away from 1 (its own
+    instantiation) against the oracle, inflow and sort between: 15 steps of
+    sums in another order."""
+    c = ps.preset(1)
+    c.nx, c.ny, c.nz = 16, 12, 24
+    c.ppc = 6
+    c.dx, c.dt = dx, c.dt * dx
+    c.absorb[2] = 3
+    c.ballistic_lo[2], c.ballistic_hi[2] = 7.0 * dx, (c.nz - 3.0) * dx
+    c.inflow_every, c.sort_every = 4, 6
+    for a in range(3):
+        c.tile[a] = tile[a]
+    g, o = ps.Simulation(c), Oracle(c)
+    for s in (g, o):
+        s.load_particles()
+    for s in (g, o):
+        s.begin()
+        s.step(15)
+    for k in FIELDS:
+        assert rel_l2(g.download_field(k), o.download_field(k)) <= 1e-12, k
+    for sp in (0, 1):
+        assert g.particle_count(sp) == o.particle_count(sp)
