@@ -7,6 +7,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include "pic_fused.h"
 #include "pic_internal.h"
 #include "pic_tiles.h"
 
@@ -836,25 +837,6 @@ namespace pic {
 // ---------------------------------------------------------------------------
 // thrust_fave (:5124-5285) accumulated over pic_step's steps
 
-// acc[q] += qn * (sum over the nb workgroups' partials of quantity q), the
-// workgroups summed in a fixed order
-constexpr int kFinish = 1024;
-__global__ __launch_bounds__(kFinish) void k_thrust_finish(const double *__restrict__ part,
-                                                           int nb, double qn, double *acc) {
-  __shared__ double sh[6][kFinish];
-  double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int b = threadIdx.x; b < nb; b += kFinish)
-    for (int q = 0; q < 6; ++q) v[q] += part[(int64_t)b * 6 + q];
-  for (int q = 0; q < 6; ++q) sh[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int st = kFinish / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st)
-      for (int q = 0; q < 6; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x < 6) acc[threadIdx.x] += qn * sh[threadIdx.x][0];
-}
-
 // the force parts of the diagnostics partials (particle quantities 8..13,
 // already multiplied by q_s w dx^3) of both species added to acc
 __global__ __launch_bounds__(64) void k_thrust_from_diag(const double *__restrict__ pf,
@@ -874,11 +856,17 @@ __global__ void k_fill_zero(double *p, int n) {
   if (i < n) p[i] = 0.0;
 }
 
-int thrust_add(pic_ctx *ctx, int sp, int nb, double qn) {
-  k_thrust_finish<<<1, kFinish, 0, ctx->stream>>>(ctx->thrust_part, nb, qn,
-                                                  ctx->thrust_acc + 6 * sp);
-  PIC_LAUNCH_CHECK(ctx);
-  return 0;
+ThrustFinish thrust_finish_args(const pic_ctx *ctx) {
+  const pic_config &c = ctx->cfg;
+  ThrustFinish f;
+  for (int sp = 0; sp < 2; ++sp) {
+    f.part[sp] = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
+    f.nb[sp] = ctx->thrust_nb[sp];
+    const double qs = sp == PIC_ION ? c.q : -c.q;
+    f.qn[sp] = qs * c.weight[sp] * c.dx * c.dx * c.dx;
+  }
+  f.acc = ctx->thrust_acc;
+  return f;
 }
 
 // the pending force from the current state, by the diagnostics' own particle
@@ -892,23 +880,6 @@ static int thrust_settle(pic_ctx *ctx) {
   PIC_LAUNCH_CHECK(ctx);
   ctx->thrust_pending = 0;
   ctx->thrust_steps++;
-  return 0;
-}
-
-// keep the end-of-step total B for the fused force of the next pass: the
-// FP64 B planes into thrust_bprev, the FP32 form's total-B planes into the
-// upper half of their own 6-plane block
-static int thrust_keep_b(pic_ctx *ctx) {
-  const int64_t pl = ctx->geom.plane;
-  if (is_f64(ctx)) {
-    PIC_HIP(ctx, hipMemcpyAsync(ctx->thrust_bprev, fields<double>(ctx).f[PIC_BX],
-                                3 * pl * sizeof(double), hipMemcpyDeviceToDevice,
-                                ctx->stream));
-  } else {
-    float *bt = f32::total_b(ctx);
-    PIC_HIP(ctx, hipMemcpyAsync(bt + 3 * pl, bt, 3 * pl * sizeof(float),
-                                hipMemcpyDeviceToDevice, ctx->stream));
-  }
   return 0;
 }
 
@@ -935,7 +906,7 @@ extern "C" int pic_thrust_ave_enable(pic_ctx *ctx, int on) {
     if (ctx->thrust_part) (void)hipFree(ctx->thrust_part);
     ctx->thrust_part = nullptr;
     ctx->thrust_part_slots = 0;
-    PIC_HIP(ctx, hipMalloc(&ctx->thrust_part, (size_t)slots * 6 * sizeof(double)));
+    PIC_HIP(ctx, hipMalloc(&ctx->thrust_part, (size_t)slots * 12 * sizeof(double)));
     ctx->thrust_part_slots = slots;
   }
   if (is_f64(ctx) && !ctx->thrust_bprev)
@@ -1025,8 +996,15 @@ extern "C" int pic_step(pic_ctx *ctx, int nsteps) {
     }
     return 0;
   };
+  // a field launch of the step, timed
+#define FIELD(cls, fn, ...)                          \
+  do {                                               \
+    timing_begin(ctx, cls);                          \
+    rc = DISPATCH(fn, __VA_ARGS__);                  \
+    timing_end(ctx, cls);                            \
+    TRY(rc);                                         \
+  } while (0)
   for (int s = 0; s < nsteps; ++s) {
-    TRY(pic_renew_grid(ctx));
     const bool sort_due = ctx->c_sort > c.sort_every - 1;
     const bool add_due = ctx->c_add > c.inflow_every - 1;
     const bool inflow_first = !f64 && sort_due && add_due;
@@ -1039,12 +1017,12 @@ extern "C" int pic_step(pic_ctx *ctx, int nsteps) {
       ctx->c_add = 0;
     }
     if (inflow_first) TRY(sort_both());
-    if (ctx->thrust_pending) {
-      TRY(thrust_keep_b(ctx));
-      ctx->thrust_now = 1;
-    }
-    TRY(pic_renew_b_half(ctx));
-    TRY(pic_halo_b(ctx));
+    // renew_grid zeroes phi (:2552); the deposits are zeroed with the first
+    // B half step, nothing before it reads them
+    if (ctx->phi) TRY(poisson_zero_phi(ctx));
+    FIELD(PIC_T_FIELD_B, step_b1, ctx, ctx->thrust_pending != 0);
+    ctx->thrust_now = ctx->thrust_pending;
+    ctx->thrust_nb[0] = ctx->thrust_nb[1] = 0;
     for (int sp = 0; sp < 2; ++sp) {
       const int tclass = !f64 && f32::pending(ctx, sp) ? PIC_T_PUSH_SORT : PIC_T_PUSH;
       timing_begin(ctx, tclass);
@@ -1056,16 +1034,16 @@ extern "C" int pic_step(pic_ctx *ctx, int nsteps) {
         return rc;
       }
     }
+    timing_begin(ctx, PIC_T_FIELD_B);
+    rc = DISPATCH(step_b2, ctx);
+    timing_end(ctx, PIC_T_FIELD_B);
     if (ctx->thrust_now) {
       ctx->thrust_now = 0;
       ctx->thrust_pending = 0;
       ctx->thrust_steps++;
     }
-    TRY(pic_renew_b_half(ctx));
-    TRY(pic_halo_b(ctx));
-    TRY(pic_fold_current(ctx));
-    TRY(pic_renew_e(ctx));
-    TRY(pic_halo_e(ctx));
+    TRY(rc);
+    FIELD(PIC_T_FIELD_E, step_e, ctx);
     if (c.poisson_every > 0 && ctx->step % c.poisson_every == 0)
       TRY(pic_poisson(ctx));  // PHI(renew_phi3; sr_phi; sr_e) :901-906
     ctx->c_sort++;
@@ -1073,6 +1051,7 @@ extern "C" int pic_step(pic_ctx *ctx, int nsteps) {
     ctx->step++;
     if (ctx->thrust_on) ctx->thrust_pending = 1;
   }
+#undef FIELD
 #undef TRY
   return 0;
 }

@@ -30,6 +30,7 @@
 #include <algorithm>
 
 #include "philox.h"
+#include "pic_fused.h"
 #include "pic_internal.h"
 #include "pic_tiles.h"
 #include "pic_tsort.h"
@@ -854,85 +855,101 @@ __device__ inline float sigma32(const Sigma32 &s, int k2, int l2, int m2) {
   return s.amp * (0.1f * sqrtf(a4) + 0.01f * sqrtf(a12));
 }
 
-// renew_b4_2 (:2580-2611) on B1: B1 <- f B1 - h (27 D1 - D3)/24/dx; the
-// total field B0 + B1 used by the gather is written alongside
-__global__ __launch_bounds__(256) void k_renew_b32(Geom g, Fields<float> F,
-                                                   float *bt, Sigma32 sg,
-                                                   float dt, float dx,
-                                                   float eps0) {
-  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
-  const int k = 2 + blockIdx.z;
-  if (m >= g.NZ + 2 || l >= g.NY + 2) return;
-  const float temp = 0.25f * dt / eps0, dth = 0.5f * dt;
-  const float c24 = 1.0f / (24.0f * dx);
-  const int64_t c = g.idx(k, l, m);
+// renew_b4_2 (:2580-2611) on B1 at interior cell c: B1 <- f B1 -
+// h (27 D1 - D3)/24/dx
+struct FieldConst {
+  float dt, dx, eps0, mu0, c;
+};
+
+__device__ inline void renew_b_cell(const Geom &g, const Fields<float> &F, const Sigma32 &sg,
+                                    const FieldConst &fc, int k, int l, int m, int64_t c,
+                                    float out[3]) {
+  const float temp = 0.25f * fc.dt / fc.eps0, dth = 0.5f * fc.dt;
+  const float c24 = 1.0f / (24.0f * fc.dx);
   const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
   const float *ex = F.f[PIC_EX], *ey = F.f[PIC_EY], *ez = F.f[PIC_EZ];
   float s, f, h;
   s = sigma32(sg, 2 * k + 1, 2 * l, 2 * m);
   f = s == 0.0f ? 1.0f : (1.f - s * temp) / (1.f + s * temp);
   h = s == 0.0f ? dth : dth / (1.f + s * temp);
-  const int64_t pl = g.plane;
-  float b1 = f * F.f[PIC_BX][c] -
-             h * c24 * (27.f * (ez[c] - ez[c - dl] - ey[c] + ey[c - 1]) -
-                        (ez[c + dl] - ez[c - 2 * dl] - ey[c + 1] + ey[c - 2]));
-  F.f[PIC_BX][c] = b1;
-  bt[c] = F.f[PIC_B0X][c] + b1;
+  out[0] = f * F.f[PIC_BX][c] -
+           h * c24 * (27.f * (ez[c] - ez[c - dl] - ey[c] + ey[c - 1]) -
+                      (ez[c + dl] - ez[c - 2 * dl] - ey[c + 1] + ey[c - 2]));
   s = sigma32(sg, 2 * k, 2 * l + 1, 2 * m);
   f = s == 0.0f ? 1.0f : (1.f - s * temp) / (1.f + s * temp);
   h = s == 0.0f ? dth : dth / (1.f + s * temp);
-  b1 = f * F.f[PIC_BY][c] -
-       h * c24 * (27.f * (ex[c] - ex[c - 1] - ez[c] + ez[c - dk]) -
-                  (ex[c + 1] - ex[c - 2] - ez[c + dk] + ez[c - 2 * dk]));
-  F.f[PIC_BY][c] = b1;
-  bt[pl + c] = F.f[PIC_B0Y][c] + b1;
+  out[1] = f * F.f[PIC_BY][c] -
+           h * c24 * (27.f * (ex[c] - ex[c - 1] - ez[c] + ez[c - dk]) -
+                      (ex[c + 1] - ex[c - 2] - ez[c + dk] + ez[c - 2 * dk]));
   s = sigma32(sg, 2 * k, 2 * l, 2 * m + 1);
   f = s == 0.0f ? 1.0f : (1.f - s * temp) / (1.f + s * temp);
   h = s == 0.0f ? dth : dth / (1.f + s * temp);
-  b1 = f * F.f[PIC_BZ][c] -
-       h * c24 * (27.f * (ey[c] - ey[c - dk] - ex[c] + ex[c - dl]) -
-                  (ey[c + dk] - ey[c - 2 * dk] - ex[c + dl] + ex[c - 2 * dl]));
-  F.f[PIC_BZ][c] = b1;
-  bt[2 * pl + c] = F.f[PIC_B0Z][c] + b1;
+  out[2] = f * F.f[PIC_BZ][c] -
+           h * c24 * (27.f * (ey[c] - ey[c - dk] - ex[c] + ex[c - dl]) -
+                      (ey[c + dk] - ey[c - 2 * dk] - ex[c + dl] + ex[c - 2 * dl]));
 }
 
-// renew_e4_2 (:2613-2652) with the curl of B1
-__global__ __launch_bounds__(256) void k_renew_e32(Geom g, Fields<float> F,
-                                                   Sigma32 sg, float dt,
-                                                   float dx, float c_light,
-                                                   float mu0) {
+// the total field B0 + B1 used by the gather is written alongside
+__global__ __launch_bounds__(256) void k_renew_b32(Geom g, Fields<float> F,
+                                                   float *bt, Sigma32 sg,
+                                                   FieldConst fc) {
   const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
   const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
   const int k = 2 + blockIdx.z;
   if (m >= g.NZ + 2 || l >= g.NY + 2) return;
-  const float temp = c_light * c_light * dt;
-  const float c24 = 1.0f / (24.0f * dx);
   const int64_t c = g.idx(k, l, m);
+  float b1[3];
+  renew_b_cell(g, F, sg, fc, k, l, m, c, b1);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    F.f[PIC_BX + q][c] = b1[q];
+    bt[q * g.plane + c] = F.f[PIC_B0X + q][c] + b1[q];
+  }
+}
+
+// renew_e4_2 (:2613-2652) with the curl of B1, at interior cell c
+__device__ inline void renew_e_cell(const Geom &g, const Fields<float> &F, const Sigma32 &sg,
+                                    const FieldConst &fc, int k, int l, int m, int64_t c,
+                                    float out[3]) {
+  const float temp = fc.c * fc.c * fc.dt;
+  const float c24 = 1.0f / (24.0f * fc.dx);
   const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
   const float *bx = F.f[PIC_BX], *by = F.f[PIC_BY], *bz = F.f[PIC_BZ];
   float s, f, h;
   s = sigma32(sg, 2 * k, 2 * l + 1, 2 * m + 1);
-  f = s == 0.0f ? 1.0f : (1.f - 0.5f * mu0 * s * temp) / (1.f + 0.5f * mu0 * s * temp);
-  h = s == 0.0f ? temp : temp / (1.f + 0.5f * mu0 * s * temp);
-  F.f[PIC_EX][c] = f * F.f[PIC_EX][c] +
+  f = s == 0.0f ? 1.0f : (1.f - 0.5f * fc.mu0 * s * temp) / (1.f + 0.5f * fc.mu0 * s * temp);
+  h = s == 0.0f ? temp : temp / (1.f + 0.5f * fc.mu0 * s * temp);
+  out[0] = f * F.f[PIC_EX][c] +
                    h * (c24 * (27.f * ((bz[c + dl] - bz[c]) - (by[c + 1] - by[c])) -
                                ((bz[c + 2 * dl] - bz[c - dl]) - (by[c + 2] - by[c - 1]))) -
-                        mu0 * (F.f[PIC_JIX][c] - F.f[PIC_JEX][c]));
+                        fc.mu0 * (F.f[PIC_JIX][c] - F.f[PIC_JEX][c]));
   s = sigma32(sg, 2 * k + 1, 2 * l, 2 * m + 1);
-  f = s == 0.0f ? 1.0f : (1.f - 0.5f * mu0 * s * temp) / (1.f + 0.5f * mu0 * s * temp);
-  h = s == 0.0f ? temp : temp / (1.f + 0.5f * mu0 * s * temp);
-  F.f[PIC_EY][c] = f * F.f[PIC_EY][c] +
+  f = s == 0.0f ? 1.0f : (1.f - 0.5f * fc.mu0 * s * temp) / (1.f + 0.5f * fc.mu0 * s * temp);
+  h = s == 0.0f ? temp : temp / (1.f + 0.5f * fc.mu0 * s * temp);
+  out[1] = f * F.f[PIC_EY][c] +
                    h * (c24 * (27.f * ((bx[c + 1] - bx[c]) - (bz[c + dk] - bz[c])) -
                                ((bx[c + 2] - bx[c - 1]) - (bz[c + 2 * dk] - bz[c - dk]))) -
-                        mu0 * (F.f[PIC_JIY][c] - F.f[PIC_JEY][c]));
+                        fc.mu0 * (F.f[PIC_JIY][c] - F.f[PIC_JEY][c]));
   s = sigma32(sg, 2 * k + 1, 2 * l + 1, 2 * m);
-  f = s == 0.0f ? 1.0f : (1.f - 0.5f * mu0 * s * temp) / (1.f + 0.5f * mu0 * s * temp);
-  h = s == 0.0f ? temp : temp / (1.f + 0.5f * mu0 * s * temp);
-  F.f[PIC_EZ][c] = f * F.f[PIC_EZ][c] +
+  f = s == 0.0f ? 1.0f : (1.f - 0.5f * fc.mu0 * s * temp) / (1.f + 0.5f * fc.mu0 * s * temp);
+  h = s == 0.0f ? temp : temp / (1.f + 0.5f * fc.mu0 * s * temp);
+  out[2] = f * F.f[PIC_EZ][c] +
                    h * (c24 * (27.f * ((by[c + dk] - by[c]) - (bx[c + dl] - bx[c])) -
                                ((by[c + 2 * dk] - by[c - dk]) - (bx[c + 2 * dl] - bx[c - dl]))) -
-                        mu0 * (F.f[PIC_JIZ][c] - F.f[PIC_JEZ][c]));
+                        fc.mu0 * (F.f[PIC_JIZ][c] - F.f[PIC_JEZ][c]));
+}
+
+__global__ __launch_bounds__(256) void k_renew_e32(Geom g, Fields<float> F, Sigma32 sg,
+                                                   FieldConst fc) {
+  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
+  const int k = 2 + blockIdx.z;
+  if (m >= g.NZ + 2 || l >= g.NY + 2) return;
+  const int64_t c = g.idx(k, l, m);
+  float e[3];
+  renew_e_cell(g, F, sg, fc, k, l, m, c, e);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) F.f[PIC_EX + q][c] = e[q];
 }
 
 // sr_b / sr_e on one rank: the reference copies the total field into the
@@ -1035,6 +1052,129 @@ __global__ void k_fx_to_f32(const unsigned long long *__restrict__ a, float *b,
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (; i < n; i += stride) b[i] = (float)((double)(long long)a[i] * inv_scale);
+}
+
+// ---------------------------------------------------------------------------
+// the step's field launches (pic_fused.h)
+
+// B half step and sr_b of cell (k, l, m); kept: the end-of-step total B goes
+// to the upper half of the bt block first
+template <bool KEEP>
+__device__ inline void b_and_guards(const Geom &g, const Fields<float> &F, float *bt,
+                                    const Sigma32 &sg, const FieldConst &fc, int k, int l,
+                                    int m) {
+  const int64_t c = g.idx(k, l, m), pl = g.plane;
+  const bool in = m >= 2 && m < g.NZ + 2;
+  float b1[3];
+  if (in) renew_b_cell(g, F, sg, fc, k, l, m, c, b1);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    float *B = F.f[PIC_BX + q], *t = bt + q * pl;
+    const float *B0 = F.f[PIC_B0X + q];
+    const float b0 = B0[c], old = t[c];
+    const float b = in ? b1[q] : B[c], tot = in ? b0 + b1[q] : old;
+    if (KEEP) t[3 * pl + c] = old;
+    if (in) {
+      B[c] = b;
+      t[c] = tot;
+    }
+    // a guard's B1 is B1(src) + B0(src) - B0(guard); the corner continues
+    // from the x image
+    float v0 = b, p0 = b0, v1 = 0.0f, p1 = 0.0f;
+    bool first = true;
+    images(g, k, l, c, [&](int64_t d, int64_t s) {
+      const float bd = B0[d];
+      const float v = s == c ? v0 + (p0 - bd) : v1 + (p1 - bd);
+      if (first) {  // the x image, where there is one (a corner needs it)
+        v1 = v;
+        p1 = bd;
+        first = false;
+      }
+      if (KEEP) t[3 * pl + d] = t[d];
+      B[d] = v;
+      t[d] = tot;
+    });
+  }
+}
+
+// renew_grid, thrust_fave's copy of the total B, the first B half step, sr_b
+template <bool DET, bool KEEP>
+__global__ __launch_bounds__(256) void k_step_b1(Geom g, CellBlocks cb, Fields<float> F,
+                                                 unsigned long long *fx, float *bt,
+                                                 Sigma32 sg, FieldConst fc) {
+  int k, l, m;
+  if (!cb.cell(g, blockIdx.x, k, l, m)) return;
+  const int64_t c = g.idx(k, l, m);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    if (DET)
+      fx[q * g.plane + c] = 0ull;
+    else
+      F.f[PIC_JIX + q][c] = 0.0f;
+  }
+  if (interior_column(g, k, l)) b_and_guards<KEEP>(g, F, bt, sg, fc, k, l, m);
+}
+
+// The second B half step and sr_b; sr_current2 (DET: from the fixed-point
+// planes, with the conversion of every deposit); thrust_fave's sums.  Blocks
+// below tb finish the thrust, then fb blocks fold, the rest are cells.
+template <bool DET>
+__global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<float> F,
+                                                 const unsigned long long *__restrict__ fx,
+                                                 double inv_s, float *bt, Sigma32 sg,
+                                                 FieldConst fc, int tb, ThrustFinish tf,
+                                                 int fb) {
+  int b = blockIdx.x;
+  if (b < tb) {
+    thrust_finish(tf, b);
+    return;
+  }
+  b -= tb;
+  const auto conv = [&](int q, int64_t i) {
+    return (float)((double)(long long)fx[q * g.plane + i] * inv_s);
+  };
+  if (b < fb) {
+    const int64_t t = (int64_t)b * 256 + threadIdx.x;
+    if (t >= (int64_t)fold_groups(g) * g.SZ) return;
+    const int m = (int)(t % g.SZ), grp = (int)(t / g.SZ);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      float *f = F.f[PIC_JIX + q];
+      fold_group(
+          g, grp, m, [&](int64_t i) { return DET ? conv(q, i) : f[i]; },
+          [&](int64_t i, float v, bool changed) {
+            if (DET || changed) f[i] = v;
+          });
+    }
+    return;
+  }
+  b -= fb;
+  int k, l, m;
+  if (!cb.cell(g, b, k, l, m)) return;
+  if (DET && unfolded_column(g, k, l)) {
+    const int64_t c = g.idx(k, l, m);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) F.f[PIC_JIX + q][c] = conv(q, c);
+  }
+  if (interior_column(g, k, l)) b_and_guards<false>(g, F, bt, sg, fc, k, l, m);
+}
+
+// the E step and sr_e
+__global__ __launch_bounds__(256) void k_step_e(Geom g, CellBlocks cb, Fields<float> F,
+                                                Sigma32 sg, FieldConst fc) {
+  int k, l, m;
+  if (!cb.cell(g, blockIdx.x, k, l, m) || !interior_column(g, k, l)) return;
+  const int64_t c = g.idx(k, l, m);
+  const bool in = m >= 2 && m < g.NZ + 2;
+  float e[3];
+  if (in) renew_e_cell(g, F, sg, fc, k, l, m, c, e);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    float *E = F.f[PIC_EX + q];
+    const float v = in ? e[q] : E[c];
+    if (in) E[c] = v;
+    images(g, k, l, c, [&](int64_t d, int64_t) { E[d] = v; });
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1664,22 +1804,23 @@ int finish_deposit(pic_ctx *ctx) {
   return 0;
 }
 
-int renew_b_half(pic_ctx *ctx) {
+static FieldConst field_const(const pic_ctx *ctx) {
   const pic_config &c = ctx->cfg;
+  return FieldConst{(float)c.dt, (float)c.dx, (float)c.eps0, (float)c.mu0, (float)c.c};
+}
+
+int renew_b_half(pic_ctx *ctx) {
   dim3 b, gr = interior_grid(ctx->geom, b);
   k_renew_b32<<<gr, b, 0, ctx->stream>>>(ctx->geom, fields<float>(ctx),
-                                         st(ctx)->bt, sigma_f(ctx), (float)c.dt,
-                                         (float)c.dx, (float)c.eps0);
+                                         st(ctx)->bt, sigma_f(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
 
 int renew_e(pic_ctx *ctx) {
-  const pic_config &c = ctx->cfg;
   dim3 b, gr = interior_grid(ctx->geom, b);
   k_renew_e32<<<gr, b, 0, ctx->stream>>>(ctx->geom, fields<float>(ctx),
-                                         sigma_f(ctx), (float)c.dt,
-                                         (float)c.dx, (float)c.c, (float)c.mu0);
+                                         sigma_f(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1696,6 +1837,43 @@ int halo(pic_ctx *ctx, int first) {
                ctx->stream>>>(g, a, b, c, a0, b0, c0, bt);
   k_halo_y32<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
                ctx->stream>>>(g, a, b, c, a0, b0, c0, bt);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+int step_b1(pic_ctx *ctx, bool keep_b) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  State32 *S = st(ctx);
+  const auto kern = S->fx ? (keep_b ? k_step_b1<true, true> : k_step_b1<true, false>)
+                          : (keep_b ? k_step_b1<false, true> : k_step_b1<false, false>);
+  kern<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<float>(ctx), S->fx, S->bt, sigma_f(ctx), field_const(ctx));
+  PIC_LAUNCH_CHECK(ctx);
+  S->fx_dirty = false;
+  return 0;
+}
+
+int step_b2(pic_ctx *ctx) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  State32 *S = st(ctx);
+  const int tb = ctx->thrust_now ? 12 : 0;
+  const int fb = (int)div_up((int64_t)fold_groups(g) * g.SZ, kBlock);
+  const auto kern = S->fx ? k_step_b2<true> : k_step_b2<false>;
+  kern<<<(unsigned)(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<float>(ctx), S->fx, 1.0 / S->fx_scale, S->bt, sigma_f(ctx),
+      field_const(ctx), tb, thrust_finish_args(ctx), fb);
+  PIC_LAUNCH_CHECK(ctx);
+  S->fx_dirty = false;
+  return 0;
+}
+
+int step_e(pic_ctx *ctx) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  k_step_e<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<float>(ctx), sigma_f(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1837,7 +2015,7 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     if ((int64_t)nb > ctx->thrust_part_slots)
       return set_error(ctx, PIC_E_CAPACITY, "thrust: %u workgroups, %lld partial slots",
                        nb, (long long)ctx->thrust_part_slots);
-    tp = ctx->thrust_part;
+    tp = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
     // the kept end-of-step B is the upper half of the 6-plane bt block
     kp.bprev = (uint32_t)(3 * ctx->geom.plane * sizeof(float));
     // farthest a particle moved from its tile since the sort, beyond the
@@ -1906,17 +2084,11 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     ctx->cur[sp] = 1 - ctx->cur[sp];
     S->pending[sp] = false;
   }
-  if (thrust) {
-    const pic_config &c = ctx->cfg;
-    const double qs = sp == PIC_ION ? c.q : -c.q;
-    return thrust_add(ctx, sp, (int)nb, qs * c.weight[sp] * c.dx * c.dx * c.dx);
-  }
+  if (thrust) ctx->thrust_nb[sp] = (int)nb;  // finished by step_b2
   return 0;
 }
 
 int particle_boundary(pic_ctx *ctx, int sp) { return push(ctx, sp, 0, 0, 1); }
-
-float *total_b(pic_ctx *ctx) { return st(ctx)->bt; }
 
 // stable compaction of live particles (tile ranges become invalid)
 static int compact(pic_ctx *ctx, int sp) {

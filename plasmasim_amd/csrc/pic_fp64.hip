@@ -13,6 +13,7 @@
 #include <string.h>
 
 #include "philox.h"
+#include "pic_fused.h"
 #include "pic_internal.h"
 #include "pic_tsort.h"
 #include "pic_tiles.h"
@@ -37,19 +38,18 @@ __device__ inline double sigma_at(const SigmaProfile &s, int k2, int l2,
   return s.amp * (0.1 * sqrt(a4) + 0.01 * sqrt(a12));
 }
 
-// renew_b4_2 (:2580-2611)
-__global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F,
-                                                 SigmaProfile sg, double dt,
-                                                 double dx, double eps0) {
-  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
-  const int k = 2 + blockIdx.z;
-  if (m >= g.NZ + 2 || l >= g.NY + 2) return;
-  const double temp = 1. / eps0 * dt * 0.5 * 0.5;
-  const double dth = 0.5 * dt;
+struct FieldConst {
+  double dt, dx, eps0, mu0, c;
+};
+
+// renew_b4_2 (:2580-2611) at interior cell c
+__device__ inline void renew_b_cell(const Geom &g, const Fields<double> &F,
+                                    const SigmaProfile &sg, const FieldConst &fc, int k,
+                                    int l, int m, int64_t c, double out[3]) {
+  const double temp = 1. / fc.eps0 * fc.dt * 0.5 * 0.5;
+  const double dth = 0.5 * fc.dt;
   const double temp_24 = 1. / 24.;
-  const double inv_dx = 1. / dx;
-  const int64_t c = g.idx(k, l, m);
+  const double inv_dx = 1. / fc.dx;
   const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
   const double *ex = F.f[PIC_EX], *ey = F.f[PIC_EY], *ez = F.f[PIC_EZ];
   double f, h, s;
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F,
   h = s == 0.0 ? dth : dth / (1. + s * temp);
   {
     const double b0 = F.f[PIC_B0X][c];
-    F.f[PIC_BX][c] =
+    out[0] =
         b0 + f * (F.f[PIC_BX][c] - b0) -
         h * temp_24 *
             (27. * (ez[c] - ez[c - dl] - ey[c] + ey[c - 1]) -
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F,
   h = s == 0.0 ? dth : dth / (1. + s * temp);
   {
     const double b0 = F.f[PIC_B0Y][c];
-    F.f[PIC_BY][c] =
+    out[1] =
         b0 + f * (F.f[PIC_BY][c] - b0) -
         h * temp_24 *
             (27. * (ex[c] - ex[c - 1] - ez[c] + ez[c - dk]) -
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F,
   h = s == 0.0 ? dth : dth / (1. + s * temp);
   {
     const double b0 = F.f[PIC_B0Z][c];
-    F.f[PIC_BZ][c] =
+    out[2] =
         b0 + f * (F.f[PIC_BZ][c] - b0) -
         h * temp_24 *
             (27. * (ey[c] - ey[c - dk] - ex[c] + ex[c - dl]) -
@@ -92,20 +92,27 @@ __global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F,
   }
 }
 
-// renew_e4_2 (:2613-2652); the curl acts on B - B0 recomputed per term, as
-// the reference writes it.
-__global__ __launch_bounds__(256) void k_renew_e(Geom g, Fields<double> F,
-                                                 SigmaProfile sg, double dt,
-                                                 double dx, double c_light,
-                                                 double mu0) {
+__global__ __launch_bounds__(256) void k_renew_b(Geom g, Fields<double> F, SigmaProfile sg,
+                                                 FieldConst fc) {
   const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
   const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
   const int k = 2 + blockIdx.z;
   if (m >= g.NZ + 2 || l >= g.NY + 2) return;
-  const double temp = c_light * c_light * dt;
-  const double temp_24 = 1. / 24.;
-  const double inv_dx = 1. / dx;
   const int64_t c = g.idx(k, l, m);
+  double b[3];
+  renew_b_cell(g, F, sg, fc, k, l, m, c, b);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) F.f[PIC_BX + q][c] = b[q];
+}
+
+// renew_e4_2 (:2613-2652) at interior cell c; the curl acts on B - B0
+// recomputed per term, as the reference writes it.
+__device__ inline void renew_e_cell(const Geom &g, const Fields<double> &F,
+                                    const SigmaProfile &sg, const FieldConst &fc, int k,
+                                    int l, int m, int64_t c, double out[3]) {
+  const double temp = fc.c * fc.c * fc.dt;
+  const double temp_24 = 1. / 24.;
+  const double inv_dx = 1. / fc.dx;
   const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
   const double *bx = F.f[PIC_BX], *by = F.f[PIC_BY], *bz = F.f[PIC_BZ];
   const double *b0x = F.f[PIC_B0X], *b0y = F.f[PIC_B0Y], *b0z = F.f[PIC_B0Z];
@@ -113,38 +120,51 @@ __global__ __launch_bounds__(256) void k_renew_e(Geom g, Fields<double> F,
 #define D1(B, B0, a, b) (B[a] - B0[a] - B[b] + B0[b])
 
   s = sigma_at(sg, 2 * k, 2 * l + 1, 2 * m + 1);
-  f = s == 0.0 ? 1.0 : (1. - 0.5 * mu0 * s * temp) / (1. + 0.5 * mu0 * s * temp);
-  h = s == 0.0 ? temp : temp / (1. + 0.5 * mu0 * s * temp);
-  F.f[PIC_EX][c] =
+  f = s == 0.0 ? 1.0 : (1. - 0.5 * fc.mu0 * s * temp) / (1. + 0.5 * fc.mu0 * s * temp);
+  h = s == 0.0 ? temp : temp / (1. + 0.5 * fc.mu0 * s * temp);
+  out[0] =
       f * F.f[PIC_EX][c] +
       h * (temp_24 *
                (27. * (D1(bz, b0z, c + dl, c) - D1(by, b0y, c + 1, c)) -
                 (D1(bz, b0z, c + 2 * dl, c - dl) - D1(by, b0y, c + 2, c - 1))) *
                inv_dx -
-           mu0 * (F.f[PIC_JIX][c] - F.f[PIC_JEX][c]));
+           fc.mu0 * (F.f[PIC_JIX][c] - F.f[PIC_JEX][c]));
 
   s = sigma_at(sg, 2 * k + 1, 2 * l, 2 * m + 1);
-  f = s == 0.0 ? 1.0 : (1. - 0.5 * mu0 * s * temp) / (1. + 0.5 * mu0 * s * temp);
-  h = s == 0.0 ? temp : temp / (1. + 0.5 * mu0 * s * temp);
-  F.f[PIC_EY][c] =
+  f = s == 0.0 ? 1.0 : (1. - 0.5 * fc.mu0 * s * temp) / (1. + 0.5 * fc.mu0 * s * temp);
+  h = s == 0.0 ? temp : temp / (1. + 0.5 * fc.mu0 * s * temp);
+  out[1] =
       f * F.f[PIC_EY][c] +
       h * (temp_24 *
                (27. * (D1(bx, b0x, c + 1, c) - D1(bz, b0z, c + dk, c)) -
                 (D1(bx, b0x, c + 2, c - 1) - D1(bz, b0z, c + 2 * dk, c - dk))) *
                inv_dx -
-           mu0 * (F.f[PIC_JIY][c] - F.f[PIC_JEY][c]));
+           fc.mu0 * (F.f[PIC_JIY][c] - F.f[PIC_JEY][c]));
 
   s = sigma_at(sg, 2 * k + 1, 2 * l + 1, 2 * m);
-  f = s == 0.0 ? 1.0 : (1. - 0.5 * mu0 * s * temp) / (1. + 0.5 * mu0 * s * temp);
-  h = s == 0.0 ? temp : temp / (1. + 0.5 * mu0 * s * temp);
-  F.f[PIC_EZ][c] =
+  f = s == 0.0 ? 1.0 : (1. - 0.5 * fc.mu0 * s * temp) / (1. + 0.5 * fc.mu0 * s * temp);
+  h = s == 0.0 ? temp : temp / (1. + 0.5 * fc.mu0 * s * temp);
+  out[2] =
       f * F.f[PIC_EZ][c] +
       h * (temp_24 *
                (27. * (D1(by, b0y, c + dk, c) - D1(bx, b0x, c + dl, c)) -
                 (D1(by, b0y, c + 2 * dk, c - dk) - D1(bx, b0x, c + 2 * dl, c - dl))) *
                inv_dx -
-           mu0 * (F.f[PIC_JIZ][c] - F.f[PIC_JEZ][c]));
+           fc.mu0 * (F.f[PIC_JIZ][c] - F.f[PIC_JEZ][c]));
 #undef D1
+}
+
+__global__ __launch_bounds__(256) void k_renew_e(Geom g, Fields<double> F, SigmaProfile sg,
+                                                 FieldConst fc) {
+  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = 2 + blockIdx.y * blockDim.y + threadIdx.y;
+  const int k = 2 + blockIdx.z;
+  if (m >= g.NZ + 2 || l >= g.NY + 2) return;
+  const int64_t c = g.idx(k, l, m);
+  double e[3];
+  renew_e_cell(g, F, sg, fc, k, l, m, c, e);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) F.f[PIC_EX + q][c] = e[q];
 }
 
 // sr_b / sr_e on one rank (:1001-1387): copy along x over all (l,m), then
@@ -212,6 +232,93 @@ __global__ void k_fold_y(Geom g, Fields<double> F) {
     f[3 * dl] += f[(g.NY + 3) * dl];
     f[g.NY * dl] += f[0];
     f[(g.NY + 1) * dl] += f[1 * dl];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// the step's field launches (pic_fused.h)
+
+// B half step and sr_b of cell (k, l, m); kept (3 planes, or null): the
+// end-of-step total B goes there first
+__device__ inline void b_and_guards(const Geom &g, const Fields<double> &F, double *kept,
+                                    const SigmaProfile &sg, const FieldConst &fc, int k, int l,
+                                    int m) {
+  const int64_t c = g.idx(k, l, m);
+  const bool in = m >= 2 && m < g.NZ + 2;
+  double b[3];
+  if (in) renew_b_cell(g, F, sg, fc, k, l, m, c, b);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double *B = F.f[PIC_BX + q], *K = kept ? kept + q * g.plane : nullptr;
+    const double old = B[c], v = in ? b[q] : old;
+    if (K) K[c] = old;
+    if (in) B[c] = v;
+    images(g, k, l, c, [&](int64_t d, int64_t) {
+      if (K) K[d] = B[d];
+      B[d] = v;
+    });
+  }
+}
+
+// renew_grid, thrust_fave's copy of the total B, the first B half step, sr_b
+__global__ __launch_bounds__(256) void k_step_b1(Geom g, CellBlocks cb, Fields<double> F,
+                                                 double *kept, SigmaProfile sg,
+                                                 FieldConst fc) {
+  int k, l, m;
+  if (!cb.cell(g, blockIdx.x, k, l, m)) return;
+  const int64_t c = g.idx(k, l, m);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) F.f[PIC_JIX + q][c] = 0.0;
+  if (interior_column(g, k, l)) b_and_guards(g, F, kept, sg, fc, k, l, m);
+}
+
+// The second B half step and sr_b, sr_current2, thrust_fave's sums: blocks
+// below tb finish the thrust, then fb blocks fold, the rest are cells.
+__global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<double> F,
+                                                 SigmaProfile sg, FieldConst fc, int tb,
+                                                 ThrustFinish tf, int fb) {
+  int b = blockIdx.x;
+  if (b < tb) {
+    thrust_finish(tf, b);
+    return;
+  }
+  b -= tb;
+  if (b < fb) {
+    const int64_t t = (int64_t)b * 256 + threadIdx.x;
+    if (t >= (int64_t)fold_groups(g) * g.SZ) return;
+    const int m = (int)(t % g.SZ), grp = (int)(t / g.SZ);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      double *f = F.f[PIC_JIX + q];
+      fold_group(
+          g, grp, m, [&](int64_t i) { return f[i]; },
+          [&](int64_t i, double v, bool changed) {
+            if (changed) f[i] = v;
+          });
+    }
+    return;
+  }
+  b -= fb;
+  int k, l, m;
+  if (!cb.cell(g, b, k, l, m) || !interior_column(g, k, l)) return;
+  b_and_guards(g, F, nullptr, sg, fc, k, l, m);
+}
+
+// the E step and sr_e
+__global__ __launch_bounds__(256) void k_step_e(Geom g, CellBlocks cb, Fields<double> F,
+                                                SigmaProfile sg, FieldConst fc) {
+  int k, l, m;
+  if (!cb.cell(g, blockIdx.x, k, l, m) || !interior_column(g, k, l)) return;
+  const int64_t c = g.idx(k, l, m);
+  const bool in = m >= 2 && m < g.NZ + 2;
+  double e[3];
+  if (in) renew_e_cell(g, F, sg, fc, k, l, m, c, e);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double *E = F.f[PIC_EX + q];
+    const double v = in ? e[q] : E[c];
+    if (in) E[c] = v;
+    images(g, k, l, c, [&](int64_t d, int64_t) { E[d] = v; });
   }
 }
 
@@ -1049,20 +1156,23 @@ int renew_grid(pic_ctx *ctx) {
   return 0;
 }
 
-int renew_b_half(pic_ctx *ctx) {
+static FieldConst field_const(const pic_ctx *ctx) {
   const pic_config &c = ctx->cfg;
+  return FieldConst{c.dt, c.dx, c.eps0, c.mu0, c.c};
+}
+
+int renew_b_half(pic_ctx *ctx) {
   dim3 b, gr = interior_grid(ctx->geom, b);
   k_renew_b<<<gr, b, 0, ctx->stream>>>(ctx->geom, fields<double>(ctx),
-                                       sigma(ctx), c.dt, c.dx, c.eps0);
+                                       sigma(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
 
 int renew_e(pic_ctx *ctx) {
-  const pic_config &c = ctx->cfg;
   dim3 b, gr = interior_grid(ctx->geom, b);
   k_renew_e<<<gr, b, 0, ctx->stream>>>(ctx->geom, fields<double>(ctx),
-                                       sigma(ctx), c.dt, c.dx, c.c, c.mu0);
+                                       sigma(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1086,6 +1196,36 @@ int fold_current(pic_ctx *ctx) {
              ctx->stream>>>(g, F);
   k_fold_y<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
              ctx->stream>>>(g, F);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+int step_b1(pic_ctx *ctx, bool keep_b) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  k_step_b1<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<double>(ctx), keep_b ? (double *)ctx->thrust_bprev : nullptr, sigma(ctx),
+      field_const(ctx));
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+int step_b2(pic_ctx *ctx) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  const int tb = ctx->thrust_now ? 12 : 0;
+  const int fb = (int)div_up((int64_t)fold_groups(g) * g.SZ, kBlock);
+  k_step_b2<<<(unsigned)(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<double>(ctx), sigma(ctx), field_const(ctx), tb, thrust_finish_args(ctx), fb);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+int step_e(pic_ctx *ctx) {
+  const Geom &g = ctx->geom;
+  const CellBlocks cb(g);
+  k_step_e<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+      g, cb, fields<double>(ctx), sigma(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1190,7 +1330,7 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     if ((int64_t)nb > ctx->thrust_part_slots)
       return set_error(ctx, PIC_E_CAPACITY, "thrust: %u workgroups, %lld partial slots",
                        nb, (long long)ctx->thrust_part_slots);
-    tp = ctx->thrust_part;
+    tp = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
   }
   // normalised units with 32-bit byte offsets, or any dx with 64-bit ones
   const bool unit = ctx->cfg.dx == 1.0 && n < ((int64_t)1 << 29) &&
@@ -1222,11 +1362,7 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
 #undef LAUNCH2
 #undef LAUNCH
   PIC_LAUNCH_CHECK(ctx);
-  if (thrust) {
-    const pic_config &c = ctx->cfg;
-    const double qs = sp == PIC_ION ? c.q : -c.q;
-    return thrust_add(ctx, sp, (int)nb, qs * c.weight[sp] * c.dx * c.dx * c.dx);
-  }
+  if (thrust) ctx->thrust_nb[sp] = (int)nb;  // finished by step_b2
   return 0;
 }
 

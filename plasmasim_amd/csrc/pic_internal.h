@@ -139,8 +139,9 @@ struct pic_ctx {
   int thrust_now = 0;                // the running pass adds it
   int64_t thrust_steps = 0;          // steps added to thrust_acc
   double *thrust_acc = nullptr;      // device: per species E part (3), v x B part (3)
-  double *thrust_part = nullptr;     // device: 6 partials per pass workgroup
-  int64_t thrust_part_slots = 0;
+  double *thrust_part = nullptr;     // device: 6 partials per pass workgroup, per species
+  int64_t thrust_part_slots = 0;     // workgroups per species
+  int thrust_nb[2] = {0, 0};         // workgroups of this step's passes
   void *thrust_bprev = nullptr;      // device: 3 FP64 B planes (the FP32 form
                                      // keeps its copy beside its total-B planes)
 
@@ -270,6 +271,13 @@ int renew_b_half(pic_ctx *);
 int halo(pic_ctx *, int first);
 int fold_current(pic_ctx *);
 int renew_e(pic_ctx *);
+// pic_step's field launches: renew_grid (and the copy of the total B for
+// thrust_fave), the first B half step and sr_b; the second, sr_b, the
+// conversion of fixed-point deposits, sr_current2 and the thrust sums of
+// both passes; the E step and sr_e
+int step_b1(pic_ctx *, bool keep_b);
+int step_b2(pic_ctx *);
+int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
 int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
 int particle_boundary(pic_ctx *, int sp);
@@ -286,6 +294,9 @@ int renew_b_half(pic_ctx *);
 int halo(pic_ctx *, int first);
 int fold_current(pic_ctx *);
 int renew_e(pic_ctx *);
+int step_b1(pic_ctx *, bool keep_b);
+int step_b2(pic_ctx *);
+int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
 int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
 int particle_boundary(pic_ctx *, int sp);
@@ -329,12 +340,6 @@ int diagnose_partials(pic_ctx *, double *partials, unsigned long long *counts);
 }
 namespace f32 {
 int diagnose_partials(pic_ctx *, double *partials, unsigned long long *counts);
-}
-// thrust_fave: add one pass's workgroup partials (6 per workgroup, nb
-// workgroups) times qn = q_s w dx^3 to the species' running sums
-int thrust_add(pic_ctx *ctx, int sp, int nb, double qn);
-namespace f32 {
-float *total_b(pic_ctx *);  // the 3 total-B planes the gather reads
 }
 // static device scratch of the allocation-free entry points (pic_noalloc.hip):
 // resolved for the current device at pic_create
