@@ -405,6 +405,7 @@ extern "C" int pic2d_sync(pic2d_ctx *ctx) {
 extern "C" int pic2d_upload_field(pic2d_ctx *ctx, int which, const double *host) {
   if (!ctx || !host || which < 0 || which >= PIC2D_NFIELDS) return PIC_E_ARG;
   const int64_t n = ctx->g.plane;
+  ctx->guards_ok = false;
   if (ctx->f64) {
     P2_HIP(ctx, hipMemcpy(plane<double>(ctx, which), host, n * sizeof(double),
                           hipMemcpyHostToDevice));
@@ -599,8 +600,18 @@ extern "C" int pic2d_step(pic2d_ctx *ctx, int nsteps) {
       return rc;                            \
     }                                       \
   } while (0)
+#define FIELD(cls, call)                 \
+  do {                                   \
+    pic::timing_begin(&ctx->rt, cls);    \
+    rc = call;                           \
+    pic::timing_end(&ctx->rt, cls);      \
+    TRY(rc);                             \
+  } while (0)
   for (int s = 0; s < nsteps; ++s) {
-    TRY(pic2d_renew_grid(ctx));
+    // the step's own launches, where the guard rows are current; otherwise
+    // (fields just written) routine by routine
+    const bool fused = ctx->guards_ok;
+    if (!fused) TRY(pic2d_renew_grid(ctx));
     if (c.inflow_every > 0 && ctx->c_add >= c.inflow_every) {
       TRY(pic2d_inflow(ctx));
       ctx->c_add = 0;
@@ -617,8 +628,12 @@ extern "C" int pic2d_step(pic2d_ctx *ctx, int nsteps) {
       }
       ctx->c_sort = 0;
     }
-    TRY(pic2d_renew_b_half(ctx));
-    TRY(pic2d_halo(ctx));
+    if (fused) {
+      FIELD(PIC_T_FIELD_B, step_b1(ctx));
+    } else {
+      TRY(pic2d_renew_b_half(ctx));
+      TRY(pic2d_halo(ctx));
+    }
     for (int sp = 0; sp < 2; ++sp) {
       const int tclass = ctx->pending[sp] ? PIC_T_PUSH_SORT : PIC_T_PUSH;
       pic::timing_begin(&ctx->rt, tclass);
@@ -626,21 +641,28 @@ extern "C" int pic2d_step(pic2d_ctx *ctx, int nsteps) {
       pic::timing_end(&ctx->rt, tclass);
       TRY(rc);
     }
-    TRY(pic2d_fold_current(ctx));
-    TRY(pic2d_external_current(ctx, ctx->step));
-    TRY(pic2d_fold_density(ctx));
-    TRY(pic2d_renew_b_half(ctx));
-    TRY(pic2d_halo(ctx));
-    TRY(pic2d_renew_e(ctx));
-    TRY(pic2d_halo(ctx));
-    if (c.poisson_every > 0 && ctx->step % c.poisson_every == 0) {
-      TRY(pic2d_poisson(ctx));
+    const bool with_phi = c.poisson_every > 0 && ctx->step % c.poisson_every == 0;
+    if (fused) {
+      FIELD(PIC_T_FIELD_B, step_b2(ctx, ctx->step));
+      FIELD(PIC_T_FIELD_E, step_e(ctx, with_phi));
+    } else {
+      TRY(pic2d_fold_current(ctx));
+      TRY(pic2d_external_current(ctx, ctx->step));
+      TRY(pic2d_fold_density(ctx));
+      TRY(pic2d_renew_b_half(ctx));
       TRY(pic2d_halo(ctx));
+      TRY(pic2d_renew_e(ctx));
+      TRY(pic2d_halo(ctx));
+      if (with_phi) {
+        TRY(pic2d_poisson(ctx));
+        TRY(pic2d_halo(ctx));
+      }
     }
     ctx->step++;
     ctx->c_add++;
     ctx->c_sort++;
   }
+#undef FIELD
 #undef TRY
   return 0;
 }

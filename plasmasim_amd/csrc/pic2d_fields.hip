@@ -67,13 +67,11 @@ static FieldSet<T> field_set(pic2d_ctx *ctx) {
   return F;
 }
 
-// renew_b4 (:1391-1417): one thread per interior node, m fastest
+// renew_b4 (:1391-1417) of interior node (k, m)
 template <typename T>
-__global__ void k_renew_b2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
-                           T dtf, T dx, T e0) {
-  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = 2 + blockIdx.y;
-  if (m >= g.NZ + 2) return;
+__device__ inline void renew_b_node(const Geom2 &g, const FieldSet<T> &F,
+                                    const T *__restrict__ sig, T dtf, T dx, T e0, int k, int m,
+                                    T out[3]) {
   const int64_t i = g.idx(k, m), dk = g.SZ;
   const int64_t S2 = 2 * (int64_t)g.SZ;
   const T one = 1, half = 0.5, c24 = 24, c27 = 27;
@@ -94,18 +92,31 @@ __global__ void k_renew_b2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
   const T bz = F.b0z[i] + (one - s) / (one + s) * (F.bz[i] - F.b0z[i]) -
                dtf * half / (one + s) * one / c24 *
                    (c27 * (ey[i] - ey[i - dk]) - (ey[i + dk] - ey[i - 2 * dk])) / dx;
-  F.bx[i] = bx;
-  F.by[i] = by;
-  F.bz[i] = bz;
+  out[0] = bx;
+  out[1] = by;
+  out[2] = bz;
 }
 
-// renew_e4 (:1419-1449): curl of B - B0 and Ji - Je
+// one thread per interior node, m fastest
 template <typename T>
-__global__ void k_renew_e2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
-                           T dtf, T dx, T mu0, T C) {
+__global__ void k_renew_b2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
+                           T dtf, T dx, T e0) {
   const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
   const int k = 2 + blockIdx.y;
   if (m >= g.NZ + 2) return;
+  const int64_t i = g.idx(k, m);
+  T b[3];
+  renew_b_node(g, F, sig, dtf, dx, e0, k, m, b);
+  F.bx[i] = b[0];
+  F.by[i] = b[1];
+  F.bz[i] = b[2];
+}
+
+// renew_e4 (:1419-1449) of interior node (k, m): curl of B - B0 and Ji - Je
+template <typename T>
+__device__ inline void renew_e_node(const Geom2 &g, const FieldSet<T> &F,
+                                    const T *__restrict__ sig, T dtf, T dx, T mu0, T C, int k,
+                                    int m, T out[3]) {
   const int64_t i = g.idx(k, m), dk = g.SZ;
   const int64_t S2 = 2 * (int64_t)g.SZ;
   const T one = 1, half = 0.5, c24 = 24, c27 = 27;
@@ -143,9 +154,23 @@ __global__ void k_renew_e2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
                 (bz[i + 2 * dk] - b0z[i + 2 * dk] - bz[i - dk] + b0z[i - dk])) /
                dx -
            mu0 * (F.jiy[i] - F.jey[i]));
-  F.ex[i] = ex;
-  F.ey[i] = ey;
-  F.ez[i] = ez;
+  out[0] = ex;
+  out[1] = ey;
+  out[2] = ez;
+}
+
+template <typename T>
+__global__ void k_renew_e2(Geom2 g, FieldSet<T> F, const T *__restrict__ sig,
+                           T dtf, T dx, T mu0, T C) {
+  const int m = 2 + blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = 2 + blockIdx.y;
+  if (m >= g.NZ + 2) return;
+  const int64_t i = g.idx(k, m);
+  T e[3];
+  renew_e_node(g, F, sig, dtf, dx, mu0, C, k, m, e);
+  F.ex[i] = e[0];
+  F.ey[i] = e[1];
+  F.ez[i] = e[2];
 }
 
 template <typename T>
@@ -169,11 +194,13 @@ static int renew_e_t(pic2d_ctx *ctx, const T *sig) {
 }
 
 int renew_b_half(pic2d_ctx *ctx) {
+  ctx->guards_ok = false;
   return ctx->f64 ? renew_b_t<double>(ctx, ctx->sig64)
                   : renew_b_t<float>(ctx, ctx->sig32);
 }
 
 int renew_e(pic2d_ctx *ctx) {
+  ctx->guards_ok = false;
   return ctx->f64 ? renew_e_t<double>(ctx, ctx->sig64)
                   : renew_e_t<float>(ctx, ctx->sig32);
 }
@@ -203,6 +230,7 @@ int halo(pic2d_ctx *ctx) {
     k_halo2<float><<<nb, kBlock, 0, ctx->rt.stream>>>(
         ctx->g, (float *)ctx->field_mem, PIC2D_NFIELDS);
   P2_LAUNCH_CHECK(ctx);
+  ctx->guards_ok = true;
   return 0;
 }
 
@@ -239,12 +267,10 @@ __global__ void k_set2(T *__restrict__ p, int64_t i0, T v0, int64_t i1, T v1) {
   }
 }
 
-int external_current(pic2d_ctx *ctx, int64_t step) {
-  const pic2d_config &c = ctx->cfg;
-  if (c.ext_k < 0) return 0;
+// the currents of a step
+static void external_values(const pic2d_config &c, int64_t step, double &v0, double &v1) {
   const double Pi = 3.14159265358979323846;
   const double I = c.ext_current, dx = c.dx;
-  double v0, v1;
   if (step < c.ext_ramp) {
     const double w = Pi / (double)c.ext_ramp;
     v0 = -I / dx / dx * (1. + cos(w * (double)step - Pi)) / 2.;
@@ -253,6 +279,13 @@ int external_current(pic2d_ctx *ctx, int64_t step) {
     v0 = -I / dx / dx;
     v1 = I / dx / dx;
   }
+}
+
+int external_current(pic2d_ctx *ctx, int64_t step) {
+  const pic2d_config &c = ctx->cfg;
+  if (c.ext_k < 0) return 0;
+  double v0, v1;
+  external_values(c, step, v0, v1);
   const int64_t i0 = ctx->g.idx(c.ext_k, c.ext_m[0]);
   const int64_t i1 = ctx->g.idx(c.ext_k, c.ext_m[1]);
   if (ctx->f64)
@@ -269,22 +302,33 @@ int external_current(pic2d_ctx *ctx, int64_t step) {
 // renew_phi (:2589-2767): source, DST-I along z then x, division by the
 // 5-point symbol, inverse DSTs, E += grad phi
 
+// the source at solved node (kk, mm), read by the first transform
 template <typename T>
-__global__ void k_phi_rhs(Geom2 g, const T *__restrict__ ni,
-                          const T *__restrict__ ne, const T *__restrict__ ex,
-                          const T *__restrict__ ez, T *__restrict__ rho,
-                          int lox, int hix, int loz, int hiz, T q, T e0, T dx) {
-  const int mm = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kk = blockIdx.y;
-  if (mm >= g.NZ) return;
-  const int k = kk + 2, m = mm + 2;
-  T v = 0;
-  if (k >= lox && k < hix && m >= loz && m < hiz) {
+struct PhiSource {
+  Geom2 g;
+  const T *ni, *ne, *ex, *ez;
+  int lox, hix, loz, hiz;
+  T q, e0, dx;
+  __device__ inline T operator()(int kk, int mm) const {
+    const int k = kk + 2, m = mm + 2;
+    if (!(k >= lox && k < hix && m >= loz && m < hiz)) return 0;
     const int64_t i = g.idx(k, m);
-    v = -(-q * (ni[i] - ne[i]) / e0 + (ex[i + g.SZ] - ex[i]) / dx +
-          (ez[i + 1] - ez[i]) / dx);
+    return -(-q * (ni[i] - ne[i]) / e0 + (ex[i + g.SZ] - ex[i]) / dx +
+             (ez[i + 1] - ez[i]) / dx);
   }
-  rho[(int64_t)kk * g.NZ + mm] = v;
+};
+
+// E += grad phi and phi of solved node (kk, mm)
+template <typename T>
+__device__ inline void phi_node(const Geom2 &g, const T *__restrict__ rho, int kk, int mm,
+                                T &ex, T &ez, T &phi, T dx) {
+  const int64_t r = (int64_t)kk * g.NZ + mm;
+  const T ph = rho[r];
+  const T pxm = kk == 0 ? rho[(int64_t)(g.NX - 1) * g.NZ + mm] : rho[r - g.NZ];
+  const T pzm = mm == 0 ? (T)0 : rho[r - 1];
+  ex += (ph - pxm) / dx;
+  phi = ph;
+  ez += (ph - pzm) / dx;
 }
 
 template <typename T>
@@ -294,14 +338,8 @@ __global__ void k_phi_apply(Geom2 g, const T *__restrict__ rho,
   const int mm = blockIdx.x * blockDim.x + threadIdx.x;
   const int kk = blockIdx.y;
   if (mm >= g.NZ) return;
-  const int64_t r = (int64_t)kk * g.NZ + mm;
-  const T ph = rho[r];
-  const T pxm = kk == 0 ? rho[(int64_t)(g.NX - 1) * g.NZ + mm] : rho[r - g.NZ];
-  const T pzm = mm == 0 ? (T)0 : rho[r - 1];
   const int64_t i = g.idx(kk + 2, mm + 2);
-  ex[i] += (ph - pxm) / dx;
-  phi[i] = ph;
-  ez[i] += (ph - pzm) / dx;
+  phi_node(g, rho, kk, mm, ex[i], ez[i], phi[i], dx);
 }
 
 // twiddles exp(-2 pi i t / L), t < L/2, and the symbol tables
@@ -327,21 +365,22 @@ int init_poisson(pic2d_ctx *ctx) {
   return 0;
 }
 
+// the potential into rho: DST-I along z of the source, along x with the
+// division and back, along z back
 template <typename T>
-static int poisson_t(pic2d_ctx *ctx) {
+static int solve_phi(pic2d_ctx *ctx) {
   const pic2d_config &c = ctx->cfg;
   const Geom2 &g = ctx->g;
   const int NX = g.NX, NZ = g.NZ;
   T *rho = (T *)ctx->rho;
   hipStream_t st = ctx->rt.stream;
-  dim3 grid((unsigned)div_up(NZ, kBlock), (unsigned)NX);
-  k_phi_rhs<T><<<grid, kBlock, 0, st>>>(
-      g, plane<T>(ctx, PIC_NI), plane<T>(ctx, PIC_NE), plane<T>(ctx, PIC_EX),
-      plane<T>(ctx, PIC_EZ), rho, c.phi_lo[0], c.phi_hi[0], c.phi_lo[1],
-      c.phi_hi[1], (T)c.q, (T)c.eps0, (T)c.dx);
-  P2_LAUNCH_CHECK(ctx);
   using pic::Cplx;
   using pic::k_dst;
+  using pic::LineData;
+  const PhiSource<T> source{g, plane<T>(ctx, PIC_NI), plane<T>(ctx, PIC_NE),
+                            plane<T>(ctx, PIC_EX), plane<T>(ctx, PIC_EZ),
+                            c.phi_lo[0], c.phi_hi[0], c.phi_lo[1], c.phi_hi[1],
+                            (T)c.q, (T)c.eps0, (T)c.dx};
   const Cplx<T> *twx = (const Cplx<T> *)ctx->tw_x;
   const Cplx<T> *twz = (const Cplx<T> *)ctx->tw_z;
   const double *symx = (const double *)((const char *)ctx->tw_x + (size_t)NX * sizeof(Cplx<T>));
@@ -350,20 +389,27 @@ static int poisson_t(pic2d_ctx *ctx) {
   const size_t ldsz = (size_t)4 * NZ * sizeof(T), ldsx = (size_t)4 * NX * sizeof(T);
   const unsigned bz = (unsigned)div_up(NX, 2), bx = (unsigned)div_up(NZ, 2);
   const int lz = pic::ilog2_ceil(2 * NZ), lx = pic::ilog2_ceil(2 * NX);
-  // forward along z (lines k, contiguous), then along x (lines m, stride
-  // NZ) with the division, inverse along x, inverse along z
-  k_dst<T><<<bz, 256, ldsz, st>>>(rho, NZ, lz, NX, NX, NZ, 0, 1, twz, 0, nullptr,
+  // z: lines k, contiguous; x: lines m, stride NZ
+  const LineData<T> along_z{rho, NX, NZ, 0, 1}, along_x{rho, NZ, 1, 0, NZ};
+  k_dst<T><<<bz, 256, ldsz, st>>>(rho, source, NZ, lz, NX, NX, NZ, 0, 1, twz, 0, nullptr,
                                   nullptr, 0.);
-  k_dst<T><<<bx, 256, ldsx, st>>>(rho, NX, lx, NZ, NZ, 1, 0, NZ, twx, 1, symz, symx,
+  k_dst<T><<<bx, 256, ldsx, st>>>(rho, along_x, NX, lx, NZ, NZ, 1, 0, NZ, twx, 3, symz, symx,
                                   dq);
-  k_dst<T><<<bx, 256, ldsx, st>>>(rho, NX, lx, NZ, NZ, 1, 0, NZ, twx, 2, nullptr,
-                                  nullptr, 0.);
-  k_dst<T><<<bz, 256, ldsz, st>>>(rho, NZ, lz, NX, NX, NZ, 0, 1, twz, 2, nullptr,
+  k_dst<T><<<bz, 256, ldsz, st>>>(rho, along_z, NZ, lz, NX, NX, NZ, 0, 1, twz, 2, nullptr,
                                   nullptr, 0.);
   P2_LAUNCH_CHECK(ctx);
-  k_phi_apply<T><<<grid, kBlock, 0, st>>>(g, rho, plane<T>(ctx, PIC_EX),
-                                          plane<T>(ctx, PIC_EZ),
-                                          plane<T>(ctx, PIC2D_PHI), (T)c.dx);
+  return 0;
+}
+
+template <typename T>
+static int poisson_t(pic2d_ctx *ctx) {
+  int rc = solve_phi<T>(ctx);
+  if (rc) return rc;
+  ctx->guards_ok = false;
+  dim3 grid((unsigned)div_up(ctx->g.NZ, kBlock), (unsigned)ctx->g.NX);
+  k_phi_apply<T><<<grid, kBlock, 0, ctx->rt.stream>>>(
+      ctx->g, (const T *)ctx->rho, plane<T>(ctx, PIC_EX), plane<T>(ctx, PIC_EZ),
+      plane<T>(ctx, PIC2D_PHI), (T)ctx->cfg.dx);
   P2_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -371,6 +417,180 @@ static int poisson_t(pic2d_ctx *ctx) {
 int poisson(pic2d_ctx *ctx) {
   if (!ctx->rho) return err(ctx, PIC_E_STATE, "poisson: disabled by poisson_every = 0");
   return ctx->f64 ? poisson_t<double>(ctx) : poisson_t<float>(ctx);
+}
+
+// ---------------------------------------------------------------------------
+// pic2d_step's field launches.  The routines one by one are 17 launches a
+// step, most of them small: on 256^2 each costs its latency.  sr_grid copies
+// rows, so the thread that owns an interior node writes its image rows as
+// well; J, n and phi are needed in the interior only until the last sr_grid
+// of the step, which copies their rows.  These launches take the guard rows
+// of E, B and B0 as the images they are (guards_ok).
+
+// the thread's node: one row per blockIdx.y of the whole array
+__device__ inline bool node_of(const Geom2 &g, int &k, int &m) {
+  m = blockIdx.x * blockDim.x + threadIdx.x;
+  k = blockIdx.y;
+  return m < g.SZ;
+}
+
+// row k's image row, or -1 (nx >= 4: at most one)
+__device__ inline int image_row(const Geom2 &g, int k) {
+  return k < 2 || k >= g.NX + 2 ? -1 : k < 4 ? k + g.NX : k >= g.NX ? k - g.NX : -1;
+}
+
+template <typename T>
+__device__ inline void put_rows(const Geom2 &g, T *p, int k, int m, T v, bool own) {
+  if (own) p[g.idx(k, m)] = v;
+  const int r = image_row(g, k);
+  if (r >= 0) p[g.idx(r, m)] = v;
+}
+
+template <typename T>
+__device__ inline void b_rows(const Geom2 &g, const FieldSet<T> &F, const T *__restrict__ sig,
+                              T dtf, T dx, T e0, int k, int m) {
+  if (k < 2 || k >= g.NX + 2) return;
+  const bool in = m >= 2 && m < g.NZ + 2;
+  if (!in && image_row(g, k) < 0) return;
+  const int64_t i = g.idx(k, m);
+  T b[3] = {F.bx[i], F.by[i], F.bz[i]};
+  if (in) renew_b_node(g, F, sig, dtf, dx, e0, k, m, b);
+  put_rows(g, F.bx, k, m, b[0], in);
+  put_rows(g, F.by, k, m, b[1], in);
+  put_rows(g, F.bz, k, m, b[2], in);
+}
+
+// renew_grid, renew_b4, sr_grid
+template <typename T>
+__global__ void k_step2_b1(Geom2 g, FieldSet<T> F, T *zero, int nzero,
+                           const T *__restrict__ sig, T dtf, T dx, T e0) {
+  int k, m;
+  if (!node_of(g, k, m)) return;
+  for (int p = 0; p < nzero; ++p) zero[(int64_t)p * g.plane + g.idx(k, m)] = (T)0;
+  b_rows(g, F, sig, dtf, dx, e0, k, m);
+}
+
+// sr_current, external_current_perp and sr_density on the 8 planes from J,
+// renew_b4, sr_grid.  Rows 2 and NX+1 take in rows NX+2 and 1; the thread of
+// the row that takes in also sets an external current in either.
+template <typename T>
+__global__ void k_step2_b2(Geom2 g, FieldSet<T> F, T *J, const T *__restrict__ sig, T dtf,
+                           T dx, T e0, int ek, int em0, int em1, T v0, T v1) {
+  int k, m;
+  if (!node_of(g, k, m)) return;
+  const int from = k == 2 ? g.NX + 2 : k == g.NX + 1 ? 1 : -1;
+  if (from >= 0) {
+    for (int p = 0; p < 8; ++p) {
+      T *P = J + (int64_t)p * g.plane;
+      P[g.idx(k, m)] += P[g.idx(from, m)];
+    }
+  }
+  if ((m == em0 || m == em1) &&
+      (k == ek ? k != 1 && k != g.NX + 2 : from >= 0 && from == ek))
+    J[g.plane + g.idx(ek, m)] = m == em1 ? v1 : v0;
+  b_rows(g, F, sig, dtf, dx, e0, k, m);
+}
+
+// renew_e4 and sr_grid (last: with the rows of J, n and phi)
+template <typename T>
+__global__ void k_step2_e(Geom2 g, FieldSet<T> F, T *J, int ncopy, const T *__restrict__ sig,
+                          T dtf, T dx, T mu0, T C) {
+  int k, m;
+  if (!node_of(g, k, m) || k < 2 || k >= g.NX + 2) return;
+  const bool in = m >= 2 && m < g.NZ + 2;
+  const int r = image_row(g, k);
+  if (!in && r < 0) return;
+  const int64_t i = g.idx(k, m);
+  T e[3] = {F.ex[i], F.ey[i], F.ez[i]};
+  if (in) renew_e_node(g, F, sig, dtf, dx, mu0, C, k, m, e);
+  put_rows(g, F.ex, k, m, e[0], in);
+  put_rows(g, F.ey, k, m, e[1], in);
+  put_rows(g, F.ez, k, m, e[2], in);
+  if (r >= 0)
+    for (int p = 0; p < ncopy; ++p) {
+      T *P = J + (int64_t)p * g.plane;
+      P[g.idx(r, m)] = P[i];
+    }
+}
+
+// E += grad phi, phi, sr_grid with the rows of J, n and phi
+template <typename T>
+__global__ void k_step2_phi(Geom2 g, const T *__restrict__ rho, T *ex, T *ez, T *phi, T *J,
+                            int ncopy, T dx) {
+  int k, m;
+  if (!node_of(g, k, m) || k < 2 || k >= g.NX + 2) return;
+  const bool in = m >= 2 && m < g.NZ + 2;
+  const int r = image_row(g, k);
+  if (!in && r < 0) return;
+  const int64_t i = g.idx(k, m);
+  T a = ex[i], b = ez[i], p = phi[i];
+  if (in) phi_node(g, rho, k - 2, m - 2, a, b, p, dx);
+  put_rows(g, ex, k, m, a, in);
+  put_rows(g, ez, k, m, b, in);
+  put_rows(g, phi, k, m, p, in);
+  if (r >= 0)
+    for (int q = 0; q < ncopy; ++q) {
+      T *P = J + (int64_t)q * g.plane;
+      P[g.idx(r, m)] = P[i];
+    }
+}
+
+static dim3 node_grid(const Geom2 &g) {
+  return dim3((unsigned)div_up(g.SZ, kBlock), (unsigned)g.SX);
+}
+
+template <typename T>
+static int step_b1_t(pic2d_ctx *ctx, const T *sig) {
+  const pic2d_config &c = ctx->cfg;
+  k_step2_b1<T><<<node_grid(ctx->g), kBlock, 0, ctx->rt.stream>>>(
+      ctx->g, field_set<T>(ctx), plane<T>(ctx, PIC_JIX), PIC2D_PHI - PIC_JIX + 1, sig,
+      (T)c.dt, (T)c.dx, (T)c.eps0);
+  P2_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+template <typename T>
+static int step_b2_t(pic2d_ctx *ctx, const T *sig, int64_t step) {
+  const pic2d_config &c = ctx->cfg;
+  double v0 = 0, v1 = 0;
+  if (c.ext_k >= 0) external_values(c, step, v0, v1);
+  k_step2_b2<T><<<node_grid(ctx->g), kBlock, 0, ctx->rt.stream>>>(
+      ctx->g, field_set<T>(ctx), plane<T>(ctx, PIC_JIX), sig, (T)c.dt, (T)c.dx, (T)c.eps0,
+      c.ext_k, c.ext_k >= 0 ? c.ext_m[0] : -1, c.ext_k >= 0 ? c.ext_m[1] : -1, (T)v0, (T)v1);
+  P2_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+template <typename T>
+static int step_e_t(pic2d_ctx *ctx, const T *sig, bool with_phi) {
+  const pic2d_config &c = ctx->cfg;
+  T *J = plane<T>(ctx, PIC_JIX);
+  k_step2_e<T><<<node_grid(ctx->g), kBlock, 0, ctx->rt.stream>>>(
+      ctx->g, field_set<T>(ctx), J, with_phi ? 0 : PIC2D_PHI - PIC_JIX + 1, sig, (T)c.dt,
+      (T)c.dx, (T)c.mu0, (T)c.c);
+  P2_LAUNCH_CHECK(ctx);
+  if (!with_phi) return 0;
+  int rc = solve_phi<T>(ctx);
+  if (rc) return rc;
+  k_step2_phi<T><<<node_grid(ctx->g), kBlock, 0, ctx->rt.stream>>>(
+      ctx->g, (const T *)ctx->rho, plane<T>(ctx, PIC_EX), plane<T>(ctx, PIC_EZ),
+      plane<T>(ctx, PIC2D_PHI), J, 8, (T)c.dx);
+  P2_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+int step_b1(pic2d_ctx *ctx) {
+  return ctx->f64 ? step_b1_t<double>(ctx, ctx->sig64) : step_b1_t<float>(ctx, ctx->sig32);
+}
+
+int step_b2(pic2d_ctx *ctx, int64_t step) {
+  return ctx->f64 ? step_b2_t<double>(ctx, ctx->sig64, step)
+                  : step_b2_t<float>(ctx, ctx->sig32, step);
+}
+
+int step_e(pic2d_ctx *ctx, bool with_phi) {
+  return ctx->f64 ? step_e_t<double>(ctx, ctx->sig64, with_phi)
+                  : step_e_t<float>(ctx, ctx->sig32, with_phi);
 }
 
 // ---------------------------------------------------------------------------

@@ -92,6 +92,10 @@ struct pic2d_ctx {
   int64_t step = 0;
   int32_t c_add = 0, c_sort = 0;
   uint32_t inflow_event = 0;
+  // the guard rows of E, B and B0 are the images of the interior rows: set
+  // by halo and the step's own launches, cleared by whatever else writes
+  // those planes
+  bool guards_ok = false;
 
   // FP32 form: the tile sort's device lists (pic_tsort.h) and how many
   // sorts took the tile sort and the radix sort
@@ -138,6 +142,12 @@ int halo(pic2d_ctx *);
 int fold(pic2d_ctx *, int first, int count);
 int external_current(pic2d_ctx *, int64_t step);
 int poisson(pic2d_ctx *);
+// pic2d_step's field launches: renew_grid, the first renew_b4 and sr_grid;
+// sr_current, external_current_perp, sr_density, the second renew_b4 and
+// sr_grid; renew_e4, sr_grid and (with_phi) renew_phi and sr_grid
+int step_b1(pic2d_ctx *);
+int step_b2(pic2d_ctx *, int64_t step);
+int step_e(pic2d_ctx *, bool with_phi);
 int init_poisson(pic2d_ctx *);
 int diagnose_fields(pic2d_ctx *, pic2d_diag *);
 

@@ -26,39 +26,36 @@ struct Cplx {
 //   mode 1: out = S / A(l, k), 0 if A = 0   (forward, divided by the symbol
 //           A = -(sym_l[l] + sym_k[k]) / dq of the standard Laplacian)
 //   mode 2: out = 2 S / n                  (inverse)
+//   mode 3: both of 1 and then 2 on the same lines (forward, division,
+//           inverse): the lines stay with their workgroup, so nothing lies
+//           between the two transforms
+// Lines are read through src(line, element) the first time: the data
+// themselves, or the expression that a pass before would have written there.
 template <typename T>
-__global__ __launch_bounds__(256) void k_dst(T *__restrict__ data, int n, int logL,
-                                             int nlines, int ninner, int64_t sline,
-                                             int64_t souter, int64_t selem,
-                                             const Cplx<T> *__restrict__ tw, int mode,
-                                             const double *__restrict__ sym_l,
-                                             const double *__restrict__ sym_k,
-                                             double dq) {
-  extern __shared__ unsigned char lds_raw[];
-  T *re = (T *)lds_raw;
+struct LineData {
+  const T *data;
+  int ninner;
+  int64_t sline, souter, selem;
+  __device__ inline T operator()(int l, int j) const {
+    return data[(int64_t)(l / ninner) * souter + (int64_t)(l % ninner) * sline +
+                (int64_t)j * selem];
+  }
+};
+
+// one FFT of the two lines given by load_a / load_b (elements 1..n-1)
+template <typename T, typename LA, typename LB>
+__device__ inline void dst_fft(T *re, T *im, int n, int logL, const Cplx<T> *__restrict__ tw,
+                               LA load_a, LB load_b) {
   const int L = 2 * n;
-  T *im = re + L;
-  const int l0 = 2 * blockIdx.x;
-  const bool has_b = l0 + 1 < nlines;
-  const int64_t base_a = (int64_t)(l0 / ninner) * souter + (int64_t)(l0 % ninner) * sline;
-  const int64_t base_b =
-      (int64_t)((l0 + 1) / ninner) * souter + (int64_t)((l0 + 1) % ninner) * sline;
-  const T *A = data + base_a;
-  const T *B = data + base_b;
-  for (int j = threadIdx.x; j < L; j += blockDim.x) {
-    T a = 0, b = 0;
-    if (j != 0 && j != n) {
-      const int s = j < n ? j : L - j;
-      a = A[(int64_t)s * selem];
-      b = has_b ? B[(int64_t)s * selem] : (T)0;
-      if (j > n) {
-        a = -a;
-        b = -b;
-      }
-    }
+  for (int j = threadIdx.x; j < n; j += blockDim.x) {
+    // elements j and 2n - j of the odd extension (0 and n are zero)
     const int r = (int)(__brev((unsigned)j) >> (32 - logL));
+    const int r2 = (int)(__brev((unsigned)(j == 0 ? n : L - j)) >> (32 - logL));
+    const T a = j == 0 ? (T)0 : load_a(j), b = j == 0 ? (T)0 : load_b(j);
     re[r] = a;
     im[r] = b;
+    re[r2] = j == 0 ? (T)0 : -a;
+    im[r2] = j == 0 ? (T)0 : -b;
   }
   __syncthreads();
   for (int h = 1; h < L; h <<= 1) {
@@ -77,11 +74,28 @@ __global__ __launch_bounds__(256) void k_dst(T *__restrict__ data, int n, int lo
     }
     __syncthreads();
   }
-  T *OA = data + base_a;
-  T *OB = data + base_b;
+}
+
+template <typename T, typename Src>
+__global__ __launch_bounds__(256) void k_dst(T *data, Src src, int n, int logL,
+                                             int nlines, int ninner, int64_t sline,
+                                             int64_t souter, int64_t selem,
+                                             const Cplx<T> *__restrict__ tw, int mode,
+                                             const double *__restrict__ sym_l,
+                                             const double *__restrict__ sym_k,
+                                             double dq) {
+  extern __shared__ unsigned char lds_raw[];
+  T *re = (T *)lds_raw;
+  T *im = re + 2 * n;
+  const int l0 = 2 * blockIdx.x;
+  const bool has_b = l0 + 1 < nlines;
+  T *A = data + (int64_t)(l0 / ninner) * souter + (int64_t)(l0 % ninner) * sline;
+  T *B = data + (int64_t)((l0 + 1) / ninner) * souter + (int64_t)((l0 + 1) % ninner) * sline;
+  dst_fft(re, im, n, logL, tw, [&](int j) { return src(l0, j); },
+          [&](int j) { return has_b ? src(l0 + 1, j) : (T)0; });
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     T sa = -im[k] / (T)2, sb = re[k] / (T)2;
-    if (mode == 1) {
+    if (mode & 1) {
       const double Aa = -(sym_l[l0] + sym_k[k]) / dq;
       sa = Aa == 0. ? (T)0 : (T)(sa / (T)Aa);
       if (has_b) {
@@ -92,8 +106,16 @@ __global__ __launch_bounds__(256) void k_dst(T *__restrict__ data, int n, int lo
       sa = (T)2 * sa / (T)n;
       sb = (T)2 * sb / (T)n;
     }
-    OA[(int64_t)k * selem] = sa;
-    if (has_b) OB[(int64_t)k * selem] = sb;
+    A[(int64_t)k * selem] = sa;
+    if (has_b) B[(int64_t)k * selem] = sb;
+  }
+  if (mode != 3) return;
+  __syncthreads();  // this workgroup's stores before its loads
+  dst_fft(re, im, n, logL, tw, [&](int j) { return A[(int64_t)j * selem]; },
+          [&](int j) { return has_b ? B[(int64_t)j * selem] : (T)0; });
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    A[(int64_t)k * selem] = (T)2 * (-im[k] / (T)2) / (T)n;
+    if (has_b) B[(int64_t)k * selem] = (T)2 * (re[k] / (T)2) / (T)n;
   }
 }
 

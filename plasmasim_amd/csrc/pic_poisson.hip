@@ -127,17 +127,17 @@ int run(pic_ctx *ctx) {
   const Pass px{0, g.NY * g.NZ, g.NY * g.NZ, 1, 0, NYZ};
   auto launch = [&](const Pass &p, int mode) {
     const int n = N[p.axis];
+    const LineData<T> src{rho, p.ninner, p.sline, p.souter, p.selem};
     k_dst<T><<<(unsigned)div_up(p.nlines, 2), 256, (size_t)4 * n * sizeof(T), st>>>(
-        rho, n, ilog2_ceil(2 * n), p.nlines, p.ninner, p.sline, p.souter, p.selem,
-        tw[p.axis], mode, mode == 1 ? ctx->sym_yz : nullptr,
-        mode == 1 ? sym[0] : nullptr, dq);
+        rho, src, n, ilog2_ceil(2 * n), p.nlines, p.ninner, p.sline, p.souter, p.selem,
+        tw[p.axis], mode, mode == 3 ? ctx->sym_yz : nullptr,
+        mode == 3 ? sym[0] : nullptr, dq);
   };
-  // fft_z, fft_y, fft_x, division (:8360-8512), inv_fft_x, inv_fft_y,
-  // inv_fft_z (:8517-8653)
+  // fft_z, fft_y, fft_x, division (:8360-8512) and inv_fft_x in one launch,
+  // inv_fft_y, inv_fft_z (:8517-8653)
   launch(pz, 0);
   launch(py, 0);
-  launch(px, 1);
-  launch(px, 2);
+  launch(px, 3);
   launch(py, 2);
   launch(pz, 2);
   PIC_LAUNCH_CHECK(ctx);
