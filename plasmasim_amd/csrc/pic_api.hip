@@ -900,7 +900,7 @@ extern "C" int pic_thrust_ave_enable(pic_ctx *ctx, int on) {
   // workgroups of one pass: the tiles and the tail chunks of up to the
   // capacity's slots
   const int64_t boxes = tg.ntiles() == 1 ? row_geom(tg).ntiles() : tg.ntiles();
-  const int64_t slots = boxes + div_up(ctx->cap, tail_chunk(ctx->cfg.ppc, false)) + 1;
+  const int64_t slots = boxes + most_chunks(ctx->cfg.ppc, ctx->cap);
   if (!ctx->thrust_acc) PIC_HIP(ctx, hipMalloc(&ctx->thrust_acc, 16 * sizeof(double)));
   if (ctx->thrust_part_slots < slots) {
     if (ctx->thrust_part) (void)hipFree(ctx->thrust_part);

@@ -1991,7 +1991,8 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   }
   if (tr.ntiles == 0) tr.sorted_end = 0;
   tr.n = n;
-  tr.chunk = tail_chunk(ctx->cfg.ppc, ctx->geom.NX % 4 == 0 && ctx->geom.NY % 4 == 0);
+  tr.chunk = tail_chunk(ctx->cfg.ppc, ctx->geom.NX % 4 == 0 && ctx->geom.NY % 4 == 0,
+                        n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
   const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
   if (nb == 0) return settle(ctx, sp);

@@ -1319,7 +1319,7 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   }
   if (tr.ntiles == 0) tr.sorted_end = 0;
   tr.n = n;
-  tr.chunk = tail_chunk(ctx->cfg.ppc, false);
+  tr.chunk = tail_chunk(ctx->cfg.ppc, false, n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
   const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
   const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);

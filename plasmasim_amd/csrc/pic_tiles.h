@@ -19,17 +19,29 @@ constexpr int kMargin = 3;
 constexpr int kTailChunk = 2048;  // most slots per workgroup of the tail
 constexpr int kStray = 8;
 
-// Slots per workgroup of the unsorted inflow tail.  An inflow batch walks
-// its two-layer slab in blocks of 4 x 4 x 2 cells (blocked) or along y in
-// columns of 2 cells, ppc slots per cell; the window holds 3 blocks or 16
+// Slots per workgroup of the unsorted tail of `tail` slots.  An inflow batch
+// walks its two-layer slab in blocks of 4 x 4 x 2 cells (blocked) or along y
+// in columns of 2 cells, ppc slots per cell; the window holds 3 blocks or 16
 // columns (kStray cells to either side of the middle sample), so a chunk of
 // more slots than that has no window and adds every contribution to the
-// global planes.
-inline int tail_chunk(int ppc, bool blocked) {
+// global planes.  A tail too short to give every place on the chip (3
+// workgroups per CU) a chunk is cut finer: it runs last, so its longest chunk
+// is what the launch waits for, and the overflow of the in-tile inflow, some
+// hundred slots per slab tile in tile order, spans few tiles per chunk.  In
+// chunks of 2048 that overflow cost 60 us of 330 us per launch at
+// 64^3 x 32 ppc.
+constexpr int kChipSlots = 768;
+inline int tail_chunk(int ppc, bool blocked, int64_t tail) {
   const int64_t most = (int64_t)(blocked ? 64 : 32) * ppc;
   int c = kTailChunk;
-  while (c > 256 && c > most) c >>= 1;
+  while (c > 256 && (c > most || tail < (int64_t)kChipSlots * c)) c >>= 1;
   return c;
+}
+// most workgroups that a store of cap slots can need for its tail
+inline int64_t most_chunks(int ppc, int64_t cap) {
+  const int64_t c = tail_chunk(ppc, false, cap);
+  const int64_t few = (int64_t)kChipSlots * kTailChunk / 256;
+  return ((cap + c - 1) / c > few ? (cap + c - 1) / c : few) + 1;
 }
 
 struct TileRun {
@@ -58,7 +70,7 @@ inline TileGeom row_geom(const TileGeom &one) {
     t.NTX = up(NX, w);
     t.NTY = up(NY, w);
     t.NTZ = up(NZ, 8);
-    if (t.ntiles() >= 768) break;
+    if (t.ntiles() >= kChipSlots) break;
   }
   t.LX = t.LY = t.LZ = -1;
   return t;
