@@ -273,7 +273,8 @@ int pic_get_counters(const pic_ctx *ctx, int64_t *step, int32_t *c_add,
 int pic_set_counters(pic_ctx *ctx, int64_t step, int32_t c_add, int32_t c_sort);
 
 /* ---- kernel timing (HIP events on the context stream) ---- */
-#define PIC_T_PUSH 0     /* fused particle pass */
+#define PIC_T_PUSH 0     /* fused particle pass; one per species, also where
+                          * a launch takes both */
 #define PIC_T_FIELD_B 1  /* B half-step */
 #define PIC_T_FIELD_E 2  /* E step */
 #define PIC_T_SORT 3

@@ -1165,8 +1165,7 @@ int fwd_step(pic_ctx *ctx, TapeStep &ts, double *tape_fields, PD tape_p[2],
   }
   if ((rc = pic_renew_b_half(ctx))) return rc;
   if ((rc = pic_halo_b(ctx))) return rc;
-  for (int s = 0; s < 2; ++s)
-    if ((rc = push_fused(ctx, s))) return rc;
+  if ((rc = push_fused(ctx))) return rc;
   if ((rc = pic_renew_b_half(ctx))) return rc;
   if ((rc = pic_halo_b(ctx))) return rc;
   if ((rc = pic_fold_current(ctx))) return rc;

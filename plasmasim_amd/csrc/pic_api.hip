@@ -60,10 +60,11 @@ void timing_begin(pic_ctx *ctx, int which) {
   (void)hipEventRecord(ctx->tev[0][ctx->tpending], ctx->stream);
 }
 
-void timing_end(pic_ctx *ctx, int which) {
+void timing_end(pic_ctx *ctx, int which, int passes) {
   if (!timed(ctx, which)) return;
   (void)hipEventRecord(ctx->tev[1][ctx->tpending], ctx->stream);
   ctx->tclass[ctx->tpending] = which;
+  ctx->tpasses[ctx->tpending] = passes;
   ctx->tpending++;
 }
 
@@ -74,7 +75,7 @@ int timing_flush(pic_ctx *ctx) {
     float ms = 0.f;
     PIC_HIP(ctx, hipEventElapsedTime(&ms, ctx->tev[0][i], ctx->tev[1][i]));
     ctx->t_ms[ctx->tclass[i]] += ms;
-    ctx->t_n[ctx->tclass[i]] += 1;
+    ctx->t_n[ctx->tclass[i]] += ctx->tpasses[i];
   }
   ctx->tpending = 0;
   return 0;
@@ -956,10 +957,12 @@ extern "C" int pic_thrust_ave_get(pic_ctx *ctx, double F[27], int64_t *nsteps,
 }
 
 namespace pic {
-int push_fused(pic_ctx *ctx, int sp) {
-  timing_begin(ctx, PIC_T_PUSH);
-  int rc = DISPATCH(push, ctx, sp, 1, 1, 1);
-  timing_end(ctx, PIC_T_PUSH);
+int push_fused(pic_ctx *ctx) {
+  const bool sorting = !is_f64(ctx) && (f32::pending(ctx, 0) || f32::pending(ctx, 1));
+  const int tclass = sorting ? PIC_T_PUSH_SORT : PIC_T_PUSH;
+  timing_begin(ctx, tclass);
+  int rc = DISPATCH(push_both, ctx);
+  timing_end(ctx, tclass, 2);
   return rc;
 }
 }  // namespace pic
@@ -1023,16 +1026,11 @@ extern "C" int pic_step(pic_ctx *ctx, int nsteps) {
     FIELD(PIC_T_FIELD_B, step_b1, ctx, ctx->thrust_pending != 0);
     ctx->thrust_now = ctx->thrust_pending;
     ctx->thrust_nb[0] = ctx->thrust_nb[1] = 0;
-    for (int sp = 0; sp < 2; ++sp) {
-      const int tclass = !f64 && f32::pending(ctx, sp) ? PIC_T_PUSH_SORT : PIC_T_PUSH;
-      timing_begin(ctx, tclass);
-      rc = DISPATCH(push, ctx, sp, 1, 1, 1);
-      timing_end(ctx, tclass);
-      if (rc) {
-        ctx->thrust_now = 0;
-        if (!f64) (void)f32::settle_sorts(ctx);
-        return rc;
-      }
+    rc = push_fused(ctx);
+    if (rc) {
+      ctx->thrust_now = 0;
+      if (!f64) (void)f32::settle_sorts(ctx);
+      return rc;
     }
     timing_begin(ctx, PIC_T_FIELD_B);
     rc = DISPATCH(step_b2, ctx);

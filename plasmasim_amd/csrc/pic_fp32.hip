@@ -620,6 +620,20 @@ __device__ inline void thrust_store(const float (&th)[6], double *out, int bid) 
   }
 }
 
+// One species' arguments of a pass; a launch takes one species or both.
+struct SpeciesArgs32 {
+  TileGeom tg;
+  TileRun tr;
+  Particles32 P, Q;
+  const uint32_t *perm;
+  Push32 kp;
+  void *dep[4];  // jx, jy, jz, n: float planes, or fixed-point ones (DET)
+  double *thrust_part;
+};
+struct PassArgs32 {
+  SpeciesArgs32 s[2];
+};
+
 // PERM: the pass also applies a sort's permutation: slot i takes its
 // particle from slot perm[i] of the arrays Q and stores the result in P (the
 // other buffer of the species), so the sort needs no separate copy
@@ -627,21 +641,30 @@ __device__ inline void thrust_store(const float (&th)[6], double *out, int bid) 
 // columns (row_geom), its threads divided evenly over the box's columns, so
 // that all of them load at once.  31 x 27 x 45 x 8 ppc on one workgroup
 // (the one tile's) took 7.26 ms per launch; in boxes 73 us.
+// BOTH: the launch holds both species, the first nb0 workgroups the ions'.
 template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool DET, bool THRUST, bool PERM,
-          bool ROWS>
+          bool ROWS, bool BOTH>
 __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
-    Grid32 G, TileGeom tg, Particles32 P, TileRun tr, Push32 kp,
-    typename GlobT<DET>::T *jx, typename GlobT<DET>::T *jy,
-    typename GlobT<DET>::T *jz, typename GlobT<DET>::T *nd, double *thrust_part,
-    Particles32 Q, const uint32_t *__restrict__ perm) {
+    Grid32 G, PassArgs32 args, int nb0) {
   using A = typename GlobT<DET>::T;
+  const int sp = BOTH && (int)blockIdx.x >= nb0 ? 1 : 0;
+  const SpeciesArgs32 &a = args.s[sp];
+  const TileGeom &tg = a.tg;
+  const Particles32 &P = a.P, &Q = a.Q;
+  const TileRun &tr = a.tr;
+  const Push32 &kp = a.kp;
+  const uint32_t *__restrict__ perm = a.perm;
+  A *const jx = (A *)a.dep[0], *const jy = (A *)a.dep[1], *const jz = (A *)a.dep[2],
+    *const nd = (A *)a.dep[3];
+  double *const thrust_part = a.thrust_part;
   __shared__ u64 acc_mem[4 * kWin];
   __shared__ Win sw;
   __shared__ int64_t s_range[2];
   __shared__ int s_box;
   const Geom &g = G.g;
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.ntiles, BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.ntiles, (int)gridDim.x - nb0);
 
   if (tid == 0) {
     int64_t s, e;
@@ -1955,14 +1978,12 @@ static Push32 push_const(const pic_ctx *ctx, int sp) {
   return p;
 }
 
-int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
-         int do_boundary) {
-  // a pending sort permutation is applied by the fused pass only
-  const bool fused = do_push_j && do_drift_n && do_boundary;
-  if (!fused) {
-    int rc = settle(ctx, sp);
-    if (rc) return rc;
-  }
+// One species' arguments of a pass (push J / drift n / boundary); *nb is its
+// number of workgroups, 0 when there is nothing to do.
+static int prepare_pass(pic_ctx *ctx, int sp, int sel, SpeciesArgs32 &a, bool *rows,
+                        unsigned *nb) {
+  State32 *S = st(ctx);
+  *nb = 0;
   const int64_t n = ctx->n[sp];
   if (n == 0) return 0;
   // slot indices and byte offsets of the pass are 32-bit
@@ -1970,19 +1991,16 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     return set_error(ctx, PIC_E_CAPACITY,
                      "fp32 particle pass: %lld stored particles of one species "
                      "exceed 2^30 (32-bit byte offsets)", (long long)n);
-  State32 *S = st(ctx);
   TileGeom tg = tile_geom(ctx);
   add_drift_shift(tg, ctx->cfg, ctx->drift_halves[sp]);
-  ctx->drift_halves[sp] += (do_push_j ? 1 : 0) + (do_drift_n ? 1 : 0);
   TileRun tr;
   tr.tile_start = ctx->tile_start[sp];
   tr.sorted_end = ctx->sorted_end[sp];
   tr.ntiles = tr.sorted_end > 0 ? tg.ntiles() : 0;
   // one tile: boxes of rows while the sort's cell starts are current,
   // otherwise chunks as an unsorted tail
-  const bool rows = tr.ntiles == 1 && ctx->row_start[sp] &&
-                    ctx->row_end[sp] == tr.sorted_end;
-  if (rows) {
+  *rows = tr.ntiles == 1 && ctx->row_start[sp] && ctx->row_end[sp] == tr.sorted_end;
+  if (*rows) {
     tg = row_geom(tg);
     tr.tile_start = ctx->row_start[sp];
     tr.ntiles = tg.ntiles();
@@ -1994,98 +2012,135 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   tr.chunk = tail_chunk(ctx->cfg.ppc, ctx->geom.NX % 4 == 0 && ctx->geom.NY % 4 == 0,
                         n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
-  const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
-  if (nb == 0) return settle(ctx, sp);
+  const unsigned blocks = (unsigned)(tr.ntiles + tr.ntail);
+  a.tg = tg;
+  a.tr = tr;
+  Push32 &kp = a.kp;
+  kp = push_const(ctx, sp);
   // with a pending permutation the pass reads the current buffer through it
   // and writes the other one
-  const uint32_t *pm = S->pending[sp] ? pass_perm(ctx, sp) : nullptr;
-  Particles32 Q = p32(ctx, sp, ctx->cur[sp]);
-  Particles32 P = pm ? p32(ctx, sp, 1 - ctx->cur[sp]) : Q;
-  Push32 kp = push_const(ctx, sp);
-  Grid32 G = grid32(ctx);
-  const bool det = S->fx != nullptr;
-  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
-  // The fused pass always runs the instantiation that can add the previous
-  // step's thrust_fave (its push and deposit arithmetic is then the same
-  // whether or not the sum is on: the unit contracts floating-point
-  // operations freely, and two instantiations could round differently);
-  // without a partials buffer it adds nothing.
-  const bool thrust = ctx->thrust_now && sel == 7;
-  double *tp = nullptr;
-  if (thrust) {
-    if ((int64_t)nb > ctx->thrust_part_slots)
+  a.perm = S->pending[sp] ? pass_perm(ctx, sp) : nullptr;
+  a.Q = p32(ctx, sp, ctx->cur[sp]);
+  a.P = a.perm ? p32(ctx, sp, 1 - ctx->cur[sp]) : a.Q;
+  if (S->fx) {
+    const int64_t pl = ctx->geom.plane;
+    for (int c = 0; c < 3; ++c) a.dep[c] = S->fx + ((sp == PIC_ION ? 0 : 3) + c) * pl;
+    a.dep[3] = S->fx + (sp == PIC_ION ? 6 : 7) * pl;
+  } else {
+    Fields<float> F = fields<float>(ctx);
+    for (int c = 0; c < 3; ++c) a.dep[c] = F.f[(sp == PIC_ION ? PIC_JIX : PIC_JEX) + c];
+    a.dep[3] = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
+  }
+  // the fused pass adds the previous step's thrust_fave; without a partials
+  // buffer it adds nothing
+  a.thrust_part = nullptr;
+  if (ctx->thrust_now && sel == 7) {
+    if ((int64_t)blocks > ctx->thrust_part_slots)
       return set_error(ctx, PIC_E_CAPACITY, "thrust: %u workgroups, %lld partial slots",
-                       nb, (long long)ctx->thrust_part_slots);
-    tp = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
+                       blocks, (long long)ctx->thrust_part_slots);
+    a.thrust_part = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
     // the kept end-of-step B is the upper half of the 6-plane bt block
     kp.bprev = (uint32_t)(3 * ctx->geom.plane * sizeof(float));
     // farthest a particle moved from its tile since the sort, beyond the
     // window's drift shift: |v| < c per half step, h halves before this pass
     const pic_config &c = ctx->cfg;
-    const int h = ctx->drift_halves[sp] - 2;  // incremented above for this pass
+    const int h = ctx->drift_halves[sp];
     int smax = 0;
-    for (int a = 0; a < 3; ++a) smax = std::max(smax, std::abs(tg.shift[a]));
+    for (int x = 0; x < 3; ++x) smax = std::max(smax, std::abs(tg.shift[x]));
     kp.box_margin = (int)ceil(h * 0.5 * c.c * c.dt / c.dx) + smax + 1;
     // a particle that wrapped across a periodic face lies within the margin
     // of the opposite face; only while that stays outside the box may whole
     // tiles be classified
     if (kp.box_margin + 2 >= 0.2 * std::min(c.nx, c.ny)) kp.box_margin = 1 << 20;
+    ctx->thrust_nb[sp] = (int)blocks;  // finished by step_b2
   }
+  ctx->drift_halves[sp] += (sel & 4 ? 1 : 0) + (sel & 2 ? 1 : 0);
+  *nb = blocks;
+  return 0;
+}
+
+// the pass sel of one species (args.s[0], nb[1] = 0) or, fused, of both
+static int launch_pass(pic_ctx *ctx, int sel, bool perm, bool rows, const PassArgs32 &args,
+                       const unsigned nb[2]) {
+  State32 *S = st(ctx);
+  const unsigned n = nb[0] + nb[1];
+  if (n == 0) return 0;
+  const Grid32 G = grid32(ctx);
   // DET, then the pass: push and J, drift and n, the boundary, or all three
   // (only a fused pass applies a permutation, and a store sorted as one
   // tile has none to apply)
-#define L(DET, ROWS, ...)                                                              \
-  switch (sel) {                                                                       \
-    case 7:                                                                            \
-      if (pm)                                                                          \
-        k_particles32<true, true, true, DET, true, true, false>                        \
-            <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
-      else                                                                             \
-        k_particles32<true, true, true, DET, true, false, ROWS>                        \
-            <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
-      break;                                                                           \
-    case 4:                                                                            \
-      k_particles32<true, false, false, DET, false, false, ROWS>                       \
-          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
-      break;                                                                           \
-    case 2:                                                                            \
-      k_particles32<false, true, false, DET, false, false, ROWS>                       \
-          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
-      break;                                                                           \
-    case 1:                                                                            \
-      k_particles32<false, false, true, DET, false, false, ROWS>                       \
-          <<<nb, kPassBlock, 0, ctx->stream>>>(G, tg, P, tr, kp, __VA_ARGS__, tp, Q, pm); \
-      break;                                                                           \
-    default:                                                                           \
-      return set_error(ctx, PIC_E_ARG, "particle pass %d", sel);                       \
-  }
-  if (det) {
-    const int64_t pl = ctx->geom.plane;
-    unsigned long long *j = S->fx + (sp == PIC_ION ? 0 : 3) * pl,
-                       *nd = S->fx + (sp == PIC_ION ? 6 : 7) * pl;
-    if (rows) {
-      L(true, true, j, j + pl, j + 2 * pl, nd)
-    } else {
-      L(true, false, j, j + pl, j + 2 * pl, nd)
-    }
-    if (do_push_j || do_drift_n) S->fx_dirty = true;
-  } else {
-    Fields<float> F = fields<float>(ctx);
-    const int j = sp == PIC_ION ? PIC_JIX : PIC_JEX;
-    float *nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
-    if (rows) {
-      L(false, true, F.f[j], F.f[j + 1], F.f[j + 2], nd)
-    } else {
-      L(false, false, F.f[j], F.f[j + 1], F.f[j + 2], nd)
-    }
-  }
+#define F(DET, ROWS, BOTH)                                              \
+  (perm ? k_particles32<true, true, true, DET, true, true, false, BOTH> \
+        : k_particles32<true, true, true, DET, true, false, ROWS, BOTH>)
+#define L(DET, ROWS)                                                                     \
+  (sel == 7 ? (nb[1] ? F(DET, ROWS, true) : F(DET, ROWS, false))                         \
+   : sel == 4 ? k_particles32<true, false, false, DET, false, false, ROWS, false>        \
+   : sel == 2 ? k_particles32<false, true, false, DET, false, false, ROWS, false>        \
+              : k_particles32<false, false, true, DET, false, false, ROWS, false>)
+  const auto kern = S->fx ? (rows ? L(true, true) : L(true, false))
+                          : (rows ? L(false, true) : L(false, false));
 #undef L
+#undef F
+  kern<<<n, kPassBlock, 0, ctx->stream>>>(G, args, (int)nb[0]);
   PIC_LAUNCH_CHECK(ctx);
-  if (pm) {
-    ctx->cur[sp] = 1 - ctx->cur[sp];
-    S->pending[sp] = false;
+  if (S->fx && (sel & 6)) S->fx_dirty = true;
+  return 0;
+}
+
+static void pass_done(pic_ctx *ctx, int sp, const SpeciesArgs32 &a) {
+  if (!a.perm) return;
+  ctx->cur[sp] = 1 - ctx->cur[sp];
+  st(ctx)->pending[sp] = false;
+}
+
+int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
+         int do_boundary) {
+  // a pending sort permutation is applied by the fused pass only
+  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
+  if (sel != 7) {
+    int rc = settle(ctx, sp);
+    if (rc) return rc;
   }
-  if (thrust) ctx->thrust_nb[sp] = (int)nb;  // finished by step_b2
+  PassArgs32 args;
+  memset(&args, 0, sizeof args);
+  bool rows = false;
+  unsigned nb[2] = {0, 0};
+  int rc = prepare_pass(ctx, sp, sel, args.s[0], &rows, &nb[0]);
+  if (!rc) rc = launch_pass(ctx, sel, args.s[0].perm != nullptr, rows, args, nb);
+  if (rc) return rc;
+  if (nb[0]) pass_done(ctx, sp, args.s[0]);
+  return 0;
+}
+
+// The fused passes of both species, in one launch where both are in the same
+// state (tiles, boxes or chunks; a permutation or none) and leave places
+// empty (kBothBlocks).
+int push_both(pic_ctx *ctx) {
+  PassArgs32 args;
+  memset(&args, 0, sizeof args);
+  bool rows[2] = {false, false};
+  unsigned nb[2] = {0, 0};
+  for (int sp = 0; sp < 2; ++sp) {
+    int rc = prepare_pass(ctx, sp, 7, args.s[sp], &rows[sp], &nb[sp]);
+    if (rc) return rc;
+  }
+  const bool perm[2] = {args.s[0].perm != nullptr, args.s[1].perm != nullptr};
+  if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks && rows[0] == rows[1] &&
+      perm[0] == perm[1]) {
+    int rc = launch_pass(ctx, 7, perm[0], rows[0], args, nb);
+    if (rc) return rc;
+  } else {
+    for (int sp = 0; sp < 2; ++sp) {
+      PassArgs32 one = args;
+      one.s[0] = args.s[sp];
+      const unsigned n[2] = {nb[sp], 0};
+      int rc = launch_pass(ctx, 7, perm[sp], rows[sp], one, n);
+      if (rc) return rc;
+      if (nb[sp]) pass_done(ctx, sp, args.s[sp]);
+    }
+    return 0;
+  }
+  for (int sp = 0; sp < 2; ++sp) pass_done(ctx, sp, args.s[sp]);
   return 0;
 }
 

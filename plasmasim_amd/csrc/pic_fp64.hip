@@ -676,6 +676,19 @@ struct PassFields {
   double *jx, *jy, *jz, *nd;
 };
 
+// One species' arguments of a pass; a launch takes one species or both.
+struct SpeciesArgs64 {
+  TileGeom tg;
+  TileRun tr;
+  PassFields F;
+  Particles64 P;
+  PassConst kc;
+  double *thrust_part;
+};
+struct PassArgs64 {
+  SpeciesArgs64 s[2];
+};
+
 // One particle pass.  PUSH_J: hot loop A (:731-812); DRIFT_N: hot loop B
 // (:818-867); BOUNDARY: sr_particle (:2041-2531) on one rank.  The fused
 // form (all three) is exact because none of the field updates between those
@@ -688,16 +701,26 @@ struct PassFields {
 // tile, the threads divided evenly over a box's columns.  32^3 x 16 ppc in
 // chunks of 2048 slots, whose boxes fit no window, took 475 us per launch
 // and in boxes 90 us; 8 x 8 x 16 x 4 ppc 70 us and 18 us.
-template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST, bool ROWS, bool UNIT>
+// BOTH: the launch holds both species, the first nb0 workgroups the ions'.
+template <bool PUSH_J, bool DRIFT_N, bool BOUNDARY, bool THRUST, bool ROWS, bool UNIT,
+          bool BOTH>
 __global__ __launch_bounds__(256) void k_particles_tiled(
-    Geom g, TileGeom tg, PassFields F, Particles64 P, TileRun tr, PassConst kc,
-    double *thrust_part) {
+    Geom g, PassArgs64 args, int nb0) {
   using O = typename Off<UNIT>::T;
+  const int sp = BOTH && (int)blockIdx.x >= nb0 ? 1 : 0;
+  const SpeciesArgs64 &sa = args.s[sp];
+  const TileGeom &tg = sa.tg;
+  const TileRun &tr = sa.tr;
+  const PassFields &F = sa.F;
+  const Particles64 &P = sa.P;
+  const PassConst &kc = sa.kc;
+  double *const thrust_part = sa.thrust_part;
   __shared__ double acc_mem[4 * kWin64];
   __shared__ Win sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.ntiles, BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.ntiles, (int)gridDim.x - nb0);
   const double dx = UNIT ? 1.0 : kc.dx;
   if (tid == 0) {
     int64_t s, e;
@@ -1255,14 +1278,17 @@ int load_particles(pic_ctx *ctx) {
   return 0;
 }
 
-int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
-         int do_boundary) {
+// One species' arguments of a pass (push J / drift n / boundary); *nb is its
+// number of workgroups, 0 when there is nothing to do.
+static int prepare_pass(pic_ctx *ctx, int sp, int sel, SpeciesArgs64 &a, bool *rows,
+                        unsigned *nb) {
+  *nb = 0;
   const int64_t n = ctx->n[sp];
   if (n == 0) return 0;
   Fields<double> F = fields<double>(ctx);
-  Particles64 P = p64(ctx, sp, ctx->cur[sp]);
+  a.P = p64(ctx, sp, ctx->cur[sp]);
   const StepConst sc = step_const(ctx, sp);
-  PassConst kc;
+  PassConst &kc = a.kc;
   {
     const double dx = sc.dx;
     kc.dx = dx;
@@ -1278,29 +1304,28 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
     kc.qn = sc.q * sc.weight / (dx * dx * dx);
     kc.wn = sc.weight / (dx * dx * dx);
     const int N[3] = {ctx->geom.NX, ctx->geom.NY, ctx->geom.NZ};
-    for (int a = 0; a < 3; ++a) {
-      kc.blo[a] = sc.blo[a];
-      kc.bhi[a] = sc.bhi[a];
-      kc.box_lo[a] = N[a] * dx * 0.2;
-      kc.box_hi[a] = N[a] * dx * 0.8;
+    for (int x = 0; x < 3; ++x) {
+      kc.blo[x] = sc.blo[x];
+      kc.bhi[x] = sc.bhi[x];
+      kc.box_lo[x] = N[x] * dx * 0.2;
+      kc.box_hi[x] = N[x] * dx * 0.8;
     }
     kc.periodic[0] = sc.periodic[0];
     kc.periodic[1] = sc.periodic[1];
   }
-  PassFields pf;
   const double *kept = (const double *)ctx->thrust_bprev;
   for (int q = 0; q < 3; ++q) {
-    pf.e[q] = F.f[PIC_EX + q];
-    pf.b[q] = F.f[PIC_BX + q];
-    pf.bp[q] = kept + q * ctx->geom.plane;
+    a.F.e[q] = F.f[PIC_EX + q];
+    a.F.b[q] = F.f[PIC_BX + q];
+    a.F.bp[q] = kept + q * ctx->geom.plane;
   }
-  pf.jx = F.f[sp == PIC_ION ? PIC_JIX : PIC_JEX];
-  pf.jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
-  pf.jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
-  pf.nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
+  a.F.jx = F.f[sp == PIC_ION ? PIC_JIX : PIC_JEX];
+  a.F.jy = F.f[sp == PIC_ION ? PIC_JIY : PIC_JEY];
+  a.F.jz = F.f[sp == PIC_ION ? PIC_JIZ : PIC_JEZ];
+  a.F.nd = F.f[sp == PIC_ION ? PIC_NI : PIC_NE];
   TileGeom tg = tile_geom(ctx);
   add_drift_shift(tg, ctx->cfg, ctx->drift_halves[sp]);
-  ctx->drift_halves[sp] += (do_push_j ? 1 : 0) + (do_drift_n ? 1 : 0);
+  ctx->drift_halves[sp] += (sel & 4 ? 1 : 0) + (sel & 2 ? 1 : 0);
   TileRun tr;
   tr.tile_start = ctx->tile_start[sp];
   tr.sorted_end = ctx->sorted_end[sp];
@@ -1308,9 +1333,9 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   // a single tile (the reference's order): boxes of rows while the sort's
   // cell starts are current, otherwise chunks as an unsorted tail (slots of
   // the rows are 32-bit)
-  const bool rows = tr.ntiles == 1 && ctx->row_start[sp] &&
-                    ctx->row_end[sp] == tr.sorted_end && n <= ((int64_t)1 << 30);
-  if (rows) {
+  *rows = tr.ntiles == 1 && ctx->row_start[sp] && ctx->row_end[sp] == tr.sorted_end &&
+          n <= ((int64_t)1 << 30);
+  if (*rows) {
     tg = row_geom(tg);
     tr.tile_start = ctx->row_start[sp];
     tr.ntiles = tg.ntiles();
@@ -1321,48 +1346,79 @@ int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
   tr.n = n;
   tr.chunk = tail_chunk(ctx->cfg.ppc, false, n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
-  const unsigned nb = (unsigned)(tr.ntiles + tr.ntail);
-  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
+  a.tg = tg;
+  a.tr = tr;
+  const unsigned blocks = (unsigned)(tr.ntiles + tr.ntail);
   // the fused pass of pic_step adds the previous step's thrust_fave
-  const bool thrust = ctx->thrust_now && sel == 7;
-  double *tp = nullptr;
-  if (thrust) {
-    if ((int64_t)nb > ctx->thrust_part_slots)
+  a.thrust_part = nullptr;
+  if (ctx->thrust_now && sel == 7) {
+    if ((int64_t)blocks > ctx->thrust_part_slots)
       return set_error(ctx, PIC_E_CAPACITY, "thrust: %u workgroups, %lld partial slots",
-                       nb, (long long)ctx->thrust_part_slots);
-    tp = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
+                       blocks, (long long)ctx->thrust_part_slots);
+    a.thrust_part = ctx->thrust_part + (int64_t)sp * 6 * ctx->thrust_part_slots;
+    ctx->thrust_nb[sp] = (int)blocks;  // finished by step_b2
   }
+  *nb = blocks;
+  return 0;
+}
+
+// the pass sel of one species (args.s[0], nb[1] = 0) or, fused, of both
+static int launch_pass(pic_ctx *ctx, int sel, bool rows, const PassArgs64 &args,
+                       const unsigned nb[2]) {
+  const unsigned n = nb[0] + nb[1];
+  if (n == 0) return 0;
   // normalised units with 32-bit byte offsets, or any dx with 64-bit ones
-  const bool unit = ctx->cfg.dx == 1.0 && n < ((int64_t)1 << 29) &&
+  const int64_t most = ctx->n[0] > ctx->n[1] ? ctx->n[0] : ctx->n[1];
+  const bool unit = ctx->cfg.dx == 1.0 && most < ((int64_t)1 << 29) &&
                     ctx->geom.plane < ((int64_t)1 << 29);
-#define LAUNCH2(A, B, C, T, R)                                                   \
-  do {                                                                           \
-    if (unit)                                                                    \
-      k_particles_tiled<A, B, C, T, R, true><<<nb, kBlock, 0, ctx->stream>>>(    \
-          ctx->geom, tg, pf, P, tr, kc, tp);                                     \
-    else                                                                         \
-      k_particles_tiled<A, B, C, T, R, false><<<nb, kBlock, 0, ctx->stream>>>(   \
-          ctx->geom, tg, pf, P, tr, kc, tp);                                     \
-  } while (0)
-#define LAUNCH(A, B, C, T)                                                       \
-  do {                                                                           \
-    if (rows)                                                                    \
-      LAUNCH2(A, B, C, T, true);                                                 \
-    else                                                                         \
-      LAUNCH2(A, B, C, T, false);                                                \
-  } while (0)
-  switch (thrust ? 8 : sel) {
-    case 8: LAUNCH(true, true, true, true); break;
-    case 7: LAUNCH(true, true, true, false); break;
-    case 4: LAUNCH(true, false, false, false); break;
-    case 2: LAUNCH(false, true, false, false); break;
-    case 1: LAUNCH(false, false, true, false); break;
-    default: return set_error(ctx, PIC_E_ARG, "particle pass %d", sel);
-  }
-#undef LAUNCH2
-#undef LAUNCH
+#define F(ROWS, UNIT, BOTH)                                                           \
+  (ctx->thrust_now ? k_particles_tiled<true, true, true, true, ROWS, UNIT, BOTH>      \
+                   : k_particles_tiled<true, true, true, false, ROWS, UNIT, BOTH>)
+#define L(ROWS, UNIT)                                                                 \
+  (sel == 7 ? (nb[1] ? F(ROWS, UNIT, true) : F(ROWS, UNIT, false))                    \
+   : sel == 4 ? k_particles_tiled<true, false, false, false, ROWS, UNIT, false>       \
+   : sel == 2 ? k_particles_tiled<false, true, false, false, ROWS, UNIT, false>       \
+              : k_particles_tiled<false, false, true, false, ROWS, UNIT, false>)
+  const auto kern = unit ? (rows ? L(true, true) : L(false, true))
+                         : (rows ? L(true, false) : L(false, false));
+#undef L
+#undef F
+  kern<<<n, kBlock, 0, ctx->stream>>>(ctx->geom, args, (int)nb[0]);
   PIC_LAUNCH_CHECK(ctx);
-  if (thrust) ctx->thrust_nb[sp] = (int)nb;  // finished by step_b2
+  return 0;
+}
+
+int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
+         int do_boundary) {
+  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
+  PassArgs64 args;
+  memset(&args, 0, sizeof args);
+  bool rows = false;
+  unsigned nb[2] = {0, 0};
+  int rc = prepare_pass(ctx, sp, sel, args.s[0], &rows, &nb[0]);
+  return rc ? rc : launch_pass(ctx, sel, rows, args, nb);
+}
+
+// The fused passes of both species, in one launch where both are in the same
+// state (tiles, boxes or chunks) and leave places empty (kBothBlocks).
+int push_both(pic_ctx *ctx) {
+  PassArgs64 args;
+  memset(&args, 0, sizeof args);
+  bool rows[2] = {false, false};
+  unsigned nb[2] = {0, 0};
+  for (int sp = 0; sp < 2; ++sp) {
+    int rc = prepare_pass(ctx, sp, 7, args.s[sp], &rows[sp], &nb[sp]);
+    if (rc) return rc;
+  }
+  if (nb[0] && nb[1] && rows[0] == rows[1] && nb[0] + nb[1] < kBothBlocks)
+    return launch_pass(ctx, 7, rows[0], args, nb);
+  for (int sp = 0; sp < 2; ++sp) {
+    PassArgs64 one = args;
+    one.s[0] = args.s[sp];
+    const unsigned n[2] = {nb[sp], 0};
+    int rc = launch_pass(ctx, 7, rows[sp], one, n);
+    if (rc) return rc;
+  }
   return 0;
 }
 

@@ -189,6 +189,7 @@ struct pic_ctx {
   int64_t t_n[PIC_T_COUNT] = {0};
   hipEvent_t tev[2][kEventPool] = {};
   int tclass[kEventPool] = {};
+  int tpasses[kEventPool] = {};  // what the interval counts for in t_n
   int tpending = 0;
 };
 
@@ -261,7 +262,7 @@ inline TileGeom tile_geom(const pic_ctx *ctx) {
 
 // timing helpers (HIP events on the context stream)
 void timing_begin(pic_ctx *ctx, int which);
-void timing_end(pic_ctx *ctx, int which);
+void timing_end(pic_ctx *ctx, int which, int passes = 1);
 int timing_flush(pic_ctx *ctx);
 
 // per-form implementations (fp64 / fp32 translation units)
@@ -280,6 +281,7 @@ int step_b2(pic_ctx *);
 int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
 int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
+int push_both(pic_ctx *);
 int particle_boundary(pic_ctx *, int sp);
 int inflow(pic_ctx *, int sp, uint32_t event);
 int sort(pic_ctx *, int sp);
@@ -299,6 +301,7 @@ int step_b2(pic_ctx *);
 int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
 int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
+int push_both(pic_ctx *);
 int particle_boundary(pic_ctx *, int sp);
 int inflow(pic_ctx *, int sp, uint32_t event);
 int sort(pic_ctx *, int sp);
@@ -345,9 +348,9 @@ int diagnose_partials(pic_ctx *, double *partials, unsigned long long *counts);
 // resolved for the current device at pic_create
 int noalloc_init(pic_ctx *ctx);
 
-// the fused particle pass of one species (gather, push, J and n deposit,
-// particle boundary), as pic_step runs it (pic_api.hip)
-int push_fused(pic_ctx *ctx, int sp);
+// the fused particle passes of both species (gather, push, J and n deposit,
+// particle boundary), as pic_step runs them (pic_api.hip)
+int push_fused(pic_ctx *ctx);
 // adjoint state (pic_adj.hip)
 void adj_free(pic_ctx *ctx);
 

@@ -31,6 +31,7 @@ constexpr int kStray = 8;
 // chunks of 2048 that overflow cost 60 us of 330 us per launch at
 // 64^3 x 32 ppc.
 constexpr int kChipSlots = 768;
+
 inline int tail_chunk(int ppc, bool blocked, int64_t tail) {
   const int64_t most = (int64_t)(blocked ? 64 : 32) * ppc;
   int c = kTailChunk;
@@ -43,6 +44,16 @@ inline int64_t most_chunks(int ppc, int64_t cap) {
   const int64_t few = (int64_t)kChipSlots * kTailChunk / 256;
   return ((cap + c - 1) / c > few ? (cap + c - 1) / c : few) + 1;
 }
+
+// Below this many workgroups of both species, their fused passes are one
+// launch: the second species' workgroups take the places that the first one's
+// last round leaves empty, and a launch's latency goes.  Above it the
+// arguments' indirection by species costs more than that.  20 steps, one
+// launch / two: FP32 31 x 27 x 45 x 8 ppc 3.4 / 3.75 ms, 64^3 x 32 ppc (4100
+// workgroups) 14.0 / 14.1 ms, 128^3 x 64 ppc (33000) 155 / 150.5 ms; FP64
+// 8 x 8 x 16 x 4 ppc 1.10 / 1.37 ms, 32^3 x 16 ppc (2000 to 4000) 3.53 /
+// 3.60 ms, 128^3 x 64 ppc 405 / 345 ms (two waves per SIMD, not three).
+constexpr unsigned kBothBlocks = 8 * kChipSlots;
 
 struct TileRun {
   const uint32_t *tile_start;  // ntiles + 1 entries (rows: one per cell, + 1)
