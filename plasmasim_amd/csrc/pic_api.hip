@@ -738,7 +738,7 @@ extern "C" int pic_halo_e(pic_ctx *ctx) {
 extern "C" int pic_push_deposit_j(pic_ctx *ctx, int species) {
   if (!ctx || species < 0 || species > 1) return PIC_E_ARG;
   timing_begin(ctx, PIC_T_PUSH);
-  int rc = DISPATCH(push, ctx, species, 1, 0, 0);
+  int rc = DISPATCH(push, ctx, species, false);
   timing_end(ctx, PIC_T_PUSH);
   return rc;
 }
@@ -746,7 +746,7 @@ extern "C" int pic_push_deposit_j(pic_ctx *ctx, int species) {
 extern "C" int pic_drift_deposit_n(pic_ctx *ctx, int species) {
   if (!ctx || species < 0 || species > 1) return PIC_E_ARG;
   timing_begin(ctx, PIC_T_PUSH);
-  int rc = DISPATCH(push, ctx, species, 0, 1, 0);
+  int rc = DISPATCH(push, ctx, species, true);
   timing_end(ctx, PIC_T_PUSH);
   return rc;
 }
@@ -775,7 +775,7 @@ extern "C" int pic_particle_boundary(pic_ctx *ctx) {
   if (!ctx) return PIC_E_ARG;
   int rc = 0;
   timing_begin(ctx, PIC_T_OTHER);
-  for (int sp = 0; sp < 2 && !rc; ++sp) rc = DISPATCH(particle_boundary, ctx, sp);
+  rc = DISPATCH(particle_boundary, ctx);
   timing_end(ctx, PIC_T_OTHER);
   return rc;
 }

@@ -489,6 +489,19 @@ __device__ __forceinline__ void glob_coop(const Geom &g, bool pend, bool current
   } while (todo);
 }
 
+// sr_particle (:2041-2531) of cell (k, l, m): z must stay in [2, NZ+2)
+// cells; x and y wrap periodically (shift by the box length) or drop (-1).
+// Written with selects: the lanes of a wave take different branches here.
+__device__ __forceinline__ int32_t bounded(const Geom &g, const int (&periodic)[2], int k,
+                                           int l, int m) {
+  const bool inside_zs = (unsigned)(m - 2) < (unsigned)g.NZ &&
+                         (unsigned)k < (unsigned)g.SX && (unsigned)l < (unsigned)g.SY;
+  const int dk = k >= g.NX + 2 ? -g.NX : k < 2 ? g.NX : 0;
+  const int dl = l >= g.NY + 2 ? -g.NY : l < 2 ? g.NY : 0;
+  const bool dead = !inside_zs || (dk != 0 && !periodic[0]) || (dl != 0 && !periodic[1]);
+  return dead ? -1 : pack(k + dk, l + dl, m);
+}
+
 // One particle of the fused pass.  PUSH_J: hot loop A (:731-812) - ballistic
 // drift or gather + Boris, half drift, J deposit at x^{n+1/2}; DRIFT_N: hot
 // loop B (:818-867) - half drift, density deposit at x^{n+1}; BOUNDARY:
@@ -585,16 +598,7 @@ __device__ __forceinline__ void particle_step(
   }
   int32_t out = pack(k, l, m);
   if (BOUNDARY) {
-    // sr_particle (:2041-2531): z must stay in [2, NZ+2) cells; x and y
-    // wrap periodically (shift by the box length) or drop.  Written with
-    // selects: the lanes of a wave take different branches here.
-    const bool inside_zs = (unsigned)(m - 2) < (unsigned)g.NZ &&
-                           (unsigned)k < (unsigned)g.SX && (unsigned)l < (unsigned)g.SY;
-    const int dk = k >= g.NX + 2 ? -g.NX : k < 2 ? g.NX : 0;
-    const int dl = l >= g.NY + 2 ? -g.NY : l < 2 ? g.NY : 0;
-    const bool dead = !inside_zs || (dk != 0 && !kp.periodic[0]) ||
-                      (dl != 0 && !kp.periodic[1]);
-    out = dead ? -1 : pack(k + dk, l + dl, m);
+    out = bounded(g, kp.periodic, k, l, m);
   } else if (k < 0 || l < 0 || m < 0 || k >= g.SX || l >= g.SY || m >= g.SZ) {
     out = -1;  // left the array: not representable
   }
@@ -812,9 +816,11 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
       *(vf *)vat(P.ox, bo) = xs;
       *(vf *)vat(P.oy, bo) = ys;
       *(vf *)vat(P.oz, bo) = zs;
-      *(vf *)vat(P.vx, bo) = us;
-      *(vf *)vat(P.vy, bo) = vs;
-      *(vf *)vat(P.vz, bo) = ws;
+      if (PUSH_J) {  // a drift leaves the velocities
+        *(vf *)vat(P.vx, bo) = us;
+        *(vf *)vat(P.vy, bo) = vs;
+        *(vf *)vat(P.vz, bo) = ws;
+      }
     } else {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
@@ -824,9 +830,11 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
         P.ox[i] = xs[j];
         P.oy[i] = ys[j];
         P.oz[i] = zs[j];
-        P.vx[i] = us[j];
-        P.vy[i] = vs[j];
-        P.vz[i] = ws[j];
+        if (PUSH_J) {
+          P.vx[i] = us[j];
+          P.vy[i] = vs[j];
+          P.vz[i] = ws[j];
+        }
       }
     }
   }
@@ -1424,6 +1432,40 @@ __global__ void k_inflow_kill32(Geom g, Particles32 P, int64_t n) {
   }
   for (int64_t i = i0; i < n; ++i)
     if (inflow_killed(g, P, i, P.cell[i])) P.cell[i] = -1;
+}
+
+// sr_particle on its own, both species: it looks at and changes the cells
+// only.  Four slots per thread as above, 4 of the 28 bytes per particle (as
+// a particle pass it read and wrote all of them: 87 us per species at 7.1M
+// particles, now 10 us).
+struct Bound32 {
+  int32_t *cell[2];
+  int64_t n[2];
+  int nb0;  // workgroups of the ions
+  int periodic[2];
+};
+
+__global__ void k_boundary32(Geom g, Bound32 b) {
+  const int sp = (int)blockIdx.x >= b.nb0 ? 1 : 0;
+  const int64_t t = (int64_t)((int)blockIdx.x - (sp ? b.nb0 : 0)) * blockDim.x + threadIdx.x;
+  int32_t *const cell = b.cell[sp];
+  const int64_t n = b.n[sp], i0 = t * 4;
+  const auto next = [&](int32_t c) {
+    if (c < 0) return c;
+    int k, l, m;
+    unpack(c, k, l, m);
+    return bounded(g, b.periodic, k, l, m);
+  };
+  if (i0 + 4 <= n) {
+    const int4 c = *(const int4 *)(cell + i0);
+    const int4 d = {next(c.x), next(c.y), next(c.z), next(c.w)};
+    if (c.x != d.x || c.y != d.y || c.z != d.z || c.w != d.w) *(int4 *)(cell + i0) = d;
+    return;
+  }
+  for (int64_t i = i0; i < n; ++i) {
+    const int32_t c = cell[i], d = next(c);
+    if (c != d) cell[i] = d;
+  }
 }
 
 __global__ void k_live_flags32(const int32_t *__restrict__ cell, int64_t n,
@@ -2066,7 +2108,7 @@ static int launch_pass(pic_ctx *ctx, int sel, bool perm, bool rows, const PassAr
   const unsigned n = nb[0] + nb[1];
   if (n == 0) return 0;
   const Grid32 G = grid32(ctx);
-  // DET, then the pass: push and J, drift and n, the boundary, or all three
+  // DET, then the pass: push and J, drift and n, or these and the boundary
   // (only a fused pass applies a permutation, and a store sorted as one
   // tile has none to apply)
 #define F(DET, ROWS, BOTH)                                              \
@@ -2075,8 +2117,7 @@ static int launch_pass(pic_ctx *ctx, int sel, bool perm, bool rows, const PassAr
 #define L(DET, ROWS)                                                                     \
   (sel == 7 ? (nb[1] ? F(DET, ROWS, true) : F(DET, ROWS, false))                         \
    : sel == 4 ? k_particles32<true, false, false, DET, false, false, ROWS, false>        \
-   : sel == 2 ? k_particles32<false, true, false, DET, false, false, ROWS, false>        \
-              : k_particles32<false, false, true, DET, false, false, ROWS, false>)
+              : k_particles32<false, true, false, DET, false, false, ROWS, false>)
   const auto kern = S->fx ? (rows ? L(true, true) : L(true, false))
                           : (rows ? L(false, true) : L(false, false));
 #undef L
@@ -2093,23 +2134,18 @@ static void pass_done(pic_ctx *ctx, int sp, const SpeciesArgs32 &a) {
   st(ctx)->pending[sp] = false;
 }
 
-int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
-         int do_boundary) {
+// one routine's pass: push and J, or drift and n
+int push(pic_ctx *ctx, int sp, bool drift) {
   // a pending sort permutation is applied by the fused pass only
-  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
-  if (sel != 7) {
-    int rc = settle(ctx, sp);
-    if (rc) return rc;
-  }
+  int rc = settle(ctx, sp);
+  if (rc) return rc;
+  const int sel = drift ? 2 : 4;
   PassArgs32 args;
   memset(&args, 0, sizeof args);
   bool rows = false;
   unsigned nb[2] = {0, 0};
-  int rc = prepare_pass(ctx, sp, sel, args.s[0], &rows, &nb[0]);
-  if (!rc) rc = launch_pass(ctx, sel, args.s[0].perm != nullptr, rows, args, nb);
-  if (rc) return rc;
-  if (nb[0]) pass_done(ctx, sp, args.s[0]);
-  return 0;
+  rc = prepare_pass(ctx, sp, sel, args.s[0], &rows, &nb[0]);
+  return rc ? rc : launch_pass(ctx, sel, false, rows, args, nb);
 }
 
 // The fused passes of both species, in one launch where both are in the same
@@ -2144,7 +2180,23 @@ int push_both(pic_ctx *ctx) {
   return 0;
 }
 
-int particle_boundary(pic_ctx *ctx, int sp) { return push(ctx, sp, 0, 0, 1); }
+int particle_boundary(pic_ctx *ctx) {
+  int rc = settle_sorts(ctx);
+  if (rc) return rc;
+  Bound32 b;
+  int64_t nb[2];
+  for (int sp = 0; sp < 2; ++sp) {
+    b.cell[sp] = p32(ctx, sp, ctx->cur[sp]).cell;
+    b.n[sp] = ctx->n[sp];
+    b.periodic[sp] = ctx->cfg.periodic[sp];
+    nb[sp] = div_up(ctx->n[sp], 4 * kBlock);
+  }
+  b.nb0 = (int)nb[0];
+  if (nb[0] + nb[1] == 0) return 0;
+  k_boundary32<<<(unsigned)(nb[0] + nb[1]), kBlock, 0, ctx->stream>>>(ctx->geom, b);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
 
 // stable compaction of live particles (tile ranges become invalid)
 static int compact(pic_ctx *ctx, int sp) {

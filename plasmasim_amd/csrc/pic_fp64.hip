@@ -650,6 +650,60 @@ __device__ __forceinline__ int win_byte(const Win &w, int k, int l, int m) {
   return (((k - w.k0) * w.WY + (l - w.l0)) * w.WZ + (m - w.m0)) * 8;
 }
 
+// sr_particle (:2041-2531) of one particle: x and y shifted into the box;
+// false when it drops out
+template <bool UNIT>
+__device__ __forceinline__ bool bounded(const Geom &g, double dx, const int (&periodic)[2],
+                                        double &x, double &y, double z) {
+  bool dead, xhi, xlo, yhi, ylo;
+  if (UNIT) {  // the upper faces by the cells: the same comparisons
+    dead = !(z >= 2.) || (int)z >= g.NZ + 2;
+    xhi = (int)x >= g.NX + 2;
+    xlo = x < 2.;
+    yhi = (int)y >= g.NY + 2;
+    ylo = y < 2.;
+  } else {
+    const double dx2 = 2. * dx;
+    dead = !(z < (g.NZ + 2) * dx && z >= dx2);
+    xhi = x >= (g.NX + 2) * dx;
+    xlo = x < dx2;
+    yhi = y >= (g.NY + 2) * dx;
+    ylo = y < dx2;
+  }
+  dead = dead || ((xhi || xlo) && !periodic[0]) || ((yhi || ylo) && !periodic[1]);
+  if (xhi) x = x - g.NX * dx;
+  else if (xlo) x = x + g.NX * dx;
+  if (yhi) y = y - g.NY * dx;
+  else if (ylo) y = y + g.NY * dx;
+  return !dead;
+}
+
+// sr_particle on its own, both species: reads the positions, writes what
+// changes
+struct Bound64 {
+  Particles64 P[2];
+  int64_t n[2];
+  int nb0;  // workgroups of the ions
+  int periodic[2];
+};
+
+__global__ void k_boundary(Geom g, Bound64 b, double dx) {
+  const int sp = (int)blockIdx.x >= b.nb0 ? 1 : 0;
+  const int64_t i = (int64_t)((int)blockIdx.x - (sp ? b.nb0 : 0)) * blockDim.x + threadIdx.x;
+  if (i >= b.n[sp]) return;
+  const Particles64 &P = b.P[sp];
+  const double z = P.z[i];
+  if (isnan(z)) return;
+  const double x0 = P.x[i], y0 = P.y[i];
+  double x = x0, y = y0;
+  if (!bounded<false>(g, dx, b.periodic, x, y, z)) {
+    P.z[i] = __longlong_as_double(0x7ff8000000000000LL);
+    return;
+  }
+  if (x != x0) P.x[i] = x;
+  if (y != y0) P.y[i] = y;
+}
+
 // thrust_fave partials of one workgroup (six per-thread sums added over the
 // workgroup in a fixed order), stored at slot bid
 __device__ inline void thrust_store64(const double (&th)[6], double *out, int bid) {
@@ -870,26 +924,7 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
       glob_coop64(g, dep && !in_lds, false, dx, x, y, z, wn, 0.0, 0.0, F.jx, F.jy, F.jz, F.nd);
     }
     if (BOUNDARY) {
-      bool dead, xhi, xlo, yhi, ylo;
-      if (UNIT) {  // the upper faces by the cells: the same comparisons
-        dead = !(z >= 2.) || (int)z >= g.NZ + 2;
-        xhi = (int)x >= g.NX + 2;
-        xlo = x < 2.;
-        yhi = (int)y >= g.NY + 2;
-        ylo = y < 2.;
-      } else {
-        const double dx2 = 2. * dx;
-        dead = !(z < (g.NZ + 2) * dx && z >= dx2);
-        xhi = x >= (g.NX + 2) * dx;
-        xlo = x < dx2;
-        yhi = y >= (g.NY + 2) * dx;
-        ylo = y < dx2;
-      }
-      dead = dead || ((xhi || xlo) && !kc.periodic[0]) || ((yhi || ylo) && !kc.periodic[1]);
-      if (xhi) x = x - g.NX * dx;
-      else if (xlo) x = x + g.NX * dx;
-      if (yhi) y = y - g.NY * dx;
-      else if (ylo) y = y + g.NY * dx;
+      const bool dead = !bounded<UNIT>(g, dx, kc.periodic, x, y, z);
       if (dead) {
         *at(P.z, pb) = __longlong_as_double(0x7ff8000000000000LL);
         continue;
@@ -1377,8 +1412,7 @@ static int launch_pass(pic_ctx *ctx, int sel, bool rows, const PassArgs64 &args,
 #define L(ROWS, UNIT)                                                                 \
   (sel == 7 ? (nb[1] ? F(ROWS, UNIT, true) : F(ROWS, UNIT, false))                    \
    : sel == 4 ? k_particles_tiled<true, false, false, false, ROWS, UNIT, false>       \
-   : sel == 2 ? k_particles_tiled<false, true, false, false, ROWS, UNIT, false>       \
-              : k_particles_tiled<false, false, true, false, ROWS, UNIT, false>)
+              : k_particles_tiled<false, true, false, false, ROWS, UNIT, false>)
   const auto kern = unit ? (rows ? L(true, true) : L(false, true))
                          : (rows ? L(true, false) : L(false, false));
 #undef L
@@ -1388,9 +1422,9 @@ static int launch_pass(pic_ctx *ctx, int sel, bool rows, const PassArgs64 &args,
   return 0;
 }
 
-int push(pic_ctx *ctx, int sp, int do_push_j, int do_drift_n,
-         int do_boundary) {
-  const int sel = (do_push_j ? 4 : 0) | (do_drift_n ? 2 : 0) | (do_boundary ? 1 : 0);
+// one routine's pass: push and J, or drift and n
+int push(pic_ctx *ctx, int sp, bool drift) {
+  const int sel = drift ? 2 : 4;
   PassArgs64 args;
   memset(&args, 0, sizeof args);
   bool rows = false;
@@ -1422,7 +1456,21 @@ int push_both(pic_ctx *ctx) {
   return 0;
 }
 
-int particle_boundary(pic_ctx *ctx, int sp) { return push(ctx, sp, 0, 0, 1); }
+int particle_boundary(pic_ctx *ctx) {
+  Bound64 b;
+  int64_t nb[2];
+  for (int sp = 0; sp < 2; ++sp) {
+    b.P[sp] = p64(ctx, sp, ctx->cur[sp]);
+    b.n[sp] = ctx->n[sp];
+    b.periodic[sp] = ctx->cfg.periodic[sp];
+    nb[sp] = div_up(ctx->n[sp], kBlock);
+  }
+  b.nb0 = (int)nb[0];
+  if (nb[0] + nb[1] == 0) return 0;
+  k_boundary<<<(unsigned)(nb[0] + nb[1]), kBlock, 0, ctx->stream>>>(ctx->geom, b, ctx->cfg.dx);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
 
 // Stable compaction of the current buffer into the other one through the
 // flags already written to ctx->flags; returns the survivor count.

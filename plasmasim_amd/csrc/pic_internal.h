@@ -280,9 +280,9 @@ int step_b1(pic_ctx *, bool keep_b);
 int step_b2(pic_ctx *);
 int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
-int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
+int push(pic_ctx *, int sp, bool drift);
 int push_both(pic_ctx *);
-int particle_boundary(pic_ctx *, int sp);
+int particle_boundary(pic_ctx *);
 int inflow(pic_ctx *, int sp, uint32_t event);
 int sort(pic_ctx *, int sp);
 int tsort_setup(pic_ctx *);  // the tile sort's lists, at create
@@ -300,9 +300,9 @@ int step_b1(pic_ctx *, bool keep_b);
 int step_b2(pic_ctx *);
 int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
-int push(pic_ctx *, int sp, int do_push_j, int do_drift_n, int do_boundary);
+int push(pic_ctx *, int sp, bool drift);
 int push_both(pic_ctx *);
-int particle_boundary(pic_ctx *, int sp);
+int particle_boundary(pic_ctx *);
 int inflow(pic_ctx *, int sp, uint32_t event);
 int sort(pic_ctx *, int sp);
 // pic_step's tile sort: the permutation is left for the species' next fused
