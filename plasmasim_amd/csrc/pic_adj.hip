@@ -480,20 +480,140 @@ __global__ void k_add_gather_T(int64_t n, Lam L) {
   }
 }
 
-// LDS window of the transposed gather: six FP64 planes of kAdjWin nodes
-// (36 KB) around the workgroup's particles
-constexpr int kAdjWin = 768;
+// A particle's stencils along one axis: the integer and the half lattice's
+// lower node and weights.
+struct AxisT {
+  int bi, bh;
+  double i0, i1, h0, h1;
+};
 
-__global__ __launch_bounds__(256) void k_pass_T(Geom g, PD P, int64_t n, F6 F,
+template <bool UNIT>
+__device__ inline AxisT axis_t(double p, double dx) {
+  if (UNIT) dx = 1.0;
+  const double q = p / dx;
+  AxisT w;
+  w.bi = (int)q;
+  w.i0 = (w.bi + 1) * dx - p;
+  w.i1 = p - w.bi * dx;
+  w.bh = (int)(q - 0.5);
+  w.h0 = (w.bh + 1 + 0.5) * dx - p;
+  w.h1 = p - (w.bh + 0.5) * dx;
+  return w;
+}
+
+// one component's stencil: E and J are on the half lattice along the two
+// other axes, B along its own
+struct StnT {
+  int k, l, m;
+  double a0, a1, b0, b1, c0, c1;
+};
+
+template <int C>
+__device__ __forceinline__ StnT stn_t(const AxisT (&w)[3]) {
+  constexpr bool hx = (C % 3 == 0) == (C >= 3), hy = (C % 3 == 1) == (C >= 3),
+                 hz = (C % 3 == 2) == (C >= 3);
+  return StnT{hx ? w[0].bh : w[0].bi, hy ? w[1].bh : w[1].bi, hz ? w[2].bh : w[2].bi,
+              hx ? w[0].h0 : w[0].i0, hx ? w[0].h1 : w[0].i1, hy ? w[1].h0 : w[1].i0,
+              hy ? w[1].h1 : w[1].i1, hz ? w[2].h0 : w[2].i0, hz ? w[2].h1 : w[2].i1};
+}
+
+// value and position gradient of sum_n F[n] W_n (W unnormalised), axis by
+// axis: 40 operations where the eight products and their derivatives take 128
+__device__ __forceinline__ double interp_t(const Geom &g, const double *F, const StnT &s,
+                                           double gr[3]) {
+  const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
+  const double *f = F + g.idx(s.k, s.l, s.m);
+  double y[2], gy[2], gz[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const double f00 = f[i * dk], f01 = f[i * dk + 1], f10 = f[i * dk + dl],
+                 f11 = f[i * dk + dl + 1];
+    const double z0 = f00 * s.c0 + f01 * s.c1, z1 = f10 * s.c0 + f11 * s.c1;
+    y[i] = z0 * s.b0 + z1 * s.b1;
+    gy[i] = z1 - z0;
+    gz[i] = (f01 - f00) * s.b0 + (f11 - f10) * s.b1;
+  }
+  gr[0] = y[1] - y[0];
+  gr[1] = gy[0] * s.a0 + gy[1] * s.a1;
+  gr[2] = gz[0] * s.a0 + gz[1] * s.a1;
+  return y[0] * s.a0 + y[1] * s.a1;
+}
+
+// Window of the transposed gather: six FP64 planes of kAdjWin nodes (36 KB)
+// around the workgroup's particles, without those that lie more than kAdjFar
+// cells from the first (a particle that wrapped across a periodic face would
+// stretch the box over the domain); they go to the global planes.
+constexpr int kAdjWin = 768;
+constexpr int kAdjFar = 6;
+
+struct WinT {
+  int k0, l0, m0, WX, WY, WZ;
+  bool on;
+};
+
+// w * stencil into component c of the window, or straight into the plane.
+// Lane j walks the 8 nodes mirrored along the axes set in j & 7, so that
+// lanes of one cell add to different nodes at a time.
+__device__ __forceinline__ void scatter_t(const Geom &g, const WinT &w, double *win,
+                                          double *plane, const StnT &s, double v, bool in) {
+  if (in) {
+    const int sw = threadIdx.x & 7;
+    const bool mx = sw & 4, my = sw & 2, mz = sw & 1;
+    const int sy = w.WZ, sx = w.WY * w.WZ;
+    const int dx = mx ? -sx : sx, dy = my ? -sy : sy, dz = mz ? -1 : 1;
+    const int o = ((s.k - w.k0) * w.WY + (s.l - w.l0)) * w.WZ + (s.m - w.m0) +
+                  (mx ? sx : 0) + (my ? sy : 0) + (mz ? 1 : 0);
+    const double A0 = v * (mx ? s.a1 : s.a0), A1 = v * (mx ? s.a0 : s.a1);
+    const double B0 = my ? s.b1 : s.b0, B1 = my ? s.b0 : s.b1;
+    const double C0 = mz ? s.c1 : s.c0, C1 = mz ? s.c0 : s.c1;
+    const double q00 = B0 * C0, q01 = B0 * C1, q10 = B1 * C0, q11 = B1 * C1;
+    const auto add = [&](int j, double x) {
+      __hip_atomic_fetch_add((PIC_LDS double *)&win[j], x, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    add(o, A0 * q00);
+    add(o + dz, A0 * q01);
+    add(o + dy, A0 * q10);
+    add(o + dy + dz, A0 * q11);
+    add(o + dx, A1 * q00);
+    add(o + dx + dz, A1 * q01);
+    add(o + dx + dy, A1 * q10);
+    add(o + dx + dy + dz, A1 * q11);
+    return;
+  }
+  const int64_t dl = g.SZ, dk = (int64_t)g.SY * g.SZ;
+  double *p = plane + g.idx(s.k, s.l, s.m);
+  const double A0 = v * s.a0, A1 = v * s.a1;
+  gadd(p, A0 * (s.b0 * s.c0));
+  gadd(p + 1, A0 * (s.b0 * s.c1));
+  gadd(p + dl, A0 * (s.b1 * s.c0));
+  gadd(p + dl + 1, A0 * (s.b1 * s.c1));
+  gadd(p + dk, A1 * (s.b0 * s.c0));
+  gadd(p + dk + 1, A1 * (s.b0 * s.c1));
+  gadd(p + dk + dl, A1 * (s.b1 * s.c0));
+  gadd(p + dk + dl + 1, A1 * (s.b1 * s.c1));
+}
+
+// Bound by memory latency and the window's upkeep (64^3 x 32 ppc, 8.4M
+// particles: 144 B of tape and adjoints per particle are 0.25 ms at the copy
+// rate).  Value and gradient of the six components come from one gather, the
+// gradients waiting in registers for the transposed step; the window's index
+// arithmetic is done once per node for its six planes.  1.47 -> 0.89 ms per
+// launch; three waves per SIMD with 44 B of spill, where two (190 VGPRs, no
+// spill) took 0.97 ms and gathering the gradients again 1.00 ms.  UNIT:
+// dx = 1, where x / dx is x exactly.
+template <bool UNIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pass_T(Geom g, PD P, int64_t n, F6 F,
                                                 Lam L, int sp, PassK K,
                                                 double *lp, double *gV_out) {
   __shared__ double win[6 * kAdjWin];
-  __shared__ int bb[6];  // node box of the workgroup's gathers: lo k, l, m, hi k, l, m
+  __shared__ int bb[9];  // first particle's cell, node box: lo k, l, m, hi k, l, m
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
-  const double dx = K.dx, dth = K.dth;
+  const double dx = UNIT ? 1.0 : K.dx, dth = K.dth;
   bool live = i < n && !isnan(P.z[i]);
-  double x0[3] = {0, 0, 0}, v0[3] = {0, 0, 0}, q0[3] = {0, 0, 0};
+  double x0[3] = {0, 0, 0}, v0[3] = {0, 0, 0};
+  AxisT w0[3] = {};
   bool pushed = false;
   if (live) {
     x0[0] = P.x[i];
@@ -504,47 +624,65 @@ __global__ __launch_bounds__(256) void k_pass_T(Geom g, PD P, int64_t n, F6 F,
     v0[2] = P.vz[i];
     const bool ball = x0[0] < K.blo[0] || x0[0] > K.bhi[0] || x0[1] < K.blo[1] ||
                       x0[1] > K.bhi[1] || x0[2] < K.blo[2] || x0[2] > K.bhi[2];
-    for (int a = 0; a < 3; ++a) q0[a] = x0[a] / dx;
+    const double q0[3] = {x0[0] / dx, x0[1] / dx, x0[2] / dx};
     pushed = !ball && in_array_q(g, q0);
+    for (int a = 0; a < 3; ++a) w0[a] = axis_t<UNIT>(x0[a], dx);
   }
-  // the nodes the gathers at x0 touch: from the half-staggered base (int)(x -
-  // 1/2) to the integer base (int)(x) + 1 on each axis
+  // the box of the nodes the gathers at x0 touch: from the half lattice's
+  // base to the integer base + 1 on each axis
+  if (tid < 9) bb[tid] = tid < 3 ? 1 << 29 : tid < 6 ? 1 << 29 : -(1 << 29);
+  __syncthreads();
+  const unsigned long long any = __builtin_amdgcn_ballot_w64(pushed);
+  if (any && lane == __builtin_ctzll(any) &&
+      atomicCAS(&bb[0], 1 << 29, w0[0].bi) == 1 << 29) {
+    bb[1] = w0[1].bi;  // this wave's first particle is the anchor
+    bb[2] = w0[2].bi;
+  }
+  __syncthreads();
+  bool near = pushed;
+  for (int a = 0; a < 3; ++a) near = near && abs(w0[a].bi - bb[a]) <= kAdjFar;
   int lo[3], hi[3];
   for (int a = 0; a < 3; ++a) {
-    lo[a] = pushed ? (int)(q0[a] - 0.5) : (1 << 29);
-    hi[a] = pushed ? (int)q0[a] + 1 : -(1 << 29);
+    lo[a] = near ? w0[a].bh : (1 << 29);
+    hi[a] = near ? w0[a].bi + 1 : -(1 << 29);
   }
   for (int o = 32; o > 0; o >>= 1)
     for (int a = 0; a < 3; ++a) {
       lo[a] = min(lo[a], __shfl_xor(lo[a], o));
       hi[a] = max(hi[a], __shfl_xor(hi[a], o));
     }
-  if (tid < 3) {
-    bb[tid] = 1 << 29;
-    bb[3 + tid] = -(1 << 29);
-  }
-  __syncthreads();
   if (lane == 0)
     for (int a = 0; a < 3; ++a) {
-      atomicMin(&bb[a], lo[a]);
-      atomicMax(&bb[3 + a], hi[a]);
+      atomicMin(&bb[3 + a], lo[a]);
+      atomicMax(&bb[6 + a], hi[a]);
     }
   __syncthreads();
-  const int k0 = bb[0], l0 = bb[1], m0 = bb[2];
-  const int WX = bb[3] - k0 + 1, WY = bb[4] - l0 + 1, WZ = bb[5] - m0 + 1;
-  const bool on = bb[3] >= k0 && (int64_t)WX * WY * WZ <= kAdjWin;
-  const int WN = on ? WX * WY * WZ : 0;
-  for (int j = tid; j < 6 * WN; j += blockDim.x) win[(j / WN) * kAdjWin + j % WN] = 0.0;
+  WinT w;
+  w.k0 = bb[3];
+  w.l0 = bb[4];
+  w.m0 = bb[5];
+  w.WX = bb[6] - w.k0 + 1;
+  w.WY = bb[7] - w.l0 + 1;
+  w.WZ = bb[8] - w.m0 + 1;
+  w.on = bb[6] >= w.k0 && (int64_t)w.WX * w.WY * w.WZ <= kAdjWin;
+  const int WN = w.on ? w.WX * w.WY * w.WZ : 0;
+  for (int j = tid; j < WN; j += blockDim.x)
+#pragma unroll
+    for (int c = 0; c < 6; ++c) win[c * kAdjWin + j] = 0.0;
   __syncthreads();
   double gV = 0;
   if (live) {
-    double f[6] = {0, 0, 0, 0, 0, 0}, vp[3], x1[3];
+    double f[6] = {0, 0, 0, 0, 0, 0}, gf[6][3], vp[3], x1[3];
     if (pushed) {
-      for (int c = 0; c < 6; ++c) {
-        Stn s;
-        stencil_q(dx, x0, q0, c, s);
-        f[c] = st_value(g, F.f[c], s) * K.inv3;
-      }
+      const auto take = [&](int c, const StnT &s) {
+        f[c] = interp_t(g, F.f[c], s, gf[c]) * K.inv3;
+      };
+      take(0, stn_t<0>(w0));
+      take(1, stn_t<1>(w0));
+      take(2, stn_t<2>(w0));
+      take(3, stn_t<3>(w0));
+      take(4, stn_t<4>(w0));
+      take(5, stn_t<5>(w0));
       boris_fwd(K.bk, f, v0, vp);
     } else {
       for (int a = 0; a < 3; ++a) vp[a] = v0[a];
@@ -557,84 +695,73 @@ __global__ __launch_bounds__(256) void k_pass_T(Geom g, PD P, int64_t n, F6 F,
     const bool dep = x1[0] < (g.NX + 4) * dx && x1[0] >= 0 && x1[1] < (g.NY + 4) * dx &&
                      x1[1] >= 0 && x1[2] < (g.NZ + 4) * dx && x1[2] >= 0 &&
                      in_array_q(g, q1);
-    double *lpi = lp + 6 * i;
-    double lx[3] = {lpi[0], lpi[1], lpi[2]};
-    double lvp[3] = {lpi[3], lpi[4], lpi[5]};
+    // the slot's six adjoints as three 16-byte words (slots of 48 bytes)
+    double2 *lpi = (double2 *)(lp + 6 * i);
+    const double2 l01 = lpi[0], l23 = lpi[1], l45 = lpi[2];
+    double lx[3] = {l01.x, l01.y, l23.x};
+    double lvp[3] = {l23.y, l45.x, l45.y};
     for (int a = 0; a < 3; ++a) lvp[a] += lx[a] * dth;
     if (dep) {
-      for (int c = 0; c < 3; ++c) {
-        Stn s;
+      const AxisT w1[3] = {axis_t<UNIT>(x1[0], dx), axis_t<UNIT>(x1[1], dx),
+                           axis_t<UNIT>(x1[2], dx)};
+      const auto take = [&](int c, const StnT &s) {
         double gr[3];
-        stencil_q(dx, x1, q1, c, s);
-        const double val = st_gather(g, L.J[sp][c], s, gr);
+        const double val = interp_t(g, L.J[sp][c], s, gr);
         lvp[c] += K.qn * val;
         for (int a = 0; a < 3; ++a) lx[a] += K.qn * vp[c] * gr[a];
-      }
+      };
+      take(0, stn_t<0>(w1));
+      take(1, stn_t<1>(w1));
+      take(2, stn_t<2>(w1));
     }
     for (int a = 0; a < 3; ++a) lvp[a] += lx[a] * dth;
     double lv[3];
     if (pushed) {
       double lf[6];
       boris_T(K.bk, f, v0, lvp, lv, lf, gV);
-      for (int c = 0; c < 6; ++c) {
-        Stn s;
-        double gr[3];
-        stencil_q(dx, x0, q0, c, s);
-        st_gather(g, F.f[c], s, gr);
-        const double w = lf[c] * K.inv3;
-        for (int a = 0; a < 3; ++a) lx[a] += w * gr[a];
-        // the total B = B0 + B1 is gathered: both adjoints receive the same
-        // scatter, collected once in the scratch planes S (added to each
-        // after the pass, k_add_gather_T); it goes to the workgroup's LDS
-        // window first, each lane walking the 8 nodes in its own order so
-        // that lanes of one cell add to different nodes at a time
-        if (on) {
-          const int bi = s.b[0] - k0, bj = s.b[1] - l0, bk = s.b[2] - m0;
-          for (int t = 0; t < 8; ++t) {
-            const int nn = t ^ (lane & 7);
-            const int a = nn >> 2, b2 = (nn >> 1) & 1, c2 = nn & 1;
-            const int j = ((bi + a) * WY + (bj + b2)) * WZ + (bk + c2);
-            // selects, not s.w[.][lane-dependent index]: that form puts the
-            // stencil in private memory
-            const double wa = a ? s.w[0][1] : s.w[0][0];
-            const double wb = b2 ? s.w[1][1] : s.w[1][0];
-            const double wc = c2 ? s.w[2][1] : s.w[2][0];
-            __hip_atomic_fetch_add((PIC_LDS double *)&win[c * kAdjWin + j], w * wa * wb * wc,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          }
-        } else {
-          st_scatter(g, c < 3 ? L.E[c] : L.S[c - 3], s, w);
-        }
-      }
+      const bool in = w.on && near;
+      // the total B = B0 + B1 is gathered: both adjoints receive the same
+      // scatter, collected once in the scratch planes S (added to each after
+      // the pass, k_add_gather_T)
+      const auto give = [&](int c, const StnT &s) {
+        const double u = lf[c] * K.inv3;
+        for (int a = 0; a < 3; ++a) lx[a] += u * gf[c][a];
+        scatter_t(g, w, win + c * kAdjWin, c < 3 ? L.E[c] : L.S[c - 3], s, u, in);
+      };
+      give(0, stn_t<0>(w0));
+      give(1, stn_t<1>(w0));
+      give(2, stn_t<2>(w0));
+      give(3, stn_t<3>(w0));
+      give(4, stn_t<4>(w0));
+      give(5, stn_t<5>(w0));
     } else {
       for (int a = 0; a < 3; ++a) lv[a] = lvp[a];
     }
-    for (int a = 0; a < 3; ++a) {
-      lpi[a] = lx[a];
-      lpi[3 + a] = lv[a];
-    }
+    lpi[0] = double2{lx[0], lx[1]};
+    lpi[1] = double2{lx[2], lv[0]};
+    lpi[2] = double2{lv[1], lv[2]};
   }
-  if (on) {
+  if (w.on) {
     __syncthreads();
-    const int WYZ = WY * WZ;
-    for (int c = 0; c < 6; ++c) {
-      double *dst = c < 3 ? L.E[c] : L.S[c - 3];
-      for (int j = tid; j < WN; j += blockDim.x) {
+    const int WYZ = w.WY * w.WZ;
+    for (int j = tid; j < WN; j += blockDim.x) {
+      const int64_t at = g.idx(w.k0 + j / WYZ, w.l0 + (j / w.WZ) % w.WY, w.m0 + j % w.WZ);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) {
         const double v = win[c * kAdjWin + j];
-        if (v == 0.0) continue;
-        gadd(dst + g.idx(k0 + j / WYZ, l0 + (j / WZ) % WY, m0 + j % WZ), v);
+        if (v != 0.0) gadd((c < 3 ? L.E[c] : L.S[c - 3]) + at, v);
       }
     }
   }
   // per-block sum of the motional-field V derivative
-  __shared__ double red[256];
-  red[threadIdx.x] = gV;
+  for (int o = 32; o > 0; o >>= 1) gV += __shfl_xor(gV, o);
+  __shared__ double red[4];
+  if (lane == 0) red[tid >> 6] = gV;
   __syncthreads();
-  for (int s2 = blockDim.x / 2; s2 > 0; s2 >>= 1) {
-    if ((int)threadIdx.x < s2) red[threadIdx.x] += red[threadIdx.x + s2];
-    __syncthreads();
+  if (tid == 0) {
+    const double v = (red[0] + red[1]) + (red[2] + red[3]);
+    if (v != 0.0) gadd(gV_out, v);
   }
-  if (threadIdx.x == 0 && red[0] != 0.0) gadd(gV_out, red[0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1408,7 +1535,8 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
         pk.bk.eimf_y = -A->p[3] * c.imf[0];
         pk.bk.imf_x = c.imf[0];
         pk.bk.imf_y = c.imf[1];
-        k_pass_T<<<nb(np), 256, 0, st>>>(g, tape_pd(j, sp), np, F, L, sp, pk, lp[sp], gvd);
+        (c.dx == 1.0 ? k_pass_T<true> : k_pass_T<false>)<<<nb(np), 256, 0, st>>>(
+            g, tape_pd(j, sp), np, F, L, sp, pk, lp[sp], gvd);
       }
       k_add_gather_T<<<nb(n), kBlock, 0, st>>>(n, L);
       TRYH(hipMemsetAsync(L.J[0][0], 0, 6 * n * sizeof(double), st));
