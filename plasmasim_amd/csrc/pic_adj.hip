@@ -480,6 +480,39 @@ __global__ void k_add_gather_T(int64_t n, Lam L) {
   }
 }
 
+// One species of one tape entry: the particles as the forward holds them
+// (FP32: cells, offsets and velocities, read as the FP64 values they stand
+// for; 28 instead of 48 bytes per particle and no conversion pass).
+struct TapePart {
+  PD d;           // FP64 forward
+  Particles32 f;  // FP32 forward
+};
+
+// particle i into x, v; false for a dead slot
+template <bool F32>
+__device__ __forceinline__ bool tape_load(const TapePart &P, int64_t i, double dx,
+                                          double (&x)[3], double (&v)[3]) {
+  if (F32) {
+    const int32_t c = P.f.cell[i];
+    if (c < 0) return false;
+    x[0] = ((double)(c >> 20) + (double)P.f.ox[i]) * dx;
+    x[1] = ((double)((c >> 10) & 1023) + (double)P.f.oy[i]) * dx;
+    x[2] = ((double)(c & 1023) + (double)P.f.oz[i]) * dx;
+    v[0] = P.f.vx[i];
+    v[1] = P.f.vy[i];
+    v[2] = P.f.vz[i];
+    return true;
+  }
+  x[2] = P.d.z[i];
+  if (isnan(x[2])) return false;
+  x[0] = P.d.x[i];
+  x[1] = P.d.y[i];
+  v[0] = P.d.vx[i];
+  v[1] = P.d.vy[i];
+  v[2] = P.d.vz[i];
+  return true;
+}
+
 // A particle's stencils along one axis: the integer and the half lattice's
 // lower node and weights.
 struct AxisT {
@@ -595,33 +628,27 @@ __device__ __forceinline__ void scatter_t(const Geom &g, const WinT &w, double *
 }
 
 // Bound by memory latency and the window's upkeep (64^3 x 32 ppc, 8.4M
-// particles: 144 B of tape and adjoints per particle are 0.25 ms at the copy
+// particles: 124 B of tape and adjoints per particle are 0.2 ms at the copy
 // rate).  Value and gradient of the six components come from one gather, the
 // gradients waiting in registers for the transposed step; the window's index
 // arithmetic is done once per node for its six planes.  1.47 -> 0.89 ms per
 // launch; three waves per SIMD with 44 B of spill, where two (190 VGPRs, no
 // spill) took 0.97 ms and gathering the gradients again 1.00 ms.  UNIT:
 // dx = 1, where x / dx is x exactly.
-template <bool UNIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pass_T(Geom g, PD P, int64_t n, F6 F,
-                                                Lam L, int sp, PassK K,
-                                                double *lp, double *gV_out) {
+template <bool UNIT, bool F32>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pass_T(
+    Geom g, TapePart P, int64_t n, F6 F, Lam L, int sp, PassK K, double *lp,
+    double *gV_out) {
   __shared__ double win[6 * kAdjWin];
   __shared__ int bb[9];  // first particle's cell, node box: lo k, l, m, hi k, l, m
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const double dx = UNIT ? 1.0 : K.dx, dth = K.dth;
-  bool live = i < n && !isnan(P.z[i]);
   double x0[3] = {0, 0, 0}, v0[3] = {0, 0, 0};
+  const bool live = i < n && tape_load<F32>(P, i, dx, x0, v0);
   AxisT w0[3] = {};
   bool pushed = false;
   if (live) {
-    x0[0] = P.x[i];
-    x0[1] = P.y[i];
-    x0[2] = P.z[i];
-    v0[0] = P.vx[i];
-    v0[1] = P.vy[i];
-    v0[2] = P.vz[i];
     const bool ball = x0[0] < K.blo[0] || x0[0] > K.bhi[0] || x0[1] < K.blo[1] ||
                       x0[1] > K.bhi[1] || x0[2] < K.blo[2] || x0[2] > K.bhi[2];
     const double q0[3] = {x0[0] / dx, x0[1] / dx, x0[2] / dx};
@@ -861,6 +888,30 @@ __global__ void k_fields_to_d(int64_t n, const T *ex, const T *ey, const T *ez,
   }
 }
 
+// B0 = sum_a M_a G_a + IMF
+__global__ void k_b0(int64_t n, const double *G, double p0, double p1, double p2, double i0,
+                     double i1, double i2, double *b0) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double imf[3] = {i0, i1, i2};
+  for (int c = 0; c < 3; ++c)
+    b0[c * n + i] = p0 * G[(0 + c) * n + i] + p1 * G[(3 + c) * n + i] + p2 * G[(6 + c) * n + i] +
+                    imf[c];
+}
+
+// the forward's initial fields: B0, B = B0 (FP32 form: B - B0 = 0), E = 0
+template <typename T>
+__global__ void k_init_fields(int64_t n, Fields<T> F, const double *b0, int b_total) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int c = 0; c < 3; ++c) {
+    const double b = b0[c * n + i];
+    F.f[PIC_B0X + c][i] = (T)b;
+    F.f[PIC_BX + c][i] = b_total ? (T)b : (T)0;
+    F.f[PIC_EX + c][i] = (T)0;
+  }
+}
+
 // F6 (E, total B) from a tape entry (E, B1) and B0
 __global__ void k_tape_to_f6(int64_t n, const double *tp, const double *b0, F6 F) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -871,35 +922,30 @@ __global__ void k_tape_to_f6(int64_t n, const double *tp, const double *b0, F6 F
   }
 }
 
-// FP32 particles into FP64 reference coordinates; dead -> z = NaN
-__global__ void k_p32_to_d(Particles32 Q, int64_t n, double dx, PD P) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// a tape entry of the FP32 forward: four slots per thread (whole 16-byte
+// words: the buffers are as long as the particle store)
+__global__ void k_tape_p32(Particles32 Q, int64_t n, Particles32 P) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= n) return;
-  const int32_t c = Q.cell[i];
-  if (c < 0) {
-    P.x[i] = P.y[i] = 0.0;
-    P.z[i] = __longlong_as_double(0x7ff8000000000000ll);
-    P.vx[i] = P.vy[i] = P.vz[i] = 0.0;
-    return;
-  }
-  const int k = c >> 20, l = (c >> 10) & 1023, m = c & 1023;
-  P.x[i] = ((double)k + (double)Q.ox[i]) * dx;
-  P.y[i] = ((double)l + (double)Q.oy[i]) * dx;
-  P.z[i] = ((double)m + (double)Q.oz[i]) * dx;
-  P.vx[i] = Q.vx[i];
-  P.vy[i] = Q.vy[i];
-  P.vz[i] = Q.vz[i];
+  *(int4 *)(P.cell + i) = *(const int4 *)(Q.cell + i);
+  *(float4 *)(P.ox + i) = *(const float4 *)(Q.ox + i);
+  *(float4 *)(P.oy + i) = *(const float4 *)(Q.oy + i);
+  *(float4 *)(P.oz + i) = *(const float4 *)(Q.oz + i);
+  *(float4 *)(P.vx + i) = *(const float4 *)(Q.vx + i);
+  *(float4 *)(P.vy + i) = *(const float4 *)(Q.vy + i);
+  *(float4 *)(P.vz + i) = *(const float4 *)(Q.vz + i);
 }
 
 // per-block sums: out[b] = sum over [lo, hi) of lp[6 i + 5] (v_z adjoint),
-// the slots zeroed afterwards when zero_after is set; alive[] filter
+// the slots zeroed afterwards when zero_after is set; z or cell: without the
+// dead slots
 __global__ __launch_bounds__(256) void k_sum_vz(double *lp, int64_t lo, int64_t hi,
-                                                const double *z, int zero_after,
-                                                double *out) {
+                                                const double *z, const int32_t *cell,
+                                                int zero_after, double *out) {
   double v = 0;
   for (int64_t i = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < hi;
        i += (int64_t)gridDim.x * blockDim.x) {
-    if (z && isnan(z[i])) continue;
+    if ((z && isnan(z[i])) || (cell && cell[i] < 0)) continue;
     v += lp[6 * i + 5];
     if (zero_after)
       for (int a = 0; a < 6; ++a) lp[6 * i + a] = 0.0;
@@ -950,6 +996,7 @@ __global__ __launch_bounds__(256) void k_dot_g(int64_t n, Lam L, const double *G
 struct Ckpt {
   void *fields = nullptr;
   void *parts[2] = {nullptr, nullptr};
+  int64_t room[2] = {0, 0};  // slots that parts holds
   uint32_t *tiles[2] = {nullptr, nullptr};
   int64_t n[2], sorted_end[2];
   int cur[2];
@@ -968,6 +1015,40 @@ struct TapeStep {
   int64_t n[2], lo[2], hi[2], nb[2], na[2];
 };
 
+// Buffers of the reverse sweep: the particle adjoints (and their copy across
+// a sort), the tape of one segment and the permutations of the sorts in it.
+// Kept for the next sweep of the context where they are no more than
+// kKeepBytes: allocating and freeing them took from 20 ms to 2.5 s of a
+// 90 ms sweep at 64^3 x 32 ppc.
+constexpr size_t kKeepBytes = (size_t)32 << 30;
+struct Sweep {
+  double *lp[2] = {nullptr, nullptr}, *lq[2] = {nullptr, nullptr};
+  std::vector<double *> tf;
+  std::vector<char *> tpart;
+  std::vector<uint32_t *> perm;
+  size_t bytes = 0;
+  template <typename T>
+  hipError_t want(T *&p, size_t b) {
+    if (p) return hipSuccess;
+    const hipError_t e = hipMalloc(&p, b);
+    if (e == hipSuccess) bytes += b;
+    return e;
+  }
+  void release() {
+    for (int s = 0; s < 2; ++s) {
+      if (lp[s]) (void)hipFree(lp[s]);
+      if (lq[s]) (void)hipFree(lq[s]);
+    }
+    for (double *p : tf)
+      if (p) (void)hipFree(p);
+    for (char *p : tpart)
+      if (p) (void)hipFree(p);
+    for (uint32_t *p : perm)
+      if (p) (void)hipFree(p);
+    *this = Sweep();
+  }
+};
+
 struct AdjState {
   double p[4];
   int nsteps = 0, ckpt = 0, nq = 0;
@@ -979,7 +1060,11 @@ struct AdjState {
   double *f6 = nullptr;  // 6 planes: the F6 scratch (device)
   double *tmp = nullptr; // 6 planes: field conversion (device)
   double *red = nullptr; // reduction partials (device, 4096)
-  std::vector<Ckpt> ck;
+  double *part = nullptr;  // the loss terms of every step (device)
+  int64_t part_n = 0;
+  std::vector<Ckpt> ck;  // the first nck hold the last forward's checkpoints
+  int nck = 0;
+  Sweep w;
 };
 
 AdjState *state(pic_ctx *ctx) { return (AdjState *)ctx->adj; }
@@ -1084,15 +1169,18 @@ int ensure_state(pic_ctx *ctx) {
   return 0;
 }
 
-void free_ckpts(AdjState *A) {
-  for (Ckpt &c : A->ck) {
+// keep the buffers of the first `keep` checkpoints
+void free_ckpts(AdjState *A, size_t keep) {
+  for (size_t j = keep; j < A->ck.size(); ++j) {
+    Ckpt &c = A->ck[j];
     if (c.fields) (void)hipFree(c.fields);
     for (int s = 0; s < 2; ++s) {
       if (c.parts[s]) (void)hipFree(c.parts[s]);
       if (c.tiles[s]) (void)hipFree(c.tiles[s]);
     }
   }
-  A->ck.clear();
+  if (A->ck.size() > keep) A->ck.resize(keep);
+  A->nck = 0;
 }
 
 size_t slot_bytes(const pic_ctx *ctx) {
@@ -1123,7 +1211,7 @@ void sub_arrays(const pic_ctx *ctx, void *buf, int64_t cap, char **ptr, size_t *
 }
 
 int save_ckpt(pic_ctx *ctx, Ckpt &c) {
-  PIC_HIP(ctx, hipMalloc(&c.fields, ctx->field_bytes));
+  if (!c.fields) PIC_HIP(ctx, hipMalloc(&c.fields, ctx->field_bytes));
   PIC_HIP(ctx, hipMemcpyAsync(c.fields, ctx->field_mem, ctx->field_bytes,
                               hipMemcpyDeviceToDevice, ctx->stream));
   const int nt = tile_geom(ctx).ntiles();
@@ -1133,7 +1221,13 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
     c.cur[s] = ctx->cur[s];
     c.drift_halves[s] = ctx->drift_halves[s];
     const int64_t n = ctx->n[s];
-    PIC_HIP(ctx, hipMalloc(&c.parts[s], (size_t)(n + 1) * slot_bytes(ctx)));
+    if (c.room[s] < n + 1) {
+      if (c.parts[s]) (void)hipFree(c.parts[s]);
+      c.parts[s] = nullptr;
+      c.room[s] = 0;
+      PIC_HIP(ctx, hipMalloc(&c.parts[s], (size_t)(n + 1) * slot_bytes(ctx)));
+      c.room[s] = n + 1;
+    }
     char *src[7], *dst[7];
     size_t esz[7];
     int cnt;
@@ -1143,7 +1237,8 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
       if (n > 0)
         PIC_HIP(ctx, hipMemcpyAsync(dst[j], src[j], n * esz[j], hipMemcpyDeviceToDevice,
                                     ctx->stream));
-    PIC_HIP(ctx, hipMalloc(&c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t)));
+    if (!c.tiles[s])
+      PIC_HIP(ctx, hipMalloc(&c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t)));
     PIC_HIP(ctx, hipMemcpyAsync(c.tiles[s], ctx->tile_start[s], (size_t)(nt + 1) * sizeof(uint32_t),
                                 hipMemcpyDeviceToDevice, ctx->stream));
   }
@@ -1211,23 +1306,15 @@ int fields_to_d(pic_ctx *ctx, double *out) {
   return 0;
 }
 
-// the loss term of the live state
-int force_now(pic_ctx *ctx, AdjState *A, double *F) {
+// the loss term of the live state: nb(nq) partial sums into out (device)
+int force_now(pic_ctx *ctx, AdjState *A, double *out) {
   int rc = fields_to_d(ctx, A->tmp);
   if (rc) return rc;
   const int64_t n = ncell(ctx);
   k_tape_to_f6<<<nb(n), kBlock, 0, ctx->stream>>>(n, A->tmp, A->b0, f6_view(ctx, A->f6));
-  const unsigned blocks = nb(A->nq);
-  k_force<<<blocks, kBlock, 0, ctx->stream>>>(ctx->geom, f6_view(ctx, A->f6),
-                                              sphere(ctx, A), A->red);
+  k_force<<<nb(A->nq), kBlock, 0, ctx->stream>>>(ctx->geom, f6_view(ctx, A->f6),
+                                                 sphere(ctx, A), out);
   PIC_LAUNCH_CHECK(ctx);
-  std::vector<double> h(blocks);
-  PIC_HIP(ctx, hipMemcpyAsync(h.data(), A->red, blocks * sizeof(double),
-                              hipMemcpyDeviceToHost, ctx->stream));
-  PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  double s = 0;
-  for (double v : h) s += v;
-  *F = s;
   return 0;
 }
 
@@ -1235,11 +1322,12 @@ int force_now(pic_ctx *ctx, AdjState *A, double *F) {
 // its permutation into perm[s] when given), the inflow appended to the
 // store (its ranges recorded), and, when tape_fields is given, the tape
 // entry (after the inflow, before the first half step)
-int fwd_step(pic_ctx *ctx, TapeStep &ts, double *tape_fields, PD tape_p[2],
+int fwd_step(pic_ctx *ctx, TapeStep &ts, double *tape_fields, TapePart tape_p[2],
              uint32_t *const perm[2]) {
   const pic_config &c = ctx->cfg;
+  const bool f64 = c.precision == PIC_FP64;
   int rc;
-  if ((rc = pic_renew_grid(ctx))) return rc;
+  if (ctx->phi && (rc = poisson_zero_phi(ctx))) return rc;  // renew_grid (:2552)
   ts.sorted = 0;
   if (ctx->c_sort > c.sort_every - 1) {
     ctx->c_sort = 0;
@@ -1278,26 +1366,22 @@ int fwd_step(pic_ctx *ctx, TapeStep &ts, double *tape_fields, PD tape_p[2],
       if (c.precision == PIC_FP64) {
         const Particles64 P = p64(ctx, s, ctx->cur[s]);
         const double *src[6] = {P.x, P.y, P.z, P.vx, P.vy, P.vz};
-        double *dst[6] = {tape_p[s].x, tape_p[s].y, tape_p[s].z, tape_p[s].vx,
-                          tape_p[s].vy, tape_p[s].vz};
+        double *dst[6] = {tape_p[s].d.x, tape_p[s].d.y, tape_p[s].d.z,
+                          tape_p[s].d.vx, tape_p[s].d.vy, tape_p[s].d.vz};
         for (int j = 0; j < 6; ++j)
           PIC_HIP(ctx, hipMemcpyAsync(dst[j], src[j], n * sizeof(double),
                                       hipMemcpyDeviceToDevice, ctx->stream));
       } else {
-        k_p32_to_d<<<nb(n), kBlock, 0, ctx->stream>>>(p32(ctx, s, ctx->cur[s]), n, c.dx,
-                                                      tape_p[s]);
+        k_tape_p32<<<nb(div_up(n, 4)), kBlock, 0, ctx->stream>>>(p32(ctx, s, ctx->cur[s]), n,
+                                                                 tape_p[s].f);
         PIC_LAUNCH_CHECK(ctx);
       }
     }
   }
-  if ((rc = pic_renew_b_half(ctx))) return rc;
-  if ((rc = pic_halo_b(ctx))) return rc;
+  if ((rc = f64 ? f64::step_b1(ctx, false) : f32::step_b1(ctx, false))) return rc;
   if ((rc = push_fused(ctx))) return rc;
-  if ((rc = pic_renew_b_half(ctx))) return rc;
-  if ((rc = pic_halo_b(ctx))) return rc;
-  if ((rc = pic_fold_current(ctx))) return rc;
-  if ((rc = pic_renew_e(ctx))) return rc;
-  if ((rc = pic_halo_e(ctx))) return rc;
+  if ((rc = f64 ? f64::step_b2(ctx) : f32::step_b2(ctx))) return rc;
+  if ((rc = f64 ? f64::step_e(ctx) : f32::step_e(ctx))) return rc;
   ctx->c_sort++;
   ctx->c_add++;
   ctx->step++;
@@ -1324,7 +1408,9 @@ double sum_partials(pic_ctx *ctx, const double *dev, int count, int stride, int 
 void adj_free(pic_ctx *ctx) {
   AdjState *A = state(ctx);
   if (!A) return;
-  free_ckpts(A);
+  free_ckpts(A, 0);
+  A->w.release();
+  if (A->part) (void)hipFree(A->part);
   if (A->G) (void)hipFree(A->G);
   if (A->b0) (void)hipFree(A->b0);
   if (A->lam) (void)hipFree(A->lam);
@@ -1356,29 +1442,37 @@ extern "C" int pic_adj_forward(pic_ctx *ctx, const double params[4], int nsteps,
   rc = ensure_state(ctx);
   if (rc) return rc;
   AdjState *A = state(ctx);
-  free_ckpts(A);
+  A->have_forward = false;
+  free_ckpts(A, (size_t)div_up(nsteps, ckpt_every));
+  const int64_t terms = (int64_t)nsteps * nb(nquad);
+  if (A->part_n < terms) {
+    if (A->part) (void)hipFree(A->part);
+    A->part = nullptr;
+    A->part_n = 0;
+    PIC_HIP(ctx, hipMalloc(&A->part, (size_t)terms * sizeof(double)));
+    A->part_n = terms;
+  }
   for (int a = 0; a < 4; ++a) A->p[a] = params[a];
   A->nsteps = nsteps;
   A->ckpt = ckpt_every;
   A->R = radius;
   A->nq = nquad;
-  A->have_forward = false;
   // parameters: B0 = sum_a M_a G_a + IMF, B = B0, E = 0; V
   const pic_config &c = ctx->cfg;
   const int64_t n = ncell(ctx);
-  std::vector<double> G(9 * n), b0(3 * n), zero(n, 0.0);
-  PIC_HIP(ctx, hipMemcpy(G.data(), A->G, 9 * n * sizeof(double), hipMemcpyDeviceToHost));
-  for (int comp = 0; comp < 3; ++comp)
-    for (int64_t i = 0; i < n; ++i)
-      b0[comp * n + i] = params[0] * G[(0 + comp) * n + i] + params[1] * G[(3 + comp) * n + i] +
-                         params[2] * G[(6 + comp) * n + i] + c.imf[comp];
-  PIC_HIP(ctx, hipMemcpy(A->b0, b0.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice));
-  for (int comp = 0; comp < 3; ++comp)
-    if ((rc = pic_upload_field(ctx, PIC_B0X + comp, b0.data() + comp * n))) return rc;
-  for (int comp = 0; comp < 3; ++comp)
-    if ((rc = pic_upload_field(ctx, PIC_BX + comp, b0.data() + comp * n))) return rc;
-  for (int comp = 0; comp < 3; ++comp)
-    if ((rc = pic_upload_field(ctx, PIC_EX + comp, zero.data()))) return rc;
+  k_b0<<<nb(n), kBlock, 0, ctx->stream>>>(n, A->G, params[0], params[1], params[2], c.imf[0],
+                                          c.imf[1], c.imf[2], A->b0);
+  if (c.precision == PIC_FP64) {
+    k_init_fields<double><<<nb(n), kBlock, 0, ctx->stream>>>(n, fields<double>(ctx), A->b0, 1);
+    PIC_LAUNCH_CHECK(ctx);
+  } else {
+    k_init_fields<float><<<nb(n), kBlock, 0, ctx->stream>>>(n, fields<float>(ctx), A->b0, 0);
+    PIC_LAUNCH_CHECK(ctx);
+    // the FP32 form's uploads and downloads take B0 from the host's copy
+    PIC_HIP(ctx, hipMemcpyAsync(ctx->b0_host, A->b0, 3 * n * sizeof(double),
+                                hipMemcpyDeviceToHost, ctx->stream));
+    if ((rc = f32::refresh_total_b(ctx))) return rc;
+  }
   ctx->cfg.vdrift[2] = params[3];
   ctx->adj_mode = 1;
   ctx->step = 0;
@@ -1387,16 +1481,24 @@ extern "C" int pic_adj_forward(pic_ctx *ctx, const double params[4], int nsteps,
   ctx->inflow_event = 0;
   if ((rc = pic_load_particles(ctx))) return rc;
   if ((rc = pic_begin(ctx))) return rc;
-  double L = 0;
   TapeStep ts;
+  const unsigned blocks = nb(nquad);
   for (int s = 0; s < nsteps; ++s) {
     if (s % ckpt_every == 0) {
-      A->ck.emplace_back();
-      if ((rc = save_ckpt(ctx, A->ck.back()))) return rc;
+      if ((size_t)A->nck == A->ck.size()) A->ck.emplace_back();
+      if ((rc = save_ckpt(ctx, A->ck[A->nck++]))) return rc;
     }
     if ((rc = fwd_step(ctx, ts, nullptr, nullptr, nullptr))) return rc;
-    double F;
-    if ((rc = force_now(ctx, A, &F))) return rc;
+    if ((rc = force_now(ctx, A, A->part + (int64_t)s * blocks))) return rc;
+  }
+  std::vector<double> h((size_t)terms);
+  PIC_HIP(ctx, hipMemcpyAsync(h.data(), A->part, (size_t)terms * sizeof(double),
+                              hipMemcpyDeviceToHost, ctx->stream));
+  PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  double L = 0;
+  for (int s = 0; s < nsteps; ++s) {
+    double F = 0;
+    for (unsigned b = 0; b < blocks; ++b) F += h[(size_t)s * blocks + b];
     L += F / nsteps;
   }
   ctx->adj_mode = 0;
@@ -1418,45 +1520,48 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
   int rc;
   hipStream_t st = ctx->stream;
   PIC_HIP(ctx, hipMemsetAsync(A->lam, 0, 18 * n * sizeof(double), st));
-  // particle adjoints (and their copy across a sort), the tape of one
-  // segment and the permutations of the sorts in it
-  double *lp[2] = {nullptr, nullptr}, *lq[2] = {nullptr, nullptr};
-  std::vector<double *> tf(K + 1, nullptr);
-  std::vector<double *> tpart(K, nullptr);
-  std::vector<uint32_t *> perm(2 * (size_t)K, nullptr);
+  Sweep &W = A->w;
+  double *(&lp)[2] = W.lp, *(&lq)[2] = W.lq;
   std::vector<TapeStep> ts(K);
   const int64_t cap = ctx->cap;
-  auto cleanup = [&]() {
-    for (int s = 0; s < 2; ++s) {
-      if (lp[s]) (void)hipFree(lp[s]);
-      if (lq[s]) (void)hipFree(lq[s]);
-    }
-    for (uint32_t *p : perm)
-      if (p) (void)hipFree(p);
-    for (double *p : tf)
-      if (p) (void)hipFree(p);
-    for (double *p : tpart)
-      if (p) (void)hipFree(p);
+  const bool f64 = c.precision == PIC_FP64;
+  auto cleanup = [&](bool keep) {
+    if (!keep || W.bytes > kKeepBytes) W.release();
     ctx->adj_mode = 0;
   };
 #define TRY(x)          \
   do {                  \
     if ((rc = (x))) {   \
-      cleanup();        \
+      cleanup(false);   \
       return rc;        \
     }                   \
   } while (0)
 #define TRYH(x) TRY((x) == hipSuccess ? 0 : set_error(ctx, PIC_E_HIP, "adjoint: %s", #x))
+  if (W.tf.size() < (size_t)K + 1) W.tf.resize(K + 1, nullptr);
+  if (W.tpart.size() < (size_t)K) W.tpart.resize(K, nullptr);
+  if (W.perm.size() < 2 * (size_t)K) W.perm.resize(2 * (size_t)K, nullptr);
   for (int s = 0; s < 2; ++s) {
-    TRYH(hipMalloc(&lp[s], 6 * (size_t)cap * sizeof(double)));
+    TRYH(W.want(lp[s], 6 * (size_t)cap * sizeof(double)));
     TRYH(hipMemsetAsync(lp[s], 0, 6 * (size_t)cap * sizeof(double), st));
-    TRYH(hipMalloc(&lq[s], 6 * (size_t)cap * sizeof(double)));
   }
-  for (int j = 0; j <= K; ++j) TRYH(hipMalloc(&tf[j], 6 * n * sizeof(double)));
-  for (int j = 0; j < K; ++j) TRYH(hipMalloc(&tpart[j], 12 * (size_t)cap * sizeof(double)));
-  auto tape_pd = [&](int j, int s) {
-    double *b = tpart[j] + (size_t)s * 6 * cap;
-    return PD{b, b + cap, b + 2 * cap, b + 3 * cap, b + 4 * cap, b + 5 * cap};
+  for (int j = 0; j <= K; ++j) TRYH(W.want(W.tf[j], 6 * n * sizeof(double)));
+  for (int j = 0; j < K; ++j) TRYH(W.want(W.tpart[j], 2 * (size_t)cap * slot_bytes(ctx)));
+  std::vector<double *> &tf = W.tf;
+  std::vector<uint32_t *> &perm = W.perm;
+  auto tape_of = [&](int j, int s) {
+    TapePart t = {};
+    char *b = W.tpart[j] + (size_t)s * cap * slot_bytes(ctx);
+    char *p[7];
+    size_t esz[7];
+    int cnt;
+    sub_arrays(ctx, b, cap, p, esz, &cnt);
+    if (f64)
+      t.d = PD{(double *)p[0], (double *)p[1], (double *)p[2],
+               (double *)p[3], (double *)p[4], (double *)p[5]};
+    else
+      t.f = Particles32{(int32_t *)p[0], (float *)p[1], (float *)p[2], (float *)p[3],
+                        (float *)p[4], (float *)p[5], (float *)p[6]};
+    return t;
   };
   const Lam L = lam_view(ctx, A);
   const SigmaProfile sg = sigma(ctx);
@@ -1468,17 +1573,17 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
   double *gvd = A->red + 4000;  // device accumulator of the motional-field term
   TRYH(hipMemsetAsync(gvd, 0, sizeof(double), st));
   ctx->adj_mode = 1;
-  const int nseg = (int)A->ck.size();
+  const int nseg = A->nck;
   for (int seg = nseg - 1; seg >= 0; --seg) {
     const int s0 = seg * K, s1 = std::min(N, s0 + K);
     TRY(restore_ckpt(ctx, A->ck[seg]));
     for (int j = 0; j < s1 - s0; ++j) {
-      PD tp[2] = {tape_pd(j, 0), tape_pd(j, 1)};
+      TapePart tp[2] = {tape_of(j, 0), tape_of(j, 1)};
       uint32_t *pm[2] = {nullptr, nullptr};
       if (ctx->c_sort > c.sort_every - 1)  // this step begins with the sort
         for (int s = 0; s < 2; ++s) {
           uint32_t *&b = perm[2 * (size_t)j + s];
-          if (!b) TRYH(hipMalloc(&b, (size_t)cap * sizeof(uint32_t)));
+          TRYH(W.want(b, (size_t)cap * sizeof(uint32_t)));
           pm[s] = b;
         }
       TRY(fwd_step(ctx, ts[j], tf[j], tp, pm));
@@ -1535,8 +1640,9 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
         pk.bk.eimf_y = -A->p[3] * c.imf[0];
         pk.bk.imf_x = c.imf[0];
         pk.bk.imf_y = c.imf[1];
-        (c.dx == 1.0 ? k_pass_T<true> : k_pass_T<false>)<<<nb(np), 256, 0, st>>>(
-            g, tape_pd(j, sp), np, F, L, sp, pk, lp[sp], gvd);
+        const auto kern = c.dx == 1.0 ? (f64 ? k_pass_T<true, false> : k_pass_T<true, true>)
+                                      : (f64 ? k_pass_T<false, false> : k_pass_T<false, true>);
+        kern<<<nb(np), 256, 0, st>>>(g, tape_of(j, sp), np, F, L, sp, pk, lp[sp], gvd);
       }
       k_add_gather_T<<<nb(n), kBlock, 0, st>>>(n, L);
       TRYH(hipMemsetAsync(L.J[0][0], 0, 6 * n * sizeof(double), st));
@@ -1554,11 +1660,11 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
           const int64_t cnt = ts[j].hi[sp] - ts[j].lo[sp];
           if (cnt <= 0) continue;
           const int blocks = (int)std::min<int64_t>(1024, div_up(cnt, kBlock));
-          k_sum_vz<<<blocks, kBlock, 0, st>>>(lp[sp], ts[j].lo[sp], ts[j].hi[sp], nullptr, 1,
-                                              A->red);
+          k_sum_vz<<<blocks, kBlock, 0, st>>>(lp[sp], ts[j].lo[sp], ts[j].hi[sp], nullptr,
+                                              nullptr, 1, A->red);
           gV += sum_partials(ctx, A->red, blocks, 1, 0, &rc);
           if (rc) {
-            cleanup();
+            cleanup(false);
             return rc;
           }
         }
@@ -1566,6 +1672,7 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
       // slots the particles held before it
       if (ts[j].sorted)
         for (int sp = 0; sp < 2; ++sp) {
+          TRYH(W.want(lq[sp], 6 * (size_t)cap * sizeof(double)));
           TRYH(hipMemsetAsync(lq[sp], 0, 6 * (size_t)ts[j].nb[sp] * sizeof(double), st));
           if (ts[j].na[sp] > 0)
             k_unsort_lp<<<nb(ts[j].na[sp]), kBlock, 0, st>>>(
@@ -1581,10 +1688,11 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
     const int64_t cnt = ts[0].n[sp];
     if (cnt <= 0) continue;
     const int blocks = (int)std::min<int64_t>(1024, div_up(cnt, kBlock));
-    k_sum_vz<<<blocks, kBlock, 0, st>>>(lp[sp], 0, cnt, tape_pd(0, sp).z, 0, A->red);
+    const TapePart t0 = tape_of(0, sp);
+    k_sum_vz<<<blocks, kBlock, 0, st>>>(lp[sp], 0, cnt, t0.d.z, t0.f.cell, 0, A->red);
     gV += sum_partials(ctx, A->red, blocks, 1, 0, &rc);
     if (rc) {
-      cleanup();
+      cleanup(false);
       return rc;
     }
   }
@@ -1600,13 +1708,13 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
     for (int a = 0; a < 3; ++a) {
       grad[a] = sum_partials(ctx, A->red, blocks, 3, a, &rc);
       if (rc) {
-        cleanup();
+        cleanup(false);
         return rc;
       }
     }
   }
   grad[3] = gV;
-  cleanup();
+  cleanup(true);
   return 0;
 #undef TRY
 #undef TRYH

@@ -1,0 +1,74 @@
+"""The reverse sweep's buffers and units: a context that is asked again, with
+other windows and parameters, gives what a new one gives; dx away from 1 (its
+own instantiation of the transposed pass) against the oracle's gradient; the
+FP32 forward's tape, read in its own form, against the FP64 one."""
+import numpy as np
+import pytest
+
+import plasmasim_amd as ps
+from oracle_lib import Oracle
+
+pytestmark = pytest.mark.gpu
+R, NQ = 3.0, 64
+
+
+def cfg(precision=ps.PIC_FP64, dx=1.0, sort_every=20):
+    c = ps.preset(0)
+    c.precision = precision
+    c.inflow_every, c.sort_every = 3, sort_every
+    c.capacity = 16384
+    c.dx, c.dt = dx, c.dt * dx
+    c.ballistic_lo[2] *= dx
+    c.ballistic_hi[2] *= dx
+    return c
+
+
+def params(c, t=0.1):
+    M = c.dipole_m
+    return np.array([t * M, 0.9 * M, 0.3 * M, c.vdrift[2]])
+
+
+def grad(s, p, steps, window):
+    loss = s.adj_forward(p, steps, window, R, NQ)
+    return loss, s.adj_backward(1.0)
+
+
+@pytest.mark.parametrize("precision", [ps.PIC_FP64, ps.PIC_FP32])
+@pytest.mark.parametrize("sort_every", [2, 20])
+def test_repeated_sweeps_equal_fresh_ones(precision, sort_every):
+    """Buffers kept between sweeps: more steps, longer and shorter windows,
+    sorts inside a window.  FP64 atomics: sums in another order."""
+    c = cfg(precision, sort_every=sort_every)
+    s = ps.Simulation(c)
+    tol = 1e-9 if precision == ps.PIC_FP64 else 1e-5
+    for steps, window, t in ((6, 2, 0.1), (7, 5, 0.2), (4, 1, 0.1), (6, 2, 0.1)):
+        loss, g = grad(s, params(c, t), steps, window)
+        f = ps.Simulation(c)
+        lf, gf = grad(f, params(c, t), steps, window)
+        f.close()
+        assert abs(loss - lf) <= tol * abs(lf)
+        assert np.all(np.abs(g - gf) <= tol * np.abs(gf)), (steps, window, g, gf)
+    s.close()
+
+
+@pytest.mark.parametrize("dx", [1.0, 0.75])
+def test_gradient_in_other_units(dx):
+    c = cfg(dx=dx)
+    s = ps.Simulation(c)
+    loss, g = grad(s, params(c), 6, 2)
+    lo, go = Oracle(c, threads=4).adj_gradient(params(c), 6, R, NQ)
+    assert abs(loss - lo) <= 1e-10 * abs(lo)
+    assert np.all(np.abs(g - go) <= 1e-6 * np.abs(go)), (g, go)
+    s.close()
+
+
+def test_fp32_tape_gradient():
+    """The FP32 forward's gradient against the FP64 one: their trajectories
+    differ by the FP32 rounding of 6 steps."""
+    out = []
+    for precision in (ps.PIC_FP32, ps.PIC_FP64):
+        c = cfg(precision)
+        s = ps.Simulation(c)
+        out.append(grad(s, params(c), 6, 3)[1])
+        s.close()
+    assert np.all(np.abs(out[0] - out[1]) <= 1e-5 * np.abs(out[1])), out
