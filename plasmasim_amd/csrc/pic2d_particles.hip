@@ -195,28 +195,31 @@ __device__ inline void glb_add64(double *p, double v) {
 }
 
 // four node values of one deposit (shape_func_*0_* :2018-2144), to the LDS
-// window or to the plane; lanes start at different nodes (the particles of
-// a wave mostly share a cell)
+// window or to the plane; lane j takes the nodes mirrored along the axes set
+// in j & 3 (the particles of a wave mostly share a cell): the values change
+// places once, by selects
 __device__ inline void dep4_64(double *lds, double *glob, const Win2 &w,
                                const Geom2 &g, int k, int m, double v00,
                                double v10, double v01, double v11) {
-  const double v[4] = {v00, v10, v01, v11};
-  const int sw = threadIdx.x & 3;
   // the gate keeps nodes inside the array (for dx = 1 exactly; the check
   // only guards against x/dx rounding up to the gate's bound)
   if (k < 0 || m < 0 || k + 1 >= g.SX || m + 1 >= g.SZ) return;
   if (w.holds(k, m)) {
-    const int i = (k - w.k0) * w.WZ + (m - w.m0);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int id = n ^ sw;
-      lds_add64(lds + i + ((id & 1) ? w.WZ : 0) + (id >> 1), v[id]);
-    }
+    const bool mk = threadIdx.x & 1, mm = threadIdx.x & 2;
+    const double a0 = mk ? v10 : v00, a1 = mk ? v00 : v10;
+    const double b0 = mk ? v11 : v01, b1 = mk ? v01 : v11;
+    const int dk = mk ? -w.WZ : w.WZ, dm = mm ? -1 : 1;
+    double *p = lds + (k - w.k0) * w.WZ + (m - w.m0) + (mk ? w.WZ : 0) + (mm ? 1 : 0);
+    lds_add64(p, mm ? b0 : a0);
+    lds_add64(p + dk, mm ? b1 : a1);
+    lds_add64(p + dm, mm ? a0 : b0);
+    lds_add64(p + dk + dm, mm ? a1 : b1);
   } else {
-    const int64_t i = g.idx(k, m);
-#pragma unroll
-    for (int n = 0; n < 4; ++n)
-      glb_add64(glob + i + ((n & 1) ? g.SZ : 0) + (n >> 1), v[n]);
+    double *p = glob + g.idx(k, m);
+    glb_add64(p, v00);
+    glb_add64(p + g.SZ, v10);
+    glb_add64(p + 1, v01);
+    glb_add64(p + g.SZ + 1, v11);
   }
 }
 
@@ -272,7 +275,9 @@ struct Dep64 {
 // PUSH_J: hot loop A (:665-720); DRIFT: the half drift of loop B; DEP_N: the
 // density deposit of loop B (:752-788) or, without DRIFT, of the pre-loop
 // pass (:586-612); BOUNDARY: the exchange and delete sweep (:812-901)
-template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY>
+// UNIT: dx = 1, where x / dx and w * dx are x and w exactly: without the 20
+// divisions per particle.
+template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY, bool UNIT>
 __global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F,
                                                 P64 P, Run2 tr, Push2 kp,
                                                 Dep64 D) {
@@ -281,7 +286,7 @@ __global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F,
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
   const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
-  const double dx = kp.dx;
+  const double dx = UNIT ? 1.0 : kp.dx;
   if (tid == 0) {
     int64_t s, e;
     Win2 w;
@@ -878,8 +883,10 @@ int push(pic2d_ctx *ctx, int sp, int push_j, int drift_n, int boundary,
                plane<double>(ctx, jx + 2), plane<double>(ctx, nn)};
     const P64 P = p64(ctx, sp, ctx->cur[sp]);
     const Push2 kp = push_const(ctx, sp);
-#define L64(a, b, c, d) \
-  k_pass64<a, b, c, d><<<nb, 256, 0, st>>>(ctx->g, ctx->tg, F, P, tr, kp, D)
+    const bool unit = ctx->cfg.dx == 1.0;
+#define L64(a, b, c, d)                                           \
+  (unit ? k_pass64<a, b, c, d, true> : k_pass64<a, b, c, d, false>) \
+      <<<nb, 256, 0, st>>>(ctx->g, ctx->tg, F, P, tr, kp, D)
     switch (sel) {
       case 7: L64(true, true, true, true); break;
       case 4: L64(true, false, false, false); break;
