@@ -30,6 +30,8 @@ namespace pic2d {
 
 using pic::kMargin;
 using pic::kTailChunk;
+using pic::part_range;
+using pic::tile_split;
 using pic::xcd_remap;
 
 constexpr int kWin2 = 1024;  // LDS window capacity in nodes per quantity
@@ -38,11 +40,15 @@ constexpr int kWin2 = 1024;  // LDS window capacity in nodes per quantity
 #define PIC_GLB __attribute__((address_space(1)))
 typedef unsigned long long u64;
 
+constexpr int kPlaces2 = 1024;  // workgroups on the chip: 33 KB windows, four per CU
+
 struct Run2 {
   const uint32_t *tile_start;  // ntiles + 1
   int ntiles;
   int64_t sorted_end;
   int64_t n;
+  int split;  // workgroups per tile
+  __host__ __device__ inline int parts() const { return ntiles * split; }
 };
 
 struct Win2 {
@@ -59,16 +65,18 @@ template <typename CellOf>
 __device__ inline void setup2(int bid, const Run2 &tr, const Tile2 &tg,
                               CellOf cell_of, int64_t &s, int64_t &e, Win2 &w) {
   int ak0, ak1, am0, am1;
-  if (bid < tr.ntiles) {
-    s = tr.tile_start[bid];
-    e = tr.tile_start[bid + 1];
-    const int tx = bid / tg.NTZ, tz = bid % tg.NTZ;
+  if (bid < tr.parts()) {
+    const int t = bid / tr.split;
+    s = tr.tile_start[t];
+    e = tr.tile_start[t + 1];
+    part_range(bid % tr.split, tr.split, s, e);
+    const int tx = t / tg.NTZ, tz = t % tg.NTZ;
     ak0 = 2 + tx * tg.TX;
     ak1 = ak0 + tg.TX - 1;
     am0 = 2 + tz * tg.TZ;
     am1 = am0 + tg.TZ - 1;
   } else {
-    const int c = bid - tr.ntiles;
+    const int c = bid - tr.parts();
     s = tr.sorted_end + (int64_t)c * kTailChunk;
     e = s + kTailChunk < tr.n ? s + kTailChunk : tr.n;
     ak0 = am0 = 1 << 30;
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F,
   __shared__ Win2 sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
+  const int bid = xcd_remap(blockIdx.x, tr.parts(), (int)gridDim.x);
   const double dx = UNIT ? 1.0 : kp.dx;
   if (tid == 0) {
     int64_t s, e;
@@ -709,7 +717,7 @@ __global__ __launch_bounds__(256) void k_pass32(Geom2 g, Tile2 tg, F32Fields F,
   __shared__ Win2 sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.ntiles, (int)gridDim.x);
+  const int bid = xcd_remap(blockIdx.x, tr.parts(), (int)gridDim.x);
   if (tid == 0) {
     int64_t s, e;
     Win2 w;
@@ -855,7 +863,9 @@ static Run2 run_of(pic2d_ctx *ctx, int sp, unsigned *nblocks) {
   tr.sorted_end = ctx->sorted_end[sp];
   tr.n = ctx->n[sp];
   const int64_t ntail = div_up(tr.n - tr.sorted_end, kTailChunk);
-  *nblocks = (unsigned)(tr.ntiles + ntail);
+  const pic2d_config &c = ctx->cfg;
+  tr.split = tile_split(tr.ntiles, (int64_t)c.nx * c.nz * c.ppc, kPlaces2);
+  *nblocks = (unsigned)(tr.parts() + ntail);
   return tr;
 }
 

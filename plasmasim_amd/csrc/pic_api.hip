@@ -25,6 +25,11 @@ int set_error(pic_ctx *ctx, int code, const char *fmt, ...) {
   return code;
 }
 
+int pass_split(const pic_ctx *ctx) {
+  const pic_config &c = ctx->cfg;
+  return tile_split(tile_geom(ctx).ntiles(), (int64_t)c.nx * c.ny * c.nz * c.ppc, kChipSlots);
+}
+
 StepConst step_const(const pic_ctx *ctx, int sp) {
   const pic_config &c = ctx->cfg;
   StepConst k;
@@ -900,7 +905,8 @@ extern "C" int pic_thrust_ave_enable(pic_ctx *ctx, int on) {
   const TileGeom tg = tile_geom(ctx);
   // workgroups of one pass: the tiles and the tail chunks of up to the
   // capacity's slots
-  const int64_t boxes = tg.ntiles() == 1 ? row_geom(tg).ntiles() : tg.ntiles();
+  const int64_t boxes =
+      tg.ntiles() == 1 ? row_geom(tg).ntiles() : (int64_t)tg.ntiles() * pass_split(ctx);
   const int64_t slots = boxes + most_chunks(ctx->cfg.ppc, ctx->cap);
   if (!ctx->thrust_acc) PIC_HIP(ctx, hipMalloc(&ctx->thrust_acc, 16 * sizeof(double)));
   if (ctx->thrust_part_slots < slots) {

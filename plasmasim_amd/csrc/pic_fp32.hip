@@ -667,8 +667,8 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
   __shared__ int s_box;
   const Geom &g = G.g;
   const int tid = threadIdx.x;
-  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.ntiles, BOTH ? nb0 : (int)gridDim.x)
-                          : xcd_remap(blockIdx.x - nb0, tr.ntiles, (int)gridDim.x - nb0);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.parts(), BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.parts(), (int)gridDim.x - nb0);
 
   if (tid == 0) {
     int64_t s, e;
@@ -691,9 +691,9 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
       // the open box or outside it unless that range meets its faces;
       // tail chunks test each particle
       int cls = 2;
-      if (bid < tr.ntiles) {
-        const int tz = bid % tg.NTZ, ty = (bid / tg.NTZ) % tg.NTY,
-                  tx = bid / (tg.NTZ * tg.NTY);
+      if (bid < tr.parts()) {
+        const int t = bid / tr.split, tz = t % tg.NTZ, ty = (t / tg.NTZ) % tg.NTY,
+                  tx = t / (tg.NTZ * tg.NTY);
         const int T[3] = {tg.TX, tg.TY, tg.TZ}, t3[3] = {tx, ty, tz};
         bool in = true, out = false;
         for (int a = 0; a < 3; ++a) {
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
   constexpr int SH = N == 8 ? 3 : N == 4 ? 2 : N == 2 ? 1 : 0;
   // slot indices fit in int32 (the host bounds the stored count)
   int s32 = (int)s, e32 = (int)e, lane = tid, lanes = blockDim.x;
-  if (ROWS && bid < tr.ntiles) {
+  if (ROWS && bid < tr.parts()) {
     lanes = kPassBlock / (tg.TX * tg.TY);
     row_range(tr, tg, g.NX, g.NY, g.NZ, bid, tid / lanes, s32, e32);
     lane = tid % lanes;
@@ -2054,7 +2054,8 @@ static int prepare_pass(pic_ctx *ctx, int sp, int sel, SpeciesArgs32 &a, bool *r
   tr.chunk = tail_chunk(ctx->cfg.ppc, ctx->geom.NX % 4 == 0 && ctx->geom.NY % 4 == 0,
                         n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
-  const unsigned blocks = (unsigned)(tr.ntiles + tr.ntail);
+  tr.split = *rows || tr.ntiles == 0 ? 1 : pass_split(ctx);
+  const unsigned blocks = (unsigned)(tr.parts() + tr.ntail);
   a.tg = tg;
   a.tr = tr;
   Push32 &kp = a.kp;

@@ -773,8 +773,8 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
   __shared__ Win sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.ntiles, BOTH ? nb0 : (int)gridDim.x)
-                          : xcd_remap(blockIdx.x - nb0, tr.ntiles, (int)gridDim.x - nb0);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.parts(), BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.parts(), (int)gridDim.x - nb0);
   const double dx = UNIT ? 1.0 : kc.dx;
   if (tid == 0) {
     int64_t s, e;
@@ -826,7 +826,7 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
   const double dth = kc.dth;
   int64_t i0 = s + tid, i1 = e;
   int lanes = blockDim.x;
-  if (ROWS && bid < tr.ntiles) {
+  if (ROWS && bid < tr.parts()) {
     lanes = kBlock / (tg.TX * tg.TY);
     int rs, re;
     row_range(tr, tg, g.NX, g.NY, g.NZ, bid, tid / lanes, rs, re);
@@ -1381,9 +1381,10 @@ static int prepare_pass(pic_ctx *ctx, int sp, int sel, SpeciesArgs64 &a, bool *r
   tr.n = n;
   tr.chunk = tail_chunk(ctx->cfg.ppc, false, n - tr.sorted_end);
   tr.ntail = (int)div_up(n - tr.sorted_end, tr.chunk);
+  tr.split = *rows || tr.ntiles == 0 ? 1 : pass_split(ctx);
   a.tg = tg;
   a.tr = tr;
-  const unsigned blocks = (unsigned)(tr.ntiles + tr.ntail);
+  const unsigned blocks = (unsigned)(tr.parts() + tr.ntail);
   // the fused pass of pic_step adds the previous step's thrust_fave
   a.thrust_part = nullptr;
   if (ctx->thrust_now && sel == 7) {

@@ -238,6 +238,7 @@ inline SigmaProfile sigma(pic_ctx *ctx) {
   return s;
 }
 StepConst step_const(const pic_ctx *ctx, int sp);
+int pass_split(const pic_ctx *ctx);  // workgroups per tile of the particle pass
 inline TileGeom tile_geom(const pic_ctx *ctx) {
   const pic_config &c = ctx->cfg;
   TileGeom t;
