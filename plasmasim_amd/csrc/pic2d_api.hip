@@ -634,11 +634,11 @@ extern "C" int pic2d_step(pic2d_ctx *ctx, int nsteps) {
       TRY(pic2d_renew_b_half(ctx));
       TRY(pic2d_halo(ctx));
     }
-    for (int sp = 0; sp < 2; ++sp) {
-      const int tclass = ctx->pending[sp] ? PIC_T_PUSH_SORT : PIC_T_PUSH;
+    {
+      const int tclass = ctx->pending[0] || ctx->pending[1] ? PIC_T_PUSH_SORT : PIC_T_PUSH;
       pic::timing_begin(&ctx->rt, tclass);
-      rc = push(ctx, sp, 1, 1, 1, 0);
-      pic::timing_end(&ctx->rt, tclass);
+      rc = push_both(ctx);
+      pic::timing_end(&ctx->rt, tclass, 2);
       TRY(rc);
     }
     const bool with_phi = c.poisson_every > 0 && ctx->step % c.poisson_every == 0;

@@ -285,15 +285,37 @@ struct Dep64 {
 // pass (:586-612); BOUNDARY: the exchange and delete sweep (:812-901)
 // UNIT: dx = 1, where x / dx and w * dx are x and w exactly: without the 20
 // divisions per particle.
-template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY, bool UNIT>
-__global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F,
-                                                P64 P, Run2 tr, Push2 kp,
-                                                Dep64 D) {
+// One species of a pass.  BOTH: the launch holds both, the first nb0
+// workgroups the ions': the second one's workgroups take the places that the
+// last of the first leave empty, and a launch goes.  20 steps, one launch /
+// two: 64^2 x 30 ppc FP32 1.19 / 1.47 ms, 256^2 x 16 ppc 2.14 / 2.32 ms,
+// 512^2 x 36 ppc FP64 12.3 / 12.7 ms, 1024^2 x 28 ppc FP64 35.5 / 36.2 ms,
+// 2048^2 x 100 ppc FP32 (33000 workgroups) 252 / 250 ms.
+constexpr unsigned kBothBlocks2 = 16384;
+struct Species64 {
+  P64 P;
+  Run2 tr;
+  Push2 kp;
+  Dep64 D;
+};
+struct Pass64 {
+  Species64 s[2];
+};
+
+template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY, bool UNIT, bool BOTH>
+__global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F, Pass64 args,
+                                                int nb0) {
+  const int sp = BOTH && (int)blockIdx.x >= nb0 ? 1 : 0;
+  const P64 &P = args.s[sp].P;
+  const Run2 &tr = args.s[sp].tr;
+  const Push2 &kp = args.s[sp].kp;
+  const Dep64 &D = args.s[sp].D;
   __shared__ double acc[4 * kWin2];
   __shared__ Win2 sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.parts(), (int)gridDim.x);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.parts(), BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.parts(), (int)gridDim.x - nb0);
   const double dx = UNIT ? 1.0 : kp.dx;
   if (tid == 0) {
     int64_t s, e;
@@ -382,8 +404,9 @@ __global__ __launch_bounds__(256) void k_pass64(Geom2 g, Tile2 tg, F64Fields F,
 
 // ===========================================================================
 // FP32 form: int32 cell + fp32 offsets.  This translation unit rounds every
-// FP64 operation separately; the FP32 functions below may fuse.
-#pragma clang fp contract(fast)
+// FP64 operation separately; the FP32 functions below fuse by expression, so
+// that every instantiation of the pass rounds alike.
+#pragma clang fp contract(on)
 
 struct K32 {
   float T, hdt;          // q dt / (2m); dt / (2 dx)
@@ -709,15 +732,32 @@ __device__ __forceinline__ void step32(const Geom2 &g, const F32Fields &F,
 // PERM: the pass also applies a sort's permutation: slot i takes its
 // particle from slot perm[i] of Q and stores the result in P (the other
 // buffer of the species), so the sort needs no separate copy
-template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY, bool PERM>
-__global__ __launch_bounds__(256) void k_pass32(Geom2 g, Tile2 tg, F32Fields F,
-                                                P32 P, Run2 tr, K32 kp, Dep32 D,
-                                                P32 Q, const uint32_t *__restrict__ perm) {
+struct Species32 {
+  P32 P, Q;
+  const uint32_t *perm;
+  Run2 tr;
+  K32 kp;
+  Dep32 D;
+};
+struct Pass32 {
+  Species32 s[2];
+};
+
+template <bool PUSH_J, bool DRIFT, bool DEP_N, bool BOUNDARY, bool PERM, bool BOTH>
+__global__ __launch_bounds__(256) void k_pass32(Geom2 g, Tile2 tg, F32Fields F, Pass32 args,
+                                                int nb0) {
+  const int sp = BOTH && (int)blockIdx.x >= nb0 ? 1 : 0;
+  const P32 &P = args.s[sp].P, &Q = args.s[sp].Q;
+  const uint32_t *__restrict__ perm = args.s[sp].perm;
+  const Run2 &tr = args.s[sp].tr;
+  const K32 &kp = args.s[sp].kp;
+  const Dep32 &D = args.s[sp].D;
   __shared__ u64 acc[4 * kWin2];
   __shared__ Win2 sw;
   __shared__ int64_t s_range[2];
   const int tid = threadIdx.x;
-  const int bid = xcd_remap(blockIdx.x, tr.parts(), (int)gridDim.x);
+  const int bid = sp == 0 ? xcd_remap(blockIdx.x, tr.parts(), BOTH ? nb0 : (int)gridDim.x)
+                          : xcd_remap(blockIdx.x - nb0, tr.parts(), (int)gridDim.x - nb0);
   if (tid == 0) {
     int64_t s, e;
     Win2 w;
@@ -871,94 +911,148 @@ static Run2 run_of(pic2d_ctx *ctx, int sp, unsigned *nblocks) {
 
 static uint32_t *pass_perm(pic2d_ctx *ctx, int sp);
 
+static Species64 species64(pic2d_ctx *ctx, int sp, unsigned *nb) {
+  const int jx = sp == 0 ? PIC_JIX : PIC_JEX, nn = sp == 0 ? PIC_NI : PIC_NE;
+  Species64 a;
+  a.P = p64(ctx, sp, ctx->cur[sp]);
+  a.tr = run_of(ctx, sp, nb);
+  a.kp = push_const(ctx, sp);
+  a.D = {plane<double>(ctx, jx), plane<double>(ctx, jx + 1), plane<double>(ctx, jx + 2),
+         plane<double>(ctx, nn)};
+  return a;
+}
+
+static Species32 species32(pic2d_ctx *ctx, int sp, unsigned *nb) {
+  const int jx = sp == 0 ? PIC_JIX : PIC_JEX, nn = sp == 0 ? PIC_NI : PIC_NE;
+  Species32 a;
+  // with a pending permutation the pass reads the current buffer through it
+  // and writes the other one
+  a.perm = ctx->pending[sp] ? pass_perm(ctx, sp) : nullptr;
+  a.Q = p32(ctx, sp, ctx->cur[sp]);
+  a.P = a.perm ? p32(ctx, sp, 1 - ctx->cur[sp]) : a.Q;
+  a.tr = run_of(ctx, sp, nb);
+  a.D = {plane<float>(ctx, jx), plane<float>(ctx, jx + 1), plane<float>(ctx, jx + 2),
+         plane<float>(ctx, nn)};
+  const pic2d_config &c = ctx->cfg;
+  const Push2 p = push_const(ctx, sp);
+  K32 &kp = a.kp;
+  kp.T = (float)p.T;
+  kp.hdt = (float)(c.dt / (2.0 * c.dx));
+  kp.qw = (float)(p.qw / (c.dx * c.dx));
+  kp.w = (float)(p.w / (c.dx * c.dx));
+  kp.eimf_x = (float)p.eimf_x;
+  kp.eimf_y = (float)p.eimf_y;
+  for (int x = 0; x < 2; ++x) {
+    kp.blo[x] = (float)std::max(-1e30, std::min(1e30, p.blo[x] / c.dx));
+    kp.bhi[x] = (float)std::max(-1e30, std::min(1e30, p.bhi[x] / c.dx));
+  }
+  kp.fx = (float)ctx->fx_scale;
+  kp.fx_inv = 1.0 / ctx->fx_scale;
+  cell_magic(ctx->g.SZ, kp.cmag, kp.csh);
+  return a;
+}
+
+// the pass sel (8: the density of the pre-loop) of args.s[0], or the fused
+// pass (7) of both species where nb[1] > 0
+static int launch64(pic2d_ctx *ctx, int sel, const Pass64 &args, const unsigned nb[2]) {
+  if (nb[0] + nb[1] == 0) return 0;
+  const F64Fields F = {plane<double>(ctx, PIC_EX), plane<double>(ctx, PIC_EY),
+                       plane<double>(ctx, PIC_EZ), plane<double>(ctx, PIC_BX),
+                       plane<double>(ctx, PIC_BY), plane<double>(ctx, PIC_BZ)};
+  const bool unit = ctx->cfg.dx == 1.0;
+#define L(a, b, c, d, e) (unit ? k_pass64<a, b, c, d, true, e> : k_pass64<a, b, c, d, false, e>)
+  const auto kern = sel == 7   ? (nb[1] ? L(true, true, true, true, true)
+                                        : L(true, true, true, true, false))
+                    : sel == 4 ? L(true, false, false, false, false)
+                    : sel == 2 ? L(false, true, true, false, false)
+                    : sel == 1 ? L(false, false, false, true, false)
+                               : L(false, false, true, false, false);
+#undef L
+  kern<<<nb[0] + nb[1], 256, 0, ctx->rt.stream>>>(ctx->g, ctx->tg, F, args, (int)nb[0]);
+  P2_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+static int launch32(pic2d_ctx *ctx, int sel, bool perm, const Pass32 &args,
+                    const unsigned nb[2]) {
+  if (nb[0] + nb[1] == 0) return 0;
+  const F32Fields F = {plane<float>(ctx, PIC_EX), plane<float>(ctx, PIC_EY),
+                       plane<float>(ctx, PIC_EZ), plane<float>(ctx, PIC_BX),
+                       plane<float>(ctx, PIC_BY), plane<float>(ctx, PIC_BZ)};
+#define L(BOTH)                                        \
+  (perm ? k_pass32<true, true, true, true, true, BOTH> \
+        : k_pass32<true, true, true, true, false, BOTH>)
+  const auto kern = sel == 7   ? (nb[1] ? L(true) : L(false))
+                    : sel == 4 ? k_pass32<true, false, false, false, false, false>
+                    : sel == 2 ? k_pass32<false, true, true, false, false, false>
+                    : sel == 1 ? k_pass32<false, false, false, true, false, false>
+                               : k_pass32<false, false, true, false, false, false>;
+#undef L
+  kern<<<nb[0] + nb[1], 256, 0, ctx->rt.stream>>>(ctx->g, ctx->tg, F, args, (int)nb[0]);
+  P2_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
+// a routine's pass of one species
 int push(pic2d_ctx *ctx, int sp, int push_j, int drift_n, int boundary,
          int density_only) {
-  // a pending sort permutation is applied by the fused pass only
-  const bool fused = push_j && drift_n && boundary && !density_only;
-  if (!fused) {
-    int rc = settle(ctx, sp);
-    if (rc) return rc;
-  }
-  if (ctx->n[sp] == 0) return 0;
-  unsigned nb;
-  const Run2 tr = run_of(ctx, sp, &nb);
-  const int jx = sp == 0 ? PIC_JIX : PIC_JEX, nn = sp == 0 ? PIC_NI : PIC_NE;
   const int sel = density_only ? 8 : (push_j ? 4 : 0) | (drift_n ? 2 : 0) | (boundary ? 1 : 0);
-  hipStream_t st = ctx->rt.stream;
+  if (sel != 8 && sel != 4 && sel != 2 && sel != 1)
+    return err(ctx, PIC_E_ARG, "push: unsupported routine combination");
+  // a pending sort permutation is applied by the fused pass only
+  int rc = settle(ctx, sp);
+  if (rc) return rc;
+  if (ctx->n[sp] == 0) return 0;
+  unsigned nb[2] = {0, 0};
   if (ctx->f64) {
-    F64Fields F = {plane<double>(ctx, PIC_EX), plane<double>(ctx, PIC_EY),
-                   plane<double>(ctx, PIC_EZ), plane<double>(ctx, PIC_BX),
-                   plane<double>(ctx, PIC_BY), plane<double>(ctx, PIC_BZ)};
-    Dep64 D = {plane<double>(ctx, jx), plane<double>(ctx, jx + 1),
-               plane<double>(ctx, jx + 2), plane<double>(ctx, nn)};
-    const P64 P = p64(ctx, sp, ctx->cur[sp]);
-    const Push2 kp = push_const(ctx, sp);
-    const bool unit = ctx->cfg.dx == 1.0;
-#define L64(a, b, c, d)                                           \
-  (unit ? k_pass64<a, b, c, d, true> : k_pass64<a, b, c, d, false>) \
-      <<<nb, 256, 0, st>>>(ctx->g, ctx->tg, F, P, tr, kp, D)
-    switch (sel) {
-      case 7: L64(true, true, true, true); break;
-      case 4: L64(true, false, false, false); break;
-      case 2: L64(false, true, true, false); break;
-      case 1: L64(false, false, false, true); break;
-      case 8: L64(false, false, true, false); break;
-      default: return err(ctx, PIC_E_ARG, "push: unsupported routine combination");
-    }
-#undef L64
-  } else {
-    F32Fields F = {plane<float>(ctx, PIC_EX), plane<float>(ctx, PIC_EY),
-                   plane<float>(ctx, PIC_EZ), plane<float>(ctx, PIC_BX),
-                   plane<float>(ctx, PIC_BY), plane<float>(ctx, PIC_BZ)};
-    Dep32 D = {plane<float>(ctx, jx), plane<float>(ctx, jx + 1),
-               plane<float>(ctx, jx + 2), plane<float>(ctx, nn)};
-    // with a pending permutation the pass reads the current buffer through
-    // it and writes the other one
-    const uint32_t *pm = ctx->pending[sp] ? pass_perm(ctx, sp) : nullptr;
-    const P32 Q = p32(ctx, sp, ctx->cur[sp]);
-    const P32 P = pm ? p32(ctx, sp, 1 - ctx->cur[sp]) : Q;
-    const pic2d_config &c = ctx->cfg;
-    const Push2 p = push_const(ctx, sp);
-    K32 kp;
-    kp.T = (float)p.T;
-    kp.hdt = (float)(c.dt / (2.0 * c.dx));
-    kp.qw = (float)(p.qw / (c.dx * c.dx));
-    kp.w = (float)(p.w / (c.dx * c.dx));
-    kp.eimf_x = (float)p.eimf_x;
-    kp.eimf_y = (float)p.eimf_y;
-    for (int a = 0; a < 2; ++a) {
-      kp.blo[a] = (float)std::max(-1e30, std::min(1e30, p.blo[a] / c.dx));
-      kp.bhi[a] = (float)std::max(-1e30, std::min(1e30, p.bhi[a] / c.dx));
-    }
-    kp.fx = (float)ctx->fx_scale;
-    kp.fx_inv = 1.0 / ctx->fx_scale;
-    cell_magic(ctx->g.SZ, kp.cmag, kp.csh);
-#define L32(a, b, c, d) \
-  k_pass32<a, b, c, d, false><<<nb, 256, 0, st>>>(ctx->g, ctx->tg, F, P, tr, kp, D, Q, pm)
-    switch (sel) {
-      case 7:
-        if (pm)
-          k_pass32<true, true, true, true, true>
-              <<<nb, 256, 0, st>>>(ctx->g, ctx->tg, F, P, tr, kp, D, Q, pm);
-        else
-          L32(true, true, true, true);
-        break;
-      case 4: L32(true, false, false, false); break;
-      case 2: L32(false, true, true, false); break;
-      case 1: L32(false, false, false, true); break;
-      case 8: L32(false, false, true, false); break;
-      default: return err(ctx, PIC_E_ARG, "push: unsupported routine combination");
-    }
-#undef L32
-    P2_LAUNCH_CHECK(ctx);
-    if (pm) {
-      ctx->cur[sp] = 1 - ctx->cur[sp];
-      ctx->pending[sp] = false;
+    Pass64 args = {};
+    args.s[0] = species64(ctx, sp, &nb[0]);
+    return launch64(ctx, sel, args, nb);
+  }
+  Pass32 args = {};
+  args.s[0] = species32(ctx, sp, &nb[0]);
+  return launch32(ctx, sel, false, args, nb);
+}
+
+// The fused passes of both species: one launch below kBothBlocks2 workgroups
+// where both carry a sort's permutation or neither does.
+int push_both(pic2d_ctx *ctx) {
+  unsigned nb[2] = {0, 0};
+  if (ctx->f64) {
+    Pass64 args = {};
+    for (int sp = 0; sp < 2; ++sp)
+      if (ctx->n[sp] > 0) args.s[sp] = species64(ctx, sp, &nb[sp]);
+    if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2) return launch64(ctx, 7, args, nb);
+    for (int sp = 0; sp < 2; ++sp) {
+      Pass64 a = {};
+      a.s[0] = args.s[sp];
+      const unsigned one[2] = {nb[sp], 0};
+      int rc = launch64(ctx, 7, a, one);
+      if (rc) return rc;
     }
     return 0;
   }
-  P2_LAUNCH_CHECK(ctx);
-  return 0;
+  Pass32 args = {};
+  for (int sp = 0; sp < 2; ++sp)
+    if (ctx->n[sp] > 0) args.s[sp] = species32(ctx, sp, &nb[sp]);
+  const bool perm[2] = {args.s[0].perm != nullptr, args.s[1].perm != nullptr};
+  int rc = 0;
+  if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2 && perm[0] == perm[1]) {
+    rc = launch32(ctx, 7, perm[0], args, nb);
+  } else {
+    for (int sp = 0; sp < 2 && !rc; ++sp) {
+      Pass32 a = {};
+      a.s[0] = args.s[sp];
+      const unsigned one[2] = {nb[sp], 0};
+      rc = launch32(ctx, 7, perm[sp], a, one);
+    }
+  }
+  for (int sp = 0; sp < 2 && !rc; ++sp)
+    if (perm[sp]) {
+      ctx->cur[sp] = 1 - ctx->cur[sp];
+      ctx->pending[sp] = false;
+    }
+  return rc;
 }
 
 int particle_boundary(pic2d_ctx *ctx, int sp) { return push(ctx, sp, 0, 0, 1, 0); }
