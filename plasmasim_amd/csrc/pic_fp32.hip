@@ -985,85 +985,60 @@ __global__ __launch_bounds__(256) void k_renew_e32(Geom g, Fields<float> F, Sigm
 
 // sr_b / sr_e on one rank: the reference copies the total field into the
 // guards.  For B this form stores B1 = B - B0 and B0 is not periodic, so the
-// guard receives B1(src) + B0(src) - B0(guard); E planes pass b0 = nullptr.
-__device__ inline void copy_total(float *f, const float *b0, float *bt,
-                                  int64_t dst, int64_t src) {
-  if (b0) {
-    f[dst] = f[src] + (b0[src] - b0[dst]);
-    bt[dst] = bt[src];
-  } else {
-    f[dst] = f[src];
-  }
+// guard receives B1(src) + B0(src) - B0(guard), the corner from the x image
+// (images of cell c with B1 = v, B0 = p and total B tot; kept as below).
+template <bool KEEP>
+__device__ inline void b_images(const Geom &g, float *B, const float *B0, float *t, int k,
+                                int l, int64_t c, float v, float p, float tot) {
+  float v1 = 0.0f, p1 = 0.0f;
+  bool first = true;
+  images(g, k, l, c, [&](int64_t d, int64_t s) {
+    const float bd = B0[d];
+    const float w = s == c ? v + (p - bd) : v1 + (p1 - bd);
+    if (first) {  // the x image, where there is one (a corner needs it)
+      v1 = w;
+      p1 = bd;
+      first = false;
+    }
+    if (KEEP) t[3 * g.plane + d] = t[d];
+    B[d] = w;
+    t[d] = tot;
+  });
 }
 
-__global__ void k_halo_x32(Geom g, float *a, float *b, float *c,
-                           const float *a0, const float *b0, const float *c0,
-                           float *bt) {
+// the guard columns of the three planes from `first`; bt: B, else E
+__global__ void k_halo32(Geom g, Fields<float> F, int first, float *bt) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SY * g.SZ;
-  if (i >= n) return;
-  const int64_t dk = n;
-  float *p[3] = {a, b, c};
-  const float *p0[3] = {a0, b0, c0};
+  if (i >= (int64_t)fold_groups(g) * g.SZ) return;
+  int k, l;
+  edge_column(g, (int)(i / g.SZ), k, l);
+  const int64_t c = g.idx(k, l, (int)(i % g.SZ));
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    float *t = bt ? bt + q * g.plane : nullptr;
-    copy_total(p[q], p0[q], t, i, i + g.NX * dk);
-    copy_total(p[q], p0[q], t, i + dk, i + (g.NX + 1) * dk);
-    copy_total(p[q], p0[q], t, i + (g.NX + 2) * dk, i + 2 * dk);
-    copy_total(p[q], p0[q], t, i + (g.NX + 3) * dk, i + 3 * dk);
+    float *f = F.f[first + q];
+    const float v = f[c];
+    if (bt) {
+      const float *b0 = F.f[PIC_B0X + q];
+      float *t = bt + q * g.plane;
+      b_images<false>(g, f, b0, t, k, l, c, v, b0[c], t[c]);
+    } else {
+      images(g, k, l, c, [&](int64_t d, int64_t) { f[d] = v; });
+    }
   }
 }
 
-__global__ void k_halo_y32(Geom g, float *a, float *b, float *c,
-                           const float *a0, const float *b0, const float *c0,
-                           float *bt) {
+// sr_current2
+__global__ void k_fold32(Geom g, Fields<float> F) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SX * g.SZ;
-  if (i >= n) return;
-  const int k = (int)(i / g.SZ), m = (int)(i % g.SZ);
-  const int64_t dl = g.SZ;
-  const int64_t o = g.idx(k, 0, m);
-  float *p[3] = {a, b, c};
-  const float *p0[3] = {a0, b0, c0};
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    float *t = bt ? bt + q * g.plane : nullptr;
-    copy_total(p[q], p0[q], t, o, o + g.NY * dl);
-    copy_total(p[q], p0[q], t, o + dl, o + (g.NY + 1) * dl);
-    copy_total(p[q], p0[q], t, o + (g.NY + 2) * dl, o + 2 * dl);
-    copy_total(p[q], p0[q], t, o + (g.NY + 3) * dl, o + 3 * dl);
-  }
-}
-
-__global__ void k_fold_x32(Geom g, Fields<float> F) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SY * g.SZ;
-  if (i >= n) return;
-  const int64_t dk = n;
+  if (i >= (int64_t)fold_groups(g) * g.SZ) return;
 #pragma unroll
   for (int q = PIC_JIX; q <= PIC_NE; ++q) {
-    float *f = F.f[q] + i;
-    f[2 * dk] += f[(g.NX + 2) * dk];
-    f[3 * dk] += f[(g.NX + 3) * dk];
-    f[g.NX * dk] += f[0];
-    f[(g.NX + 1) * dk] += f[dk];
-  }
-}
-
-__global__ void k_fold_y32(Geom g, Fields<float> F) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SX * g.SZ;
-  if (i >= n) return;
-  const int k = (int)(i / g.SZ), m = (int)(i % g.SZ);
-  const int64_t dl = g.SZ;
-#pragma unroll
-  for (int q = PIC_JIX; q <= PIC_NE; ++q) {
-    float *f = F.f[q] + g.idx(k, 0, m);
-    f[2 * dl] += f[(g.NY + 2) * dl];
-    f[3 * dl] += f[(g.NY + 3) * dl];
-    f[g.NY * dl] += f[0];
-    f[(g.NY + 1) * dl] += f[dl];
+    float *f = F.f[q];
+    fold_group(
+        g, (int)(i / g.SZ), (int)(i % g.SZ), [&](int64_t j) { return f[j]; },
+        [&](int64_t j, float v, bool changed) {
+          if (changed) f[j] = v;
+        });
   }
 }
 
@@ -1109,22 +1084,7 @@ __device__ inline void b_and_guards(const Geom &g, const Fields<float> &F, float
       B[c] = b;
       t[c] = tot;
     }
-    // a guard's B1 is B1(src) + B0(src) - B0(guard); the corner continues
-    // from the x image
-    float v0 = b, p0 = b0, v1 = 0.0f, p1 = 0.0f;
-    bool first = true;
-    images(g, k, l, c, [&](int64_t d, int64_t s) {
-      const float bd = B0[d];
-      const float v = s == c ? v0 + (p0 - bd) : v1 + (p1 - bd);
-      if (first) {  // the x image, where there is one (a corner needs it)
-        v1 = v;
-        p1 = bd;
-        first = false;
-      }
-      if (KEEP) t[3 * pl + d] = t[d];
-      B[d] = v;
-      t[d] = tot;
-    });
+    b_images<KEEP>(g, B, B0, t, k, l, c, b, b0, tot);
   }
 }
 
@@ -1892,16 +1852,9 @@ int renew_e(pic_ctx *ctx) {
 
 int halo(pic_ctx *ctx, int first) {
   const Geom &g = ctx->geom;
-  Fields<float> F = fields<float>(ctx);
-  float *a = F.f[first], *b = F.f[first + 1], *c = F.f[first + 2];
-  const bool isb = first == PIC_BX;
-  const float *a0 = isb ? F.f[PIC_B0X] : nullptr, *b0 = isb ? F.f[PIC_B0Y] : nullptr,
-              *c0 = isb ? F.f[PIC_B0Z] : nullptr;
-  float *bt = isb ? st(ctx)->bt : nullptr;
-  k_halo_x32<<<(unsigned)div_up((int64_t)g.SY * g.SZ, kBlock), kBlock, 0,
-               ctx->stream>>>(g, a, b, c, a0, b0, c0, bt);
-  k_halo_y32<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
-               ctx->stream>>>(g, a, b, c, a0, b0, c0, bt);
+  k_halo32<<<(unsigned)div_up((int64_t)fold_groups(g) * g.SZ, kBlock), kBlock, 0,
+             ctx->stream>>>(g, fields<float>(ctx), first,
+                            first == PIC_BX ? st(ctx)->bt : nullptr);
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
@@ -1945,11 +1898,8 @@ int step_e(pic_ctx *ctx) {
 
 int fold_current(pic_ctx *ctx) {
   const Geom &g = ctx->geom;
-  Fields<float> F = fields<float>(ctx);
-  k_fold_x32<<<(unsigned)div_up((int64_t)g.SY * g.SZ, kBlock), kBlock, 0,
-               ctx->stream>>>(g, F);
-  k_fold_y32<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
-               ctx->stream>>>(g, F);
+  k_fold32<<<(unsigned)div_up((int64_t)fold_groups(g) * g.SZ, kBlock), kBlock, 0,
+             ctx->stream>>>(g, fields<float>(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }

@@ -167,71 +167,34 @@ __global__ __launch_bounds__(256) void k_renew_e(Geom g, Fields<double> F, Sigma
   for (int q = 0; q < 3; ++q) F.f[PIC_EX + q][c] = e[q];
 }
 
-// sr_b / sr_e on one rank (:1001-1387): copy along x over all (l,m), then
-// along y over all (k,m) in a second launch so that corners see the x pass.
-__global__ void k_halo_x(Geom g, double *a, double *b, double *c) {
+// sr_b / sr_e on one rank (:1001-1387): the guard columns of the three planes
+// from `first`
+__global__ void k_halo(Geom g, Fields<double> F, int first) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SY * g.SZ;
-  if (i >= n) return;
-  const int64_t dk = n;
-  double *p[3] = {a, b, c};
+  if (i >= (int64_t)fold_groups(g) * g.SZ) return;
+  int k, l;
+  edge_column(g, (int)(i / g.SZ), k, l);
+  const int64_t c = g.idx(k, l, (int)(i % g.SZ));
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    double *f = p[q] + i;
-    f[0] = f[g.NX * dk];
-    f[1 * dk] = f[(g.NX + 1) * dk];
-    f[(g.NX + 2) * dk] = f[2 * dk];
-    f[(g.NX + 3) * dk] = f[3 * dk];
+    double *f = F.f[first + q];
+    const double v = f[c];
+    images(g, k, l, c, [&](int64_t d, int64_t) { f[d] = v; });
   }
 }
 
-__global__ void k_halo_y(Geom g, double *a, double *b, double *c) {
+// sr_current2 (:1805-2039) on one rank, 8 planes
+__global__ void k_fold(Geom g, Fields<double> F) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SX * g.SZ;
-  if (i >= n) return;
-  const int k = (int)(i / g.SZ), m = (int)(i % g.SZ);
-  const int64_t dl = g.SZ;
-  double *p[3] = {a, b, c};
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    double *f = p[q] + g.idx(k, 0, m);
-    f[0] = f[g.NY * dl];
-    f[1 * dl] = f[(g.NY + 1) * dl];
-    f[(g.NY + 2) * dl] = f[2 * dl];
-    f[(g.NY + 3) * dl] = f[3 * dl];
-  }
-}
-
-// sr_current2 (:1805-2039) on one rank: 2,3 += N+2,N+3 then N,N+1 += 0,1
-// along x over all (l,m); then along y over all (k,m).  8 planes.
-__global__ void k_fold_x(Geom g, Fields<double> F) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SY * g.SZ;
-  if (i >= n) return;
-  const int64_t dk = n;
+  if (i >= (int64_t)fold_groups(g) * g.SZ) return;
 #pragma unroll
   for (int q = PIC_JIX; q <= PIC_NE; ++q) {
-    double *f = F.f[q] + i;
-    f[2 * dk] += f[(g.NX + 2) * dk];
-    f[3 * dk] += f[(g.NX + 3) * dk];
-    f[g.NX * dk] += f[0];
-    f[(g.NX + 1) * dk] += f[1 * dk];
-  }
-}
-
-__global__ void k_fold_y(Geom g, Fields<double> F) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)g.SX * g.SZ;
-  if (i >= n) return;
-  const int k = (int)(i / g.SZ), m = (int)(i % g.SZ);
-  const int64_t dl = g.SZ;
-#pragma unroll
-  for (int q = PIC_JIX; q <= PIC_NE; ++q) {
-    double *f = F.f[q] + g.idx(k, 0, m);
-    f[2 * dl] += f[(g.NY + 2) * dl];
-    f[3 * dl] += f[(g.NY + 3) * dl];
-    f[g.NY * dl] += f[0];
-    f[(g.NY + 1) * dl] += f[1 * dl];
+    double *f = F.f[q];
+    fold_group(
+        g, (int)(i / g.SZ), (int)(i % g.SZ), [&](int64_t j) { return f[j]; },
+        [&](int64_t j, double v, bool changed) {
+          if (changed) f[j] = v;
+        });
   }
 }
 
@@ -1237,23 +1200,16 @@ int renew_e(pic_ctx *ctx) {
 
 int halo(pic_ctx *ctx, int first) {
   const Geom &g = ctx->geom;
-  Fields<double> F = fields<double>(ctx);
-  double *a = F.f[first], *b = F.f[first + 1], *c = F.f[first + 2];
-  k_halo_x<<<(unsigned)div_up((int64_t)g.SY * g.SZ, kBlock), kBlock, 0,
-             ctx->stream>>>(g, a, b, c);
-  k_halo_y<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
-             ctx->stream>>>(g, a, b, c);
+  k_halo<<<(unsigned)div_up((int64_t)fold_groups(g) * g.SZ, kBlock), kBlock, 0,
+           ctx->stream>>>(g, fields<double>(ctx), first);
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
 
 int fold_current(pic_ctx *ctx) {
   const Geom &g = ctx->geom;
-  Fields<double> F = fields<double>(ctx);
-  k_fold_x<<<(unsigned)div_up((int64_t)g.SY * g.SZ, kBlock), kBlock, 0,
-             ctx->stream>>>(g, F);
-  k_fold_y<<<(unsigned)div_up((int64_t)g.SX * g.SZ, kBlock), kBlock, 0,
-             ctx->stream>>>(g, F);
+  k_fold<<<(unsigned)div_up((int64_t)fold_groups(g) * g.SZ, kBlock), kBlock, 0,
+           ctx->stream>>>(g, fields<double>(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }

@@ -49,6 +49,19 @@ __device__ inline void images(const Geom &g, int k, int l, int64_t c, Put put) {
   if (x && y) put(c + x + y, c + x);
 }
 
+// interior column e < fold_groups(g) that has images
+__device__ inline void edge_column(const Geom &g, int e, int &k, int &l) {
+  const auto edge = [](int p, int n) { return p < 2 ? 2 + p : n + p - 2; };
+  if (e < 4 * g.NY) {
+    k = edge(e & 3, g.NX);
+    l = 2 + (e >> 2);
+  } else {
+    e -= 4 * g.NY;
+    k = 4 + (e >> 2);
+    l = edge(e & 3, g.NY);
+  }
+}
+
 // columns that no fold reads or writes
 __device__ inline bool unfolded_column(const Geom &g, int k, int l) {
   return k >= 4 && k < g.NX && l >= 4 && l < g.NY;
