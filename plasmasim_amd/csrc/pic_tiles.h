@@ -98,7 +98,10 @@ __device__ inline void part_range(int p, int n, int64_t &s, int64_t &e) {
 // store, found in the table of each cell's first slot that the sort leaves.
 // Boxes may reach over the grid's upper faces (the sizes need not divide).
 // 4 x 4 x 8 is the largest box whose window fits both forms; where that
-// gives fewer boxes than the chip holds workgroups (3 per CU), 2 x 2 x 8.
+// gives fewer than 300 boxes (both species' run together), 2 x 2 x 8.  20
+// steps, small / large boxes: 336 large ones of 31 x 27 x 45 x 8 ppc FP32
+// 3.25 / 2.28 ms, 500 of 40^3 x 4 ppc FP32 3.56 / 2.11 ms and FP64 3.3 /
+// 2.54 ms; 256 of 32^3 x 16 ppc FP64 the same.
 inline TileGeom row_geom(const TileGeom &one) {
   const auto up = [](int a, int b) { return (a + b - 1) / b; };
   TileGeom t = one;
@@ -109,7 +112,7 @@ inline TileGeom row_geom(const TileGeom &one) {
     t.NTX = up(NX, w);
     t.NTY = up(NY, w);
     t.NTZ = up(NZ, 8);
-    if (t.ntiles() >= kChipSlots) break;
+    if (t.ntiles() >= 300) break;
   }
   t.LX = t.LY = t.LZ = -1;
   return t;
