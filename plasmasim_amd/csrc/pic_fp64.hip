@@ -457,6 +457,57 @@ __device__ __forceinline__ double gather1o(const double *F, O i, O dl, O dk, dou
   return p1 + p2 + p3 + p4;
 }
 
+// gather1o's loads and its products and sums, apart from each other
+template <typename O>
+__device__ __forceinline__ void load8o(const double *F, O i, O dl, O dk, double (&v)[8]) {
+  const double *f0 = at(F, i), *f1 = at(F, i + dl), *f2 = at(F, i + dk),
+               *f3 = at(F, i + dk + dl);
+  v[0] = f0[0], v[1] = f0[1], v[2] = f1[0], v[3] = f1[1];
+  v[4] = f2[0], v[5] = f2[1], v[6] = f3[0], v[7] = f3[1];
+}
+__device__ __forceinline__ double sum8o(const double (&v)[8], double wa0, double wa1,
+                                        double wb0, double wb1, double wc0, double wc1) {
+  const double p1 = v[0] * (wa0 * wb0 * wc0) + v[1] * (wa0 * wb0 * wc1);
+  const double p2 = v[2] * (wa0 * wb1 * wc0) + v[3] * (wa0 * wb1 * wc1);
+  const double p3 = v[4] * (wa1 * wb0 * wc0) + v[5] * (wa1 * wb0 * wc1);
+  const double p4 = v[6] * (wa1 * wb1 * wc0) + v[7] * (wa1 * wb1 * wc1);
+  return p1 + p2 + p3 + p4;
+}
+
+// The six components at a particle in a stated order: two components' loads
+// are in flight ahead of the one summed.  Left alone, the compiler waits for
+// each load before it issues the next in a kernel with the force; all six at
+// once take 249 registers, which costs a wave per SIMD, two take 165.
+template <typename O>
+__device__ __forceinline__ void gather6o(const double *const (&E)[3],
+                                         const double *const (&B)[3], O o, O hx, O hy, O hz,
+                                         O dl, O dk, const AxisW &X, const AxisW &Y,
+                                         const AxisW &Z, double inv_dx3, double (&f)[6]) {
+  const O ox = o - hx, oy = o - hy, oz = o - hz;
+  double u[8], v[8];
+  load8o<O>(E[0], oy - hz, dl, dk, u);
+  load8o<O>(E[1], ox - hz, dl, dk, v);
+  __builtin_amdgcn_sched_barrier(0);
+  f[0] = sum8o(u, X.iu, X.il, Y.hu, Y.hl, Z.hu, Z.hl) * inv_dx3;
+  __builtin_amdgcn_sched_barrier(0);
+  load8o<O>(E[2], ox - hy, dl, dk, u);
+  __builtin_amdgcn_sched_barrier(0);
+  f[1] = sum8o(v, X.hu, X.hl, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+  __builtin_amdgcn_sched_barrier(0);
+  load8o<O>(B[0], ox, dl, dk, v);
+  __builtin_amdgcn_sched_barrier(0);
+  f[2] = sum8o(u, X.hu, X.hl, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+  __builtin_amdgcn_sched_barrier(0);
+  load8o<O>(B[1], oy, dl, dk, u);
+  __builtin_amdgcn_sched_barrier(0);
+  f[3] = sum8o(v, X.hu, X.hl, Y.iu, Y.il, Z.iu, Z.il) * inv_dx3;
+  __builtin_amdgcn_sched_barrier(0);
+  load8o<O>(B[2], oz, dl, dk, v);
+  __builtin_amdgcn_sched_barrier(0);
+  f[4] = sum8o(u, X.iu, X.il, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+  f[5] = sum8o(v, X.iu, X.il, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+}
+
 // The lane's walk over the 8 nodes of a stencil in the LDS window: lane j
 // takes them mirrored along the axes set in j & 7, so that lanes holding
 // particles of one cell add to different nodes.
@@ -818,45 +869,72 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
         const O o = (((O)X.bi * g.SY + Y.bi) * g.SZ + Z.bi) * 8;
         const O hx = X.bh != X.bi ? fk : 0, hy = Y.bh != Y.bi ? fl : 0,
                 hz = Z.bh != Z.bi ? 8 : 0;
-        const O ox = o - hx, oy = o - hy, oz = o - hz;
-        double f[6];
-        const auto take_e = [&]() {
-          f[0] = gather1o<O>(F.e[0], oy - hz, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.hu, Z.hl) * inv_dx3;
-          f[1] = gather1o<O>(F.e[1], ox - hz, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
-          f[2] = gather1o<O>(F.e[2], ox - hy, fl, fk, X.hu, X.hl, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
-        };
-        const auto take_b = [&](const double *const (&B)[3], double (&o3)[3]) {
-          o3[0] = gather1o<O>(B[0], ox, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.iu, Z.il) * inv_dx3;
-          o3[1] = gather1o<O>(B[1], oy, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
-          o3[2] = gather1o<O>(B[2], oz, fl, fk, X.iu, X.il, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
-        };
-        double b3[3];
-        // a wave without box particles takes E and B in one go: around the
-        // force's branch the two gathers wait for memory one after the other
-        // (128^3 x 64 ppc, 20 steps with the force: 346 ms, so 324 ms)
-        if (THRUST && __builtin_amdgcn_ballot_w64(box) != 0) {
-          take_e();
+        // (not with both species in one launch or dx != 1: the form below
+        // keeps three waves there, this one takes 169 to 209 registers)
+        if (THRUST && UNIT && !BOTH) {
+          double f[6];
+          // the force takes its own E: shared with the push, the E gather
+          // comes before the force's branch and the push's B after it, and
+          // every particle waits for memory twice (128^3 x 64 ppc, 20 steps:
+          // 324 ms in the other branch's form, so 301 ms)
           if (box) {
-            double bp[3];
-            take_b(F.bp, bp);
+            // the weights of x and the offset renamed, so that neither the
+            // node weights nor the E loads are formed once for both
+            AxisW XB = X;
+            O ob = o;
+            asm("" : "+v"(XB.iu), "+v"(XB.il), "+v"(XB.hu), "+v"(XB.hl), "+v"(ob));
+            gather6o<O>(F.e, F.bp, ob, hx, hy, hz, fl, fk, XB, Y, Z, inv_dx3, f);
             th[0] += f[0];
             th[1] += f[1];
             th[2] += f[2];
-            th[3] += vy * bp[2] - vz * bp[1];
-            th[4] += vz * bp[0] - vx * bp[2];
-            th[5] += vx * bp[1] - vy * bp[0];
+            th[3] += vy * f[5] - vz * f[4];
+            th[4] += vz * f[3] - vx * f[5];
+            th[5] += vx * f[4] - vy * f[3];
           }
-          // (kept apart from the push's: the compiler would otherwise form
-          // the node weights once for both and hold them in 70 registers)
-          asm("" : "+v"(X.iu), "+v"(X.il), "+v"(X.hu), "+v"(X.hl));
-          if (push) take_b(F.b, b3);
+          if (push) {
+            gather6o<O>(F.e, F.b, o, hx, hy, hz, fl, fk, X, Y, Z, inv_dx3, f);
+            boris(kc, f, vx, vy, vz);
+          }
         } else {
-          take_e();
-          take_b(F.b, b3);
-        }
-        if (push) {
-          for (int q = 0; q < 3; ++q) f[3 + q] = b3[q];
-          boris(kc, f, vx, vy, vz);
+          const O ox = o - hx, oy = o - hy, oz = o - hz;
+          double f[6];
+          const auto take_e = [&]() {
+            f[0] = gather1o<O>(F.e[0], oy - hz, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.hu, Z.hl) * inv_dx3;
+            f[1] = gather1o<O>(F.e[1], ox - hz, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+            f[2] = gather1o<O>(F.e[2], ox - hy, fl, fk, X.hu, X.hl, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+          };
+          const auto take_b = [&](const double *const (&B)[3], double (&o3)[3]) {
+            o3[0] = gather1o<O>(B[0], ox, fl, fk, X.hu, X.hl, Y.iu, Y.il, Z.iu, Z.il) * inv_dx3;
+            o3[1] = gather1o<O>(B[1], oy, fl, fk, X.iu, X.il, Y.hu, Y.hl, Z.iu, Z.il) * inv_dx3;
+            o3[2] = gather1o<O>(B[2], oz, fl, fk, X.iu, X.il, Y.iu, Y.il, Z.hu, Z.hl) * inv_dx3;
+          };
+          double b3[3];
+          // a wave without box particles does not enter the force's branch
+          // (128^3 x 64 ppc, 20 steps with the force: 346 ms, so 324 ms)
+          if (THRUST && __builtin_amdgcn_ballot_w64(box) != 0) {
+            take_e();
+            if (box) {
+              double bp[3];
+              take_b(F.bp, bp);
+              th[0] += f[0];
+              th[1] += f[1];
+              th[2] += f[2];
+              th[3] += vy * bp[2] - vz * bp[1];
+              th[4] += vz * bp[0] - vx * bp[2];
+              th[5] += vx * bp[1] - vy * bp[0];
+            }
+            // (kept apart from the push's: the compiler would otherwise form
+            // the node weights once for both and hold them in 70 registers)
+            asm("" : "+v"(X.iu), "+v"(X.il), "+v"(X.hu), "+v"(X.hl));
+            if (push) take_b(F.b, b3);
+          } else {
+            take_e();
+            take_b(F.b, b3);
+          }
+          if (push) {
+            for (int q = 0; q < 3; ++q) f[3 + q] = b3[q];
+            boris(kc, f, vx, vy, vz);
+          }
         }
       }
       x += vx * kc.dt * 0.5;
