@@ -483,8 +483,8 @@ extern "C" int pic_create(const pic_config *cfg, pic_ctx **out) {
   {
     const int nt = tile_geom(ctx).ntiles();
     for (int sp = 0; sp < 2; ++sp) {
-      CREATE_HIP(hipMalloc(&ctx->tile_start[sp], (size_t)(nt + 1) * sizeof(uint32_t)));
-      CREATE_HIP(hipMemset(ctx->tile_start[sp], 0, (size_t)(nt + 1) * sizeof(uint32_t)));
+      CREATE_HIP(hipMalloc(&ctx->tile_start[sp], (size_t)(nt + 2) * sizeof(uint32_t)));
+      CREATE_HIP(hipMemset(ctx->tile_start[sp], 0, (size_t)(nt + 2) * sizeof(uint32_t)));
       if (nt == 1 && ncell_in < ((int64_t)1 << 30))
         CREATE_HIP(hipMalloc(&ctx->row_start[sp], (size_t)(ncell_in + 1) * sizeof(uint32_t)));
     }

@@ -1515,9 +1515,10 @@ __global__ void k_gather32(Particles32 dst, Particles32 src,
 
 __global__ __launch_bounds__(256) void k_sort_keys32(
     Geom g, TileGeom tg, const int32_t *__restrict__ cell, int64_t n,
-    uint32_t *keys) {
+    uint32_t *keys, uint32_t *zero) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  if (i == 0 && zero) *zero = 0;
   const uint32_t ncell = (uint32_t)g.NX * g.NY * g.NZ;
   uint32_t key = ncell;
   const int32_t c = cell[i];
@@ -2325,8 +2326,10 @@ static int sort_impl(pic_ctx *ctx, int sp, bool defer) {
     }
   }
   ctx->sort_radix_count++;
+  const TileGeom bg = row_geom(tg);
+  const bool boxes = ctx->row_start[sp] && boxes_filled(n, bg.ntiles());
   k_sort_keys32<<<(unsigned)div_up(n, kBlock), kBlock, 0, ctx->stream>>>(
-      g, tg, src.cell, n, ctx->keys);
+      g, tg, src.cell, n, ctx->keys, boxes ? ctx->tile_start[sp] + nt + 1 : nullptr);
   PIC_LAUNCH_CHECK(ctx);
   const uint32_t ncell = (uint32_t)g.NX * g.NY * g.NZ;
   int bits = 1;
@@ -2336,15 +2339,16 @@ static int sort_impl(pic_ctx *ctx, int sp, bool defer) {
   rc = tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
                    ctx->tile_start[sp]);
   if (rc) return rc;
-  if (ctx->row_start[sp] &&
-      (rc = tile_bounds(ctx, ctx->keys_alt, n, 1u, (int)ncell, ctx->row_start[sp])))
+  if (boxes && (rc = cell_starts(ctx, ctx->keys_alt, n, bg, ctx->row_start[sp],
+                                 ctx->tile_start[sp] + nt + 1)))
     return rc;
   // the kept count is the start of the drop tile
   PIC_HIP(ctx, hipMemcpyAsync(ctx->host_counter, ctx->tile_start[sp] + nt,
-                              sizeof(uint32_t), hipMemcpyDeviceToHost,
+                              2 * sizeof(uint32_t), hipMemcpyDeviceToHost,
                               ctx->stream));
   PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const int64_t valid = (int64_t)(*(uint32_t *)ctx->host_counter);
+  const int64_t valid = (int64_t)((uint32_t *)ctx->host_counter)[0];
+  const int64_t most = (int64_t)((uint32_t *)ctx->host_counter)[1];
   Particles32 dst = p32(ctx, sp, 1 - ctx->cur[sp]);
   if (valid > 0)
     k_gather32<<<(unsigned)div_up(valid, 4 * kBlock), kBlock, 0, ctx->stream>>>(
@@ -2353,7 +2357,7 @@ static int sort_impl(pic_ctx *ctx, int sp, bool defer) {
   ctx->cur[sp] = 1 - ctx->cur[sp];
   ctx->n[sp] = valid;
   ctx->sorted_end[sp] = valid;
-  ctx->row_end[sp] = valid;
+  ctx->row_end[sp] = boxes && boxes_even(valid, bg.ntiles(), most) ? valid : 0;
   return 0;
 }
 

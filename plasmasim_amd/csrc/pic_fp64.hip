@@ -1091,12 +1091,15 @@ __global__ void k_gather_particles(Particles64 dst, Particles64 src,
 // sorting key (:7488-7497): ((int)(x/dx)-2, (int)(y/dx)-2, (int)(z/dx)-2),
 // tile-major (the reference's lexicographic order with m fastest when one
 // tile spans the interior); particles outside the interior (and dead ones)
-// get the key ncell and are dropped after the sort.
+// get the key ncell and are dropped after the sort.  zero (may be null): a
+// word to clear for the kernels that follow.
 __global__ __launch_bounds__(256) void k_sort_keys(Geom g, TileGeom tg,
                                                    Particles64 P, int64_t n,
-                                                   double dx, uint32_t *keys) {
+                                                   double dx, uint32_t *keys,
+                                                   uint32_t *zero) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  if (i == 0 && zero) *zero = 0;
   const uint32_t ncell = (uint32_t)g.NX * g.NY * g.NZ;
   uint32_t key = ncell;
   const double x = P.x[i], y = P.y[i], z = P.z[i];
@@ -1629,8 +1632,10 @@ int sort(pic_ctx *ctx, int sp) {
   Particles64 src = p64(ctx, sp, ctx->cur[sp]);
   const TileGeom tg = tile_geom(ctx);
   const int nt = tg.ntiles();
+  const TileGeom bg = row_geom(tg);
+  const bool boxes = ctx->row_start[sp] && boxes_filled(n, bg.ntiles());
   k_sort_keys<<<(unsigned)div_up(n, kBlock), kBlock, 0, ctx->stream>>>(
-      g, tg, src, n, ctx->cfg.dx, ctx->keys);
+      g, tg, src, n, ctx->cfg.dx, ctx->keys, boxes ? ctx->tile_start[sp] + nt + 1 : nullptr);
   PIC_LAUNCH_CHECK(ctx);
   const uint32_t ncell = (uint32_t)g.NX * g.NY * g.NZ;
   if (ctx->ts64 && ctx->sorted_end[sp] > 0 && ctx->sorted_end[sp] <= n) {
@@ -1662,15 +1667,16 @@ int sort(pic_ctx *ctx, int sp) {
   rc = tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
                    ctx->tile_start[sp]);
   if (rc) return rc;
-  if (ctx->row_start[sp] &&
-      (rc = tile_bounds(ctx, ctx->keys_alt, n, 1u, (int)ncell, ctx->row_start[sp])))
+  if (boxes && (rc = cell_starts(ctx, ctx->keys_alt, n, bg, ctx->row_start[sp],
+                                 ctx->tile_start[sp] + nt + 1)))
     return rc;
   // the kept count is the start of the drop tile
   PIC_HIP(ctx, hipMemcpyAsync(ctx->host_counter, ctx->tile_start[sp] + nt,
-                              sizeof(uint32_t), hipMemcpyDeviceToHost,
+                              2 * sizeof(uint32_t), hipMemcpyDeviceToHost,
                               ctx->stream));
   PIC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const int64_t valid = (int64_t)(*(uint32_t *)ctx->host_counter);
+  const int64_t valid = (int64_t)((uint32_t *)ctx->host_counter)[0];
+  const int64_t most = (int64_t)((uint32_t *)ctx->host_counter)[1];
   Particles64 dst = p64(ctx, sp, 1 - ctx->cur[sp]);
   if (valid > 0)
     k_gather_particles<<<(unsigned)div_up(valid, kBlock), kBlock, 0,
@@ -1679,7 +1685,7 @@ int sort(pic_ctx *ctx, int sp) {
   ctx->cur[sp] = 1 - ctx->cur[sp];
   ctx->n[sp] = valid;
   ctx->sorted_end[sp] = valid;
-  ctx->row_end[sp] = valid;
+  ctx->row_end[sp] = boxes && boxes_even(valid, bg.ntiles(), most) ? valid : 0;
   return 0;
 }
 

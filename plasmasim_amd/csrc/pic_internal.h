@@ -147,11 +147,13 @@ struct pic_ctx {
 
   // sort tiles: per-species particle ranges of each tile after the last
   // sort; [0, sorted_end) is tile-sorted, later slots are the inflow tail
-  uint32_t *tile_start[2] = {nullptr, nullptr};   // ntiles + 1 per species
+  // (ntiles + 1 entries per species, then the fullest box's population)
+  uint32_t *tile_start[2] = {nullptr, nullptr};
   int64_t sorted_end[2] = {0, 0};
   // one tile over the interior: each cell's first slot after the last sort
   // (cells + 1 entries), valid while row_end == sorted_end > 0; whatever
-  // sets sorted_end other than a sort sets row_end to 0
+  // sets sorted_end other than a sort sets row_end to 0, and so does a sort
+  // of a store that does not fill its boxes (boxes_filled)
   uint32_t *row_start[2] = {nullptr, nullptr};
   int64_t row_end[2] = {0, 0};
   int32_t drift_halves[2] = {0, 0};  // half-step drifts since the tile sort
@@ -374,5 +376,9 @@ int poisson_download_phi(pic_ctx *ctx, double *host);
 // >= nt * cpt are dropped slots and land in tile nt)
 int tile_bounds(pic_ctx *ctx, const uint32_t *skeys, int64_t n, uint32_t cpt,
                 int nt, uint32_t *tile_start);
+// cell_start[0..cells] from the keys of a one-tile sort; *most, zero before,
+// becomes the population of the fullest of the boxes (row_geom)
+int cell_starts(pic_ctx *ctx, const uint32_t *skeys, int64_t n, const TileGeom &boxes,
+                uint32_t *cell_start, uint32_t *most);
 
 }  // namespace pic

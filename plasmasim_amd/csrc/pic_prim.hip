@@ -334,4 +334,67 @@ int tile_bounds(pic_ctx *ctx, const uint32_t *skeys, int64_t n, uint32_t cpt,
   return 0;
 }
 
+// cell_start[c] for c = 0..cells: the first slot of cell c or above, each
+// entry by a search of its own, whatever the store's distribution.  (Filling
+// the empty cells between two particles from the second one's thread, as
+// k_tile_bounds does for tiles, takes 10 ms and more where many cells in a
+// row are empty.)  Threads are grouped by box (t: 32 or 128 cells each), so
+// that *most becomes the population of the fullest one.
+
+// first slot in [lo, hi) whose key is >= key, else hi: eighths, whose seven
+// loads are in flight together (bound by the chain of loads: 20 in halves
+// for 10^6 slots, 7 so)
+__device__ inline int64_t first_at_least(const uint32_t *__restrict__ keys, int64_t lo,
+                                         int64_t hi, uint32_t key) {
+  while (hi - lo > 8) {
+    const int64_t step = (hi - lo) >> 3;
+    int below = 0;
+#pragma unroll
+    for (int j = 1; j < 8; ++j) below += keys[lo + j * step] < key;
+    if (below < 7) hi = lo + (below + 1) * step;
+    if (below > 0) lo += below * step + 1;
+  }
+  int below = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) below += lo + j < hi && keys[lo + j] < key;
+  return lo + below;
+}
+
+__global__ __launch_bounds__(256) void k_cell_starts(const uint32_t *__restrict__ keys,
+                                                     int64_t n, TileGeom t, int NX, int NY,
+                                                     int NZ, uint32_t *cell_start,
+                                                     uint32_t *most) {
+  __shared__ uint32_t sum[256 / 32];
+  const int per = t.TX * t.TY * t.TZ, tid = threadIdx.x;
+  if (tid < 256 / 32) sum[tid] = 0;
+  __syncthreads();
+  const int b = blockIdx.x * (256 / per) + tid / per, r = tid % per;
+  const int k = b / (t.NTZ * t.NTY) * t.TX + r / (t.TY * t.TZ);
+  const int l = b / t.NTZ % t.NTY * t.TY + r / t.TZ % t.TY;
+  const int m = b % t.NTZ * t.TZ + r % t.TZ;
+  if (k < NX && l < NY && m < NZ) {
+    const uint32_t c = ((uint32_t)k * NY + l) * NZ + m;
+    const int64_t s = first_at_least(keys, 0, n, c);
+    const int64_t near = s + 64 < n ? s + 64 : n;  // most cells end here
+    const int64_t e = near == n || keys[near - 1] > c
+                          ? first_at_least(keys, s, near, c + 1)
+                          : first_at_least(keys, near, n, c + 1);
+    cell_start[c] = (uint32_t)s;
+    if (c + 1 == (uint32_t)NX * NY * NZ) cell_start[c + 1] = (uint32_t)e;
+    if (e > s) atomicAdd(&sum[tid / per], (uint32_t)(e - s));
+  }
+  __syncthreads();
+  if (tid < 256 / per && sum[tid] > *(volatile uint32_t *)most) atomicMax(most, sum[tid]);
+}
+
+int cell_starts(pic_ctx *ctx, const uint32_t *skeys, int64_t n, const TileGeom &boxes,
+                uint32_t *cell_start, uint32_t *most) {
+  const Geom &g = ctx->geom;
+  const int64_t threads = (int64_t)boxes.ntiles() * (boxes.TX * boxes.TY * boxes.TZ);
+  k_cell_starts<<<(unsigned)div_up(threads, 256), 256, 0, ctx->stream>>>(
+      skeys, n, boxes, g.NX, g.NY, g.NZ, cell_start, most);
+  PIC_LAUNCH_CHECK(ctx);
+  return 0;
+}
+
 }  // namespace pic

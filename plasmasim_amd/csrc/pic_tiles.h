@@ -118,6 +118,21 @@ inline TileGeom row_geom(const TileGeom &one) {
   return t;
 }
 
+// Whether a store of n particles takes its boxes; else it goes in chunks, as
+// an unsorted tail.  Every box pays for its window, so the store must hold 32
+// particles per box: two steps, chunks / boxes, with 16 and with 32 per box:
+// 128^3 FP64 1.85 / 1.88 and 2.73 / 1.93 ms, FP32 1.86 / 2.02 and 3.03 / 2.16
+// ms; 32^3 FP64 0.127 / 0.129 and 0.162 / 0.128 ms; with 1 per box at 128^3
+// 0.78 / 1.49 and 0.48 / 1.18 ms.  And one workgroup takes the fullest box
+// (most particles): it must not hold more than 8 times a workgroup's share.
+// 64^3, 500000 particles within a cube, chunks / boxes: 32^3 cells (3 times)
+// FP64 0.58 / 0.45, FP32 0.46 / 0.36 ms; 16^3 cells (24 times) 0.40 / 1.11 and
+// 0.35 / 0.76 ms; 4 x 4 x 8 cells 0.36 / 14 and 0.32 / 9.9 ms.
+inline bool boxes_filled(int64_t n, int64_t boxes) { return n >= 32 * boxes; }
+inline bool boxes_even(int64_t n, int64_t boxes, int64_t most) {
+  return most * (boxes < kChipSlots ? boxes : kChipSlots) <= 8 * n;
+}
+
 // slot range of column r (< TX * TY) of box bid
 __device__ inline void row_range(const TileRun &tr, const TileGeom &tg, int NX, int NY,
                                  int NZ, int bid, int r, int &s, int &e) {
