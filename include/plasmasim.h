@@ -309,6 +309,13 @@ int pic_timing_reset(pic_ctx *ctx);
  * step and deposit, the particle adjoints carried back across each sort),
  * returning dloss * dL/dp.  The context is left at the end of the last
  * recomputed segment.
+ *
+ * Device memory: the checkpoints of the last forward, and after a backward
+ * its own buffers (particle adjoints, tape of ckpt_every steps; at most 32
+ * GiB, else they are freed), stay with the context for the next sweep.  A
+ * forward with a shorter ckpt_every frees what that window does not use, an
+ * allocation of this context that finds the card full frees the sweep's
+ * buffers first, and pic_destroy frees everything.
  */
 int pic_adj_forward(pic_ctx *ctx, const double params[4], int nsteps,
                     int ckpt_every, double radius, int nquad, double *loss);

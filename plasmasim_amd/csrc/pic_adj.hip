@@ -1019,33 +1019,74 @@ struct TapeStep {
 // a sort), the tape of one segment and the permutations of the sorts in it.
 // Kept for the next sweep of the context where they are no more than
 // kKeepBytes: allocating and freeing them took from 20 ms to 2.5 s of a
-// 90 ms sweep at 64^3 x 32 ppc.
+// 90 ms sweep at 64^3 x 32 ppc.  A forward gives back what a window as long
+// as its own does not use, and an allocation of the context that the card
+// has no room for all of it (device_malloc).
 constexpr size_t kKeepBytes = (size_t)32 << 30;
 struct Sweep {
+  size_t lp_bytes = 0, tf_bytes = 0, tpart_bytes = 0, perm_bytes = 0;  // of one buffer
   double *lp[2] = {nullptr, nullptr}, *lq[2] = {nullptr, nullptr};
   std::vector<double *> tf;
   std::vector<char *> tpart;
-  std::vector<uint32_t *> perm;
-  size_t bytes = 0;
+  std::vector<uint32_t *> perm;   // by step and species
+  std::vector<uint32_t *> spare;  // permutations no step of the sweep holds
+  bool running = false, swapped = false;  // a sweep runs; it has used lq
+  size_t bytes() const {
+    const auto held = [](const auto &v) {
+      size_t c = 0;
+      for (const auto p : v) c += p != nullptr;
+      return c;
+    };
+    size_t c = 0;
+    for (int s = 0; s < 2; ++s) c += (lp[s] != nullptr) + (lq[s] != nullptr);
+    return c * lp_bytes + held(tf) * tf_bytes + held(tpart) * tpart_bytes +
+           (held(perm) + spare.size()) * perm_bytes;
+  }
   template <typename T>
-  hipError_t want(T *&p, size_t b) {
-    if (p) return hipSuccess;
-    const hipError_t e = hipMalloc(&p, b);
-    if (e == hipSuccess) bytes += b;
-    return e;
+  static bool drop(T *&p) {
+    if (!p) return false;
+    (void)hipFree(p);
+    p = nullptr;
+    return true;
+  }
+  template <typename T>
+  static bool shorten(std::vector<T *> &v, size_t n) {
+    bool any = false;
+    for (size_t j = n; j < v.size(); ++j) any |= drop(v[j]);
+    if (v.size() > n) v.resize(n);
+    return any;
+  }
+  void finish() {
+    for (uint32_t *&p : perm)
+      if (p) spare.push_back(p);
+    perm.clear();
+    running = swapped = false;
+  }
+  void trim(size_t K) {
+    shorten(tf, K + 1);
+    shorten(tpart, K);
+    shorten(spare, 2 * K);
   }
   void release() {
+    finish();
     for (int s = 0; s < 2; ++s) {
-      if (lp[s]) (void)hipFree(lp[s]);
-      if (lq[s]) (void)hipFree(lq[s]);
+      drop(lp[s]);
+      drop(lq[s]);
     }
-    for (double *p : tf)
-      if (p) (void)hipFree(p);
-    for (char *p : tpart)
-      if (p) (void)hipFree(p);
-    for (uint32_t *p : perm)
-      if (p) (void)hipFree(p);
-    *this = Sweep();
+    trim(0);
+    shorten(tf, 0);
+  }
+  // gives back what no running sweep uses; false if that is nothing
+  bool give_back() {
+    if (!running) {
+      const bool any = bytes() > 0;
+      release();
+      return any;
+    }
+    bool any = shorten(spare, 0);
+    if (!swapped)
+      for (int s = 0; s < 2; ++s) any |= drop(lq[s]);
+    return any;
   }
 };
 
@@ -1068,6 +1109,14 @@ struct AdjState {
 };
 
 AdjState *state(pic_ctx *ctx) { return (AdjState *)ctx->adj; }
+
+// one of the sweep's buffers, if it is not there yet
+template <typename T>
+int want(pic_ctx *ctx, T *&p, size_t bytes) {
+  if (p) return 0;
+  PIC_HIP(ctx, device_malloc(ctx, &p, bytes));
+  return 0;
+}
 
 int64_t ncell(const pic_ctx *ctx) {
   return (int64_t)ctx->geom.SX * ctx->geom.SY * ctx->geom.SZ;
@@ -1211,7 +1260,7 @@ void sub_arrays(const pic_ctx *ctx, void *buf, int64_t cap, char **ptr, size_t *
 }
 
 int save_ckpt(pic_ctx *ctx, Ckpt &c) {
-  if (!c.fields) PIC_HIP(ctx, hipMalloc(&c.fields, ctx->field_bytes));
+  if (!c.fields) PIC_HIP(ctx, device_malloc(ctx, &c.fields, ctx->field_bytes));
   PIC_HIP(ctx, hipMemcpyAsync(c.fields, ctx->field_mem, ctx->field_bytes,
                               hipMemcpyDeviceToDevice, ctx->stream));
   const int nt = tile_geom(ctx).ntiles();
@@ -1225,7 +1274,7 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
       if (c.parts[s]) (void)hipFree(c.parts[s]);
       c.parts[s] = nullptr;
       c.room[s] = 0;
-      PIC_HIP(ctx, hipMalloc(&c.parts[s], (size_t)(n + 1) * slot_bytes(ctx)));
+      PIC_HIP(ctx, device_malloc(ctx, &c.parts[s], (size_t)(n + 1) * slot_bytes(ctx)));
       c.room[s] = n + 1;
     }
     char *src[7], *dst[7];
@@ -1238,7 +1287,7 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
         PIC_HIP(ctx, hipMemcpyAsync(dst[j], src[j], n * esz[j], hipMemcpyDeviceToDevice,
                                     ctx->stream));
     if (!c.tiles[s])
-      PIC_HIP(ctx, hipMalloc(&c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t)));
+      PIC_HIP(ctx, device_malloc(ctx, &c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t)));
     PIC_HIP(ctx, hipMemcpyAsync(c.tiles[s], ctx->tile_start[s], (size_t)(nt + 1) * sizeof(uint32_t),
                                 hipMemcpyDeviceToDevice, ctx->stream));
   }
@@ -1405,6 +1454,14 @@ double sum_partials(pic_ctx *ctx, const double *dev, int count, int stride, int 
 
 }  // namespace
 
+hipError_t device_malloc_bytes(pic_ctx *ctx, void **p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  AdjState *A = state(ctx);
+  if (e != hipErrorOutOfMemory || !A || !A->w.give_back()) return e;
+  (void)hipGetLastError();  // answered by what was given back
+  return hipMalloc(p, bytes);
+}
+
 void adj_free(pic_ctx *ctx) {
   AdjState *A = state(ctx);
   if (!A) return;
@@ -1443,13 +1500,14 @@ extern "C" int pic_adj_forward(pic_ctx *ctx, const double params[4], int nsteps,
   if (rc) return rc;
   AdjState *A = state(ctx);
   A->have_forward = false;
+  A->w.trim((size_t)ckpt_every);
   free_ckpts(A, (size_t)div_up(nsteps, ckpt_every));
   const int64_t terms = (int64_t)nsteps * nb(nquad);
   if (A->part_n < terms) {
     if (A->part) (void)hipFree(A->part);
     A->part = nullptr;
     A->part_n = 0;
-    PIC_HIP(ctx, hipMalloc(&A->part, (size_t)terms * sizeof(double)));
+    PIC_HIP(ctx, device_malloc(ctx, &A->part, (size_t)terms * sizeof(double)));
     A->part_n = terms;
   }
   for (int a = 0; a < 4; ++a) A->p[a] = params[a];
@@ -1526,7 +1584,8 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
   const int64_t cap = ctx->cap;
   const bool f64 = c.precision == PIC_FP64;
   auto cleanup = [&](bool keep) {
-    if (!keep || W.bytes > kKeepBytes) W.release();
+    W.finish();
+    if (!keep || W.bytes() > kKeepBytes) W.release();
     ctx->adj_mode = 0;
   };
 #define TRY(x)          \
@@ -1537,15 +1596,21 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
     }                   \
   } while (0)
 #define TRYH(x) TRY((x) == hipSuccess ? 0 : set_error(ctx, PIC_E_HIP, "adjoint: %s", #x))
-  if (W.tf.size() < (size_t)K + 1) W.tf.resize(K + 1, nullptr);
-  if (W.tpart.size() < (size_t)K) W.tpart.resize(K, nullptr);
-  if (W.perm.size() < 2 * (size_t)K) W.perm.resize(2 * (size_t)K, nullptr);
+  W.trim((size_t)K);
+  W.running = true;
+  W.lp_bytes = 6 * (size_t)cap * sizeof(double);
+  W.tf_bytes = 6 * n * sizeof(double);
+  W.tpart_bytes = 2 * (size_t)cap * slot_bytes(ctx);
+  W.perm_bytes = (size_t)cap * sizeof(uint32_t);
+  W.tf.resize((size_t)K + 1, nullptr);
+  W.tpart.resize((size_t)K, nullptr);
+  W.perm.assign(2 * (size_t)K, nullptr);
   for (int s = 0; s < 2; ++s) {
-    TRYH(W.want(lp[s], 6 * (size_t)cap * sizeof(double)));
-    TRYH(hipMemsetAsync(lp[s], 0, 6 * (size_t)cap * sizeof(double), st));
+    TRY(want(ctx, lp[s], W.lp_bytes));
+    TRYH(hipMemsetAsync(lp[s], 0, W.lp_bytes, st));
   }
-  for (int j = 0; j <= K; ++j) TRYH(W.want(W.tf[j], 6 * n * sizeof(double)));
-  for (int j = 0; j < K; ++j) TRYH(W.want(W.tpart[j], 2 * (size_t)cap * slot_bytes(ctx)));
+  for (int j = 0; j <= K; ++j) TRY(want(ctx, W.tf[j], W.tf_bytes));
+  for (int j = 0; j < K; ++j) TRY(want(ctx, W.tpart[j], W.tpart_bytes));
   std::vector<double *> &tf = W.tf;
   std::vector<uint32_t *> &perm = W.perm;
   auto tape_of = [&](int j, int s) {
@@ -1583,7 +1648,11 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
       if (ctx->c_sort > c.sort_every - 1)  // this step begins with the sort
         for (int s = 0; s < 2; ++s) {
           uint32_t *&b = perm[2 * (size_t)j + s];
-          TRYH(W.want(b, (size_t)cap * sizeof(uint32_t)));
+          if (!b && !W.spare.empty()) {
+            b = W.spare.back();
+            W.spare.pop_back();
+          }
+          TRY(want(ctx, b, W.perm_bytes));
           pm[s] = b;
         }
       TRY(fwd_step(ctx, ts[j], tf[j], tp, pm));
@@ -1672,7 +1741,8 @@ extern "C" int pic_adj_backward(pic_ctx *ctx, double dloss, double grad[4]) {
       // slots the particles held before it
       if (ts[j].sorted)
         for (int sp = 0; sp < 2; ++sp) {
-          TRYH(W.want(lq[sp], 6 * (size_t)cap * sizeof(double)));
+          W.swapped = true;
+          TRY(want(ctx, lq[sp], W.lp_bytes));
           TRYH(hipMemsetAsync(lq[sp], 0, 6 * (size_t)ts[j].nb[sp] * sizeof(double), st));
           if (ts[j].na[sp] > 0)
             k_unsort_lp<<<nb(ts[j].na[sp]), kBlock, 0, st>>>(

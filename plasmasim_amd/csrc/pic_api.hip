@@ -908,21 +908,21 @@ extern "C" int pic_thrust_ave_enable(pic_ctx *ctx, int on) {
   const int64_t boxes =
       tg.ntiles() == 1 ? row_geom(tg).ntiles() : (int64_t)tg.ntiles() * pass_split(ctx);
   const int64_t slots = boxes + most_chunks(ctx->cfg.ppc, ctx->cap);
-  if (!ctx->thrust_acc) PIC_HIP(ctx, hipMalloc(&ctx->thrust_acc, 16 * sizeof(double)));
+  if (!ctx->thrust_acc) PIC_HIP(ctx, device_malloc(ctx, &ctx->thrust_acc, 16 * sizeof(double)));
   if (ctx->thrust_part_slots < slots) {
     if (ctx->thrust_part) (void)hipFree(ctx->thrust_part);
     ctx->thrust_part = nullptr;
     ctx->thrust_part_slots = 0;
-    PIC_HIP(ctx, hipMalloc(&ctx->thrust_part, (size_t)slots * 12 * sizeof(double)));
+    PIC_HIP(ctx, device_malloc(ctx, &ctx->thrust_part, (size_t)slots * 12 * sizeof(double)));
     ctx->thrust_part_slots = slots;
   }
   if (is_f64(ctx) && !ctx->thrust_bprev)
-    PIC_HIP(ctx, hipMalloc(&ctx->thrust_bprev, 3 * (size_t)g.plane * esz));
+    PIC_HIP(ctx, device_malloc(ctx, &ctx->thrust_bprev, 3 * (size_t)g.plane * esz));
   if (ctx->diag_partial_cap < kDiagPartials) {
     if (ctx->diag_partial) (void)hipFree(ctx->diag_partial);
     ctx->diag_partial = nullptr;
     ctx->diag_partial_cap = 0;
-    PIC_HIP(ctx, hipMalloc(&ctx->diag_partial, kDiagPartials * sizeof(double)));
+    PIC_HIP(ctx, device_malloc(ctx, &ctx->diag_partial, kDiagPartials * sizeof(double)));
     ctx->diag_partial_cap = kDiagPartials;
   }
   k_fill_zero<<<1, 64, 0, ctx->stream>>>(ctx->thrust_acc, 16);

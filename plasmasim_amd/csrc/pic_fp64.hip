@@ -1742,7 +1742,7 @@ int diagnose(pic_ctx *ctx, pic_diag *out) {
   if (ctx->diag_partial_cap < need) {
     if (ctx->diag_partial) (void)hipFree(ctx->diag_partial);
     ctx->diag_partial = nullptr;
-    PIC_HIP(ctx, hipMalloc(&ctx->diag_partial, need * sizeof(double)));
+    PIC_HIP(ctx, device_malloc(ctx, &ctx->diag_partial, need * sizeof(double)));
     ctx->diag_partial_cap = need;
   }
   double *pf = ctx->diag_partial;

@@ -356,6 +356,16 @@ int noalloc_init(pic_ctx *ctx);
 int push_fused(pic_ctx *ctx);
 // adjoint state (pic_adj.hip)
 void adj_free(pic_ctx *ctx);
+// hipMalloc for a context's calls after its creation: where the card has no
+// room, what the adjoint keeps for its next sweep is given back first
+hipError_t device_malloc_bytes(pic_ctx *ctx, void **p, size_t bytes);
+template <typename T>
+inline hipError_t device_malloc(pic_ctx *ctx, T **p, size_t bytes) {
+  void *v = nullptr;
+  const hipError_t e = device_malloc_bytes(ctx, &v, bytes);
+  if (e == hipSuccess) *p = (T *)v;
+  return e;
+}
 
 // device-wide building blocks, hand-written (pic_prim.hip)
 // stable selection: idx_out[0..*count) = indices i < n with flags[i] != 0

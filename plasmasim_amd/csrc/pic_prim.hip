@@ -241,7 +241,7 @@ int ensure_prim_tmp(pic_ctx *ctx, size_t bytes) {
   if (ctx->prim_tmp) PIC_HIP(ctx, hipFree(ctx->prim_tmp));
   ctx->prim_tmp = nullptr;
   ctx->prim_tmp_bytes = 0;
-  PIC_HIP(ctx, hipMalloc(&ctx->prim_tmp, bytes));
+  PIC_HIP(ctx, device_malloc(ctx, &ctx->prim_tmp, bytes));
   ctx->prim_tmp_bytes = bytes;
   return 0;
 }

@@ -398,13 +398,13 @@ inline void release(Bufs &B) {
 inline int reserve(pic_ctx *rt, Bufs &B, int nt, int64_t pool) {
   if (B.ntiles >= nt && B.pool >= pool) return 0;
   release(B);
-  PIC_HIP(rt, hipMalloc(&B.stay, (size_t)nt * sizeof(uint32_t)));
-  PIC_HIP(rt, hipMalloc(&B.mcount, (size_t)2 * nt * sizeof(uint32_t)));
+  PIC_HIP(rt, device_malloc(rt, &B.stay, (size_t)nt * sizeof(uint32_t)));
+  PIC_HIP(rt, device_malloc(rt, &B.mcount, (size_t)2 * nt * sizeof(uint32_t)));
   B.ndesc = B.mcount + nt;
-  PIC_HIP(rt, hipMalloc(&B.desc, (size_t)nt * kDescCap * sizeof(uint4)));
-  PIC_HIP(rt, hipMalloc(&B.movers, (size_t)pool * sizeof(uint2)));
-  PIC_HIP(rt, hipMalloc(&B.start, (size_t)(nt + 1) * sizeof(uint32_t)));
-  PIC_HIP(rt, hipMalloc(&B.flag, 2 * sizeof(uint32_t)));
+  PIC_HIP(rt, device_malloc(rt, &B.desc, (size_t)nt * kDescCap * sizeof(uint4)));
+  PIC_HIP(rt, device_malloc(rt, &B.movers, (size_t)pool * sizeof(uint2)));
+  PIC_HIP(rt, device_malloc(rt, &B.start, (size_t)(nt + 1) * sizeof(uint32_t)));
+  PIC_HIP(rt, device_malloc(rt, &B.flag, 2 * sizeof(uint32_t)));
   B.ntiles = nt;
   B.pool = pool;
   return 0;

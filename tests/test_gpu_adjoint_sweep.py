@@ -4,6 +4,7 @@ own instantiation of the transposed pass) against the oracle's gradient; the
 FP32 forward's tape, read in its own form, against the FP64 one."""
 import numpy as np
 import pytest
+import torch
 
 import plasmasim_amd as ps
 from oracle_lib import Oracle
@@ -49,6 +50,27 @@ def test_repeated_sweeps_equal_fresh_ones(precision, sort_every):
         assert abs(loss - lf) <= tol * abs(lf)
         assert np.all(np.abs(g - gf) <= tol * np.abs(gf)), (steps, window, g, gf)
     s.close()
+
+
+def test_kept_buffers_are_those_of_the_last_window():
+    """After a sweep over long windows and one over short ones a context holds
+    what one that has only seen the short ones holds: a forward gives back
+    the tape of 7 steps of 2 x 262144 slots (103 MB)."""
+    def used(windows):
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        c = cfg(ps.PIC_FP32)
+        c.capacity = 262144
+        s = ps.Simulation(c)
+        for w in windows:
+            grad(s, params(c), 8, w)
+        left = torch.cuda.mem_get_info()[0]
+        s.close()
+        return free - left
+
+    used([1])  # what the process loads and keeps on first use
+    one, both = used([1]), used([8, 1])
+    assert both - one <= 16 << 20, (one, both)
 
 
 @pytest.mark.parametrize("dx", [1.0, 0.75])
