@@ -998,7 +998,8 @@ struct Ckpt {
   void *parts[2] = {nullptr, nullptr};
   int64_t room[2] = {0, 0};  // slots that parts holds
   uint32_t *tiles[2] = {nullptr, nullptr};
-  int64_t n[2], sorted_end[2];
+  uint32_t *rows[2] = {nullptr, nullptr};  // one tile: the cell starts
+  int64_t n[2], sorted_end[2], row_end[2];
   int cur[2];
   int32_t drift_halves[2];
   int64_t step;
@@ -1226,6 +1227,7 @@ void free_ckpts(AdjState *A, size_t keep) {
     for (int s = 0; s < 2; ++s) {
       if (c.parts[s]) (void)hipFree(c.parts[s]);
       if (c.tiles[s]) (void)hipFree(c.tiles[s]);
+      if (c.rows[s]) (void)hipFree(c.rows[s]);
     }
   }
   if (A->ck.size() > keep) A->ck.resize(keep);
@@ -1259,6 +1261,13 @@ void sub_arrays(const pic_ctx *ctx, void *buf, int64_t cap, char **ptr, size_t *
   }
 }
 
+// bytes of a species' cell starts: a segment is recomputed in the boxes that
+// its forward ran in, with the same grouping of the deposits
+size_t row_bytes(const pic_ctx *ctx) {
+  const Geom &g = ctx->geom;
+  return ((size_t)g.NX * g.NY * g.NZ + 1) * sizeof(uint32_t);
+}
+
 int save_ckpt(pic_ctx *ctx, Ckpt &c) {
   if (!c.fields) PIC_HIP(ctx, device_malloc(ctx, &c.fields, ctx->field_bytes));
   PIC_HIP(ctx, hipMemcpyAsync(c.fields, ctx->field_mem, ctx->field_bytes,
@@ -1267,6 +1276,7 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
   for (int s = 0; s < 2; ++s) {
     c.n[s] = ctx->n[s];
     c.sorted_end[s] = ctx->sorted_end[s];
+    c.row_end[s] = ctx->row_end[s];
     c.cur[s] = ctx->cur[s];
     c.drift_halves[s] = ctx->drift_halves[s];
     const int64_t n = ctx->n[s];
@@ -1290,6 +1300,11 @@ int save_ckpt(pic_ctx *ctx, Ckpt &c) {
       PIC_HIP(ctx, device_malloc(ctx, &c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t)));
     PIC_HIP(ctx, hipMemcpyAsync(c.tiles[s], ctx->tile_start[s], (size_t)(nt + 1) * sizeof(uint32_t),
                                 hipMemcpyDeviceToDevice, ctx->stream));
+    if (c.row_end[s] > 0) {
+      if (!c.rows[s]) PIC_HIP(ctx, device_malloc(ctx, &c.rows[s], row_bytes(ctx)));
+      PIC_HIP(ctx, hipMemcpyAsync(c.rows[s], ctx->row_start[s], row_bytes(ctx),
+                                  hipMemcpyDeviceToDevice, ctx->stream));
+    }
   }
   c.step = ctx->step;
   c.c_add = ctx->c_add;
@@ -1306,7 +1321,7 @@ int restore_ckpt(pic_ctx *ctx, const Ckpt &c) {
   for (int s = 0; s < 2; ++s) {
     ctx->n[s] = c.n[s];
     ctx->sorted_end[s] = c.sorted_end[s];
-    ctx->row_end[s] = 0;  // the cell starts are those of a later sort
+    ctx->row_end[s] = c.row_end[s];
     ctx->cur[s] = c.cur[s];
     ctx->drift_halves[s] = c.drift_halves[s];
     const int64_t n = c.n[s];
@@ -1321,6 +1336,9 @@ int restore_ckpt(pic_ctx *ctx, const Ckpt &c) {
                                     ctx->stream));
     PIC_HIP(ctx, hipMemcpyAsync(ctx->tile_start[s], c.tiles[s], (size_t)(nt + 1) * sizeof(uint32_t),
                                 hipMemcpyDeviceToDevice, ctx->stream));
+    if (c.row_end[s] > 0)
+      PIC_HIP(ctx, hipMemcpyAsync(ctx->row_start[s], c.rows[s], row_bytes(ctx),
+                                  hipMemcpyDeviceToDevice, ctx->stream));
   }
   ctx->step = c.step;
   ctx->c_add = c.c_add;

@@ -343,7 +343,9 @@ extern "C" int pic_checkpoint_load(pic_ctx *ctx, const char *path) {
     ctx->sorted_end[s] = same_tiles && h.ntiles > 0 ? h.sorted_end[s] : 0;
     ctx->row_end[s] = 0;  // the file holds no cell starts
     // the windows of restored tiles follow the drift from where the writer's
-    // stood, so a resumed run deposits exactly as an uninterrupted one
+    // stood, so a resumed run of a tiled store groups its deposits as an
+    // uninterrupted one; a one-tile store runs in chunks until its next sort
+    // (the same sums in another order, fixed-point deposits bit for bit)
     ctx->drift_halves[s] = ctx->sorted_end[s] > 0 ? h.drift_halves[s] : 0;
   }
   if (!f64) return f32::state_restored(ctx);

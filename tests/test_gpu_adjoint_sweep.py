@@ -73,6 +73,32 @@ def test_kept_buffers_are_those_of_the_last_window():
     assert both - one <= 16 << 20, (one, both)
 
 
+def test_one_tile_segments_run_in_the_forwards_boxes():
+    """A recomputed segment of a one-tile store groups its deposits as its
+    forward did: at nodes that the particles of a single box reach the current
+    of the first step is the forward's, bit for bit (one fixed-point sum of a
+    workgroup, one add to the plane; without the cell starts the contributions
+    arrive one by one).  Boxes are 4 x 4 x 8 cells, and no particle crosses
+    half a cell: nodes 2 along x and y and 2 to 5 along z of each, without the
+    boxes at the z faces, where the inflow's chunks add too."""
+    c = ps.preset(1)
+    c.nx, c.ny, c.nz, c.ppc = 32, 32, 40, 8
+    c.precision = ps.PIC_FP32
+    c.inflow_every = c.sort_every = 1000
+    s = ps.Simulation(c)
+    s.adj_forward(params(c), 1, 1, R, NQ)
+    planes = ("jix", "jiy", "jiz", "jex", "jey", "jez")
+    a = [s.download_field(k) for k in planes]
+    s.adj_backward(1.0)
+    node = [np.arange(2, n + 2) for n in (c.nx, c.ny, c.nz)]
+    z = np.arange(8, c.nz - 8)
+    box = np.ix_(node[0][2::4], node[1][2::4], node[2][z[np.isin(z % 8, (2, 3, 4, 5))]])
+    for k, j in zip(planes, a):
+        assert np.count_nonzero(j[box]), k
+        assert np.array_equal(s.download_field(k)[box], j[box]), k
+    s.close()
+
+
 @pytest.mark.parametrize("dx", [1.0, 0.75])
 def test_gradient_in_other_units(dx):
     c = cfg(dx=dx)
