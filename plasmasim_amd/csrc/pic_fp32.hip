@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(256) void k_step_b1(Geom g, CellBlocks cb, Fields<f
                                                  unsigned long long *fx, float *bt,
                                                  Sigma32 sg, FieldConst fc) {
   int k, l, m;
-  if (!cb.cell(g, blockIdx.x, k, l, m)) return;
+  if (!cb.cell(g, block_index(), threadIdx.x, k, l, m)) return;
   const int64_t c = g.idx(k, l, m);
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
@@ -1115,7 +1115,7 @@ __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<f
                                                  double inv_s, float *bt, Sigma32 sg,
                                                  FieldConst fc, int tb, ThrustFinish tf,
                                                  int fb) {
-  int b = blockIdx.x;
+  int b = block_index();
   if (b < tb) {
     thrust_finish(tf, b);
     return;
@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<f
   }
   b -= fb;
   int k, l, m;
-  if (!cb.cell(g, b, k, l, m)) return;
+  if (!cb.cell(g, b, threadIdx.x, k, l, m)) return;
   if (DET && unfolded_column(g, k, l)) {
     const int64_t c = g.idx(k, l, m);
 #pragma unroll
@@ -1154,7 +1154,7 @@ __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<f
 __global__ __launch_bounds__(256) void k_step_e(Geom g, CellBlocks cb, Fields<float> F,
                                                 Sigma32 sg, FieldConst fc) {
   int k, l, m;
-  if (!cb.cell(g, blockIdx.x, k, l, m) || !interior_column(g, k, l)) return;
+  if (!cb.cell(g, block_index(), threadIdx.x, k, l, m) || !interior_column(g, k, l)) return;
   const int64_t c = g.idx(k, l, m);
   const bool in = m >= 2 && m < g.NZ + 2;
   float e[3];
@@ -1866,7 +1866,7 @@ int step_b1(pic_ctx *ctx, bool keep_b) {
   State32 *S = st(ctx);
   const auto kern = S->fx ? (keep_b ? k_step_b1<true, true> : k_step_b1<true, false>)
                           : (keep_b ? k_step_b1<false, true> : k_step_b1<false, false>);
-  kern<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+  kern<<<block_grid(cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<float>(ctx), S->fx, S->bt, sigma_f(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   S->fx_dirty = false;
@@ -1880,7 +1880,7 @@ int step_b2(pic_ctx *ctx) {
   const int tb = ctx->thrust_now ? 12 : 0;
   const int fb = (int)div_up((int64_t)fold_groups(g) * g.SZ, kBlock);
   const auto kern = S->fx ? k_step_b2<true> : k_step_b2<false>;
-  kern<<<(unsigned)(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
+  kern<<<block_grid(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<float>(ctx), S->fx, 1.0 / S->fx_scale, S->bt, sigma_f(ctx),
       field_const(ctx), tb, thrust_finish_args(ctx), fb);
   PIC_LAUNCH_CHECK(ctx);
@@ -1891,7 +1891,7 @@ int step_b2(pic_ctx *ctx) {
 int step_e(pic_ctx *ctx) {
   const Geom &g = ctx->geom;
   const CellBlocks cb(g);
-  k_step_e<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+  k_step_e<<<block_grid(cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<float>(ctx), sigma_f(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;

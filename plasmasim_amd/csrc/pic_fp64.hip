@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void k_step_b1(Geom g, CellBlocks cb, Fields<d
                                                  double *kept, SigmaProfile sg,
                                                  FieldConst fc) {
   int k, l, m;
-  if (!cb.cell(g, blockIdx.x, k, l, m)) return;
+  if (!cb.cell(g, block_index(), threadIdx.x, k, l, m)) return;
   const int64_t c = g.idx(k, l, m);
 #pragma unroll
   for (int q = 0; q < 8; ++q) F.f[PIC_JIX + q][c] = 0.0;
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256) void k_step_b1(Geom g, CellBlocks cb, Fields<d
 __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<double> F,
                                                  SigmaProfile sg, FieldConst fc, int tb,
                                                  ThrustFinish tf, int fb) {
-  int b = blockIdx.x;
+  int b = block_index();
   if (b < tb) {
     thrust_finish(tf, b);
     return;
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<d
   }
   b -= fb;
   int k, l, m;
-  if (!cb.cell(g, b, k, l, m) || !interior_column(g, k, l)) return;
+  if (!cb.cell(g, b, threadIdx.x, k, l, m) || !interior_column(g, k, l)) return;
   b_and_guards(g, F, nullptr, sg, fc, k, l, m);
 }
 
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(256) void k_step_b2(Geom g, CellBlocks cb, Fields<d
 __global__ __launch_bounds__(256) void k_step_e(Geom g, CellBlocks cb, Fields<double> F,
                                                 SigmaProfile sg, FieldConst fc) {
   int k, l, m;
-  if (!cb.cell(g, blockIdx.x, k, l, m) || !interior_column(g, k, l)) return;
+  if (!cb.cell(g, block_index(), threadIdx.x, k, l, m) || !interior_column(g, k, l)) return;
   const int64_t c = g.idx(k, l, m);
   const bool in = m >= 2 && m < g.NZ + 2;
   double e[3];
@@ -1311,7 +1311,7 @@ int fold_current(pic_ctx *ctx) {
 int step_b1(pic_ctx *ctx, bool keep_b) {
   const Geom &g = ctx->geom;
   const CellBlocks cb(g);
-  k_step_b1<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+  k_step_b1<<<block_grid(cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<double>(ctx), keep_b ? (double *)ctx->thrust_bprev : nullptr, sigma(ctx),
       field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
@@ -1323,7 +1323,7 @@ int step_b2(pic_ctx *ctx) {
   const CellBlocks cb(g);
   const int tb = ctx->thrust_now ? 12 : 0;
   const int fb = (int)div_up((int64_t)fold_groups(g) * g.SZ, kBlock);
-  k_step_b2<<<(unsigned)(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
+  k_step_b2<<<block_grid(tb + fb + cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<double>(ctx), sigma(ctx), field_const(ctx), tb, thrust_finish_args(ctx), fb);
   PIC_LAUNCH_CHECK(ctx);
   return 0;
@@ -1332,7 +1332,7 @@ int step_b2(pic_ctx *ctx) {
 int step_e(pic_ctx *ctx) {
   const Geom &g = ctx->geom;
   const CellBlocks cb(g);
-  k_step_e<<<(unsigned)cb.count(g), kBlock, 0, ctx->stream>>>(
+  k_step_e<<<block_grid(cb.count(g)), kBlock, 0, ctx->stream>>>(
       g, cb, fields<double>(ctx), sigma(ctx), field_const(ctx));
   PIC_LAUNCH_CHECK(ctx);
   return 0;

@@ -19,17 +19,29 @@
 
 namespace pic {
 
-// cell of thread (tx, ty) of cell block b: 64 x 4 threads over (m, l), one k
+// The blocks of a step's field launch, of 256 threads, as a grid of rows: a
+// launch may not have 2^32 threads along one dimension, which short columns
+// reach first (nz = 8: at 6.7e7 columns, 64 threads each).  Blocks past the
+// last one have no cell.
+constexpr int64_t kGridRow = (int64_t)1 << 23;
+__host__ inline dim3 block_grid(int64_t blocks) {
+  const int64_t rows = div_up(blocks, kGridRow);
+  return dim3((unsigned)(rows > 1 ? kGridRow : blocks), (unsigned)rows);
+}
+__device__ inline int block_index() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
+// cell of thread t of cell block b: 64 x 4 threads over (m, l), one k
 struct CellBlocks {
   int gx, gy;  // blocks along m and l
   __host__ inline CellBlocks(const Geom &g)
       : gx((g.SZ + 63) / 64), gy((g.SY + 3) / 4) {}
-  __host__ inline int count(const Geom &g) const { return gx * gy * g.SX; }
-  __device__ inline bool cell(const Geom &g, int b, int &k, int &l, int &m) const {
-    m = (b % gx) * 64 + (int)(threadIdx.x & 63);
-    l = (b / gx) % gy * 4 + (int)(threadIdx.x >> 6);
+  __host__ inline int64_t count(const Geom &g) const { return (int64_t)gx * gy * g.SX; }
+  __host__ __device__ inline bool cell(const Geom &g, int b, int t, int &k, int &l,
+                                       int &m) const {
+    m = (b % gx) * 64 + (t & 63);
+    l = (b / gx) % gy * 4 + (t >> 6);
     k = b / (gx * gy);
-    return m < g.SZ && l < g.SY;
+    return m < g.SZ && l < g.SY && k < g.SX;
   }
 };
 
