@@ -1664,12 +1664,10 @@ int sort(pic_ctx *ctx, int sp) {
   while (bits < 32 && ((uint64_t)1 << bits) <= ncell) ++bits;
   int rc = sort_keys(ctx, ctx->keys, ctx->keys_alt, ctx->idx, n, bits);
   if (rc) return rc;
-  rc = tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
-                   ctx->tile_start[sp]);
+  rc = boxes ? cell_starts(ctx, ctx->keys_alt, n, bg, ctx->row_start[sp], ctx->tile_start[sp])
+             : tile_bounds(ctx, ctx->keys_alt, n, (uint32_t)(tg.TX * tg.TY * tg.TZ), nt,
+                           ctx->tile_start[sp]);
   if (rc) return rc;
-  if (boxes && (rc = cell_starts(ctx, ctx->keys_alt, n, bg, ctx->row_start[sp],
-                                 ctx->tile_start[sp] + nt + 1)))
-    return rc;
   // the kept count is the start of the drop tile
   PIC_HIP(ctx, hipMemcpyAsync(ctx->host_counter, ctx->tile_start[sp] + nt,
                               2 * sizeof(uint32_t), hipMemcpyDeviceToHost,

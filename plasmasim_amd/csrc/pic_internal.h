@@ -386,9 +386,9 @@ int poisson_download_phi(pic_ctx *ctx, double *host);
 // >= nt * cpt are dropped slots and land in tile nt)
 int tile_bounds(pic_ctx *ctx, const uint32_t *skeys, int64_t n, uint32_t cpt,
                 int nt, uint32_t *tile_start);
-// cell_start[0..cells] from the keys of a one-tile sort; *most, zero before,
-// becomes the population of the fullest of the boxes (row_geom)
+// the same of a one-tile sort, with cell_start[0..cells] and, in tile[2] (zero
+// before), the population of the fullest of the boxes (row_geom)
 int cell_starts(pic_ctx *ctx, const uint32_t *skeys, int64_t n, const TileGeom &boxes,
-                uint32_t *cell_start, uint32_t *most);
+                uint32_t *cell_start, uint32_t *tile);
 
 }  // namespace pic

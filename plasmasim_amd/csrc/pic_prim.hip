@@ -340,8 +340,8 @@ int tile_bounds(pic_ctx *ctx, const uint32_t *skeys, int64_t n, uint32_t cpt,
 // as k_tile_bounds does for tiles, took 25 ms for 200000 particles in 4^3 of
 // 128^3 cells.  The search takes 43 us for 10^6 particles on 128^3 cells, 7 us
 // for 65536 on 32^3; in eighths, with seven loads in flight, the same.)
-// Threads are grouped by box (t: 32 or 128 cells each), so that *most becomes
-// the population of the fullest one.
+// Threads are grouped by box (t: 32 or 128 cells each).  tile: the one tile's
+// bounds, and the population of the fullest box (0 before).
 __device__ inline int64_t first_at_least(const uint32_t *__restrict__ keys, int64_t lo,
                                          int64_t hi, uint32_t key) {
   while (lo < hi) {
@@ -357,7 +357,7 @@ __device__ inline int64_t first_at_least(const uint32_t *__restrict__ keys, int6
 __global__ __launch_bounds__(256) void k_cell_starts(const uint32_t *__restrict__ keys,
                                                      int64_t n, TileGeom t, int NX, int NY,
                                                      int NZ, uint32_t *cell_start,
-                                                     uint32_t *most) {
+                                                     uint32_t *tile) {
   __shared__ uint32_t sum[256 / 32];
   const int per = t.TX * t.TY * t.TZ, tid = threadIdx.x;
   if (tid < 256 / 32) sum[tid] = 0;
@@ -374,19 +374,21 @@ __global__ __launch_bounds__(256) void k_cell_starts(const uint32_t *__restrict_
                           ? first_at_least(keys, s, near, c + 1)
                           : first_at_least(keys, near, n, c + 1);
     cell_start[c] = (uint32_t)s;
-    if (c + 1 == (uint32_t)NX * NY * NZ) cell_start[c + 1] = (uint32_t)e;
+    if (c == 0) tile[0] = 0;
+    if (c + 1 == (uint32_t)NX * NY * NZ) cell_start[c + 1] = tile[1] = (uint32_t)e;
     if (e > s) atomicAdd(&sum[tid / per], (uint32_t)(e - s));
   }
   __syncthreads();
-  if (tid < 256 / per && sum[tid] > *(volatile uint32_t *)most) atomicMax(most, sum[tid]);
+  if (tid < 256 / per && sum[tid] > *(volatile uint32_t *)(tile + 2))
+    atomicMax(tile + 2, sum[tid]);
 }
 
 int cell_starts(pic_ctx *ctx, const uint32_t *skeys, int64_t n, const TileGeom &boxes,
-                uint32_t *cell_start, uint32_t *most) {
+                uint32_t *cell_start, uint32_t *tile) {
   const Geom &g = ctx->geom;
   const int64_t threads = (int64_t)boxes.ntiles() * (boxes.TX * boxes.TY * boxes.TZ);
   k_cell_starts<<<(unsigned)div_up(threads, 256), 256, 0, ctx->stream>>>(
-      skeys, n, boxes, g.NX, g.NY, g.NZ, cell_start, most);
+      skeys, n, boxes, g.NX, g.NY, g.NZ, cell_start, tile);
   PIC_LAUNCH_CHECK(ctx);
   return 0;
 }
