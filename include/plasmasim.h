@@ -273,13 +273,17 @@ int pic_get_counters(const pic_ctx *ctx, int64_t *step, int32_t *c_add,
 int pic_set_counters(pic_ctx *ctx, int64_t step, int32_t c_add, int32_t c_sort);
 
 /* ---- kernel timing (HIP events on the context stream) ---- */
-#define PIC_T_PUSH 0     /* fused particle pass; one per species, also where
-                          * a launch takes both */
+/* Inside pic_step a B half-step's launch also holds renew_grid (the first) or
+ * the fold, the conversion of fixed-point deposits and thrust_fave's sums
+ * (the second), and sr_b; the E step's launch holds sr_e.  The routines called
+ * one by one (pic_halo_b, pic_fold_current, ...) have launches of their own. */
+#define PIC_T_PUSH 0     /* fused particle pass; counted once per species,
+                          * also where a launch takes both */
 #define PIC_T_FIELD_B 1  /* B half-step */
-#define PIC_T_FIELD_E 2  /* E step */
+#define PIC_T_FIELD_E 2  /* E step; the Poisson correction */
 #define PIC_T_SORT 3
 #define PIC_T_INFLOW 4
-#define PIC_T_OTHER 5    /* halos, fold, zeroing */
+#define PIC_T_OTHER 5    /* the routines' halos, fold and zeroing */
 #define PIC_T_PUSH_SORT 6 /* fused particle pass applying pic_step's sort
                              permutation (FP32 form) */
 #define PIC_T_COUNT 7

@@ -634,13 +634,7 @@ extern "C" int pic2d_step(pic2d_ctx *ctx, int nsteps) {
       TRY(pic2d_renew_b_half(ctx));
       TRY(pic2d_halo(ctx));
     }
-    {
-      const int tclass = ctx->pending[0] || ctx->pending[1] ? PIC_T_PUSH_SORT : PIC_T_PUSH;
-      pic::timing_begin(&ctx->rt, tclass);
-      rc = push_both(ctx);
-      pic::timing_end(&ctx->rt, tclass, 2);
-      TRY(rc);
-    }
+    TRY(push_both(ctx));
     const bool with_phi = c.poisson_every > 0 && ctx->step % c.poisson_every == 0;
     if (fused) {
       FIELD(PIC_T_FIELD_B, step_b2(ctx, ctx->step));

@@ -155,7 +155,7 @@ int diagnose_fields(pic2d_ctx *, pic2d_diag *);
 int load_particles(pic2d_ctx *);
 int push(pic2d_ctx *, int sp, int push_j, int drift_n, int boundary,
          int density_only);
-int push_both(pic2d_ctx *);  // the fused passes of both species
+int push_both(pic2d_ctx *);  // the fused passes of both species, timed each in its class
 int particle_boundary(pic2d_ctx *, int sp);
 int inflow(pic2d_ctx *, int sp, uint32_t event);
 int sort(pic2d_ctx *, int sp);

@@ -1022,12 +1022,19 @@ int push_both(pic2d_ctx *ctx) {
     Pass64 args = {};
     for (int sp = 0; sp < 2; ++sp)
       if (ctx->n[sp] > 0) args.s[sp] = species64(ctx, sp, &nb[sp]);
-    if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2) return launch64(ctx, 7, args, nb);
+    if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2) {
+      pic::timing_begin(&ctx->rt, PIC_T_PUSH);
+      const int rc = launch64(ctx, 7, args, nb);
+      pic::timing_end(&ctx->rt, PIC_T_PUSH, 2);
+      return rc;
+    }
     for (int sp = 0; sp < 2; ++sp) {
       Pass64 a = {};
       a.s[0] = args.s[sp];
       const unsigned one[2] = {nb[sp], 0};
-      int rc = launch64(ctx, 7, a, one);
+      pic::timing_begin(&ctx->rt, PIC_T_PUSH);
+      const int rc = launch64(ctx, 7, a, one);
+      pic::timing_end(&ctx->rt, PIC_T_PUSH);
       if (rc) return rc;
     }
     return 0;
@@ -1036,15 +1043,21 @@ int push_both(pic2d_ctx *ctx) {
   for (int sp = 0; sp < 2; ++sp)
     if (ctx->n[sp] > 0) args.s[sp] = species32(ctx, sp, &nb[sp]);
   const bool perm[2] = {args.s[0].perm != nullptr, args.s[1].perm != nullptr};
+  const int tclass[2] = {perm[0] ? PIC_T_PUSH_SORT : PIC_T_PUSH,
+                         perm[1] ? PIC_T_PUSH_SORT : PIC_T_PUSH};
   int rc = 0;
   if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2 && perm[0] == perm[1]) {
+    pic::timing_begin(&ctx->rt, tclass[0]);
     rc = launch32(ctx, 7, perm[0], args, nb);
+    pic::timing_end(&ctx->rt, tclass[0], 2);
   } else {
     for (int sp = 0; sp < 2 && !rc; ++sp) {
       Pass32 a = {};
       a.s[0] = args.s[sp];
       const unsigned one[2] = {nb[sp], 0};
+      pic::timing_begin(&ctx->rt, tclass[sp]);
       rc = launch32(ctx, 7, perm[sp], a, one);
+      pic::timing_end(&ctx->rt, tclass[sp]);
     }
   }
   for (int sp = 0; sp < 2 && !rc; ++sp)

@@ -963,14 +963,7 @@ extern "C" int pic_thrust_ave_get(pic_ctx *ctx, double F[27], int64_t *nsteps,
 }
 
 namespace pic {
-int push_fused(pic_ctx *ctx) {
-  const bool sorting = !is_f64(ctx) && (f32::pending(ctx, 0) || f32::pending(ctx, 1));
-  const int tclass = sorting ? PIC_T_PUSH_SORT : PIC_T_PUSH;
-  timing_begin(ctx, tclass);
-  int rc = DISPATCH(push_both, ctx);
-  timing_end(ctx, tclass, 2);
-  return rc;
-}
+int push_fused(pic_ctx *ctx) { return DISPATCH(push_both, ctx); }
 }  // namespace pic
 
 // fdtd() step loop (:687-949) with loops A and B and the particle boundary

@@ -2113,16 +2113,22 @@ int push_both(pic_ctx *ctx) {
     if (rc) return rc;
   }
   const bool perm[2] = {args.s[0].perm != nullptr, args.s[1].perm != nullptr};
+  const int tclass[2] = {perm[0] ? PIC_T_PUSH_SORT : PIC_T_PUSH,
+                         perm[1] ? PIC_T_PUSH_SORT : PIC_T_PUSH};
   if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks && rows[0] == rows[1] &&
       perm[0] == perm[1]) {
+    timing_begin(ctx, tclass[0]);
     int rc = launch_pass(ctx, 7, perm[0], rows[0], args, nb);
+    timing_end(ctx, tclass[0], 2);
     if (rc) return rc;
   } else {
     for (int sp = 0; sp < 2; ++sp) {
       PassArgs32 one = args;
       one.s[0] = args.s[sp];
       const unsigned n[2] = {nb[sp], 0};
+      timing_begin(ctx, tclass[sp]);
       int rc = launch_pass(ctx, 7, perm[sp], rows[sp], one, n);
+      timing_end(ctx, tclass[sp]);
       if (rc) return rc;
       if (nb[sp]) pass_done(ctx, sp, args.s[sp]);
     }
@@ -2263,11 +2269,6 @@ int settle(pic_ctx *ctx, int sp) {
   ctx->cur[sp] = 1 - ctx->cur[sp];
   S->pending[sp] = false;
   return 0;
-}
-
-bool pending(const pic_ctx *ctx, int sp) {
-  const State32 *S = (const State32 *)ctx->form_state;
-  return S && S->pending[sp];
 }
 
 int settle_sorts(pic_ctx *ctx) {

@@ -1495,13 +1495,19 @@ int push_both(pic_ctx *ctx) {
     int rc = prepare_pass(ctx, sp, 7, args.s[sp], &rows[sp], &nb[sp]);
     if (rc) return rc;
   }
-  if (nb[0] && nb[1] && rows[0] == rows[1] && nb[0] + nb[1] < kBothBlocks)
-    return launch_pass(ctx, 7, rows[0], args, nb);
+  if (nb[0] && nb[1] && rows[0] == rows[1] && nb[0] + nb[1] < kBothBlocks) {
+    timing_begin(ctx, PIC_T_PUSH);
+    int rc = launch_pass(ctx, 7, rows[0], args, nb);
+    timing_end(ctx, PIC_T_PUSH, 2);
+    return rc;
+  }
   for (int sp = 0; sp < 2; ++sp) {
     PassArgs64 one = args;
     one.s[0] = args.s[sp];
     const unsigned n[2] = {nb[sp], 0};
+    timing_begin(ctx, PIC_T_PUSH);
     int rc = launch_pass(ctx, 7, rows[sp], one, n);
+    timing_end(ctx, PIC_T_PUSH);
     if (rc) return rc;
   }
   return 0;

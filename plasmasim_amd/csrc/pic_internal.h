@@ -284,7 +284,7 @@ int step_b2(pic_ctx *);
 int step_e(pic_ctx *);
 int load_particles(pic_ctx *);
 int push(pic_ctx *, int sp, bool drift);
-int push_both(pic_ctx *);
+int push_both(pic_ctx *);  // timed, each pass in its own class
 int particle_boundary(pic_ctx *);
 int inflow(pic_ctx *, int sp, uint32_t event);
 int sort(pic_ctx *, int sp);
@@ -314,7 +314,6 @@ int sort(pic_ctx *, int sp);
 int sort_for_pass(pic_ctx *, int sp);
 int settle(pic_ctx *, int sp);
 int settle_sorts(pic_ctx *);
-bool pending(const pic_ctx *, int sp);
 int diagnose(pic_ctx *, pic_diag *);
 int count_live(pic_ctx *, int sp, int64_t *n);
 int upload_particles(pic_ctx *, int sp, int64_t n, const double *const *h);
