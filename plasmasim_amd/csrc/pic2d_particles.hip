@@ -1018,6 +1018,12 @@ int push(pic2d_ctx *ctx, int sp, int push_j, int drift_n, int boundary,
 // where both carry a sort's permutation or neither does.
 int push_both(pic2d_ctx *ctx) {
   unsigned nb[2] = {0, 0};
+  // a pass that has run has applied its species' permutation, whatever
+  // becomes of the other species'
+  const auto applied = [&](int sp) {
+    ctx->cur[sp] = 1 - ctx->cur[sp];
+    ctx->pending[sp] = false;
+  };
   if (ctx->f64) {
     Pass64 args = {};
     for (int sp = 0; sp < 2; ++sp)
@@ -1045,27 +1051,25 @@ int push_both(pic2d_ctx *ctx) {
   const bool perm[2] = {args.s[0].perm != nullptr, args.s[1].perm != nullptr};
   const int tclass[2] = {perm[0] ? PIC_T_PUSH_SORT : PIC_T_PUSH,
                          perm[1] ? PIC_T_PUSH_SORT : PIC_T_PUSH};
-  int rc = 0;
   if (nb[0] && nb[1] && nb[0] + nb[1] < kBothBlocks2 && perm[0] == perm[1]) {
     pic::timing_begin(&ctx->rt, tclass[0]);
-    rc = launch32(ctx, 7, perm[0], args, nb);
+    const int rc = launch32(ctx, 7, perm[0], args, nb);
     pic::timing_end(&ctx->rt, tclass[0], 2);
-  } else {
-    for (int sp = 0; sp < 2 && !rc; ++sp) {
-      Pass32 a = {};
-      a.s[0] = args.s[sp];
-      const unsigned one[2] = {nb[sp], 0};
-      pic::timing_begin(&ctx->rt, tclass[sp]);
-      rc = launch32(ctx, 7, perm[sp], a, one);
-      pic::timing_end(&ctx->rt, tclass[sp]);
-    }
+    for (int sp = 0; sp < 2 && !rc; ++sp)
+      if (perm[sp]) applied(sp);
+    return rc;
   }
-  for (int sp = 0; sp < 2 && !rc; ++sp)
-    if (perm[sp]) {
-      ctx->cur[sp] = 1 - ctx->cur[sp];
-      ctx->pending[sp] = false;
-    }
-  return rc;
+  for (int sp = 0; sp < 2; ++sp) {
+    Pass32 a = {};
+    a.s[0] = args.s[sp];
+    const unsigned one[2] = {nb[sp], 0};
+    pic::timing_begin(&ctx->rt, tclass[sp]);
+    const int rc = launch32(ctx, 7, perm[sp], a, one);
+    pic::timing_end(&ctx->rt, tclass[sp]);
+    if (rc) return rc;
+    if (perm[sp]) applied(sp);
+  }
+  return 0;
 }
 
 int particle_boundary(pic2d_ctx *ctx, int sp) { return push(ctx, sp, 0, 0, 1, 0); }
