@@ -71,6 +71,47 @@ def test_fp64_sum_matches_oracle(preset, steps):
         assert np.abs(F4[:15]).max() > 0
 
 
+# 8192 workgroups of both species together: a launch for each, as on large
+# grids (below 6144 one launch takes both), on tiles and on a one-tile
+# store's boxes, each instantiation of the FP64 pass
+@pytest.mark.parametrize("n, tile, ppc", [((32, 32, 32), 2, 6), ((64, 64, 128), 0, 1)])
+@pytest.mark.parametrize("dx", [1.0, 0.75])
+@pytest.mark.parametrize("thrust", [True, False])
+def test_fp64_launch_per_species_against_the_oracle(n, tile, ppc, dx, thrust):
+    """Fields to 1e-12 (sums in another order), the force's sum to 1e-9 of its
+    largest component, sorts and inflows between."""
+    c = ps.preset(1)
+    c.precision = ps.PIC_FP64
+    c.nx, c.ny, c.nz = n
+    c.ppc = ppc
+    c.dx, c.dt = dx, c.dt * dx
+    c.ballistic_lo[2], c.ballistic_hi[2] = 8.0 * dx, (c.nz - 4.0) * dx
+    c.inflow_every, c.sort_every = 3, 5
+    for a in range(3):
+        c.tile[a] = tile
+    g, o = started(c), Oracle(c, threads=8)
+    o.load_particles()
+    o.begin()
+    g.thrust_ave(thrust)
+    steps, ref = 7, np.zeros(15)
+    for _ in range(steps):
+        o.step(1)
+        if thrust:
+            ref += np.asarray(o.diagnose()["force"])
+    g.step(steps)
+    for k in FIELDS:
+        assert rel_l2(g.download_field(k), o.download_field(k)) <= 1e-12, k
+    for sp in (0, 1):
+        assert g.particle_count(sp) == o.particle_count(sp)
+    if thrust:
+        F, done = g.thrust_ave_get()
+        scale = np.abs(ref).max()
+        assert done == steps and scale > 0
+        assert np.abs(F[:15] - ref).max() <= 1e-9 * scale, np.abs(F[:15] - ref) / scale
+    g.close()
+    o.close()
+
+
 def test_reset_and_reenable():
     c = ps.preset(1)
     c.precision = ps.PIC_FP64
