@@ -56,40 +56,14 @@ struct Stn {
   double w[3][2];
 };
 
-// q = p / dx, computed once per position by callers that build several
-// stencils at it
-__device__ inline void stencil_q(double dx, const double p[3], const double q[3], int c,
-                                 Stn &s) {
+__device__ inline void stencil(double dx, const double p[3], int c, Stn &s) {
   for (int a = 0; a < 3; ++a) {
     const double h = kStg[c][a] ? 0.5 : 0.0;
-    const int k = (int)(q[a] - h);
+    const int k = (int)(p[a] / dx - h);
     s.b[a] = k;
     s.w[a][0] = (k + 1 + h) * dx - p[a];
     s.w[a][1] = p[a] - (k + h) * dx;
   }
-}
-
-__device__ inline void stencil(double dx, const double p[3], int c, Stn &s) {
-  const double q[3] = {p[0] / dx, p[1] / dx, p[2] / dx};
-  stencil_q(dx, p, q, c, s);
-}
-
-// value and position gradient of sum_n F[n] W_n (W unnormalised)
-__device__ inline double st_gather(const Geom &g, const double *F, const Stn &s,
-                                   double gr[3]) {
-  double v = 0;
-  gr[0] = gr[1] = gr[2] = 0;
-#pragma unroll
-  for (int n = 0; n < 8; ++n) {
-    const int i = n >> 2, j = (n >> 1) & 1, k = n & 1;
-    const double f = F[g.idx(s.b[0] + i, s.b[1] + j, s.b[2] + k)];
-    const double wx = s.w[0][i], wy = s.w[1][j], wz = s.w[2][k];
-    v += f * wx * wy * wz;
-    gr[0] += f * (i ? 1.0 : -1.0) * wy * wz;
-    gr[1] += f * wx * (j ? 1.0 : -1.0) * wz;
-    gr[2] += f * wx * wy * (k ? 1.0 : -1.0);
-  }
-  return v;
 }
 
 __device__ inline double st_value(const Geom &g, const double *F, const Stn &s) {
@@ -574,8 +548,13 @@ __device__ __forceinline__ double interp_t(const Geom &g, const double *F, const
 
 // Window of the transposed gather: six FP64 planes of kAdjWin nodes (36 KB)
 // around the workgroup's particles, without those that lie more than kAdjFar
-// cells from the first (a particle that wrapped across a periodic face would
-// stretch the box over the domain); they go to the global planes.
+// cells from the anchor (a particle that wrapped across a periodic face would
+// stretch the box over the domain); they go to the global planes.  The anchor
+// is the first pushed particle of whichever wave is first to store it: a
+// workgroup's particles are neighbours after the sort, so any wave's will do.
+// Where that particle itself wrapped or strayed, nearly all others of its
+// workgroup take the global path, 48 atomics each; which ones the window sums
+// is therefore the same from run to run only up to such workgroups.
 constexpr int kAdjWin = 768;
 constexpr int kAdjFar = 6;
 
@@ -662,7 +641,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   const unsigned long long any = __builtin_amdgcn_ballot_w64(pushed);
   if (any && lane == __builtin_ctzll(any) &&
       atomicCAS(&bb[0], 1 << 29, w0[0].bi) == 1 << 29) {
-    bb[1] = w0[1].bi;  // this wave's first particle is the anchor
+    bb[1] = w0[1].bi;
     bb[2] = w0[2].bi;
   }
   __syncthreads();

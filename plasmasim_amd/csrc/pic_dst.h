@@ -23,12 +23,11 @@ struct Cplx {
 // and is taken as zero (sinft sets y[1] = 0).  Radix-2 decimation-in-time in
 // LDS (4n values of T), input in bit-reversed order.
 //   mode 0: out = S                        (forward)
-//   mode 1: out = S / A(l, k), 0 if A = 0   (forward, divided by the symbol
-//           A = -(sym_l[l] + sym_k[k]) / dq of the standard Laplacian)
 //   mode 2: out = 2 S / n                  (inverse)
-//   mode 3: both of 1 and then 2 on the same lines (forward, division,
-//           inverse): the lines stay with their workgroup, so nothing lies
-//           between the two transforms
+//   mode 3: S / A(l, k), 0 if A = 0 (forward, divided by the symbol A =
+//           -(sym_l[l] + sym_k[k]) / dq of the standard Laplacian), then
+//           mode 2 of that: the lines stay with their workgroup, so nothing
+//           lies between the two transforms
 // Lines are read through src(line, element) the first time: the data
 // themselves, or the expression that a pass before would have written there.
 template <typename T>
@@ -95,7 +94,7 @@ __global__ __launch_bounds__(256) void k_dst(T *data, Src src, int n, int logL,
           [&](int j) { return has_b ? src(l0 + 1, j) : (T)0; });
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     T sa = -im[k] / (T)2, sb = re[k] / (T)2;
-    if (mode & 1) {
+    if (mode == 3) {
       const double Aa = -(sym_l[l0] + sym_k[k]) / dq;
       sa = Aa == 0. ? (T)0 : (T)(sa / (T)Aa);
       if (has_b) {

@@ -681,7 +681,6 @@ __global__ __launch_bounds__(kPassBlock) PIC_WAVES32 void k_particles32(
                  return true;
                },
                s, e, w);
-    if (!(PUSH_J || DRIFT_N)) w.on = false;
     sw = w;
     s_range[0] = s;
     s_range[1] = e;

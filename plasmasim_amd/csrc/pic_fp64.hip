@@ -803,7 +803,6 @@ __global__ __launch_bounds__(256) void k_particles_tiled(
                  return true;
                },
                s, e, w);
-    if (!(PUSH_J || DRIFT_N)) w.on = false;
     sw = w;
     s_range[0] = s;
     s_range[1] = e;
