@@ -261,8 +261,8 @@ int pic_poisson(pic_ctx *ctx);
 
 /* Species sorts done so far by each method: the FP32 form sorts with the
  * tile sort (particles still tile-sorted since the last sort, each tile's
- * movers within its list) and otherwise, as the FP64 form always does, with
- * a radix sort of (key, slot) pairs.  Both give the stable key order. */
+ * movers within its list), the FP64 form on its keys, and otherwise with a
+ * radix sort of (key, slot) pairs.  Both give the stable key order. */
 int pic_sort_stats(const pic_ctx *ctx, int64_t *tile, int64_t *radix);
 
 /* Step counter (c) and cadence counters (c_add, c_thrust).  pic_step keeps

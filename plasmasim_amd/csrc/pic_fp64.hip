@@ -402,16 +402,17 @@ __device__ inline bool in_array(const Geom &g, double x, double y, double z,
 // particle pass: one workgroup per sort tile, J and n accumulated in an LDS
 // window with FP64 atomics, then added to the planes (see pic_tiles.h)
 //
-// No unit is saturated (128^3 x 64 ppc: VALU 41 %, LDS 42 %, L1 46 % busy at
-// three waves per SIMD), the waves wait on each in turn; the pass is written
-// for few instructions (830 per particle) with the reference's operations and
-// rounding: one stencil per position shared by the gathers and the previous
+// No unit is saturated (128^3 x 64 ppc with the force: VALU and LDS 47 % busy
+// at three waves per SIMD), half of the waves' cycles are waits for memory; the
+// pass is written for few instructions (867 per particle) with the reference's
+// operations and rounding: one stencil per position shared by the gathers and the previous
 // step's force; constants formed on the host; each lane's walk of the
 // stencils set up once per workgroup, one swap of the weights per axis; and
 // in normalised units (UNIT: dx = 1, where x / dx and w * dx are x and w
 // exactly; planes and arrays below 4 GiB) no divisions by dx and 32-bit byte
 // offsets from uniform bases.  165 VGPRs, from 239 at two waves per SIMD.
-// 20 steps at 128^3 x 64 ppc 377 -> 345 ms, at 32^3 x 16 ppc 7.1 -> 5.8 ms.
+// 20 steps at 128^3 x 64 ppc 377 -> 345 ms, at 32^3 x 16 ppc 7.1 -> 5.8 ms; with
+// the ordered gathers (gather6o) 295 ms.
 
 constexpr int kWin64 = 1400;  // window capacity in nodes (4 x double each)
 

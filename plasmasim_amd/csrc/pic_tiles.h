@@ -49,10 +49,11 @@ inline int64_t most_chunks(int ppc, int64_t cap) {
 // launch: the second species' workgroups take the places that the first one's
 // last round leaves empty, and a launch's latency goes.  Above it the
 // arguments' indirection by species costs more than that.  20 steps, one
-// launch / two: FP32 31 x 27 x 45 x 8 ppc 3.4 / 3.75 ms, 64^3 x 32 ppc (4100
-// workgroups) 14.0 / 14.1 ms, 128^3 x 64 ppc (33000) 155 / 150.5 ms; FP64
-// 8 x 8 x 16 x 4 ppc 1.10 / 1.37 ms, 32^3 x 16 ppc (2000 to 4000) 3.53 /
-// 3.60 ms, 128^3 x 64 ppc 405 / 345 ms (two waves per SIMD, not three).
+// launch / two: FP32 31 x 27 x 45 x 8 ppc 1.62 / 1.82 ms, 64^3 x 32 ppc (4100
+// workgroups) 14.1 / 14.6 ms, 128^3 x 64 ppc (33000) 154 / 149.5 ms; FP64
+// 8 x 8 x 16 x 4 ppc 0.53 / 0.58 ms, 32^3 x 16 ppc (2000 to 4000) 4.66 /
+// 4.80 ms, 128^3 x 64 ppc 332 / 294 ms (with a species per launch the force
+// gathers its own E).
 constexpr unsigned kBothBlocks = 8 * kChipSlots;
 
 struct TileRun {
