@@ -1177,18 +1177,14 @@ void unit_fields_host(const pic_config &c, const Geom &g, double *G) {
       }
 }
 
-int ensure_state(pic_ctx *ctx) {
-  if (ctx->adj) return 0;
-  AdjState *A = new (std::nothrow) AdjState();
-  if (!A) return set_error(ctx, PIC_E_NOMEM, "adjoint state");
-  ctx->adj = A;
+int fill_state(pic_ctx *ctx, AdjState *A) {
   const int64_t n = ncell(ctx);
-  PIC_HIP(ctx, hipMalloc(&A->G, 9 * n * sizeof(double)));
-  PIC_HIP(ctx, hipMalloc(&A->b0, 3 * n * sizeof(double)));
-  PIC_HIP(ctx, hipMalloc(&A->lam, 18 * n * sizeof(double)));
-  PIC_HIP(ctx, hipMalloc(&A->f6, 6 * n * sizeof(double)));
-  PIC_HIP(ctx, hipMalloc(&A->tmp, 6 * n * sizeof(double)));
-  PIC_HIP(ctx, hipMalloc(&A->red, 4096 * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->G, 9 * n * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->b0, 3 * n * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->lam, 18 * n * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->f6, 6 * n * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->tmp, 6 * n * sizeof(double)));
+  PIC_HIP(ctx, device_malloc(ctx, &A->red, 4096 * sizeof(double)));
   double *h = (double *)malloc(9 * n * sizeof(double));
   if (!h) return set_error(ctx, PIC_E_NOMEM, "adjoint unit fields");
   unit_fields_host(ctx->cfg, ctx->geom, h);
@@ -1196,6 +1192,17 @@ int ensure_state(pic_ctx *ctx) {
   free(h);
   PIC_HIP(ctx, e);
   return 0;
+}
+
+// whole or not at all: the kernels take its planes as they are
+int ensure_state(pic_ctx *ctx) {
+  if (ctx->adj) return 0;
+  AdjState *A = new (std::nothrow) AdjState();
+  if (!A) return set_error(ctx, PIC_E_NOMEM, "adjoint state");
+  ctx->adj = A;
+  const int rc = fill_state(ctx, A);
+  if (rc) adj_free(ctx);
+  return rc;
 }
 
 // keep the buffers of the first `keep` checkpoints
@@ -1452,11 +1459,12 @@ double sum_partials(pic_ctx *ctx, const double *dev, int count, int stride, int 
 }  // namespace
 
 hipError_t device_malloc_bytes(pic_ctx *ctx, void **p, size_t bytes) {
-  const hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = hipMalloc(p, bytes);
   AdjState *A = state(ctx);
-  if (e != hipErrorOutOfMemory || !A || !A->w.give_back()) return e;
-  (void)hipGetLastError();  // answered by what was given back
-  return hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && A && A->w.give_back()) e = hipMalloc(p, bytes);
+  // the caller has the error: the next launch's check must not find it again
+  (void)hipGetLastError();
+  return e;
 }
 
 void adj_free(pic_ctx *ctx) {
